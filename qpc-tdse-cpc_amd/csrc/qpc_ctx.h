@@ -59,6 +59,8 @@ struct qpc_ctx {
     int64_t eprim_cap = 0;
     // {S, X} pairs of the coupling sweeps' right-hand sides, X = 1/r, d/dr, r
     cplx *sxR = nullptr, *sxD = nullptr, *sxL = nullptr;
+    // the same pairs as the factorisations read them (qpc::launch_factor_bands)
+    cplx *fxR = nullptr, *fxD = nullptr, *fxL = nullptr;
     // t-SURFF (qpc_upload_tsurff): tables on the device, the accumulated
     // amplitudes work[kr][kt][kp], and the Volkov clock (time, int A dt)
     bool have_tsf = false, tsf_on = false, have_tsf_xy = false;

@@ -370,33 +370,33 @@ int ep_factor(qpc_ctx* c, int set, int64_t k) {
     // a complex symmetric sweep's tables (ts: tables of time point t at
     // position t * np of its block; shared tables: the nprim primaries)
     const int64_t trs = c->geo.trf_elems;
-    auto sym_tables = [&](int op, const double* X, int restart) {
+    auto sym_tables = [&](int op, const cplx* fx, int restart) {
         const int64_t slot = ep_slot(op, 0);
         cplx* tab = T.tabR + slot * np * cte;
         cplx* trf = T.trfR + slot * np * trs;
         if (E.rmap[op]) {
-            qpc::launch_factor_sym(c->fstream, c->S, X, E.eprim[op], sc + ep_sc(op, 0), 2, (int)E.nprim[op], c->geo,
+            qpc::launch_factor_sym(c->fstream, fx, E.eprim[op], sc + ep_sc(op, 0), 2, (int)E.nprim[op], c->geo,
                                    tab, 0, restart, np);
             qpc::launch_transfer_c(c->fstream, tab, trf, (int)E.nprim[op], 2, np, c->geo);
         } else {
-            qpc::launch_factor_sym(c->fstream, c->S, X, E.eig + op * ML + E.p0, sc + ep_sc(op, 0), 2, (int)np, c->geo,
+            qpc::launch_factor_sym(c->fstream, fx, E.eig + op * ML + E.p0, sc + ep_sc(op, 0), 2, (int)np, c->geo,
                                    tab, 0, restart);
             qpc::launch_transfer_c(c->fstream, tab, trf, (int)(2 * np), c->geo);
         }
     };
     if (E.lg) {
         TimedLaunch tl(c, QPC_K_FACTOR, c->fstream);
-        for (int op : {EP_X1, EP_Y1}) sym_tables(op, c->rpow1, c->restart_l);
+        for (int op : {EP_X1, EP_Y1}) sym_tables(op, c->fxL, c->restart_l);
     } else {
         TimedLaunch tl(c, QPC_K_FACTOR, c->fstream);
         for (int op = 0; op < 4; ++op) {
             const double* eig = E.eig + op * ML + E.p0;
             const int64_t slot = ep_slot(op, 0);
             if (ep_is_d(op))
-                qpc::launch_factor_asy(c->fstream, c->S, c->rdif, eig, sc + ep_sc(op, 0), 2, (int)np, c->geo,
+                qpc::launch_factor_asy(c->fstream, c->fxD, eig, sc + ep_sc(op, 0), 2, (int)np, c->geo,
                                        T.tabD + slot * np * te, 0, c->restart_d);
             else
-                sym_tables(op, c->rinv, 0);
+                sym_tables(op, c->fxR, 0);
         }
         qpc::launch_transfer_r(c->fstream, T.tabD, T.trfD, (int)(4 * np), c->geo);
     }

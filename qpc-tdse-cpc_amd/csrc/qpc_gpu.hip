@@ -279,23 +279,23 @@ int factor_batch(qpc_ctx* c, int ts, int64_t t0, int64_t n, int64_t pos = 0, boo
         const int64_t ML = c->ML;
         if (c->batch) {
             if (c->n_rprim > 0)  // one table per shot and distinct |eigenvalue|
-                qpc::launch_factor_sym(c->fstream, c->S, c->rinv, c->d_eprim + t0 * c->n_rprim, c->d_ones, (int)n,
+                qpc::launch_factor_sym(c->fstream, c->fxR, c->d_eprim + t0 * c->n_rprim, c->d_ones, (int)n,
                                        (int)c->n_rprim, c->geo, T.tabR, c->n_rprim, 0, ML);
             else
-                qpc::launch_factor_sym(c->fstream, c->S, c->rinv, c->d_e + (c->run_cap + t0) * ML, c->d_ones,
+                qpc::launch_factor_sym(c->fstream, c->fxR, c->d_e + (c->run_cap + t0) * ML, c->d_ones,
                                        (int)n, (int)ML, c->geo, T.tabR, ML);
         } else if (c->gauge == 1) {
             // length gauge: S + i e r with the Y10 eigenvalues only
             const double* dL = c->d_ifdt + c->run_cap + t0;
-            qpc::launch_factor_sym(c->fstream, c->S, c->rpow1, c->yeig, dL, (int)n, (int)ML, c->geo, T.tabR, 0,
+            qpc::launch_factor_sym(c->fstream, c->fxL, c->yeig, dL, (int)n, (int)ML, c->geo, T.tabR, 0,
                                    c->restart_l);
         } else {
             const double* dR = c->d_ifdt + c->run_cap + t0;
             if (c->n_rprim > 0)  // one table per distinct |eigenvalue|, in the first slots of each time point
-                qpc::launch_factor_sym(c->fstream, c->S, c->rinv, c->qeig_prim, dR, (int)n, (int)c->n_rprim, c->geo,
+                qpc::launch_factor_sym(c->fstream, c->fxR, c->qeig_prim, dR, (int)n, (int)c->n_rprim, c->geo,
                                        T.tabR, 0, 0, ML);
             else
-                qpc::launch_factor_sym(c->fstream, c->S, c->rinv, c->qeig, dR, (int)n, (int)ML, c->geo, T.tabR);
+                qpc::launch_factor_sym(c->fstream, c->fxR, c->qeig, dR, (int)n, (int)ML, c->geo, T.tabR);
         }
         if (c->gauge != 1 && c->n_rprim > 0)
             qpc::launch_transfer_c(c->fstream, T.tabR, T.trfR, (int)c->n_rprim, (int)n, ML, c->geo);
@@ -312,10 +312,10 @@ int factor_batch(qpc_ctx* c, int ts, int64_t t0, int64_t n, int64_t pos = 0, boo
         TimedLaunch tl(c, QPC_K_FACTOR, ds);
         const int64_t ML = c->ML;
         if (c->batch)
-            qpc::launch_factor_asy(ds, c->S, c->rdif, c->d_e + t0 * ML, c->d_ones, (int)n, (int)ML, c->geo, T.tabD,
+            qpc::launch_factor_asy(ds, c->fxD, c->d_e + t0 * ML, c->d_ones, (int)n, (int)ML, c->geo, T.tabD,
                                    ML, c->restart_d);
         else
-            qpc::launch_factor_asy(ds, c->S, c->rdif, c->yeig, c->d_ifdt + t0, (int)n, (int)ML, c->geo, T.tabD, 0,
+            qpc::launch_factor_asy(ds, c->fxD, c->yeig, c->d_ifdt + t0, (int)n, (int)ML, c->geo, T.tabD, 0,
                                    c->restart_d);
         qpc::launch_transfer_r(ds, T.tabD, T.trfD, (int)(n * ML), c->geo);
         TRY(launch_check(c, "factor_batch"));
@@ -643,7 +643,7 @@ static int create_impl(const qpc_dims* d, int64_t n_shots, int64_t tb_cap, qpc_c
     c->geo = qpc::make_geom((int)c->N, (int)c->p);
     c->tb_cap = tb_cap;
     const size_t ntab = (size_t)c->geo.tab_elems, nctab = (size_t)c->geo.ctab_elems;
-    const size_t ntrf = (size_t)c->geo.trf_elems;
+    const size_t ntrf = (size_t)c->geo.trf_elems, nfx = (size_t)qpc::factor_elems(c->geo);
     if ((rc = dev_alloc(c, &c->spare, nstate)) || (rc = dev_alloc(c, &c->vbuf, nstate)) ||
         (rc = dev_alloc(c, &c->tab_free, nl * nctab)) ||
         (rc = dev_alloc(c, &c->trf_free, nl * ntrf)) || (rc = dev_alloc(c, &c->tab_mask, ntab)) ||
@@ -657,6 +657,7 @@ static int create_impl(const qpc_dims* d, int64_t n_shots, int64_t tb_cap, qpc_c
         (rc = dev_alloc(c, &c->rdifd, band)) || (rc = dev_alloc(c, &c->maskd, band)) ||
         (rc = dev_alloc(c, &c->rpow1d, band)) || (rc = dev_alloc(c, &c->sxR, band)) ||
         (rc = dev_alloc(c, &c->sxD, band)) || (rc = dev_alloc(c, &c->sxL, band)) ||
+        (rc = dev_alloc(c, &c->fxR, nfx)) || (rc = dev_alloc(c, &c->fxD, nfx)) || (rc = dev_alloc(c, &c->fxL, nfx)) ||
         (rc = dev_alloc(c, &c->yeig, (size_t)c->ML)) ||
         (rc = dev_alloc(c, &c->qeig, (size_t)c->ML)) || (rc = dev_alloc(c, &c->y10, (size_t)c->ML)) ||
         (rc = dev_alloc(c, &c->yprj, (size_t)c->ML * c->L)) || (rc = dev_alloc(c, &c->qprj, (size_t)c->ML * c->L)) ||
@@ -699,7 +700,7 @@ int qpc_destroy(qpc_ctx* c) {
                     c->qeig,
                     c->y10, c->yprj, c->qprj, c->merged, c->coef, c->tmpc, c->spare, c->vbuf, c->red,
                     c->tab_free, c->trf_free, c->tab_mask, c->trf_mask, c->d_ifdt, c->Sd, c->rinvd, c->rdifd, c->maskd, c->upperd,
-                    c->rpow1d, c->sxR, c->sxD, c->sxL, c->tsf_ib, c->tsf_b0, c->tsf_br, c->tsf_kr, c->tsf_ckt,
+                    c->rpow1d, c->sxR, c->sxD, c->sxL, c->fxR, c->fxD, c->fxL, c->tsf_ib, c->tsf_b0, c->tsf_br, c->tsf_kr, c->tsf_ckt,
                     c->tsf_j0, c->tsf_jr, c->tsf_pm, c->tsf_Y, c->tsf_tmp, c->tsf_work, c->tsf_stx, c->tsf_sty,
                     c->tsf_pm1, c->tsf_pm2, c->rtY, c->rtYt, c->rtM, c->rtMh, c->rtQ, c->rtQh,
                     c->Wp, c->ppart, c->pchan, c->pcnt, c->pout, c->Hd, c->q10, c->kU, c->kpart, c->kcoef,
@@ -756,6 +757,9 @@ int qpc_upload_radial(qpc_ctx* c, const double* S, const double* chol, const dou
     qpc::launch_band_pair(c->stream, c->Sd, c->rinvd, c->sxR, n, p);
     qpc::launch_band_pair(c->stream, c->Sd, c->rdifd, c->sxD, n, p);
     qpc::launch_band_pair(c->stream, c->Sd, c->rpow1d, c->sxL, n, p);
+    qpc::launch_factor_bands(c->stream, c->S, c->rinv, c->fxR, c->geo);
+    qpc::launch_factor_bands(c->stream, c->S, c->rdif, c->fxD, c->geo);
+    qpc::launch_factor_bands(c->stream, c->S, c->rpow1, c->fxL, c->geo);
     c->S_h.assign(S, S + band);
     c->rdif_h.assign(rdif, rdif + band);
     if (rpow1) c->rpow1_h.assign(rpow1, rpow1 + band);

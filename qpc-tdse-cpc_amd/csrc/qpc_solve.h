@@ -177,9 +177,17 @@ void launch_band_diag_r(hipStream_t s, const double* src, double* dst, int n, in
 void launch_band_pair(hipStream_t s, const double* S, const double* X, cplx* dst, int N, int p);
 void launch_band_diag_c(hipStream_t s, const cplx* src, cplx* dst, int n, int N, int p);
 
+// The band operands of the factorisations: entry j of column c = 24 g + s is
+// fx[(s * (p+1) + j) * factor_cols + g] = {S, X}(c-j, c), so that lanes of
+// consecutive partitions read consecutive entries (factor_elems entries)
+inline __host__ __device__ int factor_cols(const Geom& g) { return g.P + 2; }
+inline int64_t factor_elems(const Geom& g) { return (int64_t)kPM * (g.hw + 1) * factor_cols(g); }
+// from row-major S and X (N * (p+1))
+void launch_factor_bands(hipStream_t s, const double* S, const double* X, cplx* fx, Geom geo);
+
 // reference-order LU of (S + ifet X) for nt time points x nch channels
-// (cn_propagate_kernel_avx1 elimination, propagate.hpp:33-86) on row-major
-// S, X; ifdt[t] is the per-time-point scalar of cn_hl_propagate1/2
+// (cn_propagate_kernel_avx1 elimination, propagate.hpp:33-86) on the band
+// operands fx; ifdt[t] is the per-time-point scalar of cn_hl_propagate1/2
 // (propagate.hpp:343,400).  Tables of (t, ch) at (t * nch + ch) * ctab_elems
 // (launch_factor_sym: complex symmetric rows) or * tab_elems (launch_factor_asy:
 // real LU rows), with e = eig[t*eig_tstride + ch] * ifdt[t] (eig_tstride 0:
@@ -187,11 +195,10 @@ void launch_band_diag_c(hipStream_t s, const cplx* src, cplx* dst, int n, int N,
 // restarted elimination above each partition (0: kRestart).  tab_tstride:
 // tables per time point in the layout (0: nch), so that nch of them can be
 // written into room for more.
-void launch_factor_sym(hipStream_t s, const double* S, const double* X, const double* eig, const double* ifdt,
-                       int nt, int nch, Geom geo, cplx* tab, int64_t eig_tstride = 0, int restart = 0,
-                       int64_t tab_tstride = 0);
-void launch_factor_asy(hipStream_t s, const double* S, const double* X, const double* eig, const double* ifdt,
-                       int nt, int nch, Geom geo, double* tab, int64_t eig_tstride = 0, int restart = 0);
+void launch_factor_sym(hipStream_t s, const cplx* fx, const double* eig, const double* ifdt, int nt, int nch, Geom geo,
+                       cplx* tab, int64_t eig_tstride = 0, int restart = 0, int64_t tab_tstride = 0);
+void launch_factor_asy(hipStream_t s, const cplx* fx, const double* eig, const double* ifdt, int nt, int nch, Geom geo,
+                       double* tab, int64_t eig_tstride = 0, int restart = 0);
 
 // ---- host ------------------------------------------------------------------
 // Reach of the recurrences of A = S + e X (row-major bands N*(p+1)): asym 0,

@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 namespace qpc {
@@ -1084,15 +1085,25 @@ __global__ __launch_bounds__(256) void k_band_diag(const T* __restrict__ src, T*
 }
 
 // ---------------------------------------------------------------------------
-// reference-order LU of b = S + ifet X (propagate.hpp:33-86), one lane per
-// (time point, channel, partition).  A lane restarts the elimination
-// `restart` rows above its partition (as if the matrix began there) and
-// writes the table rows of its own partition.  The last P U rows live in a
-// register ring of P + 1 slots (row i in slot (i - start) mod (P+1)); the row
-// loop is unrolled by the ring length so that every slot index is a
-// constant.  The lower panel of row i (S and X of rows i-P..i-1, the rows
-// just eliminated) comes from a second register ring at p = 7 and is read
-// again from the band arrays, where it is in cache, at p = 8.
+// LU of A = S + ifet X in the reference's elimination order
+// (propagate.hpp:33-86), one lane per (time point, channel, partition).  A
+// lane restarts the elimination `restart` rows above its partition (as if the
+// matrix began there) and writes the table rows of its own partition.
+//
+// The elimination is right-looking: the lane keeps the window of the Schur
+// complement that row i touches (rows and columns i .. i+P) in registers; row
+// r's entries sit in slot (r - start) mod RS, and the row loop is unrolled by
+// the RS slots so that every slot index is a constant.  A symmetric
+// matrix (S + i e X) needs the upper triangle only, P(P+1)/2 products per row
+// where the row-by-row elimination forms P^2.  Column i + P of the band
+// enters the window at step i; its {S, X} entries (launch_factor_bands) lie
+// partition-interleaved, so that a wave's load is one contiguous run instead of
+// 64 lines 24 rows apart, and the next column is loaded a whole step ahead.
+// One time point is bound by the chain of rows (reciprocal, scale, update of
+// the next pivot): 31 channels of N = 1000 take 41 us (S + i e X, was 134) and
+// 31 us (S + e X, was 71).  A batch is bound by the products and the table
+// writes: 32 time points of N = 3000, 41 tables of S + i e X 167 us (was
+// 434), 81 of S + e X 307 us (was 596).
 template <int SYM>
 struct FactorTypes;
 template <>
@@ -1106,135 +1117,141 @@ struct FactorTypes<1> {
 
 __device__ inline cplx frcp(cplx b) { return crecip(b); }
 __device__ inline double frcp(double b) { return 1.0 / b; }
+__device__ inline cplx fmulx(cplx a, cplx b) {
+    return {fma(-a.im, b.im, a.re * b.re), fma(a.im, b.re, a.re * b.im)};
+}
+__device__ inline double fmulx(double a, double b) { return a * b; }
+// a - t x
+__device__ inline cplx fsubx(cplx a, cplx t, cplx x) { return tmsub(a, t, x); }
+__device__ inline double fsubx(double a, double t, double x) { return fma(-t, x, a); }
 
 template <int SYM, int P>
-__global__ __launch_bounds__(kLane) void k_factor(const double* __restrict__ S, const double* __restrict__ X,
-                                                  const double* __restrict__ eig, int64_t eig_tstride,
-                                                  const double* __restrict__ ifdt, int nch, Geom geo, int restart,
-                                                  typename FactorTypes<SYM>::T* __restrict__ tab, int64_t tstride) {
+__global__ __launch_bounds__(kLane, P == 7 ? 2 : 1) void k_factor(const cplx* __restrict__ fx, const double* __restrict__ eig,
+                                                  int64_t eig_tstride, const double* __restrict__ ifdt, Geom geo,
+                                                  int restart, typename FactorTypes<SYM>::T* __restrict__ tab,
+                                                  int64_t tstride) {
     using T = typename FactorTypes<SYM>::T;
-    constexpr int nd = P, ne = P + 1, RS = P + 1;
+    constexpr int NE = P + 1;
+    // slots: a divisor of kPM, so that the rounds of rows end with the partition
+    constexpr int RS = P == 7 ? 8 : 12;
+    static_assert(RS > P && kPM % RS == 0, "slot count");
     const int g = blockIdx.x * kLane + threadIdx.x;
     const int ch = blockIdx.y, t = blockIdx.z;
     if (g >= geo.P) return;
-    const int N = geo.N;
+    const int FP = factor_cols(geo);
     const double e = eig[(int64_t)t * eig_tstride + ch] * ifdt[t];
-    // SYM 0 (S + i e X, X symmetric) writes complex symmetric rows [u(i,0..P-1), 1/pivot]:
-    // for a symmetric matrix the unit upper factor's rows are the columns of
-    // L in A = L D L^T and the pivots are D; SYM 1 writes real LU rows
+    // SYM 0 writes complex symmetric rows [E_1..E_P, 1/pivot] (for a symmetric
+    // matrix the unit upper factor's rows are the columns of L in A = L D L^T);
+    // SYM 1 writes real LU rows
     constexpr int ROW = TabFmt<T, P>::row;
     T* Tg = tab + ((int64_t)t * tstride + ch) * TabFmt<T, P>::elems(geo) + part_col<T, P>(g);
     const int r0 = g * kPM;
-    const int start = r0 > restart ? r0 - restart : 0;
-    const int end = min(N, r0 + kPM);
-    T u[RS][nd];
-    // p = 7: entries 1..P of the upper bands of the last RS rows (the lower
-    // panel of later rows) stay in a register ring beside u; p = 8 reads them
-    // again from the band arrays (the rings would not fit the registers)
-    constexpr bool WRING = P == 7;
-    double ws[WRING ? RS : 1][nd], wx[WRING ? RS : 1][nd];
+    // whole rounds of RS rows above the partition (r0 is a multiple of RS too)
+    const int above = (restart + RS - 1) / RS * RS;
+    const int start = r0 > above ? r0 - above : 0;
+    // column entries of the band from column `start` on
+    int sc = start % kPM, gc = start / kPM;
+    auto column = [&](cplx (&q)[NE]) {
+        const cplx* b = fx + ((int64_t)sc * NE * FP + gc);
+#pragma unroll
+        for (int j = 0; j < NE; ++j) q[j] = b[j * FP];
+        if (++sc == kPM) {
+            sc = 0;
+            ++gc;
+        }
+    };
+    T wu[RS][NE];                    // wu[slot(r)][j] = A(r, r+j)
+    double wl[SYM ? RS : 1][NE];     // wl[slot(r)][j] = A(r+j, r), j >= 1 (SYM 1)
 #pragma unroll
     for (int s = 0; s < RS; ++s)
 #pragma unroll
-        for (int k = 0; k < nd; ++k) {
-            u[s][k] = tzero(T{});
-            if constexpr (WRING) {
-                ws[s][k] = 0.0;
-                wx[s][k] = 0.0;
-            }
+        for (int j = 0; j < NE; ++j) {
+            wu[s][j] = tzero(T{});
+            if constexpr (SYM) wl[s][j] = 0.0;
         }
-    for (int i0 = start; i0 < end; i0 += RS) {
+    auto put = [&](int slot, int j, cplx q) {
+        if constexpr (SYM == 0) {
+            wu[slot][j] = cplx{q.re, e * q.im};  // s + ifet r, ifet = i e
+        } else {
+            wu[slot][j] = fma(e, q.im, q.re);
+            if (j) wl[slot][j] = fma(-e, q.im, q.re);  // antisymmetric below the diagonal
+        }
+    };
+    cplx nx[NE];
+#pragma unroll
+    for (int c = 0; c < P; ++c) {  // columns start .. start+P-1 of the rows that exist
+        column(nx);
+#pragma unroll
+        for (int j = 0; j <= c; ++j) put(c - j, j, nx[j]);
+    }
+    column(nx);
+    // RS rows from row i on; STORE writes their table rows.  No branch inside:
+    // the compiler moves updates across one to their last use, which keeps
+    // every row's operands live
+    auto round = [&](int i, auto store) {
 #pragma unroll
         for (int s = 0; s < RS; ++s) {
-            const int i = i0 + s;
-            if (i < end) {
-                const int avail = i - start;  // rows above i in the restarted matrix
-                double sr[ne], xr[ne], sl[nd], xl[nd];
+            // a row at a time: later rows' column loads ahead of these products
+            // would need registers for all of them
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int j = 0; j < ne; ++j) {
-                    sr[j] = S[(int64_t)i * ne + j];
-                    xr[j] = X[(int64_t)i * ne + j];
-                }
-                // entry j of the upper bands of row i-j (clamped index: rows
-                // above the restart are zeroed below)
+            for (int j = 0; j < NE; ++j) put((s + P - j) % RS, j, nx[j]);
+            column(nx);
+            const T rp = frcp(wu[s][0]);
+            T u[NE];
 #pragma unroll
-                for (int j = 1; j <= nd; ++j) {
-                    if constexpr (WRING) {
-                        const int slot = (s - j + RS) % RS;  // row i-j
-                        sl[j - 1] = ws[slot][j - 1];
-                        xl[j - 1] = wx[slot][j - 1];
-                    } else {
-                        const int64_t k = (int64_t)max(i - j, 0) * ne + j;
-                        sl[j - 1] = S[k];
-                        xl[j - 1] = X[k];
-                    }
-                }
-                if constexpr (WRING) {
+            for (int k = 1; k < NE; ++k) u[k] = fmulx(wu[s][k], rp);
+            if constexpr (decltype(store)::value) {
+                T* o = Tg + (int64_t)(i + s - r0) * ROW * kLane;
+                if constexpr (SYM == 0) {
 #pragma unroll
-                    for (int j = 1; j < ne; ++j) {
-                        ws[s][j - 1] = sr[j];
-                        wx[s][j - 1] = xr[j];
-                    }
-                }
-                T b[2 * nd + 1];
-                // lower panel: column i-j (propagate.hpp:35-53)
+                    for (int k = 1; k < NE; ++k) o[(int64_t)(k - 1) * kLane] = u[k];
+                    o[(int64_t)P * kLane] = rp;
+                } else {
+                    // multiplier of column i-j: entry j of row i-j, final since step i-j
 #pragma unroll
-                for (int j = 1; j <= nd; ++j) {
-                    if (j > avail) {
-                        b[nd - j] = tzero(T{});
-                    } else {
-                        const double sv = sl[j - 1], rv = xl[j - 1];
-                        if constexpr (SYM == 0) b[nd - j] = cplx{sv, e * rv};  // s + ifet r, ifet = i e
-                        else b[nd - j] = sv - e * rv;                            // s - ifet r (antisymmetric)
-                    }
-                }
-                // upper (propagate.hpp:55-62)
+                    for (int j = 1; j < NE; ++j) o[(int64_t)(j - 1) * kLane] = wl[(s - j + RS) % RS][j];
+                    o[(int64_t)P * kLane] = rp;
 #pragma unroll
-                for (int j = 0; j < ne; ++j) {
-                    if constexpr (SYM == 0) b[nd + j] = cplx{sr[j], e * xr[j]};
-                    else b[nd + j] = sr[j] + e * xr[j];
-                }
-                const int l = avail < nd ? nd - avail : 0;
-                // elimination with the previous U rows (propagate.hpp:67-71)
-#pragma unroll
-                for (int j = 0; j < nd; ++j) {
-                    if (j >= l) {
-                        const int slot = (s + j + 1) % RS;  // row i+j-P
-#pragma unroll
-                        for (int k = 0; k < nd; ++k) b[j + k + 1] = b[j + k + 1] - b[j] * u[slot][k];
-                    }
-                }
-                // u(i,:) = b / pivot (propagate.hpp:72-75), via one reciprocal
-                const T rp = frcp(b[nd]);
-#pragma unroll
-                for (int j = 0; j < nd; ++j) u[s][j] = b[j + nd + 1] * rp;
-                if (i >= r0) {
-                    T* o = Tg + (int64_t)(i - r0) * ROW * kLane;
-                    if constexpr (SYM == 0) {
-#pragma unroll
-                        for (int k = 1; k <= nd; ++k) o[(int64_t)(k - 1) * kLane] = i + k < N ? u[s][k - 1] : tzero(T{});
-                        o[(int64_t)nd * kLane] = rp;
-                    } else {
-#pragma unroll
-                        for (int j = 1; j <= nd; ++j) o[(int64_t)(j - 1) * kLane] = b[nd - j];  // multiplier of column i-j
-                        o[(int64_t)nd * kLane] = rp;
-#pragma unroll
-                        for (int k = 1; k <= nd; ++k)
-                            o[(int64_t)(nd + k) * kLane] = i + k < N ? u[s][k - 1] : tzero(T{});
-                        o[(int64_t)(ROW - 1) * kLane] = tone(T{});
-                    }
+                    for (int k = 1; k < NE; ++k) o[(int64_t)(P + k) * kLane] = u[k];
+                    o[(int64_t)(ROW - 1) * kLane] = tone(T{});
                 }
             }
-        }
-    }
-    // identity padding rows of the last partition
-    for (int i = max(N, r0); i < r0 + kPM; ++i) {
-        T* o = Tg + (int64_t)(i - r0) * ROW * kLane;
+            // A(i+a, i+b) -= A(i+a, i) u(i, i+b)
 #pragma unroll
-        for (int q = 0; q < ROW; ++q) o[(int64_t)q * kLane] = tzero(T{});
-        o[(int64_t)nd * kLane] = tone(T{});
-        o[(int64_t)(ROW - 1) * kLane] = tone(T{});
-    }
+            for (int a = 1; a < NE; ++a)
+#pragma unroll
+                for (int b = SYM ? 1 : a; b < NE; ++b) {
+                    if constexpr (SYM == 0) {
+                        T& w = wu[(s + a) % RS][b - a];
+                        w = fsubx(w, wu[s][a], u[b]);
+                    } else {
+                        T& w = b >= a ? wu[(s + a) % RS][b - a] : wl[(s + b) % RS][a - b];
+                        w = fsubx(w, wl[s][a], u[b]);
+                    }
+                }
+        }
+    };
+    int i = start;
+#pragma unroll 1
+    for (; i < r0; i += RS) round(i, std::false_type{});
+#pragma unroll 1
+    for (; i < r0 + kPM; i += RS) round(i, std::true_type{});
+}
+
+// fx[(s * (p+1) + j) * FP + g] = {S, X}(c-j, c) of column c = 24 g + s, zero
+// above the first row; columns from N on are the identity's (the table rows
+// of the last partition's padding)
+__global__ __launch_bounds__(256) void k_factor_bands(const double* __restrict__ S, const double* __restrict__ X,
+                                                      cplx* __restrict__ fx, int N, int ne, int FP) {
+    const int id = blockIdx.x * 256 + threadIdx.x;
+    if (id >= kPM * ne * FP) return;
+    const int g = id % FP, j = id / FP % ne, s = id / FP / ne;
+    const int c = g * kPM + s, r = c - j;
+    cplx v = {0.0, 0.0};
+    if (c >= N) v.re = j == 0 ? 1.0 : 0.0;
+    else if (r >= 0) v = {S[(int64_t)r * ne + j], X[(int64_t)r * ne + j]};
+    fx[id] = v;
 }
 
 }  // namespace
@@ -1411,26 +1428,28 @@ void launch_band_diag_c(hipStream_t s, const cplx* src, cplx* dst, int n, int N,
                        p + 1);
 }
 
-void launch_factor_sym(hipStream_t s, const double* S, const double* X, const double* eig, const double* ifdt, int nt,
-                       int nch, Geom geo, cplx* tab, int64_t eig_tstride, int restart, int64_t tab_tstride) {
-    const int rs = restart > 0 ? restart : kRestart;
-    const int64_t ts = tab_tstride > 0 ? tab_tstride : nch;
-    if (geo.hw == 8)
-        hipLaunchKernelGGL((k_factor<0, 8>), dim3(geo.NG, nch, nt), dim3(kLane), 0, s, S, X, eig, eig_tstride, ifdt,
-                           nch, geo, rs, tab, ts);
-    else
-        hipLaunchKernelGGL((k_factor<0, 7>), dim3(geo.NG, nch, nt), dim3(kLane), 0, s, S, X, eig, eig_tstride, ifdt,
-                           nch, geo, rs, tab, ts);
+void launch_factor_bands(hipStream_t s, const double* S, const double* X, cplx* fx, Geom geo) {
+    const int total = kPM * (geo.hw + 1) * factor_cols(geo);
+    hipLaunchKernelGGL(k_factor_bands, dim3((total + 255) / 256), dim3(256), 0, s, S, X, fx, geo.N, geo.hw + 1,
+                       factor_cols(geo));
 }
-void launch_factor_asy(hipStream_t s, const double* S, const double* X, const double* eig, const double* ifdt, int nt,
-                       int nch, Geom geo, double* tab, int64_t eig_tstride, int restart) {
+template <int SYM>
+static void factor_launch(hipStream_t s, const cplx* fx, const double* eig, const double* ifdt, int nt, int nch, Geom geo,
+                          typename FactorTypes<SYM>::T* tab, int64_t eig_tstride, int restart, int64_t ts) {
     const int rs = restart > 0 ? restart : kRestart;
+    const dim3 grid(geo.NG, nch, nt);
     if (geo.hw == 8)
-        hipLaunchKernelGGL((k_factor<1, 8>), dim3(geo.NG, nch, nt), dim3(kLane), 0, s, S, X, eig, eig_tstride, ifdt,
-                           nch, geo, rs, tab, (int64_t)nch);
+        hipLaunchKernelGGL((k_factor<SYM, 8>), grid, dim3(kLane), 0, s, fx, eig, eig_tstride, ifdt, geo, rs, tab, ts);
     else
-        hipLaunchKernelGGL((k_factor<1, 7>), dim3(geo.NG, nch, nt), dim3(kLane), 0, s, S, X, eig, eig_tstride, ifdt,
-                           nch, geo, rs, tab, (int64_t)nch);
+        hipLaunchKernelGGL((k_factor<SYM, 7>), grid, dim3(kLane), 0, s, fx, eig, eig_tstride, ifdt, geo, rs, tab, ts);
+}
+void launch_factor_sym(hipStream_t s, const cplx* fx, const double* eig, const double* ifdt, int nt, int nch, Geom geo,
+                       cplx* tab, int64_t eig_tstride, int restart, int64_t tab_tstride) {
+    factor_launch<0>(s, fx, eig, ifdt, nt, nch, geo, tab, eig_tstride, restart, tab_tstride > 0 ? tab_tstride : nch);
+}
+void launch_factor_asy(hipStream_t s, const cplx* fx, const double* eig, const double* ifdt, int nt, int nch, Geom geo,
+                       double* tab, int64_t eig_tstride, int restart) {
+    factor_launch<1>(s, fx, eig, ifdt, nt, nch, geo, tab, eig_tstride, restart, nch);
 }
 
 // ---------------------------------------------------------------------------

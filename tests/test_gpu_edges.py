@@ -1,0 +1,47 @@
+"""Steps at the sizes where the partitioned kernels have edges, against the
+oracle: fewer rows than one partition (24), whole and ragged last partitions,
+grids shorter than the factorisation's restart and the carry, one and two wave
+groups of partitions (1536 rows), both spline orders.  Bar: relative L2 <=
+1e-12 per call, the parity bar of single steps."""
+import numpy as np
+import pytest
+
+from _cfg import make_oracle, mixed_state, rel_l2, shape, upload_from_oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _pair(N, p, L, M=1, m0=0):
+    import qpc_gpu
+    cfg = shape(N, L, 0.2 * N, M=M, m0=m0, p=p)
+    o = make_oracle(cfg)
+    prop = qpc_gpu.Propagator(N, p, L, M, m0, cfg["dt"])
+    upload_from_oracle(prop, o)
+    return o, prop
+
+
+@pytest.mark.parametrize("p", [7, 8])
+@pytest.mark.parametrize("N", [18, 23, 24, 25, 48, 71, 97, 145, 191, 1535, 1536, 1537])
+def test_steps_at_partition_edges(N, p):
+    print(f"case: edges N={N} p={p}", flush=True)
+    o, prop = _pair(N, p, 3)
+    c = mixed_state(o, seed=N + p, amp=0.3)
+    prop.set_state(c)
+    for kind, a in (("vg", (0.7, 0.9)), ("vg", (0.9, -0.4)), ("free", None), ("lg", (0.05, 0.03)), ("mask", None)):
+        ref = np.ascontiguousarray(prop.get_state())
+        if kind == "vg":
+            o.step(ref, *a)
+            prop.propagate(*a)
+        elif kind == "lg":
+            o.step_lg(ref, *a)
+            prop.propagate_lg(*a)
+        elif kind == "free":
+            o.step_free(ref)
+            prop.propagate()
+        else:
+            o.mask(ref)
+            prop.mask()
+        err = rel_l2(prop.get_state(), ref)
+        print(f"  {kind} {a}: rel L2 {err:.2e}", flush=True)
+        assert err <= 1e-12
+    prop.close()
