@@ -414,8 +414,8 @@ int  qpc_run_lgwr(qpc_ctx* ctx, const double* extab, const double* eytab, int64_
  * launch shape).  The partitioned solves cut each channel's partitions into
  * segments, one work-group each; seg_add adds segments beyond the fewest
  * that hold them (more work-groups, each with the carry's halo partitions
- * again), and grids of at most stage_grid work-groups stage the transfer sets
- * in LDS with four waves per work-group.  Neither changes the result (the
+ * again), and grids of at most stage_grid work-groups stage table rows in
+ * LDS, with eight waves per work-group.  Neither changes the result (the
  * segments are exact, the two paths share their arithmetic).
  * qpc_autotune runs the with-field steps [it0, it0+nsteps) of the field
  * table (as qpc_run, or qpc_run_batch with its stride for a batch context;

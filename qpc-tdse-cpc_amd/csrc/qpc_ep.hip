@@ -369,7 +369,7 @@ int ep_factor(qpc_ctx* c, int set, int64_t k) {
     const int64_t te = c->geo.tab_elems, cte = c->geo.ctab_elems;
     // a complex symmetric sweep's tables (ts: tables of time point t at
     // position t * np of its block; shared tables: the nprim primaries)
-    const int64_t trs = c->geo.trf_elems;
+    const int64_t trs = c->geo.ctrf_elems;
     auto sym_tables = [&](int op, const cplx* fx, int restart) {
         const int64_t slot = ep_slot(op, 0);
         cplx* tab = T.tabR + slot * np * cte;
@@ -412,7 +412,8 @@ int ep_sweep(qpc_ctx* c, int set, int64_t k, int op, int tf, cplx* buf) {
     const int64_t np = E.p1 - E.p0;
     if (np <= 0) return QPC_OK;
     const auto& T = E.set[set];
-    const int64_t te = c->geo.tab_elems, cte = c->geo.ctab_elems, tr = c->geo.trf_elems;
+    const int64_t te = c->geo.tab_elems, cte = c->geo.ctab_elems;
+    const int64_t tr = c->geo.trf_elems, ctr = c->geo.ctrf_elems;
     const int64_t slot = ep_slot(op, tf);
     qpc::RhsArgs ra{};
     ra.sx = E.lg ? c->sxL : ep_is_d(op) ? c->sxD : c->sxR;
@@ -441,13 +442,13 @@ int ep_sweep(qpc_ctx* c, int set, int64_t k, int op, int tf, cplx* buf) {
     // in place (z in, z out): the right-hand side goes through vbuf
     TimedLaunch tl(c, QPC_K_EP_SWEEP);
     if (E.lg)
-        qpc::launch_rsolve_c(c->stream, kind, ra, T.tabR + slot * np * cte, T.trfR + slot * np * tr, tm, z, c->vbuf, z,
+        qpc::launch_rsolve_c(c->stream, kind, ra, T.tabR + slot * np * cte, T.trfR + slot * np * ctr, tm, z, c->vbuf, z,
                              (int)np, c->geo, c->pk_l);
     else if (ep_is_d(op))
         qpc::launch_rsolve_r(c->stream, kind, ra, T.tabD + slot * np * te, T.trfD + slot * np * tr, tm, z, c->vbuf, z,
                              (int)np, c->geo, c->pk_d);
     else
-        qpc::launch_rsolve_c(c->stream, kind, ra, T.tabR + slot * np * cte, T.trfR + slot * np * tr, tm, z, c->vbuf, z,
+        qpc::launch_rsolve_c(c->stream, kind, ra, T.tabR + slot * np * cte, T.trfR + slot * np * ctr, tm, z, c->vbuf, z,
                              (int)np, c->geo);
     return launch_check(c, "ep sweep");
 }
@@ -634,7 +635,8 @@ int ep_prepare(qpc_ctx* c, int isub, bool lg) {
     QPC_HIP_CHECK(c, hipStreamSynchronize(c->fstream));
     const size_t mm = (size_t)ML * ML;
     const int64_t np = E.p1 - E.p0;
-    const size_t te = (size_t)c->geo.tab_elems, cte = (size_t)c->geo.ctab_elems, tr = (size_t)c->geo.trf_elems;
+    const size_t te = (size_t)c->geo.tab_elems, cte = (size_t)c->geo.ctab_elems, tr = (size_t)c->geo.trf_elems,
+                 ctr = (size_t)c->geo.ctrf_elems;
     int rc = QPC_OK;
     if (!E.eig) {
         if ((rc = dev_alloc(c, &E.eig, 4 * (size_t)ML)) || (rc = dev_alloc(c, &E.tx1, mm)) ||
@@ -662,7 +664,7 @@ int ep_prepare(qpc_ctx* c, int isub, bool lg) {
         T.pending = false;
         if (np > 0 && !lg && ((rc = dev_alloc(c, &T.tabD, 4 * np * te)) || (rc = dev_alloc(c, &T.trfD, 4 * np * tr))))
             return rc;
-        if (np > 0 && ((rc = dev_alloc(c, &T.tabR, 4 * np * cte)) || (rc = dev_alloc(c, &T.trfR, 4 * np * tr))))
+        if (np > 0 && ((rc = dev_alloc(c, &T.tabR, 4 * np * cte)) || (rc = dev_alloc(c, &T.trfR, 4 * np * ctr))))
             return rc;
     }
     E.lg = lg;

@@ -27,7 +27,8 @@ int rot_cplx(qpc_ctx* c, const cplx* Pt, const cplx* src, cplx* dst) {
 // per-batch table pointers of time point t
 inline int64_t tabsz_r(const qpc_ctx* c) { return c->ML * c->geo.tab_elems; }   // real LU tables (D-part)
 inline int64_t tabsz_c(const qpc_ctx* c) { return c->ML * c->geo.ctab_elems; }  // complex symmetric (R-part)
-inline int64_t trfsz(const qpc_ctx* c) { return c->ML * c->geo.trf_elems; }
+inline int64_t trfsz_r(const qpc_ctx* c) { return c->ML * c->geo.trf_elems; }
+inline int64_t trfsz_c(const qpc_ctx* c) { return c->ML * c->geo.ctrf_elems; }
 
 // cn_hl_propagate2 (D-part, propagate.hpp:388-441) on rotated channels:
 // run time point t, whose tables are entry t - t0 of table set ts
@@ -63,7 +64,7 @@ int solve_D(qpc_ctx* c, int ts, int64_t t0, int64_t t, const cplx* in, cplx* out
     TRY(wg_order(c, c->dorder, c->pk_d, [](int64_t ch) { return (int)ch; }, tm));
     const int64_t k = t - t0;
     TimedLaunch tl(c, QPC_K_CN_D);
-    qpc::launch_rsolve_r(c->stream, qpc::RHS_SX_ASY, ra, c->ts[ts].tabD + k * tabsz_r(c), c->ts[ts].trfD + k * trfsz(c),
+    qpc::launch_rsolve_r(c->stream, qpc::RHS_SX_ASY, ra, c->ts[ts].tabD + k * tabsz_r(c), c->ts[ts].trfD + k * trfsz_r(c),
                          tm, in, c->vbuf, out, (int)c->ML, c->geo, c->pk_d);
     return launch_check(c, "solve_D");
 }
@@ -93,7 +94,7 @@ int solve_R(qpc_ctx* c, int ts, int64_t t0, int64_t t, const cplx* in, cplx* out
     }
     const int64_t k = t - t0;
     TimedLaunch tl(c, QPC_K_CN_R);
-    qpc::launch_rsolve_c(c->stream, qpc::RHS_SX_SYM, ra, c->ts[ts].tabR + k * tabsz_c(c), c->ts[ts].trfR + k * trfsz(c),
+    qpc::launch_rsolve_c(c->stream, qpc::RHS_SX_SYM, ra, c->ts[ts].tabR + k * tabsz_c(c), c->ts[ts].trfR + k * trfsz_c(c),
                          tm, in, c->vbuf, out, (int)c->ML, c->geo);
     return launch_check(c, "solve_R");
 }
@@ -108,7 +109,7 @@ int solve_L(qpc_ctx* c, int ts, int64_t t0, int64_t t, const cplx* in, cplx* out
     const qpc::TabMap tm{0, (int)c->L, (int)c->m0};
     const int64_t k = t - t0;
     TimedLaunch tl(c, QPC_K_CN_R);
-    qpc::launch_rsolve_c(c->stream, qpc::RHS_SX_SYM, ra, c->ts[ts].tabR + k * tabsz_c(c), c->ts[ts].trfR + k * trfsz(c),
+    qpc::launch_rsolve_c(c->stream, qpc::RHS_SX_SYM, ra, c->ts[ts].tabR + k * tabsz_c(c), c->ts[ts].trfR + k * trfsz_c(c),
                          tm, in, c->vbuf, out, (int)c->ML, c->geo, c->pk_l);
     return launch_check(c, "solve_L");
 }
@@ -268,9 +269,9 @@ int factor_batch(qpc_ctx* c, int ts, int64_t t0, int64_t n, int64_t pos = 0, boo
     const qpc_ctx::TableSet& S = c->ts[ts];
     qpc_ctx::TableSet T = S;  // the set's tables from position pos on
     T.tabD = S.tabD + pos * tabsz_r(c);
-    T.trfD = S.trfD + pos * trfsz(c);
+    T.trfD = S.trfD + pos * trfsz_r(c);
     T.tabR = S.tabR + pos * tabsz_c(c);
-    T.trfR = S.trfR + pos * trfsz(c);
+    T.trfR = S.trfR + pos * trfsz_c(c);
     if (wait_set && T.pending) QPC_HIP_CHECK(c, hipStreamWaitEvent(c->fstream, T.freed, 0));
     // the R-part tables and transfer sets first (ready_r), then the D-part's
     // (ready): a step reads the R part of its t_f tables before the D part
@@ -499,12 +500,12 @@ int ready(qpc_ctx* c, bool need_mask) {
 int alloc_zsets(qpc_ctx* c) {
     if (c->ts[0].tabD) return QPC_OK;
     const size_t ntab = (size_t)c->geo.tab_elems, nctab = (size_t)c->geo.ctab_elems;
-    const size_t ntrf = (size_t)c->geo.trf_elems;
+    const size_t ntrf = (size_t)c->geo.trf_elems, nctrf = (size_t)c->geo.ctrf_elems;
     const size_t nt = (size_t)c->tb_cap * c->ML;
     for (auto& T : c->ts) {
         int rc = QPC_OK;
         if ((rc = dev_alloc(c, &T.tabD, nt * ntab)) || (rc = dev_alloc(c, &T.trfD, nt * ntrf)) ||
-            (rc = dev_alloc(c, &T.tabR, nt * nctab)) || (rc = dev_alloc(c, &T.trfR, nt * ntrf)))
+            (rc = dev_alloc(c, &T.tabR, nt * nctab)) || (rc = dev_alloc(c, &T.trfR, nt * nctrf)))
             return rc;
     }
     QPC_HIP_CHECK(c, hipStreamSynchronize(c->stream));
@@ -646,7 +647,7 @@ static int create_impl(const qpc_dims* d, int64_t n_shots, int64_t tb_cap, qpc_c
     const size_t ntrf = (size_t)c->geo.trf_elems, nfx = (size_t)qpc::factor_elems(c->geo);
     if ((rc = dev_alloc(c, &c->spare, nstate)) || (rc = dev_alloc(c, &c->vbuf, nstate)) ||
         (rc = dev_alloc(c, &c->tab_free, nl * nctab)) ||
-        (rc = dev_alloc(c, &c->trf_free, nl * ntrf)) || (rc = dev_alloc(c, &c->tab_mask, ntab)) ||
+        (rc = dev_alloc(c, &c->trf_free, nl * (size_t)c->geo.ctrf_elems)) || (rc = dev_alloc(c, &c->tab_mask, ntab)) ||
         (rc = dev_alloc(c, &c->trf_mask, ntrf)))
         return fail(rc);
     if ((rc = dev_alloc(c, &c->S, band)) || (rc = dev_alloc(c, &c->chol, band)) || (rc = dev_alloc(c, &c->rinv, band)) ||

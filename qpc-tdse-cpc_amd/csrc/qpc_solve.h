@@ -8,16 +8,17 @@
 //
 // Real LU tables (D-part sweeps, S + e X with X antisymmetric; absorber
 // chol(S)), 2(p+1) coefficients per row [F_1..F_p, rdf, G_1..G_p, rdb]:
-//   forward   y_i = rdf_i * (v_i - sum_{j=1..p} F_ij y_{i-j})
-//   backward  x_i = rdb_i * y_i   - sum_{k=1..p} G_ik x_{i+k}
+//   forward   y_i = rdf_i * (v_i - sum_{j=1..p} F_j(i-j) y_{i-j})
+//   backward  x_i = rdb_i * y_i   - sum_{k=1..p} G_k(i) x_{i+k}
+// F_k(i) is the entry of column i of L in row i + k: a row done, its multiples
+// go to the p rows below.
 //
 // Complex symmetric tables (R-part sweeps S + i e X with X symmetric, and the
 // field-free S + i dt/2 H_l), A = L D L^T with L unit lower, p+1 coefficients
 // per row [E_1..E_p, rD] with E_k(i) = L(i+k, i) and rD_i = 1 / D_i:
 //   forward   z_i = v_i - sum_{j=1..p} E_j(i-j) z_{i-j},   y_i = rD_i z_i
 //   backward  x_i = y_i - sum_{k=1..p} E_k(i) x_{i+k}
-// The forward coefficients of row i are entries of the p rows above it, so
-// one row serves both directions: half the bytes of an LU row.
+// One row serves both directions: half the bytes of an LU row.
 //
 // Rows are cut into partitions of kPM rows (the last one padded with identity
 // rows: F = G = E = 0, rdf = rdb = rD = 1, v = 0, which leaves rows < N
@@ -36,11 +37,18 @@
 // kPKMax partitions runs the sequential solve (one lane per channel over all
 // rows), exact for any e.  The result equals the sequential solve to rounding.
 //
+// The state between partitions: forward, what the rows of a partition
+// contribute to the first p rows of the next; backward, the first p values of
+// a partition.  With these, the backward transfer matrix of a complex symmetric
+// partition is the transpose of its forward one, and one set serves both.
+//
 // Device layout ("partition-interleaved"): lanes of a wave own 64 consecutive
-// partitions, so element (partition g, row s of the partition, coefficient q)
-// of a table with R coefficients per row sits at
-// ((g/64 * kPM + s) * R + q) * 64 + g%64: every table or transfer access of a
-// wave is one contiguous 64-element run.
+// partitions, so unit (partition g, row s of the partition, unit q) of a table
+// with R units of 16 bytes per row sits at ((g/64 * kPM + s) * R + q) * 64 +
+// g%64: every table access of a wave is one contiguous run of 1 KB.  A unit is
+// a complex coefficient, or two real ones: (F_1, F_2), (F_3, F_4), .. with rdf
+// after the last, then the G and rdb alike.  Transfer entry e of partition g is
+// element ((g/64 * D + dir) * p^2 + e) * 64 + g%64 (D = 1 complex, 2 real).
 #pragma once
 #include "qpc_common.h"
 
@@ -52,8 +60,8 @@ constexpr int kPKD = 8;        // default carry look-back of the D-part solves (
 constexpr int kPKMax = 28;     // deepest partitioned carry (seg_max 8); deeper reaches run sequentially
 constexpr int kLane = 64;      // partitions per wave group
 constexpr int kMaxGroups = 4;  // wave groups per channel: N <= 4 * 64 * 24 = 6144
-// solve segments: up to seg_max(PK) partitions per 64-lane work-group, plus
-// PK halo partitions on either side
+// solve segments of a channel of more than 64 partitions: up to seg_max(PK)
+// partitions per 64-lane work-group, plus PK halo partitions on either side
 constexpr int seg_max(int pk) { return kLane - 2 * pk; }
 // default factorisation restart: a partition's LU rows are rebuilt from
 // kRestart rows above it, where the elimination state has contracted to
@@ -63,18 +71,22 @@ constexpr int kRestart = 64;
 // band half-widths the kernels are built for
 inline bool width_supported(int p) { return p == 7 || p == 8; }
 
-// grids of at most this many solve work-groups stage the transfer sets in LDS
-// (four waves per work-group, the right-hand side formed in the launch)
+// grids of at most this many solve work-groups stage table rows in LDS
+// (eight waves per work-group, the right-hand side formed in the launch)
 constexpr int64_t kStageGrid = 512;
+
+// units (two doubles) per direction of a real LU row: p coefficients and a diagonal
+constexpr int real_units(int p) { return (p + 2) / 2; }
 
 struct Geom {
     int N;      // rows of the operator
     int P;      // partitions
     int NG;     // wave groups (ceil(P / 64)); the solve uses 64 * NG lanes per channel
     int hw;     // band half-width p
-    int64_t tab_elems;   // elements per real table  (NG * 64 * kPM * 2(p+1))
+    int64_t tab_elems;   // doubles per real table (NG * 64 * kPM * 4 real_units(p))
     int64_t ctab_elems;  // elements per complex symmetric table (NG * 64 * kPM * (p+1))
-    int64_t trf_elems;   // elements per transfer set (NG * 64 * 2 * p^2)
+    int64_t trf_elems;   // elements per real transfer set (NG * 64 * 2 * p^2)
+    int64_t ctrf_elems;  // elements per complex symmetric transfer set (NG * 64 * p^2)
     // launch shape of the partitioned solves (the autotuner's choices; the
     // result does not depend on them): segments per channel beyond the fewest
     // that hold the partitions, and the staged-grid limit
@@ -90,9 +102,10 @@ inline Geom make_geom(int N, int p) {
     g.hw = p;
     g.P = (N + kPM - 1) / kPM;
     g.NG = (g.P + kLane - 1) / kLane;
-    g.tab_elems = (int64_t)g.NG * kLane * kPM * 2 * (p + 1);
+    g.tab_elems = (int64_t)g.NG * kLane * kPM * 4 * real_units(p);
     g.ctab_elems = (int64_t)g.NG * kLane * kPM * (p + 1);
     g.trf_elems = (int64_t)g.NG * kLane * 2 * p * p;
+    g.ctrf_elems = (int64_t)g.NG * kLane * p * p;
     return g;
 }
 
@@ -122,8 +135,8 @@ struct TabMap {
     int L, m0;
     const int* map = nullptr;
     // optional order of the (segment, channel) work-groups of a partitioned
-    // solve: work-group i (linear, segment fastest) runs order[i] = ch * nseg
-    // + seg.  Work-groups are dealt to the XCDs round-robin by linear id, so
+    // solve: work-group i (linear, segment fastest) runs order[i] = ch << 8 |
+    // seg.  Work-groups are dealt to the XCDs round-robin by linear id, so
     // an order that gives the channels of one shared table ids of one residue
     // mod 8 keeps them on one XCD and its L2 (solve_order builds it).
     const int* order = nullptr;
@@ -142,7 +155,7 @@ void solve_order(const int* tab, int nch, int nseg, int* order);
 void launch_rhs(hipStream_t s, int rhs, const RhsArgs& ra, TabMap tm, const cplx* zin, cplx* vout, int nch, Geom geo);
 // x = A^-1 v for nch channels; tab/trf hold the tables and transfer sets of
 // every table id, strides geo.ctab_elems (complex symmetric) or
-// geo.tab_elems (real LU) and geo.trf_elems; role is the RhsKind of the
+// geo.tab_elems (real LU) and geo.ctrf_elems or geo.trf_elems; role is the RhsKind of the
 // operator (kernel name only).  vin and zout may not alias.  pk is the carry
 // depth in partitions (0: the operator's default, kPKS or kPKD; > kPKMax:
 // the sequential solve).
@@ -152,7 +165,7 @@ void launch_bsolve_r(hipStream_t s, int role, const double* tab, const double* t
                      cplx* zout, int nch, Geom geo, int pk = 0);
 
 // v = B z (the RhsKind role with the bands of ra) and x = A^-1 v in one call.
-// On grids that stage the transfer sets in LDS, and when zin and zout do not
+// On grids that stage table rows in LDS, and when zin and zout do not
 // overlap, the solve forms v itself; otherwise launch_rhs writes v into vbuf
 // (nch * N) and the solve reads it.
 void launch_rsolve_c(hipStream_t s, int role, const RhsArgs& ra, const cplx* tab, const cplx* trf, TabMap tm,

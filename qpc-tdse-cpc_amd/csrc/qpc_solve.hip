@@ -11,41 +11,77 @@
 namespace qpc {
 namespace {
 
-__device__ inline cplx tmul(double a, cplx b) { return {a * b.re, a * b.im}; }
 // a + t x with fused multiply-adds (4 for complex t, 2 for real t)
 __device__ inline cplx tmac(cplx a, cplx t, cplx x) {
     return {fma(-t.im, x.im, fma(t.re, x.re, a.re)), fma(t.im, x.re, fma(t.re, x.im, a.im))};
 }
 __device__ inline cplx tmac(cplx a, double t, cplx x) { return {fma(t, x.re, a.re), fma(t, x.im, a.im)}; }
-// a - t x with fused multiply-adds
+// a - t x with fused multiply-adds (4 for complex t, 2 for real t)
 __device__ inline cplx tmsub(cplx a, cplx t, cplx x) {
     return {fma(t.im, x.im, fma(-t.re, x.re, a.re)), fma(-t.im, x.re, fma(-t.re, x.im, a.im))};
 }
+__device__ inline cplx tmsub(cplx a, double t, cplx x) { return {fma(-t, x.re, a.re), fma(-t, x.im, a.im)}; }
+__device__ inline cplx tmulf(cplx a, cplx b) {
+    return {fma(-a.im, b.im, a.re * b.re), fma(a.im, b.re, a.re * b.im)};
+}
+// a complex number in LDS: 16-byte aligned, so that it moves in one access
+struct alignas(16) lcplx {
+    double re, im;
+    __device__ operator cplx() const { return {re, im}; }
+};
+__device__ inline lcplx lc(cplx a) { return {a.re, a.im}; }
 __device__ inline double tzero(double) { return 0.0; }
 __device__ inline cplx tzero(cplx) { return {0.0, 0.0}; }
 __device__ inline double tone(double) { return 1.0; }
 __device__ inline cplx tone(cplx) { return {1.0, 0.0}; }
 
-// row length and table stride of the two table formats (qpc_solve.h)
+// The two table formats (qpc_solve.h) in units of 16 bytes: UF units per row
+// and direction, `row` units per row, the backward ones from unit boff on.
+// coef(c, k): the coefficient k = 1..P of a row's units; diag: its diagonal.
 template <class TF, int P>
 struct TabFmt;
 template <int P>
 struct TabFmt<double, P> {
-    static constexpr int row = 2 * (P + 1);
-    __host__ __device__ static int64_t elems(const Geom& g) { return g.tab_elems; }
+    static constexpr bool SYM = false;
+    static constexpr int UF = real_units(P), row = 2 * UF, boff = UF;
+    __host__ __device__ static int64_t units(const Geom& g) { return g.tab_elems / 2; }
+    __host__ __device__ static int64_t trf_elems(const Geom& g) { return g.trf_elems; }
+    __device__ static double coef(const cplx (&c)[UF], int k) { return k & 1 ? c[(k - 1) / 2].re : c[(k - 1) / 2].im; }
+    __device__ static double diag(const cplx (&c)[UF]) { return P & 1 ? c[UF - 1].im : c[UF - 1].re; }
 };
 template <int P>
 struct TabFmt<cplx, P> {
-    static constexpr int row = P + 1;
-    __host__ __device__ static int64_t elems(const Geom& g) { return g.ctab_elems; }
+    static constexpr bool SYM = true;
+    static constexpr int UF = P + 1, row = P + 1, boff = 0;
+    __host__ __device__ static int64_t units(const Geom& g) { return g.ctab_elems; }
+    __host__ __device__ static int64_t trf_elems(const Geom& g) { return g.ctrf_elems; }
+    __device__ static cplx coef(const cplx (&c)[UF], int k) { return c[k - 1]; }
+    __device__ static cplx diag(const cplx (&c)[UF]) { return c[P]; }
 };
-// first element of partition g's column in a table
+// first unit of partition g's column in a table
 template <class TF, int P>
 __device__ inline int64_t part_col(int g) {
     return (int64_t)(g >> 6) * kPM * TabFmt<TF, P>::row * kLane + (g & 63);
 }
+// its byte offset
+template <class TF, int P>
+__device__ inline unsigned part_off(int g) {
+    return (unsigned)part_col<TF, P>(g) * 16u;
+}
+// the units of one direction of a real row from its coefficients 1..P and diagonal
 template <int P>
-constexpr int trf_n() { return P * P; }  // transfer matrix entries
+__device__ inline void put_real(cplx* o, const double* f, double d) {
+#pragma unroll
+    for (int u = 0; u < P / 2; ++u) o[(int64_t)u * kLane] = cplx{f[2 * u], f[2 * u + 1]};
+    o[(int64_t)(real_units(P) - 1) * kLane] = P & 1 ? cplx{f[P - 1], d} : cplx{d, 0.0};
+}
+// 16 bytes per lane from global memory straight into LDS (to + lane), and the
+// wait for all of them
+__device__ inline void lds_load16(const cplx* from, lcplx* to) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)from,
+                                     (__attribute__((address_space(3))) void*)to, 16, 0, 0);
+}
+__device__ inline void lds_load_wait() { __builtin_amdgcn_s_waitcnt(0x0f70); }  // vmcnt(0)
 
 __device__ inline int table_of(const TabMap& tm, int ch) {
     if (tm.mode == 4) return tm.map[ch] & kMapIdx;
@@ -160,300 +196,278 @@ struct SBandRow {
     }
 };
 
-// LDS slot of row s of partition g in the row-staging buffer: the partition
-// index is XOR-swizzled with s so that row-ordered accesses (consecutive s of
-// one g) and partition-ordered accesses (consecutive g of one s) both spread
-// over the banks without padding
-__device__ inline int sv_slot(int s, int g, int NT) { return s * NT + (g ^ s); }
-
-// forward recurrence over the kPM rows of partition g of a real LU table
-// from state h (h[j] = y_{r0-1-j}); v/y rows live in the row-staging buffer.
-// Table rows are fetched in blocks of RB rows, every load of a block issued
-// before its first use.
-template <bool STORE, int P>
-__device__ inline void fwd_pass(const double* __restrict__ Tg, cplx* sv, int NT, int g, cplx (&h)[P]) {
-    constexpr int R = TabFmt<double, P>::row;
-    constexpr int RB = 12;  // rows per block
-    // the block loop stays rolled: the whole solve kernel must fit the
-    // instruction cache (a fully unrolled solve is ~100 KB of code)
-#pragma unroll 1
-    for (int s0 = 0; s0 < kPM; s0 += RB) {
-        double c[RB][P + 1];
-#pragma unroll
-        for (int b = 0; b < RB; ++b)
-#pragma unroll
-            for (int q = 0; q <= P; ++q)
-                if (s0 + b < kPM) c[b][q] = Tg[(int64_t)((s0 + b) * R + q) * kLane];
-        cplx vr[RB];
-#pragma unroll
-        for (int b = 0; b < RB; ++b)
-            if (s0 + b < kPM) vr[b] = sv[sv_slot(s0 + b, g, NT)];
-#pragma unroll
-        for (int b = 0; b < RB; ++b) {
-            const int s = s0 + b;
-            if (s < kPM) {
-                cplx acc = vr[b];
-#pragma unroll
-                for (int j = 0; j < P; ++j) acc -= tmul(c[b][j], h[j]);
-                const cplx y = tmul(c[b][P], acc);
-#pragma unroll
-                for (int j = P - 1; j > 0; --j) h[j] = h[j - 1];
-                h[0] = y;
-                if (STORE) sv[sv_slot(s, g, NT)] = y;
-            }
-        }
-    }
-}
-
-// backward recurrence over the rows of partition g of a real LU table from
-// state h (h[k] = x_{r0+kPM+k})
-template <bool STORE, int P>
-__device__ inline void bwd_pass(const double* __restrict__ Tg, cplx* sv, int NT, int g, cplx (&h)[P]) {
-    constexpr int R = TabFmt<double, P>::row;
-    constexpr int RB = 12;
-#pragma unroll 1
-    for (int s0 = kPM - 1; s0 >= 0; s0 -= RB) {
-        double c[RB][P + 1];
-#pragma unroll
-        for (int b = 0; b < RB; ++b)
-#pragma unroll
-            for (int q = 0; q <= P; ++q)
-                if (s0 - b >= 0) c[b][q] = Tg[(int64_t)((s0 - b) * R + P + 1 + q) * kLane];
-        cplx yr[RB];
-#pragma unroll
-        for (int b = 0; b < RB; ++b)
-            if (s0 - b >= 0) yr[b] = sv[sv_slot(s0 - b, g, NT)];
-#pragma unroll
-        for (int b = 0; b < RB; ++b) {
-            const int s = s0 - b;
-            if (s >= 0) {
-                cplx x = tmul(c[b][P], yr[b]);
-#pragma unroll
-                for (int k = 0; k < P; ++k) x -= tmul(c[b][k], h[k]);
-#pragma unroll
-                for (int k = P - 1; k > 0; --k) h[k] = h[k - 1];
-                h[0] = x;
-                if (STORE) sv[sv_slot(s, g, NT)] = x;
-            }
-        }
-    }
-}
-
-// Complex symmetric tables.  The forward coefficient of z_{i-1-j} in row i
-// is E_{j+1} of row i-1-j.  The sequential solve and the transfer kernels
-// keep a register ring of, for each of the P rows above, the entries later
-// rows still need: ring[m][k] = E_{k+1}(i-1-m) for k >= m; at a partition's
-// first row it holds the last P rows of the partition before.
-template <int P>
-struct SymRing {
-    static constexpr int R = P + 1;
-    cplx r[P][P];
-    __device__ inline void clear() {
-#pragma unroll
-        for (int m = 0; m < P; ++m)
-#pragma unroll
-            for (int k = m; k < P; ++k) r[m][k] = {0.0, 0.0};
-    }
-    // the last P rows of the partition whose table column starts at Tq
-    __device__ inline void load_tail(const cplx* __restrict__ Tq) {
-#pragma unroll
-        for (int m = 0; m < P; ++m)
-#pragma unroll
-            for (int k = m; k < P; ++k) r[m][k] = Tq[(int64_t)((kPM - 1 - m) * R + k) * kLane];
-    }
-    // row i done: its entries e[0..P-1] become ring row 0
-    __device__ inline void push(const cplx (&e)[P + 1]) {
-#pragma unroll
-        for (int m = P - 1; m > 0; --m)
-#pragma unroll
-            for (int k = m; k < P; ++k) r[m][k] = r[m - 1][k];
-#pragma unroll
-        for (int k = 0; k < P; ++k) r[0][k] = e[k];
-    }
-};
-
-// Forward recurrence over the kPM rows of partition g of a complex symmetric
-// table from state h (h[j] = z_{r0-1-j}); pass B (STORE) writes y = rD z.
-// The coefficient of z_{i-1-j} in row i is E_{j+1} of row i-1-j: the
-// coefficients are gathered from the rows above, a row of the partition
-// before (column Tp) for the first rows of the partition.  Pass A starts
-// from the zero state, where those entries multiply zeros; the first
-// partition has none before, and any finite entry (Tp = Tg) does the same.
-template <bool STORE, int P>
-__device__ inline void fwd_pass_gs(const cplx* __restrict__ Tg, const cplx* __restrict__ Tp, cplx* sv, int NT, int g,
-                                   cplx (&h)[P]) {
-    constexpr int R = P + 1;
-    constexpr int RB = 6;  // rows per block: 6(P+1) loads in flight (a wave counts at most 63)
-    static_assert(kPM % RB == 0, "a pass is a whole number of blocks");
-#pragma unroll 1
-    for (int s0 = 0; s0 < kPM; s0 += RB) {
-        cplx c[RB][R];
-#pragma unroll
-        for (int b = 0; b < RB; ++b) {
-#pragma unroll
-            for (int q = 0; q < P; ++q) {
-                const int rr = s0 + b - 1 - q;
-                const cplx* a = rr >= 0 ? Tg + (int64_t)(rr * R + q) * kLane : Tp + (int64_t)((kPM + rr) * R + q) * kLane;
-                c[b][q] = *a;
-            }
-            c[b][P] = Tg[(int64_t)((s0 + b) * R + P) * kLane];
-        }
-        cplx vr[RB];
-#pragma unroll
-        for (int b = 0; b < RB; ++b) vr[b] = sv[sv_slot(s0 + b, g, NT)];
-#pragma unroll
-        for (int b = 0; b < RB; ++b) {
-            cplx acc = vr[b];
-#pragma unroll
-            for (int j = 0; j < P; ++j) acc = tmsub(acc, c[b][j], h[j]);
-#pragma unroll
-            for (int j = P - 1; j > 0; --j) h[j] = h[j - 1];
-            h[0] = acc;
-            if (STORE) sv[sv_slot(s0 + b, g, NT)] = c[b][P] * acc;
-        }
-    }
-}
-
-// backward recurrence over the rows of partition g of a complex symmetric
-// table from state h (h[k] = x_{r0+kPM+k}); the rows hold y = rD z
-template <bool STORE, int P>
-__device__ inline void bwd_pass_sym(const cplx* __restrict__ Tg, cplx* sv, int NT, int g, cplx (&h)[P]) {
-    constexpr int R = P + 1;
-    constexpr int RB = P == 7 ? 8 : 6;  // rows per block: 56 / 48 loads in flight (a wave counts at most 63)
-    static_assert(kPM % RB == 0, "a pass is a whole number of blocks");
-#pragma unroll 1
-    for (int s0 = kPM - 1; s0 >= 0; s0 -= RB) {
-        cplx c[RB][P];
-#pragma unroll
-        for (int b = 0; b < RB; ++b)
-#pragma unroll
-            for (int q = 0; q < P; ++q) c[b][q] = Tg[(int64_t)((s0 - b) * R + q) * kLane];
-        cplx yr[RB];
-#pragma unroll
-        for (int b = 0; b < RB; ++b) yr[b] = sv[sv_slot(s0 - b, g, NT)];
-#pragma unroll
-        for (int b = 0; b < RB; ++b) {
-            const int s = s0 - b;
-            cplx x = yr[b];
-#pragma unroll
-            for (int k = 0; k < P; ++k) x = tmsub(x, c[b][k], h[k]);
-#pragma unroll
-            for (int k = P - 1; k > 0; --k) h[k] = h[k - 1];
-            h[0] = x;
-            if (STORE) sv[sv_slot(s, g, NT)] = x;
-        }
-    }
-}
-
-// truncated carry by Horner: acc <- E[gp] + T[gp] acc for gp = g -/+ k,
-// k = PK..1 (partitions beyond the channel ends do not exist: exact start).
-// The first existing term starts from the zero state, so its transfer
-// product vanishes and acc = E[gp].  End state and transfer entry e of
-// partition gp are column gp - base of sE and of sT (row e).
-// Transfer entry e of partition gp: staged in LDS (column gp - base of row e)
-// or read from the transfer set in global memory.
-template <class TF, bool LDS_T, int P>
-struct TrfAt {
-    const TF* p;  // LDS: the direction's staged rows; global: the direction's set
-    int NT, base;
-    __device__ inline TF operator()(int gp, int e) const {
-        if constexpr (LDS_T) return p[e * NT + gp - base];
-        else return p[(int64_t)(gp >> 6) * 2 * trf_n<P>() * kLane + (int64_t)e * kLane + (gp & 63)];
-    }
-};
-
-template <class TF, bool LDS_T, int P>
-__device__ inline void carry(TrfAt<TF, LDS_T, P> T, const cplx* sE, int NT, int g, int dir, int NP, int base, int PK,
-                             cplx (&acc)[P]) {
-#pragma unroll
-    for (int r = 0; r < P; ++r) acc[r] = {0.0, 0.0};
-    bool started = false;
-#pragma unroll 1
-    for (int k = PK; k >= 1; --k) {
-        const int gp = dir == 0 ? g - k : g + k;
-        if (gp >= 0 && gp < NP) {
-            const int lg = gp - base;
-            if (!started) {
-#pragma unroll
-                for (int r = 0; r < P; ++r) acc[r] = sE[r * NT + lg];
-                started = true;
-                continue;
-            }
-            // the transfer matrix row by row (LDS, or global memory when
-            // LDS_T is off), each row's reads in flight together
-            cplx nv[P];
-#pragma unroll
-            for (int r = 0; r < P; ++r) {
-                TF t[P];
-#pragma unroll
-                for (int c = 0; c < P; ++c) t[c] = T(gp, r * P + c);
-                cplx a = sE[r * NT + lg];
-#pragma unroll
-                for (int c = 0; c < P; ++c) a = tmac(a, t[c], acc[c]);
-                nv[r] = a;
-            }
-#pragma unroll
-            for (int r = 0; r < P; ++r) acc[r] = nv[r];
-        }
-    }
-}
-
-// waves of a work-group on the grids that stage the transfer sets in LDS
-constexpr int kStageWaves = 4;
-
-// The carry of every staged partition spread over the kStageWaves waves of
-// a staged work-group: lane ln of each wave serves partition g = base + ln,
-// and wave w forms rows w and w + 4 of each Horner step's product; the state
-// goes through LDS (two buffers of P x NT) with one barrier per step.  The
-// same products in the same order as carry(), so the same bits.  Every wave
-// calls it (it holds barriers); lanes with active false only keep their
-// state.  Returns the buffer that holds the result.
+// ---------------------------------------------------------------------------
+// One table row of one partition and direction in registers (UF units).
+// Forward (state acc[k]: what the rows above contribute to row s + k, to be
+// added to its right-hand side): the row's value leaves the window and its
+// multiples go to the P rows below.  The state a partition hands on is what
+// its rows contribute to the first P rows of the next.
 template <class TF, int P>
-__device__ inline int carry4(TrfAt<TF, true, P> T, const cplx* sE, cplx* sA, int NT, int g, int dir, int NP, int base,
-                             int PK, int w, int ln, bool active) {
-    static_assert(P <= 2 * kStageWaves, "two rows per wave");
-    // the partitions on the dir side that exist: the first of them starts the chain
-    const int ks = !active ? 0 : dir == 0 ? min(PK, g) : min(PK, NP - 1 - g);
+__device__ inline cplx fwd_row(const cplx (&c)[TabFmt<TF, P>::UF], cplx v, cplx (&acc)[P]) {
+    using F = TabFmt<TF, P>;
+    const cplx z = {v.re + acc[0].re, v.im + acc[0].im};
+    cplx y;  // what the lower rows' updates take, and the stored row
+    if constexpr (F::SYM) y = z;
+    else y = {F::diag(c) * z.re, F::diag(c) * z.im};
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int r = w + kStageWaves * i;
-        if (r < P) sA[r * NT + ln] = ks > 0 ? sE[r * NT + (dir == 0 ? g - ks : g + ks) - base] : cplx{0.0, 0.0};
+    for (int k = 1; k < P; ++k) acc[k - 1] = tmsub(acc[k], F::coef(c, k), y);
+    acc[P - 1] = tmsub(cplx{0.0, 0.0}, F::coef(c, P), y);
+    if constexpr (F::SYM) return tmulf(F::diag(c), z);
+    else return y;
+}
+// Backward (state h[k] = x_{s+1+k}): x_s from the stored row, oldest term
+// first, so that only the last product waits for x_{s+1}
+template <class TF, int P>
+__device__ inline cplx bwd_row(const cplx (&c)[TabFmt<TF, P>::UF], cplx y, cplx (&h)[P]) {
+    using F = TabFmt<TF, P>;
+    cplx x = y;
+    if constexpr (!F::SYM) x = {F::diag(c) * y.re, F::diag(c) * y.im};
+#pragma unroll
+    for (int k = P; k >= 1; --k) x = tmsub(x, F::coef(c, k), h[k - 1]);
+#pragma unroll
+    for (int k = P - 1; k > 0; --k) h[k] = h[k - 1];
+    h[0] = x;
+    return x;
+}
+
+// ---------------------------------------------------------------------------
+// Rows of a partition are taken in blocks of RB.  The units of the block in
+// hand sit in registers; as soon as a row is done its registers are filled
+// with the same row of the next block, so that a block's loads are in flight
+// while the block before runs.  Blocks [LB0, LB1) of a staged work-group come
+// from LDS, the others from the table.  The block loops stay rolled and there
+// is no branch between rows: a branch costs a wave about as much as six FP64
+// operations, and code that is not in the instruction cache costs twice its
+// run time, so the solves of a step together must stay within it (64 KB).
+template <class TF, int P>
+struct Blocks {
+    static constexpr int RB = 4, NB = kPM / RB;
+    static constexpr int LB0 = 1, LB1 = P == 7 ? 4 : 3;  // what the LDS holds beside the rows and states
+    static constexpr int LR = (LB1 - LB0) * RB;          // staged rows
+    static constexpr int UF = TabFmt<TF, P>::UF, UT = TabFmt<TF, P>::row;
+    static_assert(kPM % RB == 0, "a pass is a whole number of blocks");
+};
+template <class TF, int P>
+using RowRegs = cplx[TabFmt<TF, P>::UF];
+template <class TF, int P>
+using BlockRegs = RowRegs<TF, P>[Blocks<TF, P>::RB];
+
+// unit k of the run at base (uniform), this lane's byte offset off
+__device__ inline cplx unit_at(const cplx* base, unsigned off, int k) {
+    return *(const cplx*)((const char*)(base + (int64_t)k * kLane) + off);
+}
+// UN units of row r of the block at p
+template <class TF, int P, int UN>
+__device__ inline void row_g(RowRegs<TF, P>& c, const cplx* p, unsigned off, int r) {
+#pragma unroll
+    for (int u = 0; u < UN; ++u) c[u] = unit_at(p, off, r * TabFmt<TF, P>::row + u);
+}
+template <class TF, int P, int UN>
+__device__ inline void block_g(BlockRegs<TF, P>& c, const cplx* p, unsigned off) {
+#pragma unroll
+    for (int r = 0; r < Blocks<TF, P>::RB; ++r) row_g<TF, P, UN>(c[r], p, off, r);
+}
+
+// The row buffer: kRowStride slots per partition (an odd count, so that lanes
+// of consecutive partitions fall on different banks), row s of slot ln at
+// ln * kRowStride + s; kRowPad slots on either side for the passes' read-ahead
+constexpr int kRowStride = kPM + 1, kRowPad = 4;
+constexpr int kRowSlots = kLane * kRowStride + 2 * kRowPad;
+__device__ inline int row_slot(int s, int ln) { return kRowPad + ln * kRowStride + s; }
+
+// the rows of one block: v[r] the row's value, written to wb[r]; the block's
+// registers are refilled from LDS (l: this lane's units) or the table (p)
+template <class TF, int P, bool L>
+__device__ inline void fwd_block(BlockRegs<TF, P>& c, cplx (&v)[Blocks<TF, P>::RB], const lcplx* rb, lcplx* wb,
+                                 const lcplx* l, const cplx* p, unsigned off, cplx (&acc)[P]) {
+    using B = Blocks<TF, P>;
+#pragma unroll
+    for (int r = 0; r < B::RB; ++r) {
+        const cplx y = fwd_row<TF, P>(c[r], v[r], acc);
+        v[r] = rb[B::RB + r];
+        wb[r] = lc(y);
+#pragma unroll
+        for (int u = 0; u < B::UF; ++u)
+            c[r][u] = L ? (cplx)l[(r * B::UF + u) * kLane] : unit_at(p, off, r * B::UT + u);
+        __builtin_amdgcn_sched_barrier(0);
     }
-    __syncthreads();
-    int cur = 0;
+}
+template <class TF, int P, bool L>
+__device__ inline void bwd_block(BlockRegs<TF, P>& c, cplx (&v)[Blocks<TF, P>::RB], const lcplx* rb, lcplx* wb,
+                                 const lcplx* l, const cplx* p, unsigned off, cplx (&h)[P]) {
+    using B = Blocks<TF, P>;
+    constexpr int UB = TabFmt<TF, P>::SYM ? P : B::UF;  // a symmetric row's diagonal is not read
+#pragma unroll
+    for (int r = B::RB - 1; r >= 0; --r) {
+        const cplx x = bwd_row<TF, P>(c[r], v[r], h);
+        v[r] = rb[r - B::RB];
+        wb[r] = lc(x);
+#pragma unroll
+        for (int u = 0; u < UB; ++u)
+            c[r][u] = L ? (cplx)l[(r * B::UF + u) * kLane] : unit_at(p, off, r * B::UT + u);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// One pass over the rows of slot ln (rows: its first row; T: the direction's
+// units of the table, uniform).  c holds the first block at entry and the
+// block at `after` at the end.  Rows are written to `out` (their own place, or
+// a scrap block of RB rows when ostep is 0).
+template <class TF, int P, bool STAGED>
+__device__ inline void fwd_pass(BlockRegs<TF, P>& c, const cplx* T, unsigned off, const lcplx* sL,
+                                const lcplx* rows, lcplx* out, int ostep, cplx (&acc)[P], const cplx* after) {
+    using B = Blocks<TF, P>;
+    cplx v[B::RB];
+#pragma unroll
+    for (int r = 0; r < B::RB; ++r) v[r] = rows[r];
+    if constexpr (STAGED) {
 #pragma unroll 1
-    for (int k = PK - 1; k >= 1; --k) {
-        const cplx* a = sA + cur * P * NT;
-        cplx* o = sA + (1 - cur) * P * NT;
-        if (k < ks) {
-            const int gp = dir == 0 ? g - k : g + k;
-            cplx acc[P];
+        for (int i = 0; i < B::LB1 - B::LB0; ++i) {
+            fwd_block<TF, P, true>(c, v, rows, out, sL, nullptr, 0, acc);
+            rows += B::RB;
+            out += ostep;
+            sL += B::RB * B::UF * kLane;
+        }
+    }
+    constexpr int G0 = STAGED ? B::LB1 : 1, GN = B::NB + 1 - G0;  // the blocks still to load: G0 .. NB-1, after
+    T += (int64_t)G0 * B::RB * B::UT * kLane;
+#pragma unroll 1
+    for (int i = 0; i < GN; ++i) {
+        fwd_block<TF, P, false>(c, v, rows, out, nullptr, i == GN - 1 ? after : T, off, acc);
+        rows += B::RB;
+        out += ostep;
+        T += B::RB * B::UT * kLane;
+    }
+}
+template <class TF, int P, bool STAGED>
+__device__ inline void bwd_pass(BlockRegs<TF, P>& c, const cplx* T, unsigned off, const lcplx* sL,
+                                const lcplx* rows, lcplx* out, int ostep, cplx (&h)[P], const cplx* after) {
+    using B = Blocks<TF, P>;
+    cplx v[B::RB];
+    rows += (B::NB - 1) * B::RB;
+    out += (ostep ? B::NB - 1 : 0) * B::RB;
 #pragma unroll
-            for (int c = 0; c < P; ++c) acc[c] = a[c * NT + ln];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int r = w + kStageWaves * i;
-                if (r < P) {
-                    TF t[P];
-#pragma unroll
-                    for (int c = 0; c < P; ++c) t[c] = T(gp, r * P + c);
-                    cplx v = sE[r * NT + gp - base];
-#pragma unroll
-                    for (int c = 0; c < P; ++c) v = tmac(v, t[c], acc[c]);
-                    o[r * NT + ln] = v;
-                }
+    for (int r = 0; r < B::RB; ++r) v[r] = rows[r];
+    sL += (B::LR - B::RB) * B::UF * kLane;
+    int b = B::NB - 2;  // the block to load next
+#pragma unroll 1
+    for (int ph = 0; ph < 2; ++ph) {
+        const int stop = STAGED && ph == 0 ? B::LB1 : -1;
+#pragma unroll 1
+        for (; b >= stop; --b) {
+            bwd_block<TF, P, false>(c, v, rows, out, nullptr, b < 0 ? after : T + b * (B::RB * B::UT * kLane), off, h);
+            rows -= B::RB;
+            out -= ostep;
+        }
+        if constexpr (!STAGED) break;
+        if (ph == 0) {
+#pragma unroll 1
+            for (; b >= B::LB0; --b) {
+                bwd_block<TF, P, true>(c, v, rows, out, sL, nullptr, 0, h);
+                rows -= B::RB;
+                out -= ostep;
+                sL -= B::RB * B::UF * kLane;
             }
-        } else {
+        }
+    }
+}
+
+// The incoming state of every partition from the pass-A end states E and the
+// partitions' own transfer matrices: s_g <- E_g + T_g s_{g-1} (g+1 backward),
+// PK - 1 times from s = E, so that s_{g-1} holds the PK partitions before g,
+// the same sums as Horner's rule over them.  A matrix is read once and stays
+// in registers; only states pass between lanes, through LDS: entry r of slot
+// ln at r * kSt + ln, with a column of zeros after the slots for the neighbour
+// that does not exist.
+constexpr int kSt = kLane + 1;
+constexpr int kWavesStaged = 8, kHelp = kWavesStaged - 1;
+
+// entry (r, c) of the direction's matrix, T the table's set (uniform); a
+// symmetric table's backward matrix is the transpose of its forward one
+template <class TF, int P>
+__device__ inline unsigned trf_off(int g) {
+    return ((unsigned)(g >> 6) * (TabFmt<TF, P>::SYM ? 1 : 2) * P * P * kLane + (g & 63)) * (unsigned)sizeof(TF);
+}
+template <class TF, int P>
+__device__ inline TF trf_at(const TF* T, unsigned off, int dir, int r, int c) {
+    constexpr bool SYM = TabFmt<TF, P>::SYM;
+    const int e = SYM ? (dir ? c * P + r : r * P + c) : dir * P * P + r * P + c;
+    return *(const TF*)((const char*)(T + (int64_t)e * kLane) + off);
+}
+// the column of slot ln's neighbour
+__device__ inline int neighbour(int ln, int n, int dir) {
+    const int nb = dir == 0 ? ln - 1 : ln + 1;
+    return nb >= 0 && nb < n ? nb : kLane;
+}
+
+// one wave: slot ln of n; e enters as the end states and leaves as the
+// incoming state
+template <class TF, int P>
+__device__ inline void carry1(const TF (&t)[P][P], lcplx* sS, int ln, int n, int dir, int PK, cplx (&e)[P]) {
+    const int q = neighbour(ln, n, dir);
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int r = w + kStageWaves * i;
-                if (r < P) o[r * NT + ln] = a[r * NT + ln];
-            }
+    for (int r = 0; r < P; ++r) sS[r * kSt + ln] = lc(e[r]);
+    __syncthreads();
+#pragma unroll 1
+    for (int k = 1; k < PK; ++k) {
+        cplx in[P];
+#pragma unroll
+        for (int c = 0; c < P; ++c) in[c] = sS[c * kSt + q];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < P; ++r) {
+            cplx a = e[r];
+#pragma unroll
+            for (int c = 0; c < P; ++c) a = tmac(a, t[r][c], in[c]);
+            sS[r * kSt + ln] = lc(a);
         }
         __syncthreads();
-        cur ^= 1;
     }
-    return cur;
+#pragma unroll
+    for (int r = 0; r < P; ++r) e[r] = sS[r * kSt + q];
+    __syncthreads();
+}
+
+// a staged work-group: the helper waves share the rows of the product (helper
+// hw has row hw, and hw + 7 of eight), wave 0 waits.  One barrier per step.
+constexpr int trf_rows(int P) { return (P + kHelp - 1) / kHelp; }
+template <class TF, int P>
+__device__ inline void carry_load(TF (&t)[trf_rows(P)][P], const TF* T, unsigned off, int dir, int hw) {
+#pragma unroll
+    for (int i = 0; i < trf_rows(P); ++i)
+#pragma unroll
+        for (int c = 0; c < P; ++c) t[i][c] = trf_at<TF, P>(T, off, dir, min(hw + kHelp * i, P - 1), c);
+}
+template <class TF, int P>
+__device__ inline void carry8(const TF (&t)[trf_rows(P)][P], const lcplx* sE, lcplx* sS, int ln, int n, int dir, int PK,
+                              int hw) {
+    const int q = neighbour(ln, n, dir);
+    cplx e[trf_rows(P)];
+#pragma unroll
+    for (int i = 0; i < trf_rows(P); ++i) e[i] = sE[min(hw + kHelp * i, P - 1) * kSt + ln];
+    const lcplx* src = sE;
+#pragma unroll 1
+    for (int k = 1; k < PK; ++k) {
+        lcplx* dst = sS + (k & 1) * P * kSt;
+        cplx in[P];
+#pragma unroll
+        for (int c = 0; c < P; ++c) in[c] = src[c * kSt + q];
+#pragma unroll
+        for (int i = 0; i < trf_rows(P); ++i) {
+            const int r = min(hw + kHelp * i, P - 1);  // (a row past the last repeats the last)
+            cplx a = e[i];
+#pragma unroll
+            for (int c = 0; c < P; ++c) a = tmac(a, t[i][c], in[c]);
+            dst[r * kSt + ln] = lc(a);
+        }
+        __syncthreads();
+        src = dst;
+    }
+}
+// the buffer that holds the result after PK - 1 steps
+template <int P>
+__device__ inline const lcplx* carried(const lcplx* sE, const lcplx* sS, int PK) {
+    return PK > 1 ? sS + ((PK - 1) & 1) * P * kSt : sE;
 }
 
 // v = B z for per-table bands (RHS_CBAND), one lane per (row, channel)
@@ -501,237 +515,264 @@ __global__ __launch_bounds__(256) void k_rhs_shared(RhsArgs ra, const cplx* __re
     }
 }
 
-// x = U^-1 L^-1 v, v = B z.  A channel's partitions are cut
-// into segments of up to SN partitions, one 64-lane work-group per (segment,
-// channel), one lane per partition, so that a channel spreads over several
-// compute units.  A work-group also runs the PK partitions on either side of
-// its segment (halo): the forward carries of its own partitions need the
-// pass-A end states of the PK partitions before them, and the backward
-// carries need the PK partitions after the segment forward-solved.  Every
-// value computed for an owned partition depends on these partitions only, so
-// the segmentation does not change a single bit of the result.  Requires
-// SN + 2 PK <= 64.  ROLE is the RhsKind of the operator.  On the small grids
-// that stage the transfer sets (LDS_T: one or two work-groups per CU) a
-// work-group has kStageWaves waves: all of them fetch the right-hand side and
-// the transfer sets and write the result, on SIMDs that would otherwise idle,
-// and wave 0 runs the passes and carries.  Both directions' transfer sets are
-// staged during forward pass A when they fit the LDS with the other buffers
-// (p = 7, and real tables); otherwise (complex tables at p = 8) the forward
-// sets are staged then and the backward sets, into the same buffer, during
-// backward pass A.
+// x = U^-1 L^-1 v, v = B z.  A channel's partitions are cut into segments of
+// up to SN partitions, one work-group each, one lane per partition; a channel
+// of at most 64 partitions is one segment.  With several segments a
+// work-group also runs the PK partitions on either side of its own (halo):
+// the forward carries need the pass-A end states of the PK partitions before
+// them, and the backward carries need the PK partitions after the segment
+// forward-solved.  Every value computed for an owned partition depends on
+// these partitions only, so the segmentation does not change a single bit of
+// the result.  Requires SN + 2 PK <= 64, or one segment.  ROLE is the RhsKind
+// of the operator.
 //
-// FUSE (LDS_T grids only): src is the state z and the work-group forms
-// v = B z itself while staging (the RhsKind ROLE with the bands of ra, the
-// same arithmetic as k_rhs / k_rhs_shared): the staged rows and P rows on
-// either side of z go to LDS, and each staged row's band entries are read
-// from L2.  Other work-groups read z rows this one owns, so src and zout may
-// not overlap.  Without FUSE, src is v.
-constexpr int kLdsBytes = 160 * 1024;
-template <class TF, int P, bool FUSE, int ND>
-constexpr int bsolve_lds() {
-    return kPM * kLane * 16 + P * kLane * 16 + ND * P * P * kLane * (int)sizeof(TF) +
-           (FUSE ? (kPM * kLane + 2 * P) * 16 : 0) + 2 * P * kLane * 16;
-}
-template <class TF, int P, bool FUSE>
-constexpr bool both_trf_fit() { return bsolve_lds<TF, P, FUSE, 2>() <= kLdsBytes; }
+// What bounds it is latency: a lane's chain is 24 rows, four times, and the
+// table rows (24 x P+1 units of 16 bytes for each of 64 partitions, 196 KB)
+// neither fit the registers nor, with the buffers, the LDS.  On the small
+// grids (STAGED: one work-group per compute unit) a work-group therefore has
+// kWavesStaged waves.  Wave 0 runs the passes; at the start it loads the first
+// block of rows into registers and 12 rows into LDS, where all four passes
+// find them, and the remaining rows come from L2 a block ahead (Blocks).
+// Meanwhile the helper waves fetch z, form v = B z (FUSE), and hold the
+// transfer matrices, with which they run the carries.  Larger grids run one
+// wave per work-group, several per compute unit, which hide each other's
+// loads.
+// Measured per launch, R, D, free and mask solves (with, in
+// brackets, four waves that shared the passes' loads through LDS): 21.6 / 18.0 / 21.4 / 17.0 us at N = 240
+// (29.6 / 22.2 / 30 / 20.7), 26.9 / 25.0 / 28.7 / 19.2 us at N = 3000 with 81
+// channels (32.2 / 27.6 / 33.8 / 22.8).  Of the 55 k cycles of a symmetric solve the
+// passes take 27 k (two thirds of it the issue of their own arithmetic), the
+// carries 7 k and the loads with the right-hand side 20 k.
+//
+// FUSE (STAGED): src is the state z and the work-group forms v = B z itself
+// (the RhsKind ROLE with the bands of ra, the same arithmetic as k_rhs /
+// k_rhs_shared) from the staged rows and P rows on either side of z in LDS;
+// other work-groups read z rows this one owns, so src and zout may not
+// overlap.  Without FUSE, src is v.
+template <class TF, int P>
+struct StageLds {
+    // z rows of a fused right-hand side, then the carry's states (two
+    // buffers) and the scrap rows of the passes that keep their input
+    static constexpr int NZ = kPM * kLane + 2 * P;
+    static constexpr int scrap = 2 * P * kSt;
+    static constexpr int sz = NZ > scrap + kLane * Blocks<TF, P>::RB ? NZ : scrap + kLane * Blocks<TF, P>::RB;
+    static constexpr int bytes = 16 * (sz + kRowSlots + P * kSt + Blocks<TF, P>::LR * Blocks<TF, P>::UT * kLane);
+    static_assert(bytes <= 160 * 1024, "LDS budget");
+};
 
-// helper waves 1..kStageWaves-1 copy transfer entries q = Q0 .. Q0+NQ-1 of the
-// staged partitions [ga, gb) into st (row q - Q0, column gl - ga)
-template <class TF, int P, int Q0, int NQ>
-__device__ inline void stage_trf(const TF* __restrict__ TR, TF* st, int tid, int ga, int gb) {
-    constexpr int NW = kStageWaves - 1, QW = (NQ + NW - 1) / NW;
-    const int ln = tid & (kLane - 1), w = tid / kLane - 1;
-    const int gl = ga + ln;
-    if (w >= 0 && gl < gb) {
-        const TF* Tr = TR + (int64_t)(gl >> 6) * 2 * trf_n<P>() * kLane + (gl & 63) + (int64_t)Q0 * kLane;
-        TF tv[QW];
-#pragma unroll
-        for (int j = 0; j < QW; ++j) tv[j] = Tr[(int64_t)min(w + j * NW, NQ - 1) * kLane];
-#pragma unroll
-        for (int j = 0; j < QW; ++j)
-            if (w + j * NW < NQ) st[(w + j * NW) * kLane + ln] = tv[j];
-    }
-}
-
-template <class TF, int ROLE, bool LDS_T, bool FUSE, int P>
-__global__ __launch_bounds__(kLane * (LDS_T ? kStageWaves : 1)) void k_bsolve(
-    const TF* __restrict__ tab, const TF* __restrict__ trf, TabMap tm, const cplx* __restrict__ src,
+template <class TF, int ROLE, bool STAGED, bool FUSE, int P>
+__global__ __launch_bounds__(kLane * (STAGED ? kWavesStaged : 1)) void k_bsolve(
+    const cplx* __restrict__ tab, const TF* __restrict__ trf, TabMap tm, const cplx* __restrict__ src,
     cplx* __restrict__ zout, Geom geo, int SN, int PK, RhsArgs ra) {
-    static_assert(LDS_T || !FUSE, "the fused right-hand side is built for the staged grids");
-    constexpr int NT = kLane;
-    constexpr int NTH = kLane * (LDS_T ? kStageWaves : 1);  // threads of the work-group
-    constexpr int KV = kPM * NT / NTH;                       // staged rows per thread
-    static_assert(kPM * NT % NTH == 0, "whole staged rows per thread");
-    constexpr int KT = trf_n<P>();
-    constexpr bool TWO = both_trf_fit<TF, P, FUSE>();
-    static_assert(!LDS_T || bsolve_lds<TF, P, FUSE, TWO ? 2 : 1>() <= kLdsBytes, "LDS budget");
-    constexpr int NZ = kPM * NT + 2 * P;  // z rows of a fused right-hand side
-    __shared__ cplx sv[kPM * NT];
-    __shared__ cplx sE[P * NT];
-    // transfer sets of the staged partitions (LDS_T only): both directions,
-    // or one direction at a time
-    __shared__ TF sT[LDS_T ? (TWO ? 2 : 1) : 1][LDS_T ? KT * NT : 1];
-    // z rows [r0 - P, r0 + NZ - P) (FUSE only; zero outside [0, N))
-    __shared__ cplx sz[FUSE ? NZ : 1];
-    // carry state of the staged partitions (LDS_T: carry4)
-    __shared__ cplx sA[LDS_T ? 2 * P * NT : 1];
+    static_assert(STAGED || !FUSE, "the fused right-hand side is built for the staged grids");
+    using F = TabFmt<TF, P>;
+    using B = Blocks<TF, P>;
+    using S = StageLds<TF, P>;
+    constexpr int NTH = kLane * (STAGED ? kWavesStaged : 1);  // threads of the work-group
+    __shared__ lcplx sv[kRowSlots];                             // the rows v, y, x
+    __shared__ lcplx sE[P * kSt];                               // end states (one wave: the carry's)
+    // z rows [r0 - P, r0 + NZ - P) (FUSE; zero outside [0, N)); then carry states and scrap rows
+    __shared__ lcplx sz[STAGED ? S::sz : kLane * B::RB];
+    __shared__ lcplx sT[STAGED ? B::LR * B::UT * kLane : 1];    // staged table rows
 
     int ch = blockIdx.y, seg = blockIdx.x;
     if (tm.order) {
         const int o = tm.order[blockIdx.y * gridDim.x + blockIdx.x];
-        ch = o / (int)gridDim.x;
-        seg = o - ch * (int)gridDim.x;
+        ch = o >> 8;
+        seg = o & 255;
     }
     const int N = geo.N, NP = geo.P;
-    const int k0 = seg * SN, k1 = min(NP, k0 + SN);  // owned partitions [k0, k1)
+    const int k0 = seg * SN, k1 = min(NP, k0 + SN);         // owned partitions [k0, k1)
     const int ga = max(0, k0 - PK), gb = min(NP, k1 + PK);  // staged partitions [ga, gb)
-    const int tid = threadIdx.x;
-    const int g = ga + tid;  // this lane's partition (wave 0)
-    const bool run = tid < kLane && g < gb;
+    const int n = gb - ga;
+    const int tid = threadIdx.x, ln = tid & (kLane - 1);
+    const int w = STAGED ? __builtin_amdgcn_readfirstlane(tid / kLane) : 0;
+    // this lane's partition; lanes past the staged ones repeat the last (their
+    // rows and states are not used)
+    const int g = min(ga + ln, gb - 1);
     const int tabid = table_of(tm, ch);
     const bool cj = conj_of(tm, ch);
-    const int64_t r0 = (int64_t)ga * kPM;  // first staged row
-    const int nrow = (gb - ga) * kPM;
-    const int nv = min(nrow, N - (int)r0);  // staged rows below N
-    cplx* xo = zout + (int64_t)ch * N + r0;
-    const TF* T0 = tab + (int64_t)tabid * TabFmt<TF, P>::elems(geo);
-    const TF* Tg = T0 + part_col<TF, P>(g);
-    // the column of the partition before (the partition itself for the first)
-    const TF* Tp = T0 + part_col<TF, P>(g > 0 ? g - 1 : 0);
-    constexpr bool SYM = TabFmt<TF, P>::row == P + 1;
-    const int w = tid / kLane, ln = tid % kLane;  // wave, lane (carry4)
+    const int r0 = ga * kPM;  // first staged row
+    const int nrow = n * kPM;
+    const int nv = min(nrow, N - r0);  // staged rows below N
+    const cplx* T = tab + (int64_t)tabid * F::units(geo);
+    const unsigned off = part_off<TF, P>(g);
+    const TF* TR = trf + (int64_t)tabid * F::trf_elems(geo);
+    const unsigned toff = trf_off<TF, P>(g);
+    const cplx* Tb = T + F::boff * kLane;                                   // backward units
+    const cplx* Tb0 = Tb + (int64_t)(B::NB - 1) * B::RB * B::UT * kLane;    // their first block
+    lcplx* rows = sv + row_slot(0, ln);
 
-    // right-hand side rows (padding rows: 0), or the z rows it is formed
-    // from (the transfer sets follow during pass A).  The row loads are
-    // unconditional (indices clamped into the channel) so that all of them
-    // are in flight at once.
-    if constexpr (FUSE) {
-        constexpr int KZ = (NZ + NTH - 1) / NTH;
-        const cplx* zc = src + (int64_t)ch * N;
-        const int zlo = (int)r0 - P;
-        cplx zr[KZ];
+    if (w == 0) {
+        BlockRegs<TF, P> c;
+        cplx h[P];
+        const lcplx* sL = sT + ln;
+        lcplx* scrap = sz + (STAGED ? S::scrap : 0) + ln * B::RB;
+        if constexpr (STAGED) {
+            block_g<TF, P, F::UF>(c, T, off);
+            // rows of blocks [LB0, LB1): straight into LDS, unit by unit
+            const cplx* Ts = T + (int64_t)B::LB0 * B::RB * B::UT * kLane;
+#pragma unroll 1
+            for (int i = 0; i < B::LR; ++i)
 #pragma unroll
-        for (int k = 0; k < KZ; ++k) zr[k] = cj_if(cj, zc[min(max(zlo + tid + k * NTH, 0), N - 1)]);
+                for (int u = 0; u < B::UT; ++u) {
+                    const int d = F::SYM || u < B::UF ? i * B::UF + u : (B::LR + i) * B::UF + u - B::UF;
+                    lds_load16((const cplx*)((const char*)(Ts + (i * B::UT + u) * kLane) + off), sT + d * kLane);
+                }
+            if (FUSE) __syncthreads();  // z in LDS
+            __syncthreads();            // v in LDS
+            lds_load_wait();
+            // the states' zero columns (the z rows they replace are done with)
+            if (ln < 2 * P) sz[ln * kSt + kLane] = lcplx{0.0, 0.0};
+            if (ln < P) sE[ln * kSt + kLane] = lcplx{0.0, 0.0};
+        } else {
+            constexpr int KB = 8;  // rows fetched together
+            const cplx* vi = src + (int64_t)ch * N + r0;
+#pragma unroll 1
+            for (int k = 0; k < kPM; k += KB) {
+                cplx vr[KB];
 #pragma unroll
-        for (int k = 0; k < KZ; ++k) {
-            const int j = tid + k * NTH, row = zlo + j;
-            if (j < NZ) sz[j] = row >= 0 && row < N ? zr[k] : cplx{0.0, 0.0};
+                for (int j = 0; j < KB; ++j) vr[j] = cj_if(cj, vi[min(tid + (k + j) * NTH, nv - 1)]);
+#pragma unroll
+                for (int j = 0; j < KB; ++j) {
+                    const int i = tid + (k + j) * NTH;
+                    if (i < nrow) sv[row_slot(i % kPM, i / kPM)] = lc(i < nv ? vr[j] : cplx{0.0, 0.0});
+                }
+            }
+            block_g<TF, P, F::UF>(c, T, off);
+            if (ln < P) sE[ln * kSt + kLane] = lcplx{0.0, 0.0};
+            __syncthreads();
+        }
+#pragma unroll
+        for (int j = 0; j < P; ++j) h[j] = {0.0, 0.0};
+        // forward: pass A from the zero state, carry, pass B
+#pragma unroll 1
+        for (int pass = 0;; ++pass) {
+            fwd_pass<TF, P, STAGED>(c, T, off, sL, rows, pass ? rows : scrap, pass ? B::RB : 0, h, pass ? Tb0 : T);
+            if (pass) break;
+            if constexpr (STAGED) {
+#pragma unroll
+                for (int j = 0; j < P; ++j) sE[j * kSt + ln] = lc(h[j]);
+                for (int k = 0; k < PK; ++k) __syncthreads();
+                const lcplx* s = carried<P>(sE, sz, PK) + neighbour(ln, n, 0);
+#pragma unroll
+                for (int j = 0; j < P; ++j) h[j] = s[j * kSt];
+            } else {
+                TF t[P][P];
+#pragma unroll
+                for (int r = 0; r < P; ++r)
+#pragma unroll
+                    for (int q = 0; q < P; ++q) t[r][q] = trf_at<TF, P>(TR, toff, 0, r, q);
+                carry1<TF, P>(t, sE, ln, n, 0, PK, h);
+            }
+        }
+        if constexpr (STAGED && !F::SYM) sL += B::LR * B::UF * kLane;
+#pragma unroll
+        for (int j = 0; j < P; ++j) h[j] = {0.0, 0.0};
+#pragma unroll 1
+        for (int pass = 0;; ++pass) {
+            bwd_pass<TF, P, STAGED>(c, Tb, off, sL, rows, pass ? rows : scrap, pass ? B::RB : 0, h, Tb0);
+            if (pass) break;
+            if constexpr (STAGED) {
+#pragma unroll
+                for (int j = 0; j < P; ++j) sE[j * kSt + ln] = lc(h[j]);
+                for (int k = 0; k < PK; ++k) __syncthreads();
+                const lcplx* s = carried<P>(sE, sz, PK) + neighbour(ln, n, 1);
+#pragma unroll
+                for (int j = 0; j < P; ++j) h[j] = s[j * kSt];
+            } else {
+                TF t[P][P];
+                const TF* Tq = TR;
+                asm volatile("" : "+s"(Tq));  // loaded here: kept from the forward carry it would fill the registers
+#pragma unroll
+                for (int r = 0; r < P; ++r)
+#pragma unroll
+                    for (int q = 0; q < P; ++q) t[r][q] = trf_at<TF, P>(Tq, toff, 1, r, q);
+                carry1<TF, P>(t, sE, ln, n, 1, PK, h);
+            }
         }
     } else {
-        const cplx* v = src + (int64_t)ch * N + r0;
-        cplx vr[KV];
+        constexpr int HT = kLane * kHelp, NR = kPM * kLane;  // helper threads, rows
+        constexpr int KH = (NR + HT - 1) / HT;               // rows per thread
+        const int ht = tid - kLane, hw = w - 1;
+        TF t[trf_rows(P)][P];
+        if constexpr (FUSE) {
+            using Row = std::conditional_t<ROLE == RHS_CBAND, CBandRow<P>, SBandRow<ROLE, P>>;
+            constexpr int KZ = (S::NZ + HT - 1) / HT;
+            const cplx* zc = src + (int64_t)ch * N;
+            const int zlo = r0 - P;
+            cplx zr[KZ];
 #pragma unroll
-        for (int k = 0; k < KV; ++k) vr[k] = cj_if(cj, v[min(tid + k * NTH, nv - 1)]);
+            for (int k = 0; k < KZ; ++k) zr[k] = cj_if(cj, zc[min(max(zlo + ht + k * HT, 0), N - 1)]);
+            // (two matrix rows beside two band rows would not fit the registers)
+            if constexpr (trf_rows(P) == 1) carry_load<TF, P>(t, TR, toff, 0, hw);
+            auto row_at = [&](int k) { return min(r0 + min(ht + k * HT, NR - 1), N - 1); };
+            auto band = [&](Row& b, int k) {
+                if constexpr (ROLE == RHS_CBAND) b.load(ra.cband + (int64_t)tabid * (P + 1) * N, row_at(k), N);
+                else b.load(ra, row_at(k), N);
+            };
+            // staged row i is channel row r0 + i, its z_{r0+i+d} sits at
+            // sz[i + P + d]; a conjugate channel forms its table's
+            // right-hand side (scalar -e)
+            const double e0 = ROLE == RHS_SX_SYM || ROLE == RHS_SX_ASY ? ra.eig[ch] * ra.ifdt : 0.0;
+            const double e = cj ? -e0 : e0;
+            auto form = [&](const Row& b, int k) {
+                const int i = min(ht + k * HT, NR - 1);  // (a row past the last repeats the last)
+                cplx zl[P], zu[P + 1], v;
 #pragma unroll
-        for (int k = 0; k < KV; ++k) {
-            const int i = tid + k * NTH;
-            if (i < nrow) sv[sv_slot(i % kPM, i / kPM, NT)] = i < nv ? vr[k] : cplx{0.0, 0.0};
-        }
-    }
-    const TF* TR = trf + (int64_t)tabid * geo.trf_elems;
-    __syncthreads();
-    if constexpr (FUSE) {
-        // v rows of the staged partitions from z in LDS: staged row i is
-        // channel row r0 + i, its z_{r0+i+d} sits at sz[i + P + d]
-        // a conjugate channel forms its table's right-hand side (scalar -e)
-        const double e0 = ROLE == RHS_SX_SYM || ROLE == RHS_SX_ASY ? ra.eig[ch] * ra.ifdt : 0.0;
-        const double e = cj ? -e0 : e0;
+                for (int j = 1; j <= P; ++j) zl[j - 1] = sz[i + P - j];
 #pragma unroll
-        for (int k = 0; k < KV; ++k) {
-            const int i = tid + k * NTH;
-            const int row = min((int)r0 + i, N - 1);  // rows from N on are padding: v = 0
-            cplx zl[P], zu[P + 1];
+                for (int q = 0; q <= P; ++q) zu[q] = sz[i + P + q];
+                if constexpr (ROLE == RHS_CBAND) v = b.apply(zl, zu, row_at(k));
+                else v = b.apply(zl, zu, e);
+                // rows from N on are padding: v = 0
+                if (i < nrow) sv[row_slot(i % kPM, i / kPM)] = lc(i < nv ? v : cplx{0.0, 0.0});
+            };
+            // band entries a row ahead of the products
+            Row b0, b1;
+            band(b0, 0);
 #pragma unroll
-            for (int j = 1; j <= P; ++j) zl[j - 1] = sz[i + P - j];
-#pragma unroll
-            for (int q = 0; q <= P; ++q) zu[q] = sz[i + P + q];
-            cplx vv;
-            if constexpr (ROLE == RHS_CBAND) {
-                CBandRow<P> b;
-                b.load(ra.cband + (int64_t)tabid * (P + 1) * N, row, N);
-                vv = b.apply(zl, zu, row);
-            } else {
-                SBandRow<ROLE, P> b;
-                b.load(ra, row, N);
-                vv = b.apply(zl, zu, e);
+            for (int k = 0; k < KZ; ++k) {
+                const int j = ht + k * HT, row = zlo + j;
+                if (j < S::NZ) sz[j] = lc(row >= 0 && row < N ? zr[k] : cplx{0.0, 0.0});
             }
-            if (i < nrow) sv[sv_slot(i % kPM, i / kPM, NT)] = i < nv ? vv : cplx{0.0, 0.0};
+            __syncthreads();
+#pragma unroll 1
+            for (int k = 0; k < KH; k += 2) {
+                band(b1, k + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                form(b0, k);
+                band(b0, min(k + 2, KH - 1));
+                __builtin_amdgcn_sched_barrier(0);
+                form(b1, k + 1);
+            }
+            if constexpr (trf_rows(P) > 1) carry_load<TF, P>(t, TR, toff, 0, hw);
+        } else {
+            const cplx* vi = src + (int64_t)ch * N + r0;
+            cplx vr[KH];
+#pragma unroll
+            for (int k = 0; k < KH; ++k) vr[k] = cj_if(cj, vi[min(ht + k * HT, nv - 1)]);
+            carry_load<TF, P>(t, TR, toff, 0, hw);
+#pragma unroll
+            for (int k = 0; k < KH; ++k) {
+                const int i = ht + k * HT;
+                if (i < nrow) sv[row_slot(i % kPM, i / kPM)] = lc(i < nv ? vr[k] : cplx{0.0, 0.0});
+            }
         }
-        __syncthreads();
-    }
-    const TrfAt<TF, LDS_T, P> Tf{LDS_T ? &sT[0][0] : TR, NT, ga};
-    const TrfAt<TF, LDS_T, P> Tb{LDS_T ? &sT[TWO ? 1 : 0][0] : TR + (int64_t)KT * kLane, NT, ga};
-
-    // forward pass A on every staged partition (wave 0).  Meanwhile the
-    // other waves fetch the staged partitions' transfer sets, which the
-    // carries read only after the next barrier.
-    if constexpr (LDS_T) stage_trf<TF, P, 0, TWO ? 2 * KT : KT>(TR, &sT[0][0], tid, ga, gb);
-    cplx h[P];
-    if (run) {
-#pragma unroll
-        for (int j = 0; j < P; ++j) h[j] = {0.0, 0.0};
-        if constexpr (SYM) fwd_pass_gs<false, P>(Tg, Tp, sv, NT, tid, h);
-        else fwd_pass<false, P>(Tg, sv, NT, tid, h);
-#pragma unroll
-        for (int j = 0; j < P; ++j) sE[j * NT + tid] = h[j];
-    }
-    __syncthreads();
-
-    // forward carry and pass B on the owned partitions and the trailing halo
-    const bool fw = run && g >= k0;
-    if constexpr (LDS_T) {
-        // every wave takes part in the carry; lane ln serves partition ga + ln
-        const int gl = ga + ln;
-        const int cur = carry4<TF, P>(Tf, sE, sA, NT, gl, 0, NP, ga, PK, w, ln, gl < gb && gl >= k0);
-        if (fw) {
-#pragma unroll
-            for (int j = 0; j < P; ++j) h[j] = sA[(cur * P + j) * NT + tid];
+        __syncthreads();  // v in LDS
+#pragma unroll 1
+        for (int dir = 0;; ++dir) {
+            __syncthreads();  // end states
+            carry8<TF, P>(t, sE, sz, ln, n, dir, PK, hw);
+            if (dir) break;
+            carry_load<TF, P>(t, TR, toff, 1, hw);
         }
-    } else if (fw) {
-        carry<TF, LDS_T, P>(Tf, sE, NT, g, 0, NP, ga, PK, h);
-    }
-    if (fw) {
-        if constexpr (SYM) fwd_pass_gs<true, P>(Tg, Tp, sv, NT, tid, h);
-        else fwd_pass<true, P>(Tg, sv, NT, tid, h);
-    }
-    __syncthreads();
-
-    // backward pass A on the same partitions; the backward transfer sets
-    // replace the forward ones now when both do not fit at once
-    if constexpr (LDS_T && !TWO) stage_trf<TF, P, KT, KT>(TR, &sT[0][0], tid, ga, gb);
-    if (fw) {
-#pragma unroll
-        for (int j = 0; j < P; ++j) h[j] = {0.0, 0.0};
-        if constexpr (SYM) bwd_pass_sym<false, P>(Tg, sv, NT, tid, h);
-        else bwd_pass<false, P>(Tg, sv, NT, tid, h);
-#pragma unroll
-        for (int j = 0; j < P; ++j) sE[j * NT + tid] = h[j];
-    }
-    __syncthreads();
-
-    // backward carry and pass B on the owned partitions
-    const bool bw = fw && g < k1;
-    if constexpr (LDS_T) {
-        const int gl = ga + ln;
-        const int cur = carry4<TF, P>(Tb, sE, sA, NT, gl, 1, NP, ga, PK, w, ln, gl < gb && gl >= k0 && gl < k1);
-        if (bw) {
-#pragma unroll
-            for (int j = 0; j < P; ++j) h[j] = sA[(cur * P + j) * NT + tid];
-        }
-    } else if (bw) {
-        carry<TF, LDS_T, P>(Tb, sE, NT, g, 1, NP, ga, PK, h);
-    }
-    if (bw) {
-        if constexpr (SYM) bwd_pass_sym<true, P>(Tg, sv, NT, tid, h);
-        else bwd_pass<true, P>(Tg, sv, NT, tid, h);
     }
     __syncthreads();
     const int i0 = (k0 - ga) * kPM, i1 = min((k1 - ga) * kPM, nv);
-#pragma unroll
-    for (int k = 0; k < KV; ++k) {
-        const int i = tid + k * NTH;
-        if (i >= i0 && i < i1) xo[i] = cj_if(cj, sv[sv_slot(i % kPM, i / kPM, NT)]);
-    }
+    cplx* xo = zout + (int64_t)ch * N + r0;
+#pragma unroll 6
+    for (int i = i0 + tid; i < i1; i += NTH) xo[i] = cj_if(cj, sv[row_slot(i % kPM, i / kPM)]);
 }
 
 // Sequential solve x = U^-1 L^-1 v over all N rows, one lane per channel:
@@ -739,273 +780,117 @@ __global__ __launch_bounds__(kLane * (LDS_T ? kStageWaves : 1)) void k_bsolve(
 // operator the tables hold).  Table rows are fetched in blocks of RB rows,
 // every load of a block issued before its first use; zout holds y between
 // the two passes.
-template <int P>
-__global__ __launch_bounds__(64) void k_seqsolve_c(const cplx* __restrict__ tab, TabMap tm,
-                                                   const cplx* __restrict__ vin, cplx* __restrict__ zout, Geom geo,
-                                                   int nch) {
-    constexpr int R = P + 1, RB = 6;
+template <class TF, int P>
+__global__ __launch_bounds__(64) void k_seqsolve(const cplx* __restrict__ tab, TabMap tm, const cplx* __restrict__ vin,
+                                                 cplx* __restrict__ zout, Geom geo, int nch) {
+    using F = TabFmt<TF, P>;
+    constexpr int RB = 6;
     const int ch = blockIdx.x * 64 + threadIdx.x;
     if (ch >= nch) return;
     const int N = geo.N;
-    const cplx* T0 = tab + (int64_t)table_of(tm, ch) * geo.ctab_elems;
+    const cplx* T0 = tab + (int64_t)table_of(tm, ch) * F::units(geo);
     const bool cj = conj_of(tm, ch);
     const cplx* v = vin + (int64_t)ch * N;
     cplx* x = zout + (int64_t)ch * N;
-    SymRing<P> ring;
-    ring.clear();
     cplx h[P];
 #pragma unroll
     for (int j = 0; j < P; ++j) h[j] = {0.0, 0.0};
     for (int i0 = 0; i0 < N; i0 += RB) {
-        cplx c[RB][R], vr[RB];
+        cplx c[RB][F::UF], vr[RB];
 #pragma unroll
         for (int b = 0; b < RB; ++b) {
             const int i = min(i0 + b, N - 1);
-            const cplx* Tq = T0 + part_col<cplx, P>(i / kPM) + (int64_t)(i % kPM) * R * kLane;
-#pragma unroll
-            for (int q = 0; q < R; ++q) c[b][q] = Tq[(int64_t)q * kLane];
+            row_g<TF, P, F::UF>(c[b], T0, part_off<TF, P>(i / kPM), i % kPM);
             vr[b] = cj_if(cj, v[i]);
         }
 #pragma unroll
-        for (int b = 0; b < RB; ++b) {
-            if (i0 + b < N) {
-                cplx acc = vr[b];
-#pragma unroll
-                for (int j = 0; j < P; ++j) acc = tmsub(acc, ring.r[j][j], h[j]);
-#pragma unroll
-                for (int j = P - 1; j > 0; --j) h[j] = h[j - 1];
-                h[0] = acc;
-                x[i0 + b] = c[b][P] * acc;
-                ring.push(c[b]);
-            }
-        }
+        for (int b = 0; b < RB; ++b)
+            if (i0 + b < N) x[i0 + b] = fwd_row<TF, P>(c[b], vr[b], h);
     }
 #pragma unroll
     for (int j = 0; j < P; ++j) h[j] = {0.0, 0.0};
     for (int i1 = N - 1; i1 >= 0; i1 -= RB) {
-        cplx c[RB][P], yr[RB];
+        cplx c[RB][F::UF], yr[RB];
 #pragma unroll
         for (int b = 0; b < RB; ++b) {
             const int i = max(i1 - b, 0);
-            const cplx* Tq = T0 + part_col<cplx, P>(i / kPM) + (int64_t)(i % kPM) * R * kLane;
-#pragma unroll
-            for (int q = 0; q < P; ++q) c[b][q] = Tq[(int64_t)q * kLane];
+            row_g<TF, P, F::UF>(c[b], T0 + F::boff * kLane, part_off<TF, P>(i / kPM), i % kPM);
             yr[b] = x[i];
         }
 #pragma unroll
-        for (int b = 0; b < RB; ++b) {
-            if (i1 - b >= 0) {
-                cplx xv = yr[b];
-#pragma unroll
-                for (int k = 0; k < P; ++k) xv = tmsub(xv, c[b][k], h[k]);
-#pragma unroll
-                for (int k = P - 1; k > 0; --k) h[k] = h[k - 1];
-                h[0] = xv;
-                x[i1 - b] = cj_if(cj, xv);
-            }
-        }
-    }
-}
-
-template <int P>
-__global__ __launch_bounds__(64) void k_seqsolve_r(const double* __restrict__ tab, TabMap tm,
-                                                   const cplx* __restrict__ vin, cplx* __restrict__ zout, Geom geo,
-                                                   int nch) {
-    constexpr int R = 2 * (P + 1), RB = 6;
-    const int ch = blockIdx.x * 64 + threadIdx.x;
-    if (ch >= nch) return;
-    const int N = geo.N;
-    const double* T0 = tab + (int64_t)table_of(tm, ch) * geo.tab_elems;
-    const bool cj = conj_of(tm, ch);  // tables shared by conjugation are complex only: false here
-    const cplx* v = vin + (int64_t)ch * N;
-    cplx* x = zout + (int64_t)ch * N;
-    cplx h[P];
-#pragma unroll
-    for (int j = 0; j < P; ++j) h[j] = {0.0, 0.0};
-    for (int i0 = 0; i0 < N; i0 += RB) {
-        double c[RB][P + 1];
-        cplx vr[RB];
-#pragma unroll
-        for (int b = 0; b < RB; ++b) {
-            const int i = min(i0 + b, N - 1);
-            const double* Tq = T0 + part_col<double, P>(i / kPM) + (int64_t)(i % kPM) * R * kLane;
-#pragma unroll
-            for (int q = 0; q <= P; ++q) c[b][q] = Tq[(int64_t)q * kLane];
-            vr[b] = cj_if(cj, v[i]);
-        }
-#pragma unroll
-        for (int b = 0; b < RB; ++b) {
-            if (i0 + b < N) {
-                cplx acc = vr[b];
-#pragma unroll
-                for (int j = 0; j < P; ++j) acc -= tmul(c[b][j], h[j]);
-                const cplx y = tmul(c[b][P], acc);
-#pragma unroll
-                for (int j = P - 1; j > 0; --j) h[j] = h[j - 1];
-                h[0] = y;
-                x[i0 + b] = y;
-            }
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < P; ++j) h[j] = {0.0, 0.0};
-    for (int i1 = N - 1; i1 >= 0; i1 -= RB) {
-        double c[RB][P + 1];
-        cplx yr[RB];
-#pragma unroll
-        for (int b = 0; b < RB; ++b) {
-            const int i = max(i1 - b, 0);
-            const double* Tq = T0 + part_col<double, P>(i / kPM) + (int64_t)(i % kPM) * R * kLane;
-#pragma unroll
-            for (int q = 0; q <= P; ++q) c[b][q] = Tq[(int64_t)(P + 1 + q) * kLane];
-            yr[b] = x[i];
-        }
-#pragma unroll
-        for (int b = 0; b < RB; ++b) {
-            if (i1 - b >= 0) {
-                cplx xv = tmul(c[b][P], yr[b]);
-#pragma unroll
-                for (int k = 0; k < P; ++k) xv -= tmul(c[b][k], h[k]);
-#pragma unroll
-                for (int k = P - 1; k > 0; --k) h[k] = h[k - 1];
-                h[0] = xv;
-                x[i1 - b] = cj_if(cj, xv);
-            }
-        }
+        for (int b = 0; b < RB; ++b)
+            if (i1 - b >= 0) x[i1 - b] = cj_if(cj, bwd_row<TF, P>(c[b], yr[b], h));
     }
 }
 
 // ---------------------------------------------------------------------------
-// transfer sets of real LU tables: one lane per (table, partition); the
-// P unit responses of each direction are propagated together so every
-// table row is read once
-template <int P>
-__global__ __launch_bounds__(kLane) void k_transfer(const double* __restrict__ tab, double* __restrict__ trf,
-                                                    Geom geo) {
-    constexpr int R = TabFmt<double, P>::row, KT = trf_n<P>();
-    const int g = blockIdx.y * kLane + threadIdx.x;
-    const int t = blockIdx.x;
-    if (g >= geo.P) return;
-    const double* Tg = tab + (int64_t)t * geo.tab_elems + part_col<double, P>(g);
-    double* out = trf + (int64_t)t * geo.trf_elems + (int64_t)((g >> 6) * 2) * KT * kLane + (g & 63);
-    for (int dir = 0; dir < 2; ++dir) {
-        double H[P][P];  // H[q][col]: state entry q of the response to unit vector col
-#pragma unroll
-        for (int q = 0; q < P; ++q)
-#pragma unroll
-            for (int col = 0; col < P; ++col) H[q][col] = q == col ? 1.0 : 0.0;
-        for (int ss = 0; ss < kPM; ++ss) {
-            const int s = dir == 0 ? ss : kPM - 1 - ss;
-            const double* c = Tg + (int64_t)(s * R + (dir == 0 ? 0 : P + 1)) * kLane;
-            double f[P + 1];
-#pragma unroll
-            for (int q = 0; q <= P; ++q) f[q] = c[(int64_t)q * kLane];
-            double y[P];
-#pragma unroll
-            for (int col = 0; col < P; ++col) {
-                double acc = 0.0;
-#pragma unroll
-                for (int q = 0; q < P; ++q) acc = acc - f[q] * H[q][col];
-                y[col] = dir == 0 ? f[P] * acc : acc;
-            }
-#pragma unroll
-            for (int q = P - 1; q > 0; --q)
-#pragma unroll
-                for (int col = 0; col < P; ++col) H[q][col] = H[q - 1][col];
-#pragma unroll
-            for (int col = 0; col < P; ++col) H[0][col] = y[col];
-        }
-        double* o = out + (int64_t)dir * KT * kLane;
-#pragma unroll
-        for (int q = 0; q < P; ++q)
-#pragma unroll
-            for (int col = 0; col < P; ++col) o[(int64_t)(q * P + col) * kLane] = H[q][col];
-    }
-}
+// Transfer matrices: one lane per (table, partition), the unit responses of
+// the state through the partition's rows, NC at a time (as many as the
+// registers hold beside the rows), the groups of columns - and, of real LU
+// tables, the two directions - in work-groups of their own.  A symmetric
+// table's backward matrix is the transpose of the forward one and is not
+// stored.  Rows are loaded in blocks of RB ahead of their products.
+template <class TF, int P>
+constexpr int trf_cols() { return TabFmt<TF, P>::SYM ? 4 : P; }
+template <class TF, int P>
+constexpr int trf_groups() { return TabFmt<TF, P>::SYM ? (P + trf_cols<TF, P>() - 1) / trf_cols<TF, P>() : 2; }
 
-// transfer sets of complex symmetric tables (the z recurrence forward, the x
-// recurrence backward); the forward responses start from the coefficients of
-// the previous partition's last rows, as the solve's pass B does.  The P unit
-// responses are propagated NC at a time (P = 8: two sweeps of 4, which keeps
-// the responses in registers), each sweep reading the partition's rows.
-template <int P>
-__global__ __launch_bounds__(kLane) void k_transfer_sym(const cplx* __restrict__ tab, cplx* __restrict__ trf,
-                                                        Geom geo, int64_t stride) {
-    constexpr int R = P + 1, KT = trf_n<P>();
-    constexpr int NC = P == 7 ? 7 : 4;
-    static_assert(P % NC == 0, "whole column groups");
-    const int g = blockIdx.y * kLane + threadIdx.x;
+__device__ inline double tsub(double a, double t, double x) { return fma(-t, x, a); }
+__device__ inline cplx tsub(cplx a, cplx t, cplx x) { return tmsub(a, t, x); }
+
+template <class TF, int P>
+__global__ __launch_bounds__(kLane) void k_transfer(const cplx* __restrict__ tab, TF* __restrict__ trf, Geom geo,
+                                                    int64_t stride) {
+    using F = TabFmt<TF, P>;
+    constexpr int NC = trf_cols<TF, P>(), RB = 4;
+    const int grp = blockIdx.y % trf_groups<TF, P>();
+    const int g = blockIdx.y / trf_groups<TF, P>() * kLane + threadIdx.x;
     const int64_t t = (int64_t)blockIdx.z * stride + blockIdx.x;  // table index
     if (g >= geo.P) return;
-    const cplx* T0 = tab + t * geo.ctab_elems;
-    const cplx* Tg = T0 + part_col<cplx, P>(g);
-    cplx* out = trf + (int64_t)t * geo.trf_elems + (int64_t)((g >> 6) * 2) * KT * kLane + (g & 63);
+    const int dir = F::SYM ? 0 : grp, c0 = F::SYM ? grp * NC : 0;
+    const cplx* T0 = tab + t * F::units(geo) + (dir ? F::boff * kLane : 0);
+    const unsigned off = part_off<TF, P>(g);
+    TF* out = trf + t * F::trf_elems(geo) + (int64_t)(g >> 6) * (F::SYM ? 1 : 2) * P * P * kLane +
+              (int64_t)dir * P * P * kLane + (g & 63);
+    TF H[P][NC];  // H[q][c]: state entry q of the response to unit vector c0 + c
+#pragma unroll
+    for (int q = 0; q < P; ++q)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) H[q][c] = q == c0 + c ? tone(TF{}) : tzero(TF{});
 #pragma unroll 1
-    for (int c0 = 0; c0 < P; c0 += NC) {
-        cplx H[P][NC];  // H[q][c]: state entry q of the response to unit vector c0 + c
-        // forward
+    for (int s0 = 0; s0 < kPM; s0 += RB) {
+        cplx e[RB][F::UF];
 #pragma unroll
-        for (int q = 0; q < P; ++q)
+        for (int b = 0; b < RB; ++b) row_g<TF, P, F::SYM ? P : F::UF>(e[b], T0, off, dir ? kPM - 1 - s0 - b : s0 + b);
 #pragma unroll
-            for (int c = 0; c < NC; ++c) H[q][c] = q == c0 + c ? cplx{1.0, 0.0} : cplx{0.0, 0.0};
-        SymRing<P> ring;
-        if (g > 0) ring.load_tail(T0 + part_col<cplx, P>(g - 1));
-        else ring.clear();
-        for (int s = 0; s < kPM; ++s) {
-            cplx e[R];
+        for (int b = 0; b < RB; ++b) {
+            if (!F::SYM && dir) {
 #pragma unroll
-            for (int q = 0; q < R; ++q) e[q] = Tg[(int64_t)(s * R + q) * kLane];
-            cplx y[NC];
+                for (int c = 0; c < NC; ++c) {
+                    TF x = tzero(TF{});
 #pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                cplx acc = {0.0, 0.0};
+                    for (int k = P; k >= 1; --k) x = tsub(x, F::coef(e[b], k), H[k - 1][c]);
 #pragma unroll
-                for (int q = 0; q < P; ++q) acc = acc - ring.r[q][q] * H[q][c];
-                y[c] = acc;
+                    for (int q = P - 1; q > 0; --q) H[q][c] = H[q - 1][c];
+                    H[0][c] = x;
+                }
+            } else {
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    TF y = H[0][c];
+                    if constexpr (!F::SYM) y = F::diag(e[b]) * y;
+#pragma unroll
+                    for (int k = 1; k < P; ++k) H[k - 1][c] = tsub(H[k][c], F::coef(e[b], k), y);
+                    H[P - 1][c] = tsub(tzero(TF{}), F::coef(e[b], P), y);
+                }
             }
-#pragma unroll
-            for (int q = P - 1; q > 0; --q)
-#pragma unroll
-                for (int c = 0; c < NC; ++c) H[q][c] = H[q - 1][c];
-#pragma unroll
-            for (int c = 0; c < NC; ++c) H[0][c] = y[c];
-            ring.push(e);
         }
-#pragma unroll
-        for (int q = 0; q < P; ++q)
-#pragma unroll
-            for (int c = 0; c < NC; ++c) out[(int64_t)(q * P + c0 + c) * kLane] = H[q][c];
-        // backward
-#pragma unroll
-        for (int q = 0; q < P; ++q)
-#pragma unroll
-            for (int c = 0; c < NC; ++c) H[q][c] = q == c0 + c ? cplx{1.0, 0.0} : cplx{0.0, 0.0};
-        for (int ss = 0; ss < kPM; ++ss) {
-            const int s = kPM - 1 - ss;
-            cplx e[P];
-#pragma unroll
-            for (int q = 0; q < P; ++q) e[q] = Tg[(int64_t)(s * R + q) * kLane];
-            cplx y[NC];
-#pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                cplx acc = {0.0, 0.0};
-#pragma unroll
-                for (int q = 0; q < P; ++q) acc = acc - e[q] * H[q][c];
-                y[c] = acc;
-            }
-#pragma unroll
-            for (int q = P - 1; q > 0; --q)
-#pragma unroll
-                for (int c = 0; c < NC; ++c) H[q][c] = H[q - 1][c];
-#pragma unroll
-            for (int c = 0; c < NC; ++c) H[0][c] = y[c];
-        }
-        cplx* o = out + (int64_t)KT * kLane;
-#pragma unroll
-        for (int q = 0; q < P; ++q)
-#pragma unroll
-            for (int c = 0; c < NC; ++c) o[(int64_t)(q * P + c0 + c) * kLane] = H[q][c];
     }
+#pragma unroll
+    for (int q = 0; q < P; ++q)
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+            if (c0 + c < P) out[(int64_t)(q * P + c0 + c) * kLane] = H[q][c];
 }
 
 // ---------------------------------------------------------------------------
@@ -1039,31 +924,29 @@ __global__ __launch_bounds__(kLane) void k_tab_ldlt(const cplx* __restrict__ low
 
 // tables from chol(S) (ed.h:182-194): c[i*ne+j] = L(i+j,i)
 template <int P>
-__global__ __launch_bounds__(kLane) void k_tab_chol(const double* __restrict__ c, double* __restrict__ tab, Geom geo) {
-    constexpr int R = TabFmt<double, P>::row, ne = P + 1;
+__global__ __launch_bounds__(kLane) void k_tab_chol(const double* __restrict__ c, cplx* __restrict__ tab, Geom geo) {
+    using F = TabFmt<double, P>;
+    constexpr int ne = P + 1;
     const int g = blockIdx.x * kLane + threadIdx.x;
     if (g >= geo.P) return;
     const int N = geo.N;
-    double* Tg = tab + part_col<double, P>(g);
+    cplx* Tg = tab + part_col<double, P>(g);
     for (int s = 0; s < kPM; ++s) {
         const int i = g * kPM + s;
-        double o[R];
-        if (i >= N) {
+        double f[P], b[P], d = 1.0;  // identity padding rows
 #pragma unroll
-            for (int q = 0; q < R; ++q) o[q] = 0.0;
-            o[P] = 1.0;
-            o[R - 1] = 1.0;
-        } else {
-            const double d = 1.0 / c[(int64_t)i * ne];
+        for (int k = 0; k < P; ++k) f[k] = b[k] = 0.0;
+        if (i < N) {
+            d = 1.0 / c[(int64_t)i * ne];
 #pragma unroll
-            for (int j = 1; j <= P; ++j) o[j - 1] = i - j >= 0 ? c[(int64_t)(i - j) * ne + j] : 0.0;
-            o[P] = d;
-#pragma unroll
-            for (int k = 1; k <= P; ++k) o[P + k] = i + k < N ? c[(int64_t)i * ne + k] * d : 0.0;
-            o[R - 1] = d;
+            for (int k = 1; k <= P; ++k)
+                if (i + k < N) {
+                    f[k - 1] = c[(int64_t)i * ne + k];
+                    b[k - 1] = f[k - 1] * d;
+                }
         }
-#pragma unroll
-        for (int q = 0; q < R; ++q) Tg[(int64_t)(s * R + q) * kLane] = o[q];
+        put_real<P>(Tg + (int64_t)s * F::row * kLane, f, d);
+        put_real<P>(Tg + (int64_t)(s * F::row + F::boff) * kLane, b, d);
     }
 }
 
@@ -1128,8 +1011,7 @@ __device__ inline double fsubx(double a, double t, double x) { return fma(-t, x,
 template <int SYM, int P>
 __global__ __launch_bounds__(kLane, P == 7 ? 2 : 1) void k_factor(const cplx* __restrict__ fx, const double* __restrict__ eig,
                                                   int64_t eig_tstride, const double* __restrict__ ifdt, Geom geo,
-                                                  int restart, typename FactorTypes<SYM>::T* __restrict__ tab,
-                                                  int64_t tstride) {
+                                                  int restart, cplx* __restrict__ tab, int64_t tstride) {
     using T = typename FactorTypes<SYM>::T;
     constexpr int NE = P + 1;
     // slots: a divisor of kPM, so that the rounds of rows end with the partition
@@ -1142,9 +1024,9 @@ __global__ __launch_bounds__(kLane, P == 7 ? 2 : 1) void k_factor(const cplx* __
     const double e = eig[(int64_t)t * eig_tstride + ch] * ifdt[t];
     // SYM 0 writes complex symmetric rows [E_1..E_P, 1/pivot] (for a symmetric
     // matrix the unit upper factor's rows are the columns of L in A = L D L^T);
-    // SYM 1 writes real LU rows
+    // SYM 1 writes real LU rows (forward: the multipliers of the rows below, backward: u)
     constexpr int ROW = TabFmt<T, P>::row;
-    T* Tg = tab + ((int64_t)t * tstride + ch) * TabFmt<T, P>::elems(geo) + part_col<T, P>(g);
+    cplx* Tg = tab + ((int64_t)t * tstride + ch) * TabFmt<T, P>::units(geo) + part_col<T, P>(g);
     const int r0 = g * kPM;
     // whole rounds of RS rows above the partition (r0 is a multiple of RS too)
     const int above = (restart + RS - 1) / RS * RS;
@@ -1202,19 +1084,14 @@ __global__ __launch_bounds__(kLane, P == 7 ? 2 : 1) void k_factor(const cplx* __
 #pragma unroll
             for (int k = 1; k < NE; ++k) u[k] = fmulx(wu[s][k], rp);
             if constexpr (decltype(store)::value) {
-                T* o = Tg + (int64_t)(i + s - r0) * ROW * kLane;
+                cplx* o = Tg + (int64_t)(i + s - r0) * ROW * kLane;
                 if constexpr (SYM == 0) {
 #pragma unroll
                     for (int k = 1; k < NE; ++k) o[(int64_t)(k - 1) * kLane] = u[k];
                     o[(int64_t)P * kLane] = rp;
                 } else {
-                    // multiplier of column i-j: entry j of row i-j, final since step i-j
-#pragma unroll
-                    for (int j = 1; j < NE; ++j) o[(int64_t)(j - 1) * kLane] = wl[(s - j + RS) % RS][j];
-                    o[(int64_t)P * kLane] = rp;
-#pragma unroll
-                    for (int k = 1; k < NE; ++k) o[(int64_t)(P + k) * kLane] = u[k];
-                    o[(int64_t)(ROW - 1) * kLane] = tone(T{});
+                    put_real<P>(o, &wl[s][1], rp);
+                    put_real<P>(o + TabFmt<T, P>::boff * kLane, &u[1], 1.0);
                 }
             }
             // A(i+a, i+b) -= A(i+a, i) u(i, i+b)
@@ -1282,19 +1159,28 @@ void launch_rhs(hipStream_t s, int rhs, const RhsArgs& ra, TabMap tm, const cplx
     else rhs_launch<7>(s, rhs, ra, tm, zin, vout, nch, geo);
 }
 
-// Largest grid whose solves stage the transfer sets in LDS (geo.stage_grid,
-// default kStageGrid), with four waves per work-group and the right-hand side
-// formed in the launch.  One such work-group fits a CU (107-157 KB of LDS),
-// so up to 512 run in at most two rounds over the 256 CUs; larger grids read
-// the transfer sets from L2 and keep several single-wave work-groups per CU
-// (64 batched shots in buckets of 468-720 channels: 7.59e8 coefficient
-// updates/s with 512, 7.01e8 with 1024, 6.81e8 with 4096).
+// Largest grid whose solves run staged (geo.stage_grid, default kStageGrid):
+// eight waves per work-group, part of the table in LDS and the right-hand side
+// formed in the launch.  One such work-group fills a CU (133-156 KB of LDS), so
+// up to 256 run at once and up to 512 in two rounds; larger grids run one wave
+// per work-group, four per CU.  Batched shots, 16 steps, N = 1200, staged
+// against one wave: 240 channels 4.61 / 5.75 ms, 320 channels 6.80 / 6.49,
+// 480 channels 7.92 / 7.96, 640 channels 11.2 / 10.0.
+
+// Partitions per segment: one segment when the channel fits a work-group (no
+// halo to run), else the fewest segments that hold them with their halos,
+// plus geo.seg_add, none empty
+static int seg_parts(const Geom& geo, int pk) {
+    const int smax = seg_max(pk), fewest = (geo.P + smax - 1) / smax;
+    int nseg = (geo.P <= kLane ? 1 : fewest) + std::max(0, geo.seg_add);
+    if (nseg > 1) nseg = std::max(nseg, fewest);
+    nseg = std::min(geo.P, nseg);
+    return (geo.P + nseg - 1) / nseg;
+}
 
 int solve_segments(const Geom& geo, int pk) {
     if (pk > kPKMax) return 0;  // the sequential solve: no segments
-    const int smax = seg_max(pk);
-    const int nseg0 = std::min(geo.P, (geo.P + smax - 1) / smax + std::max(0, geo.seg_add));
-    const int sn = (geo.P + nseg0 - 1) / nseg0;
+    const int sn = seg_parts(geo, pk);
     return (geo.P + sn - 1) / sn;
 }
 
@@ -1313,7 +1199,10 @@ void solve_order(const int* tab, int nch, int nseg, int* order) {
     int j = 0;
     for (int x = 0; x < kXcds; ++x) {
         const int n = base + (x < extra ? 1 : 0);
-        for (int k = 0; k < n; ++k) order[x + kXcds * k] = e[j++];
+        for (int k = 0; k < n; ++k) {
+            const int q = e[j++];
+            order[x + kXcds * k] = (q / nseg) << 8 | q % nseg;
+        }
     }
 }
 
@@ -1327,20 +1216,14 @@ static void bsolve(hipStream_t s, const TF* tab, const TF* trf, TabMap tm, const
             rhs_launch<P>(s, ROLE, *ra, tm, zin, vbuf, nch, geo);
             zin = vbuf;
         }
-        if constexpr (sizeof(TF) == sizeof(cplx))
-            hipLaunchKernelGGL(k_seqsolve_c<P>, dim3((nch + 63) / 64), dim3(64), 0, s, tab, tm, zin, zout, geo, nch);
-        else
-            hipLaunchKernelGGL(k_seqsolve_r<P>, dim3((nch + 63) / 64), dim3(64), 0, s, tab, tm, zin, zout, geo, nch);
+        hipLaunchKernelGGL((k_seqsolve<TF, P>), dim3((nch + 63) / 64), dim3(64), 0, s, (const cplx*)tab, tm, zin, zout,
+                           geo, nch);
         return;
     }
-    const int smax = seg_max(PK);
-    // the fewest segments that hold the partitions, plus geo.seg_add, none empty
-    const int nseg0 = std::min(geo.P, (geo.P + smax - 1) / smax + std::max(0, geo.seg_add));
-    const int sn = (geo.P + nseg0 - 1) / nseg0;  // <= smax, so sn + 2 PK <= 64
+    const int sn = seg_parts(geo, PK);
     const int nseg = (geo.P + sn - 1) / sn;
     if (tm.order && nseg != tm.order_nseg) tm.order = nullptr;  // built for another launch shape
-    // staged grids (geo.stage_grid): transfer sets in LDS, four waves, and the
-    // right-hand side formed in the launch when z and x do not overlap
+    // staged grids form the right-hand side in the launch when z and x do not overlap
     const bool staged = (int64_t)nseg * nch <= geo.stage_grid;
     const dim3 grid(nseg, nch);
     if (ra) {
@@ -1348,19 +1231,19 @@ static void bsolve(hipStream_t s, const TF* tab, const TF* trf, TabMap tm, const
         const uintptr_t a0 = (uintptr_t)zin, b0 = (uintptr_t)zout;
         const uintptr_t len = sizeof(cplx) * (uintptr_t)nch * geo.N;
         if (staged && (a0 + len <= b0 || b0 + len <= a0)) {
-            hipLaunchKernelGGL((k_bsolve<TF, ROLE, true, true, P>), grid, dim3(kLane * kStageWaves), 0, s, tab, trf,
-                               tm, zin, zout, geo, sn, PK, *ra);
+            hipLaunchKernelGGL((k_bsolve<TF, ROLE, true, true, P>), grid, dim3(kLane * kWavesStaged), 0, s,
+                               (const cplx*)tab, trf, tm, zin, zout, geo, sn, PK, *ra);
             return;
         }
         rhs_launch<P>(s, ROLE, *ra, tm, zin, vbuf, nch, geo);
         zin = vbuf;
     }
     if (staged)
-        hipLaunchKernelGGL((k_bsolve<TF, ROLE, true, false, P>), grid, dim3(kLane * kStageWaves), 0, s, tab, trf, tm,
-                           zin, zout, geo, sn, PK, RhsArgs{});
+        hipLaunchKernelGGL((k_bsolve<TF, ROLE, true, false, P>), grid, dim3(kLane * kWavesStaged), 0, s,
+                           (const cplx*)tab, trf, tm, zin, zout, geo, sn, PK, RhsArgs{});
     else
-        hipLaunchKernelGGL((k_bsolve<TF, ROLE, false, false, P>), grid, dim3(kLane), 0, s, tab, trf, tm, zin, zout,
-                           geo, sn, PK, RhsArgs{});
+        hipLaunchKernelGGL((k_bsolve<TF, ROLE, false, false, P>), grid, dim3(kLane), 0, s, (const cplx*)tab, trf, tm,
+                           zin, zout, geo, sn, PK, RhsArgs{});
 }
 
 template <class TF, int ROLE>
@@ -1394,14 +1277,18 @@ void launch_rsolve_r(hipStream_t s, int role, const RhsArgs& ra, const double* t
 void launch_transfer_c(hipStream_t s, const cplx* tab, cplx* trf, int ntab, Geom geo) {
     launch_transfer_c(s, tab, trf, ntab, 1, 0, geo);
 }
+template <class TF, int P>
+static void transfer_launch(hipStream_t s, const void* tab, TF* trf, int per_t, int nt, int64_t stride, Geom geo) {
+    hipLaunchKernelGGL((k_transfer<TF, P>), dim3(per_t, geo.NG * trf_groups<TF, P>(), nt), dim3(kLane), 0, s,
+                       (const cplx*)tab, trf, geo, stride);
+}
 void launch_transfer_c(hipStream_t s, const cplx* tab, cplx* trf, int per_t, int nt, int64_t stride, Geom geo) {
-    const dim3 grid(per_t, geo.NG, nt);
-    if (geo.hw == 8) hipLaunchKernelGGL(k_transfer_sym<8>, grid, dim3(kLane), 0, s, tab, trf, geo, stride);
-    else hipLaunchKernelGGL(k_transfer_sym<7>, grid, dim3(kLane), 0, s, tab, trf, geo, stride);
+    if (geo.hw == 8) transfer_launch<cplx, 8>(s, tab, trf, per_t, nt, stride, geo);
+    else transfer_launch<cplx, 7>(s, tab, trf, per_t, nt, stride, geo);
 }
 void launch_transfer_r(hipStream_t s, const double* tab, double* trf, int ntab, Geom geo) {
-    if (geo.hw == 8) hipLaunchKernelGGL(k_transfer<8>, dim3(ntab, geo.NG), dim3(kLane), 0, s, tab, trf, geo);
-    else hipLaunchKernelGGL(k_transfer<7>, dim3(ntab, geo.NG), dim3(kLane), 0, s, tab, trf, geo);
+    if (geo.hw == 8) transfer_launch<double, 8>(s, tab, trf, ntab, 1, 0, geo);
+    else transfer_launch<double, 7>(s, tab, trf, ntab, 1, 0, geo);
 }
 
 void launch_tab_ldlt(hipStream_t s, const cplx* lower, cplx* tab, int nl, Geom geo) {
@@ -1409,8 +1296,8 @@ void launch_tab_ldlt(hipStream_t s, const cplx* lower, cplx* tab, int nl, Geom g
     else hipLaunchKernelGGL(k_tab_ldlt<7>, dim3(geo.NG, nl), dim3(kLane), 0, s, lower, tab, geo);
 }
 void launch_tab_chol(hipStream_t s, const double* chol, double* tab, Geom geo) {
-    if (geo.hw == 8) hipLaunchKernelGGL(k_tab_chol<8>, dim3(geo.NG), dim3(kLane), 0, s, chol, tab, geo);
-    else hipLaunchKernelGGL(k_tab_chol<7>, dim3(geo.NG), dim3(kLane), 0, s, chol, tab, geo);
+    if (geo.hw == 8) hipLaunchKernelGGL(k_tab_chol<8>, dim3(geo.NG), dim3(kLane), 0, s, chol, (cplx*)tab, geo);
+    else hipLaunchKernelGGL(k_tab_chol<7>, dim3(geo.NG), dim3(kLane), 0, s, chol, (cplx*)tab, geo);
 }
 
 void launch_band_diag_r(hipStream_t s, const double* src, double* dst, int n, int N, int p) {
@@ -1435,7 +1322,7 @@ void launch_factor_bands(hipStream_t s, const double* S, const double* X, cplx* 
 }
 template <int SYM>
 static void factor_launch(hipStream_t s, const cplx* fx, const double* eig, const double* ifdt, int nt, int nch, Geom geo,
-                          typename FactorTypes<SYM>::T* tab, int64_t eig_tstride, int restart, int64_t ts) {
+                          cplx* tab, int64_t eig_tstride, int restart, int64_t ts) {
     const int rs = restart > 0 ? restart : kRestart;
     const dim3 grid(geo.NG, nch, nt);
     if (geo.hw == 8)
@@ -1449,7 +1336,7 @@ void launch_factor_sym(hipStream_t s, const cplx* fx, const double* eig, const d
 }
 void launch_factor_asy(hipStream_t s, const cplx* fx, const double* eig, const double* ifdt, int nt, int nch, Geom geo,
                        double* tab, int64_t eig_tstride, int restart) {
-    factor_launch<1>(s, fx, eig, ifdt, nt, nch, geo, tab, eig_tstride, restart, nch);
+    factor_launch<1>(s, fx, eig, ifdt, nt, nch, geo, (cplx*)tab, eig_tstride, restart, nch);
 }
 
 // ---------------------------------------------------------------------------
