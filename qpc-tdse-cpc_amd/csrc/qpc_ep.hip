@@ -17,168 +17,213 @@
 namespace {
 
 // ---- (m,l)-space rotations on the FP64 matrix cores ---------------------------
-// C (M x Nc doubles, row-major, ldc) = A' B', K terms, one 64 x 64 tile of C
-// per work-group of four waves (each 2 x 2 tiles of v_mfma_f64_16x16x4f64,
-// operand layout as k_rot's), K staged through LDS 8 at a time,
-// double-buffered: the next slice's global loads are in flight while the
-// current one is multiplied, and each k-step's LDS operands are read while
-// the previous k-step's products run.  Small tiles and slices keep many
-// work-groups per CU (the staging, not the matrix cores, sets the pace: the
-// same loop without global loads runs 1.4x faster), and slices that lie
-// wholly inside the operands take a load path with per-thread base pointers
-// and contiguous elements.  A' (M x K):
-//   AM 0: A[(ai + i) * lda + ak + k]            (real, row-major)
-//   AM 1: A[(ak + k) * lda + ai + i]            (real, transposed)
-//   AM 2: k < K0: Re P[(ai + i) * lda + ak + k], k >= K0: Im P[.. + k - K0]   (complex P)
-//   AM 3: k < K0: Re P[(ak + k) * lda + ai + i], k >= K0: -Im P[(ak + k - K0) * lda + ai + i]   (P^H)
-// B' (K x Nc doubles): row k of B for k < K0; for k >= K0 the complex row
-// k - K0 times i ({re, im} -> {-im, re}), so that with AM 2 / 3 and K = 2 K0
-// the product is the complex C = P B (or P^H B) with B, C complex rows
-// (re P B + im P (i B)).  Each sum runs over k in order.
+// C (M x Nc doubles, row-major, ldc) = A' B', one 64 x 64 tile of C per
+// work-group of four waves (each 2 x 2 tiles of v_mfma_f64_16x16x4f64, operand
+// layout as k_rot's).  A' (M x K):
+//   AM 0: A[i * lda + k]            (real, row-major)
+//   AM 1: A[k * lda + i]            (real, transposed)
+//   AM 2: P[i * lda + k]            (complex P)
+//   AM 3: conj(P[k * lda + i])      (P^H)
+// With a complex P the rows of B and C are complex, Nc = twice their length.
+//
+// K is staged through LDS a slice at a time (kGK elements), double-buffered:
+// the next slice's global loads are in flight while the current one is
+// multiplied, and each k-step's LDS operands are read while the previous
+// k-step's products run.  A complex slice brings each element of P and B once
+// and multiplies it four ways: re P B from the staged rows, im P (i B) from
+// the same registers with re and im swapped between neighbouring lanes (a DPP
+// move) and one sign flipped.  What bounds it is the matrix cores, with the
+// staging beside them: 1721 x 1721 complex by 1500 complex columns take 0.60 ms,
+// 59 TFLOP/s of the 73 that a large FP64 product reaches (as 2 K real terms, P
+// and B read twice, 0.79 ms); 651 x 651 by 1000 columns 0.10 ms (0.15).  Rows
+// and columns past the tile's edge repeat the last ones (their products are not
+// stored), so only the last slice is masked.
+//
+// A launch takes up to three products of one B row length (row groups of one
+// operator with their own K ranges): a group of few rows alone leaves the chip
+// idle for as long as its K lasts (41 rows, K = 3321: 0.34 ms).  The first
+// group's tiles start first (the longest sums); both parts are dealt to the
+// XCDs in contiguous runs of tiles, rows fastest, so that an XCD's tiles share
+// the columns of B.
 typedef double v4d __attribute__((ext_vector_type(4)));
-constexpr int kGM = 64, kGN = 64, kGK = 8;  // tile rows, tile columns, K slice
+constexpr int kGM = 64, kGN = 64, kGK = 8;  // tile rows, tile columns, K slice (elements)
+constexpr int kGGroups = 3;
+
+struct GemmGroup {
+    const double* A;
+    const double* B;
+    double* C;
+    int M, K;
+};
+struct GemmArgs {
+    GemmGroup g[kGGroups];
+    int rt[kGGroups];  // row tiles up to and including the group
+    int nct;           // column tiles
+};
+
+// v of the neighbouring lane (l ^ 1), sign flipped where neg is set
+__device__ inline double lane_pair(double v, unsigned neg) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)b, 0xB1, 0xf, 0xf, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), 0xB1, 0xf, 0xf, true) ^ neg;
+    return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
 
 template <int AM>
-__global__ __launch_bounds__(256) void k_gemm(const double* __restrict__ A, int64_t lda, int64_t ai, int64_t ak,
-                                               const double* __restrict__ B, int64_t ldb, double* __restrict__ C,
-                                               int64_t ldc, int M, int Nc, int K, int K0) {
+__global__ __launch_bounds__(256) void k_gemm(GemmArgs ga, int64_t lda, int64_t ldb, int64_t ldc, int Nc) {
+    constexpr bool TRANS = AM == 1 || AM == 3, CPLX = AM >= 2;
+    constexpr int W = CPLX ? 2 : 1;                  // doubles per element
+    constexpr int KS = kGK;
     constexpr int PA = kGM + 4, PB = kGN + 4;
-    constexpr int EA = kGM * kGK / 256, EB = kGK * kGN / 256;  // staged elements per thread
-    static_assert(EB % 2 == 0 && kGK % EA == 0 && kGM % EA == 0 && kGK * (kGN / EB) == 256, "staging map");
-    __shared__ double sA[2][kGK][PA];  // [k][i]
-    __shared__ double sB[2][kGK][PB];  // [k][j]
+    constexpr int EA = kGM * KS / 256;               // A elements per thread
+    constexpr int EB = KS * kGN / 256 / 2;           // pairs of B per thread
+    __shared__ __align__(16) double sA[2][W][KS][PA];  // [re, im][k][i]
+    __shared__ __align__(16) double sB[2][KS][PB];     // [k][j]
     const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
-    const int bm = blockIdx.y * kGM, bn = blockIdx.x * kGN;
+    // this work-group's tile
+    const int n0 = ga.rt[0] * ga.nct, id = blockIdx.x;
+    const int first = id < n0, b = id - (first ? 0 : n0), nt = first ? n0 : gridDim.x - n0;
+    const int x = b & 7, t0 = x * (nt >> 3) + min(x, nt & 7) + (b >> 3);
+    const int rf = first ? 0 : ga.rt[0], nrt = (first ? ga.rt[0] : ga.rt[kGGroups - 1]) - rf;
+    const int ct = t0 / nrt;
+    int rt = rf + t0 - ct * nrt;
+    const int gi = rt < ga.rt[0] ? 0 : rt < ga.rt[1] ? 1 : 2;
+    rt -= gi ? ga.rt[gi - 1] : 0;
+    const double* gA = ga.g[gi].A;
+    const double* gB = ga.g[gi].B;
+    double* C = ga.g[gi].C;
+    const int M = ga.g[gi].M, K = ga.g[gi].K;
+    const int bm = rt * kGM, bn = ct * kGN;
     const int wr = (w >> 1) * 32, wc = (w & 1) * 32;
-    constexpr bool TRANS = AM == 1 || AM == 3;
-    constexpr bool CPLX = AM >= 2;
-    // thread -> staged elements: A row-wise (row r, EA consecutive k) or
-    // column-wise (k, EA consecutive i); B (k, EB consecutive j)
-    constexpr int KPR = kGK / EA;  // threads per A row (row-wise)
-    const int ar = TRANS ? (tid % (kGM / EA)) * EA : tid / KPR;
-    const int akk = TRANS ? tid / (kGM / EA) : (tid % KPR) * EA;
-    constexpr int TPR = kGN / EB;
-    const int bk = tid / TPR, bj = (tid % TPR) * EB;
-    double ra[EA], rb[EB];
-    // load() only issues the global loads (addresses clamped into the
-    // operands, the element's validity and sign kept aside); store() applies
-    // them when it writes LDS after the slice's products, so no load is
-    // waited for before the multiplications that hide it
-    unsigned va = 0, na = 0, vb = 0;  // per A element: in range, negated (-Im P^H); per B pair: in range
-    bool rotb = false;
-    const bool tile_in = bm + kGM <= M && bn + kGN <= Nc;
-    const double* pa = CPLX ? (TRANS ? A + 2 * ((ak + akk) * lda + ai + bm + ar) : A + 2 * ((ai + bm + ar) * lda + ak + akk))
-                            : (TRANS ? A + ((ak + akk) * lda + ai + bm + ar) : A + ((ai + bm + ar) * lda + ak + akk));
-    const double* pb = B + bn + bj;
-    auto load = [&](int k0) {
-        if (tile_in && k0 + kGK <= K && (!CPLX || k0 + kGK <= K0 || k0 >= K0)) {
-            // the whole slice inside the operands (and inside one half of a complex K)
-            const bool imh = CPLX && k0 >= K0;
-            const int kq = imh ? k0 - K0 : k0;
-            va = (1u << EA) - 1;
-            na = (CPLX && TRANS && imh) ? va : 0;
+
+    // thread -> staged elements: A row-wise (row ar, EA consecutive k) or
+    // column-wise (k, EA consecutive i); B (k, EB consecutive pairs)
+    constexpr int TA = TRANS ? kGM / EA : KS / EA;   // threads per k (column-wise) or row (row-wise)
+    const int ar = TRANS ? (tid % TA) * EA : tid / TA;
+    const int ak = TRANS ? tid / TA : (tid % TA) * EA;
+    constexpr int TB = kGN / (2 * EB);
+    const int bk = tid / TB, bj = (tid % TB) * (2 * EB);
+    // offsets of the thread's elements along the clamped dimension
+    int ia[TRANS ? EA : 1], ib[EB];
+    if constexpr (TRANS) {
+#pragma unroll
+        for (int e = 0; e < EA; ++e) ia[e] = W * min(bm + ar + e, M - 1);
+    } else {
+        ia[0] = min(bm + ar, M - 1);
+    }
+#pragma unroll
+    for (int e = 0; e < EB; ++e) ib[e] = min(bn + bj + 2 * e, Nc - 2);  // Nc even: pairs stay whole
+    const double* pa = TRANS ? gA : gA + W * (int64_t)ia[0] * lda;
+    double ra[EA][W], rb[EB][2];
+    auto load = [&](int k0, auto last) {
+        constexpr bool LAST = decltype(last)::value;
+        if constexpr (TRANS) {
+            const double* r = pa + W * (int64_t)(LAST ? min(k0 + ak, K - 1) : k0 + ak) * lda;
+#pragma unroll
+            for (int e = 0; e < EA; ++e)
+#pragma unroll
+                for (int u = 0; u < W; ++u) ra[e][u] = r[ia[e] + u];
+        } else {
 #pragma unroll
             for (int e = 0; e < EA; ++e) {
-                if constexpr (!CPLX) ra[e] = TRANS ? pa[(int64_t)kq * lda + e] : pa[kq + e];
-                else ra[e] = TRANS ? pa[2 * ((int64_t)kq * lda + e) + (imh ? 1 : 0)] : pa[2 * (kq + e) + (imh ? 1 : 0)];
+                const double* r = pa + W * (LAST ? min(k0 + ak + e, K - 1) : k0 + ak + e);
+#pragma unroll
+                for (int u = 0; u < W; ++u) ra[e][u] = r[u];
             }
-            rotb = imh;
-            const double* br = pb + (int64_t)(kq + bk) * ldb;
-            vb = (1u << (EB / 2)) - 1;
-#pragma unroll
-            for (int e = 0; e < EB; ++e) rb[e] = br[e];
-            return;
         }
-        va = na = 0;
+        const double* b = gB + (int64_t)(LAST ? min(k0 + bk, K - 1) : k0 + bk) * ldb;
 #pragma unroll
-        for (int e = 0; e < EA; ++e) {
-            const int i = bm + ar + (TRANS ? e : 0), k = k0 + akk + (TRANS ? 0 : e);
-            const bool ok = i < M && k < K;
-            const int ic = ok ? i : 0, kc = ok ? k : 0;
-            const double* q;
-            if constexpr (!CPLX) {
-                q = TRANS ? A + ((ak + kc) * lda + ai + ic) : A + ((ai + ic) * lda + ak + kc);
-            } else {
-                const bool im = kc >= K0;
-                const int kk = im ? kc - K0 : kc;
-                q = (TRANS ? A + 2 * ((ak + kk) * lda + ai + ic) : A + 2 * ((ai + ic) * lda + ak + kk)) + (im ? 1 : 0);
-                if (im && TRANS) na |= 1u << e;
-            }
-            if (ok) va |= 1u << e;
-            ra[e] = *q;
+        for (int e = 0; e < EB; ++e) {
+            rb[e][0] = b[ib[e]];
+            rb[e][1] = b[ib[e] + 1];
         }
-        const int k = k0 + bk;
-        rotb = k >= K0;
-        const int row = k < K ? (rotb ? k - K0 : k) : 0;
-        const double* br = B + (int64_t)row * ldb;
-        vb = 0;
+        if constexpr (LAST) {
+            // terms past K: both operands zero
 #pragma unroll
-        for (int e = 0; e < EB; e += 2) {
-            const int j = bn + bj + e;
-            const bool v = k < K && j < Nc;  // Nc even: pairs stay whole
-            if (v) vb |= 1u << (e / 2);
-            const double* q = br + (v ? j : 0);
-            rb[e] = q[0];
-            rb[e + 1] = q[1];
+            for (int e = 0; e < EA; ++e)
+                if (k0 + ak + (TRANS ? 0 : e) >= K)
+#pragma unroll
+                    for (int u = 0; u < W; ++u) ra[e][u] = 0.0;
+            if (k0 + bk >= K)
+#pragma unroll
+                for (int e = 0; e < EB; ++e) rb[e][0] = rb[e][1] = 0.0;
         }
     };
     auto store = [&](int buf) {
 #pragma unroll
-        for (int e = 0; e < EA; ++e) {
-            double v = (va >> e) & 1 ? ra[e] : 0.0;
-            if ((na >> e) & 1) v = -v;
-            if (TRANS) sA[buf][akk][ar + e] = v;
-            else sA[buf][akk + e][ar] = v;
-        }
+        for (int e = 0; e < EA; ++e)
 #pragma unroll
-        for (int e = 0; e < EB; e += 2) {
-            const bool v = (vb >> (e / 2)) & 1;
-            const double re = v ? rb[e] : 0.0, im = v ? rb[e + 1] : 0.0;
-            sB[buf][bk][bj + e] = rotb ? -im : re;
-            sB[buf][bk][bj + e + 1] = rotb ? re : im;
+            for (int u = 0; u < W; ++u) {
+                if (TRANS) sA[buf][u][ak][ar + e] = ra[e][u];
+                else sA[buf][u][ak + e][ar] = ra[e][u];
+            }
+#pragma unroll
+        for (int e = 0; e < EB; ++e) {
+            sB[buf][bk][bj + 2 * e] = rb[e][0];
+            sB[buf][bk][bj + 2 * e + 1] = rb[e][1];
         }
     };
+    // im P (i B): column pair {-im, re}; P^H: -im P (i B), {im, -re}
+    const unsigned neg = (AM == 2) == ((l & 1) == 0) ? 0x80000000u : 0u;
     v4d acc[2][2];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int u = 0; u < 2; ++u) acc[t][u] = v4d{0.0, 0.0, 0.0, 0.0};
-    load(0);
-    store(0);
+    struct Ops {
+        double a[W][2], b[2];
+    };
+    auto ops = [&](Ops& o, int buf, int ks) {
+        const int k = ks * 4 + (l >> 4);
+#pragma unroll
+        for (int u = 0; u < W; ++u)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) o.a[u][t] = sA[buf][u][k][wr + t * 16 + (l & 15)];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) o.b[u] = sB[buf][k][wc + u * 16 + (l & 15)];
+    };
+    auto mul = [&](const Ops& o) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+                acc[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a[0][t], o.b[u], acc[t][u], 0, 0, 0);
+        if constexpr (CPLX) {
+            double r[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) r[u] = lane_pair(o.b[u], neg);
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+                    acc[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a[1][t], r[u], acc[t][u], 0, 0, 0);
+        }
+    };
+    const int nfull = K / KS, nsl = (K + KS - 1) / KS;
+    auto fetch = [&](int sl) {
+        if (sl < nfull) load(sl * KS, std::false_type{});
+        else load(sl * KS, std::true_type{});
+    };
+    if (nsl > 0) {
+        fetch(0);
+        store(0);
+    }
     __syncthreads();
-    int buf = 0;
-    for (int k0 = 0; k0 < K; k0 += kGK) {
-        const bool more = k0 + kGK < K;
-        if (more) load(k0 + kGK);
-        double a0[2], b0[2], a1[2], b1[2];
+    for (int sl = 0; sl < nsl; ++sl) {
+        const int buf = sl & 1;
+        const bool more = sl + 1 < nsl;
+        if (more) fetch(sl + 1);
+        Ops o0, o1;
+        ops(o0, buf, 0);
 #pragma unroll
-        for (int t = 0; t < 2; ++t) a0[t] = sA[buf][(l >> 4)][wr + t * 16 + (l & 15)];
-#pragma unroll
-        for (int u = 0; u < 2; ++u) b0[u] = sB[buf][(l >> 4)][wc + u * 16 + (l & 15)];
-#pragma unroll
-        for (int ks = 0; ks < kGK / 4; ks += 2) {
-#pragma unroll
-            for (int t = 0; t < 2; ++t) a1[t] = sA[buf][(ks + 1) * 4 + (l >> 4)][wr + t * 16 + (l & 15)];
-#pragma unroll
-            for (int u = 0; u < 2; ++u) b1[u] = sB[buf][(ks + 1) * 4 + (l >> 4)][wc + u * 16 + (l & 15)];
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int u = 0; u < 2; ++u) acc[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[t], b0[u], acc[t][u], 0, 0, 0);
-            if (ks + 2 < kGK / 4) {
-#pragma unroll
-                for (int t = 0; t < 2; ++t) a0[t] = sA[buf][(ks + 2) * 4 + (l >> 4)][wr + t * 16 + (l & 15)];
-#pragma unroll
-                for (int u = 0; u < 2; ++u) b0[u] = sB[buf][(ks + 2) * 4 + (l >> 4)][wc + u * 16 + (l & 15)];
-            }
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int u = 0; u < 2; ++u) acc[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[t], b1[u], acc[t][u], 0, 0, 0);
+        for (int ks = 0; ks < KS / 4; ks += 2) {
+            ops(o1, buf, ks + 1);
+            mul(o0);
+            if (ks + 2 < KS / 4) ops(o0, buf, ks + 2);
+            mul(o1);
         }
         if (more) store(buf ^ 1);
         __syncthreads();
-        buf ^= 1;
     }
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -194,17 +239,36 @@ __global__ __launch_bounds__(256) void k_gemm(const double* __restrict__ A, int6
         }
 }
 
+// the products of n <= kGGroups row groups in one launch (groups without rows are left out)
 template <int AM>
-int gemm(qpc_ctx* c, const double* A, int64_t lda, int64_t ai, int64_t ak, const double* B, int64_t ldb, double* C,
-         int64_t ldc, int64_t M, int64_t Nc, int64_t K, int64_t K0) {
-    if (M <= 0 || Nc <= 0) return QPC_OK;
-    if (Nc % 2 || M > (1 << 30) || Nc > (1 << 30) || K > (1 << 30)) {
+int gemm(qpc_ctx* c, const GemmGroup* g, int n, int64_t lda, int64_t ldb, int64_t ldc, int64_t Nc) {
+    GemmArgs a{};
+    int m = 0, rt = 0;
+    for (int k = 0; k < n; ++k) {
+        if (g[k].M <= 0) continue;
+        a.g[m] = g[k];
+        rt += (g[k].M + kGM - 1) / kGM;
+        a.rt[m++] = rt;
+    }
+    if (m == 0 || Nc <= 0) return QPC_OK;
+    for (int k = m; k < kGGroups; ++k) a.rt[k] = rt;
+    a.nct = (int)((Nc + kGN - 1) / kGN);
+    if (Nc % 2 || Nc > (1 << 30) || (int64_t)rt * a.nct > (1 << 30)) {
         c->set_error("rotation GEMM shape");
         return QPC_E_SHAPE;
     }
-    hipLaunchKernelGGL((k_gemm<AM>), dim3((unsigned)((Nc + kGN - 1) / kGN), (unsigned)((M + kGM - 1) / kGM)), dim3(256),
-                       0, c->stream, A, lda, ai, ak, B, ldb, C, ldc, (int)M, (int)Nc, (int)K, (int)K0);
+    hipLaunchKernelGGL((k_gemm<AM>), dim3((unsigned)(rt * a.nct)), dim3(256), 0, c->stream, a, lda, ldb, ldc, (int)Nc);
     return launch_check(c, "rotation GEMM");
+}
+
+// group of M rows: rows ai.. and columns ak.. of the projector P (W doubles
+// per element; T: transposed, columns ai.., rows ak..), B and C at their rows
+template <int AM>
+GemmGroup gemm_group(const void* P, int64_t lda, int64_t ai, int64_t ak, const cplx* B, cplx* C, int64_t M, int64_t K) {
+    constexpr bool T = AM == 1 || AM == 3;
+    const int64_t o = (T ? ak * lda + ai : ai * lda + ak) * (AM >= 2 ? 2 : 1);
+    return {(const double*)P + o, (const double*)B, (double*)C, (int)std::max<int64_t>(M, 0),
+            (int)std::max<int64_t>(K, 0)};
 }
 
 // cn_transform_hm::construct<-1,isub> / eliminate<isub,-1> of a real projector
@@ -215,15 +279,16 @@ int rot_real_construct(qpc_ctx* c, const double* P, const cplx* src, cplx* dst) 
     const int64_t n2 = 2 * c->N;
     TimedLaunch t(c, QPC_K_EP_ROT);
     // dst rows [s0, s1) = P[s0:s1, :] src
-    return gemm<0>(c, P, c->ML, E.s0, 0, (const double*)src, n2, (double*)(dst + E.s0 * c->N), n2, E.s1 - E.s0, n2,
-                   c->ML, c->ML);
+    const GemmGroup g = gemm_group<0>(P, c->ML, E.s0, 0, src, dst + E.s0 * c->N, E.s1 - E.s0, c->ML);
+    return gemm<0>(c, &g, 1, c->ML, n2, n2, n2);
 }
 int rot_real_eliminate(qpc_ctx* c, const double* P, const cplx* src, cplx* dst) {
     const auto& E = c->ep;
     const int64_t n2 = 2 * c->N, ns = E.s1 - E.s0;
     TimedLaunch t(c, QPC_K_EP_ROT);
     // dst = P[s0:s1, :]^T src[s0:s1]
-    return gemm<1>(c, P, c->ML, 0, E.s0, (const double*)(src + E.s0 * c->N), n2, (double*)dst, n2, c->ML, n2, ns, ns);
+    const GemmGroup g = gemm_group<1>(P, c->ML, 0, E.s0, src + E.s0 * c->N, dst, c->ML, ns);
+    return gemm<1>(c, &g, 1, c->ML, n2, n2, n2);
 }
 // ---- the rotations around the field-free solve, on the parity-ordered state --
 // Rows of tran_y2 / tran_y1 in the even category (catagorize's first n_even)
@@ -247,20 +312,17 @@ int rot_construct_p(qpc_ctx* c, const void* P, const cplx* src, cplx* dst) {
     const auto& E = c->ep;
     const RowGroups g = row_groups(c);
     const int64_t ML = c->ML, N = c->N, n2 = 2 * N;
-    // (row range, column block [k0, k1)) of the three groups
-    const int64_t r[3][4] = {{g.ev0, g.ev1, 0, E.n_ev}, {g.ev1, g.z1, 0, ML}, {g.z1, ML, E.n_ev, ML}};
+    // (row range, column block [k0, k1)) of the three groups, the longest sums first
+    const int64_t r[3][4] = {{g.ev1, g.z1, 0, ML}, {g.ev0, g.ev1, 0, E.n_ev}, {g.z1, ML, E.n_ev, ML}};
     TimedLaunch t(c, QPC_K_EP_ROT);
-    for (const auto& q : r) {
+    constexpr int AM = CPLX ? 2 : 0;
+    GemmGroup gg[3];
+    for (int k = 0; k < 3; ++k) {
+        const auto& q = r[k];
         const int64_t a = std::max(q[0], E.s0), b = std::min(q[1], E.s1), k0 = q[2], kn = q[3] - q[2];
-        if (b <= a) continue;
-        if (CPLX)
-            TRY(gemm<2>(c, (const double*)P, ML, a, k0, (const double*)(src + k0 * N), n2, (double*)(dst + a * N), n2,
-                        b - a, n2, 2 * kn, kn));
-        else
-            TRY(gemm<0>(c, (const double*)P, ML, a, k0, (const double*)(src + k0 * N), n2, (double*)(dst + a * N), n2,
-                        b - a, n2, kn, kn));
+        gg[k] = gemm_group<AM>(P, ML, a, k0, src + k0 * N, dst + a * N, b - a, kn);
     }
-    return QPC_OK;
+    return gemm<AM>(c, gg, 3, ML, n2, n2, n2);
 }
 // dst (parity order, all ML rows) = P[s0:s1, :]^H src[s0:s1] (^T when real):
 // the even block from the even and zero rows, the odd block from the zero and
@@ -272,20 +334,17 @@ int rot_eliminate_p(qpc_ctx* c, const void* P, const cplx* src, cplx* dst) {
     const int64_t ML = c->ML, N = c->N, n2 = 2 * N;
     const int64_t blk[2][4] = {{0, E.n_ev, g.ev0, g.z1}, {E.n_ev, ML, g.ev1, ML}};  // out rows, source rows
     TimedLaunch t(c, QPC_K_EP_ROT);
-    for (const auto& q : blk) {
+    constexpr int AM = CPLX ? 3 : 1;
+    GemmGroup gg[2];
+    for (int k = 0; k < 2; ++k) {
+        const auto& q = blk[k];
         const int64_t o0 = q[0], on = q[1] - q[0];
         const int64_t a = std::max(q[2], E.s0), b = std::min(q[3], E.s1), kn = std::max<int64_t>(0, b - a);
-        if (on <= 0) continue;
-        // an empty source range leaves the block zero (the GEMM with K = 0 writes zeros)
+        // an empty source range leaves the block zero (a product with K = 0 writes zeros)
         const int64_t k0 = kn > 0 ? a : 0;
-        if (CPLX)
-            TRY(gemm<3>(c, (const double*)P, ML, o0, k0, (const double*)(src + k0 * N), n2, (double*)(dst + o0 * N),
-                        n2, on, n2, 2 * kn, kn));
-        else
-            TRY(gemm<1>(c, (const double*)P, ML, o0, k0, (const double*)(src + k0 * N), n2, (double*)(dst + o0 * N),
-                        n2, on, n2, kn, kn));
+        gg[k] = gemm_group<AM>(P, ML, o0, k0, src + k0 * N, dst + o0 * N, on, kn);
     }
-    return QPC_OK;
+    return gemm<AM>(c, gg, 2, ML, n2, n2, n2);
 }
 
 // construct<isub,isub> / eliminate<isub,isub> of a merged complex projector:
@@ -294,10 +353,9 @@ int rot_cplx(qpc_ctx* c, bool herm, const cplx* P, const cplx* src, cplx* dst) {
     const auto& E = c->ep;
     const int64_t ns = E.s1 - E.s0, N = c->N;
     TimedLaunch t(c, QPC_K_EP_ROT);
-    const double* B = (const double*)(src + E.s0 * N);
-    double* C = (double*)(dst + E.s0 * N);
-    if (herm) return gemm<3>(c, (const double*)P, c->ML, E.s0, E.s0, B, 2 * N, C, 2 * N, ns, 2 * N, 2 * ns, ns);
-    return gemm<2>(c, (const double*)P, c->ML, E.s0, E.s0, B, 2 * N, C, 2 * N, ns, 2 * N, 2 * ns, ns);
+    const GemmGroup g = herm ? gemm_group<3>(P, c->ML, E.s0, E.s0, src + E.s0 * N, dst + E.s0 * N, ns, ns)
+                             : gemm_group<2>(P, c->ML, E.s0, E.s0, src + E.s0 * N, dst + E.s0 * N, ns, ns);
+    return herm ? gemm<3>(c, &g, 1, c->ML, 2 * N, 2 * N, 2 * N) : gemm<2>(c, &g, 1, c->ML, 2 * N, 2 * N, 2 * N);
 }
 
 // operators of the sweeps: x1 and y1 are D-parts (Y11 with d/dr), x2 and y2
@@ -822,13 +880,14 @@ int ep_build_angular(qpc_ctx* c, int isub, bool lg) {
         }
         // merged products P_b P_a^H = conj(prj_b) prj_a^T (merge_two, cn_1e.hpp:161-181)
         if (lg) {
-            TRY(gemm<2>(c, (const double*)cj[2], ML, 0, 0, (const double*)tr[0], 2 * ML, (double*)E.x1x2, 2 * ML, ML,
-                        2 * ML, 2 * ML, ML));
+            const GemmGroup g = gemm_group<2>(cj[2], ML, 0, 0, tr[0], E.x1x2, ML, ML);
+            TRY(gemm<2>(c, &g, 1, ML, 2 * ML, 2 * ML, 2 * ML));
         } else {
             cplx* out[3] = {E.x1x2, E.x2y1, E.y1y2};
-            for (int t = 0; t < 3; ++t)
-                TRY(gemm<2>(c, (const double*)cj[mg[t][0]], ML, 0, 0, (const double*)tr[mg[t][1]], 2 * ML,
-                            (double*)out[t], 2 * ML, ML, 2 * ML, 2 * ML, ML));
+            for (int t = 0; t < 3; ++t) {
+                const GemmGroup g = gemm_group<2>(cj[mg[t][0]], ML, 0, 0, tr[mg[t][1]], out[t], ML, ML);
+                TRY(gemm<2>(c, &g, 1, ML, 2 * ML, 2 * ML, 2 * ML));
+            }
         }
         QPC_HIP_CHECK(c, hipStreamSynchronize(c->stream));
         TRY(ep_plan_share(c));

@@ -45,3 +45,37 @@ def test_steps_at_partition_edges(N, p):
         print(f"  {kind} {a}: rel L2 {err:.2e}", flush=True)
         assert err <= 1e-12
     prop.close()
+
+
+@pytest.mark.parametrize("gauge", ["vgwr", "lgwr"])
+@pytest.mark.parametrize("M,L,N,isub", [(2, 4, 32, -1), (3, 3, 31, -1), (3, 5, 33, 2), (7, 9, 95, -1), (8, 8, 64, 3),
+                                        (5, 13, 48, -1), (5, 13, 50, 2), (13, 11, 40, 3)])
+def test_rotations_at_tile_edges(M, L, N, isub, gauge):
+    """Channel counts around the rotations' 64-row tiles and 8-term slices,
+    row lengths around their 64 columns, each sub-block (row groups that are
+    empty, of a few rows, of several tiles)."""
+    import pyoracle as po
+    print(f"case: rotation edges M={M} L={L} N={N} isub={isub} {gauge}", flush=True)
+    m0 = -(M // 2)
+    o, prop = _pair(N, 7, L, M, m0)
+    c = mixed_state(o, seed=N + M, amp=0.3)
+    if isub > 0:
+        c = np.where(np.repeat([il % 2 == isub - 2 for _ in range(M) for il in range(L)], N), c, 0.0)
+    c = np.ascontiguousarray(c / np.sqrt(o.norm(c)))
+    prop.set_state(c)
+    if gauge == "vgwr":
+        ang, f = po.ep_angular(M, L, m0), (0.9, 1.1, -0.5, 0.3)
+        o.set_ep(ang, isub=isub)
+        prop.upload_angular_ep(ang, isub=isub)
+        o.step_ep(c, *f)
+        prop.propagate_ep(*f)
+    else:
+        ang, f = po.lgwr_angular(M, L, m0), (0.05, 0.06, -0.03, 0.02)
+        o.set_lgwr(ang, isub=isub)
+        prop.upload_angular_lgwr(ang, isub=isub)
+        o.step_lgwr(c, *f)
+        prop.propagate_lgwr(*f)
+    err = rel_l2(prop.get_state(), c)
+    print(f"  rel L2 {err:.2e}", flush=True)
+    assert err <= 1e-12
+    prop.close()
