@@ -982,9 +982,9 @@ __global__ __launch_bounds__(256) void k_band_diag(const T* __restrict__ src, T*
 // enters the window at step i; its {S, X} entries (launch_factor_bands) lie
 // partition-interleaved, so that a wave's load is one contiguous run instead of
 // 64 lines 24 rows apart, and the next column is loaded a whole step ahead.
-// One time point is bound by the chain of rows (reciprocal, scale, update of
-// the next pivot): 31 channels of N = 1000 take 41 us (S + i e X, was 134) and
-// 31 us (S + e X, was 71).  A batch is bound by the products and the table
+// Few tables are bound by the chain of rows (reciprocal, scale, update of
+// the next pivot: 31 channels of N = 1000 take 41 us, was 134) and are left to
+// k_factor_row.  A batch is bound by the products and the table
 // writes: 32 time points of N = 3000, 41 tables of S + i e X 167 us (was
 // 434), 81 of S + e X 307 us (was 596).
 template <int SYM>
@@ -998,7 +998,10 @@ struct FactorTypes<1> {
     using T = double;
 };
 
-__device__ inline cplx frcp(cplx b) { return crecip(b); }
+__device__ inline cplx frcp(cplx b) {
+    const double d = fma(b.re, b.re, b.im * b.im);
+    return {b.re / d, -b.im / d};
+}
 __device__ inline double frcp(double b) { return 1.0 / b; }
 __device__ inline cplx fmulx(cplx a, cplx b) {
     return {fma(-a.im, b.im, a.re * b.re), fma(a.im, b.re, a.re * b.im)};
@@ -1114,6 +1117,170 @@ __global__ __launch_bounds__(kLane, P == 7 ? 2 : 1) void k_factor(const cplx* __
     for (; i < r0; i += RS) round(i, std::false_type{});
 #pragma unroll 1
     for (; i < r0 + kPM; i += RS) round(i, std::true_type{});
+}
+
+// The same elimination for few tables: 16 lanes per partition, four
+// partitions per wave.  A launch of one time point is bound by the chain of
+// rows, and k_factor's lane issues 190 (S + e X: 130) instructions per row for
+// its own partition however few waves there are.  Here lane c mod 8 of a
+// partition's 16 holds column c of the window (rows i+1 .. i+8, row r in
+// register r mod 8) and the pivot and the row's entries reach the others by DPP
+// row broadcasts, so a row takes P products per lane instead of P(P+1)/2.  Of a
+// complex symmetric matrix the lower eight lanes hold the real parts and the
+// upper eight the imaginary ones (each divides one part of 1 / pivot); of a
+// real one both halves hold the same.  The bits are k_factor's.  Once column i is the pivot its lane
+// takes column i + 8.  The columns come from LDS, where the wave stages the
+// `above` rows over its first partition and the four partitions; columns
+// before the matrix are the identity's, which changes nothing below them.
+// Per partition it takes four times k_factor's lane-instructions.  Measured
+// against k_factor, S + i e X (S + e X), one time point: 3 tables of N = 240
+// 18 us against 49 (13 against 32), 16 tables of N = 1000 19 against 41; two
+// of 37 tables of N = 361 20 against 52 (81: 18 against 34).
+template <int L>
+__device__ inline double bcast16(double v) {  // lane L of each 16
+    return __longlong_as_double(__builtin_amdgcn_mov_dpp(__double_as_longlong(v), 0x150 + L, 0xf, 0xf, true));
+}
+template <int BANKS>
+__device__ inline double swap8(double v) {  // lane l ^ 8 in the banks of four lanes of BANKS, v in the others
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    const int l = (int)(unsigned)b, h = (int)(unsigned)(b >> 32);
+    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(l, l, 0x128, 0xf, BANKS, false);
+    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(h, h, 0x128, 0xf, BANKS, false);
+    return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+template <int... I, class F>
+__device__ inline void each(std::integer_sequence<int, I...>, F f) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+constexpr int kFactorQ = 4;  // partitions per wave
+// Used up to this many waves (six per compute unit, the most its LDS holds:
+// 650 waves take 18 us, 3200 78 us and 5600 118 us where k_factor takes 35 to
+// 55), and this many restart rows (LDS: 50 KB)
+constexpr int64_t kFactorRowWaves = 1536;
+constexpr int kFactorRowAbove = 192;
+// doubles per staged column, blocks of kPM columns staged for `above` restart rows
+template <int P>
+constexpr int factor_pe() { return P == 7 ? 8 : 10; }
+inline __host__ __device__ int factor_row_blocks(int above) { return (above + kPM - 1) / kPM + kFactorQ + 1; }
+
+template <int SYM, int P>
+__global__ __launch_bounds__(kLane) void k_factor_row(const cplx* __restrict__ fx, const double* __restrict__ eig,
+                                                      int64_t eig_tstride, const double* __restrict__ ifdt, Geom geo,
+                                                      int above, cplx* __restrict__ tab, int64_t tstride) {
+    using T = typename FactorTypes<SYM>::T;
+    constexpr int NE = P + 1, PE = factor_pe<P>();
+    constexpr int ROW = TabFmt<T, P>::row;
+    extern __shared__ __align__(16) double sh[];  // [2][columns][PE]: re, im or upper, lower
+    const int g0 = blockIdx.x * kFactorQ;
+    const int ch = blockIdx.y, t = blockIdx.z;
+    const int FP = factor_cols(geo);
+    const double e = eig[(int64_t)t * eig_tstride + ch] * ifdt[t];
+    const int ln = threadIdx.x, cl = ln & 7, hf = (ln >> 3) & 1;
+    // stage whole blocks of kPM columns from block b0 on, a lane per (block, entry)
+    const int nb = factor_row_blocks(above), b0 = g0 - (nb - kFactorQ - 1), half = nb * kPM * PE;
+    for (int gb = cl; gb < nb; gb += 8)
+        for (int j = ln >> 3; j < NE; j += 8) {
+            const int b = b0 + gb;
+            const cplx* q = fx + ((int64_t)j * FP + min(max(b, 0), FP - 1));
+            cplx v[kPM];
+#pragma unroll
+            for (int k = 0; k < kPM; ++k) v[k] = q[(int64_t)k * NE * FP];
+            double* d = sh + gb * kPM * PE + j;
+#pragma unroll
+            for (int k = 0; k < kPM; ++k, d += PE) {
+                if (b < 0) v[k] = cplx{j == 0 ? 1.0 : 0.0, 0.0};
+                if constexpr (SYM == 0) {
+                    d[0] = v[k].re;
+                    d[half] = e * v[k].im;
+                } else {
+                    const double up = fma(e, v[k].im, v[k].re);
+                    d[0] = up;
+                    d[half] = j ? fma(-e, v[k].im, v[k].re) : up;  // antisymmetric below the diagonal
+                }
+            }
+        }
+    __syncthreads();
+    // (partitions past the last repeat it)
+    const int g = min(g0 + (ln >> 4), geo.P - 1);
+    const int first = (g - b0) * kPM - above;  // first row of the restarted elimination
+    const double* up = sh + first * PE + (SYM == 0 ? hf * half : 0);
+    const double* lo = sh + first * PE + half;
+    char* Tg = (char*)(tab + ((int64_t)t * tstride + ch) * TabFmt<T, P>::units(geo) + part_col<T, P>(g));
+    double w[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+        if constexpr (SYM == 0) w[r] = r <= cl ? up[cl * PE + max(cl - r, 0)] : 0.0;
+        else w[r] = r <= cl ? up[cl * PE + max(cl - r, 0)] : lo[r * PE + max(r - cl, 0)];
+    }
+    // eight rows from row i (of the staged columns) on, pivot columns at up / lo
+    auto round = [&](int i, auto store) {
+        constexpr bool STORE = decltype(store)::value;
+        each(std::make_integer_sequence<int, 8>{}, [&](auto sc) {
+            constexpr int S = decltype(sc)::value;
+            const bool mine = cl == S;          // the pivot column's lane
+            const int b1 = (cl - S - 1) & 7;    // column i + 1 + b1 (P = 7: 7 is the pivot's lane)
+            const double* nu = up + (S + 8) * PE;  // column i + 8
+            double a0 = w[S];
+            char* o = Tg + (int64_t)(i + S - above) * ROW * kLane * 16;
+            if constexpr (SYM == 0) {
+                const double pr = bcast16<S>(a0), pi = bcast16<S + 8>(a0);
+                if (mine) {
+                    a0 = P == 8 ? nu[P] : 0.0;
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) w[(S + 1 + k) & 7] = nu[7 - k];
+                }
+                // 1 / pivot = (pr - i pi) / |pivot|^2, a part in either half
+                const double q0 = (hf ? -pi : pr) / fma(pr, pr, pi * pi);
+                const double qr = bcast16<0>(q0), qi = bcast16<8>(q0);
+                const double ar = swap8<0xc>(a0), ai = swap8<0x3>(a0);
+                // u = a / pivot (k_factor's order of operations: the same bits);
+                // the lower half multiplies by (re u, -im u), the upper by (im u, re u)
+                const double ur = fma(-ai, qi, ar * qr), ui = fma(ai, qr, ar * qi);
+                const double x1 = hf ? ui : ur, x2 = hf ? ur : -ui;
+                if constexpr (STORE) {
+                    *(double*)(o + (b1 * kLane * 16 + hf * 8)) = P == 7 && mine ? q0 : x1;
+                    if (P == 8 && cl == 0) *(double*)(o + (P * kLane * 16 + hf * 8)) = q0;
+                }
+                each(std::make_integer_sequence<int, P>{}, [&](auto ac) {
+                    constexpr int a = decltype(ac)::value + 1, c = (S + a) & 7;
+                    double& v = w[(S + a) & 7];
+                    v = fma(-bcast16<c>(a0), x1, v);
+                    v = fma(-bcast16<c + 8>(a0), x2, v);
+                });
+            } else {
+                const double* nl = lo + (S + 8) * PE;
+                double l[NE];
+                l[0] = bcast16<S>(a0);
+#pragma unroll
+                for (int a = 1; a < 8; ++a) l[a] = bcast16<S>(w[(S + a) & 7]);
+                if constexpr (P == 8) l[8] = nl[8];
+                // row i + 8 of the columns i + 1 .. i + 8, then column i + 8
+                w[S] = nl[(7 - b1) & 7];
+                if (mine) {
+                    a0 = P == 8 ? nu[P] : 0.0;
+#pragma unroll
+                    for (int k = 0; k < 7; ++k) w[(S + 1 + k) & 7] = nu[7 - k];
+                }
+                const double rp = 1.0 / l[0];
+                const double u = a0 * rp;
+                if constexpr (STORE) {
+                    if (cl == 0) put_real<P>((cplx*)o, l + 1, rp);
+                    char* ob = o + (int64_t)TabFmt<T, P>::boff * kLane * 16;
+                    *(double*)(ob + ((b1 >> 1) * kLane * 16 + (b1 & 1) * 8)) = P == 7 && mine ? 1.0 : u;
+                    if (P == 8 && cl == 0) *(cplx*)(ob + (P / 2) * kLane * 16) = cplx{1.0, 0.0};
+                }
+#pragma unroll
+                for (int a = 1; a < NE; ++a) w[(S + a) & 7] = fma(-l[a], u, w[(S + a) & 7]);
+            }
+        });
+        up += 8 * PE;
+        lo += 8 * PE;
+    };
+    int i = 0;
+#pragma unroll 1
+    for (; i < above; i += 8) round(i, std::false_type{});
+#pragma unroll 1
+    for (; i < above + kPM; i += 8) round(i, std::true_type{});
 }
 
 // fx[(s * (p+1) + j) * FP + g] = {S, X}(c-j, c) of column c = 24 g + s, zero
@@ -1320,15 +1487,25 @@ void launch_factor_bands(hipStream_t s, const double* S, const double* X, cplx* 
     hipLaunchKernelGGL(k_factor_bands, dim3((total + 255) / 256), dim3(256), 0, s, S, X, fx, geo.N, geo.hw + 1,
                        factor_cols(geo));
 }
+template <int SYM, int P>
+static void factor_launch_p(hipStream_t s, const cplx* fx, const double* eig, const double* ifdt, int nt, int nch,
+                            Geom geo, cplx* tab, int64_t eig_tstride, int rs, int64_t ts) {
+    const int above = (rs + 7) / 8 * 8;
+    const int64_t groups = (geo.P + kFactorQ - 1) / kFactorQ;
+    if (groups * nch * nt <= kFactorRowWaves && above <= kFactorRowAbove)
+        hipLaunchKernelGGL((k_factor_row<SYM, P>), dim3((unsigned)groups, nch, nt), dim3(kLane),
+                           sizeof(double) * 2 * factor_row_blocks(above) * kPM * factor_pe<P>(), s, fx, eig, eig_tstride, ifdt,
+                           geo, above, tab, ts);
+    else
+        hipLaunchKernelGGL((k_factor<SYM, P>), dim3(geo.NG, nch, nt), dim3(kLane), 0, s, fx, eig, eig_tstride, ifdt,
+                           geo, rs, tab, ts);
+}
 template <int SYM>
 static void factor_launch(hipStream_t s, const cplx* fx, const double* eig, const double* ifdt, int nt, int nch, Geom geo,
                           cplx* tab, int64_t eig_tstride, int restart, int64_t ts) {
     const int rs = restart > 0 ? restart : kRestart;
-    const dim3 grid(geo.NG, nch, nt);
-    if (geo.hw == 8)
-        hipLaunchKernelGGL((k_factor<SYM, 8>), grid, dim3(kLane), 0, s, fx, eig, eig_tstride, ifdt, geo, rs, tab, ts);
-    else
-        hipLaunchKernelGGL((k_factor<SYM, 7>), grid, dim3(kLane), 0, s, fx, eig, eig_tstride, ifdt, geo, rs, tab, ts);
+    if (geo.hw == 8) factor_launch_p<SYM, 8>(s, fx, eig, ifdt, nt, nch, geo, tab, eig_tstride, rs, ts);
+    else factor_launch_p<SYM, 7>(s, fx, eig, ifdt, nt, nch, geo, tab, eig_tstride, rs, ts);
 }
 void launch_factor_sym(hipStream_t s, const cplx* fx, const double* eig, const double* ifdt, int nt, int nch, Geom geo,
                        cplx* tab, int64_t eig_tstride, int restart, int64_t tab_tstride) {

@@ -79,3 +79,25 @@ def test_rotations_at_tile_edges(M, L, N, isub, gauge):
     print(f"  rel L2 {err:.2e}", flush=True)
     assert err <= 1e-12
     prop.close()
+
+
+@pytest.mark.parametrize("p", [7, 8])
+def test_batched_and_single_time_points_agree(p):
+    """The tables of a run's time points are factorised together, those of
+    single steps one time point at a time, by different kernels: 16 steps
+    either way (20 R-part tables and 40 D-part tables of 25 partitions)."""
+    N, L, nt = 600, 40, 16
+    print(f"case: batched against single time points N={N} L={L} p={p}", flush=True)
+    o, prop = _pair(N, p, L)
+    a = 0.8 * np.sin(0.3 * np.arange(nt + 1)) + 0.1
+    c = mixed_state(o, seed=p, amp=0.3)
+    prop.set_state(c)
+    prop.run(a, nt, 0, nt, use_mask=False)
+    ref = prop.get_state().copy()
+    prop.set_state(c)
+    for k in range(nt):
+        prop.propagate(a[k], a[k + 1])
+    err = rel_l2(prop.get_state(), ref)
+    print(f"  rel L2 {err:.2e}", flush=True)
+    assert err <= 1e-12
+    prop.close()
