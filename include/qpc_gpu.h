@@ -365,7 +365,7 @@ int  qpc_observe_batch(qpc_ctx* ctx, int what, double* out);
  * (binsrc/sphTDSE.cpp:921-951): with-field steps with
  * (axtab[it], axtab[it+1], aytab[it], aytab[it+1]) while it < nt_field,
  * field-free steps afterwards, the absorber after each step when use_mask;
- * it returns when the work is queued (qpc_sync waits).  The eight coupling
+ * both return when the work is queued (qpc_sync waits).  The eight coupling
  * sweeps of a step are factorised on a second stream one step ahead.
  * QPC_E_NUMERIC when A(t)*dt leaves the range of the D-part sweeps
  * (as qpc_step). */

@@ -21,9 +21,6 @@ struct qpc_ctx {
     int64_t N = 0, p = 0, ne = 0, L = 0, M = 0, m0 = 0, lmax = 0, ML = 0;
     hipStream_t stream = nullptr;   // the step sequence
     hipStream_t fstream = nullptr;  // coupling-sweep factorisations, one batch ahead
-    // the D-part factorisation of a per-step call, beside the R part's on fstream
-    hipStream_t dstream = nullptr;
-    hipEvent_t put_done = nullptr;  // the per-step scalars are on the device (fstream)
     int device = 0;
     std::string err;
 
@@ -96,7 +93,6 @@ struct qpc_ctx {
         double *tabD = nullptr, *trfD = nullptr;
         cplx *tabR = nullptr, *trfR = nullptr;
         hipEvent_t ready = nullptr;  // factorisation done (fstream)
-        hipEvent_t ready_r = nullptr;  // its R-part (length gauge: all) tables and transfers done
         hipEvent_t freed = nullptr;  // last step that reads the set issued (stream)
         bool pending = false;        // freed has been recorded
     } ts[2];
@@ -105,12 +101,13 @@ struct qpc_ctx {
     std::vector<double> h_dD, h_dR;
     // the per-step entry points keep their last A(t_f) (or E(t_f)): its tables
     // are at position step_slot (0..2) of table set 0 (-1: none), its value
-    // step_a; slot_read[k] marks the end of the last step that read position k
+    // step_a; position k was last read by the step that recorded
+    // step_done[slot_read[k]] at its end (-1: none since the last idle)
     int64_t step_slot = -1;
     double step_a = 0.0;
     int step_gauge = 0;
-    hipEvent_t slot_read[3] = {nullptr, nullptr, nullptr};
-    bool slot_rec[3] = {false, false, false};
+    hipEvent_t step_done[3] = {nullptr, nullptr, nullptr};  // steps in turn
+    int slot_read[3] = {-1, -1, -1}, step_next = 0;
     double yeig_max = 0.0;  // largest |eigenvalue| of the D-part rotation
     // host copies of S, d/dr and r (row-major bands) for the sweep plans
     std::vector<double> S_h, rdif_h, rpow1_h;
@@ -210,8 +207,7 @@ struct qpc_ctx {
             bool pending = false;
         } set[2];
         std::vector<double> h_sc;    // per step: [x1 ti, x1 tf, y1 ti, y1 tf, x2 ti, x2 tf, y2 ti, y2 tf]
-        double* d_sc = nullptr;      // device copy, [run_cap][8]
-        int64_t run_cap = 0;
+        int step_set = 0;            // table set of the next per-step call
         bool have = false;
     } ep;
     bool have_radial = false, have_hc = false, have_ang = false, have_mask = false, have_state = false;

@@ -402,16 +402,6 @@ int ep_set_scalars(qpc_ctx* c, const double* ax, const double* ay, int64_t nstep
     // for this run's scalars
     if (E.lg) TRY(qpc_host::plan_l_part(c, emax));
     else TRY(qpc_host::plan_d_part(c, emax));
-    if (nsteps > E.run_cap) {
-        if (E.d_sc) QPC_HIP_CHECK(c, hipFree(E.d_sc));
-        E.d_sc = nullptr;
-        E.run_cap = 0;
-        QPC_HIP_CHECK(c, hipMalloc((void**)&E.d_sc, sizeof(double) * 8 * nsteps));
-        E.run_cap = nsteps;
-    }
-    QPC_HIP_CHECK(c, hipMemcpyAsync(E.d_sc, E.h_sc.data(), sizeof(double) * 8 * nsteps, hipMemcpyHostToDevice,
-                                    c->stream));
-    QPC_HIP_CHECK(c, hipStreamSynchronize(c->stream));
     return QPC_OK;
 }
 
@@ -423,40 +413,39 @@ int ep_factor(qpc_ctx* c, int set, int64_t k) {
     const int64_t np = E.p1 - E.p0, ML = c->ML;
     if (np <= 0) return QPC_OK;
     if (T.pending) QPC_HIP_CHECK(c, hipStreamWaitEvent(c->fstream, T.freed, 0));
-    const double* sc = E.d_sc + k * 8;
-    const int64_t te = c->geo.tab_elems, cte = c->geo.ctab_elems;
-    // a complex symmetric sweep's tables (ts: tables of time point t at
-    // position t * np of its block; shared tables: the nprim primaries)
-    const int64_t trs = c->geo.ctrf_elems;
-    auto sym_tables = [&](int op, const cplx* fx, int restart) {
-        const int64_t slot = ep_slot(op, 0);
-        cplx* tab = T.tabR + slot * np * cte;
-        cplx* trf = T.trfR + slot * np * trs;
-        if (E.rmap[op]) {
-            qpc::launch_factor_sym(c->fstream, fx, E.eprim[op], sc + ep_sc(op, 0), 2, (int)E.nprim[op], c->geo,
-                                   tab, 0, restart, np);
-            qpc::launch_transfer_c(c->fstream, tab, trf, (int)E.nprim[op], 2, np, c->geo);
+    const double* sc = &E.h_sc[(size_t)k * 8];
+    const int64_t te = c->geo.tab_elems, cte = c->geo.ctab_elems, tr = c->geo.trf_elems, ctr = c->geo.ctrf_elems;
+    // tables of time point t at position t * np of an operator's block (shared
+    // tables: the nprim primaries)
+    qpc::FactorJob jobs[4];
+    int n = 0;
+    for (int op = 0; op < 4; ++op) {
+        if (E.lg && !ep_is_d(op)) continue;
+        const int64_t slot = ep_slot(op, 0) * np;
+        qpc::FactorJob& J = jobs[n++];
+        J.ifdt[0] = sc[ep_sc(op, 0)];
+        J.ifdt[1] = sc[ep_sc(op, 1)];
+        J.tstride = np;
+        J.real = ep_is_d(op) && !E.lg;
+        if (J.real) {
+            J.fx = c->fxD;
+            J.restart = c->restart_d;
+            J.eig = E.eig + op * ML + E.p0;
+            J.nch = (int)np;
+            J.tab = T.tabD + slot * te;
+            J.trf = T.trfD + slot * tr;
         } else {
-            qpc::launch_factor_sym(c->fstream, fx, E.eig + op * ML + E.p0, sc + ep_sc(op, 0), 2, (int)np, c->geo,
-                                   tab, 0, restart);
-            qpc::launch_transfer_c(c->fstream, tab, trf, (int)(2 * np), c->geo);
+            J.fx = E.lg ? c->fxL : c->fxR;
+            J.restart = E.lg ? c->restart_l : 0;
+            J.eig = E.rmap[op] ? E.eprim[op] : E.eig + op * ML + E.p0;
+            J.nch = (int)(E.rmap[op] ? E.nprim[op] : np);
+            J.tab = T.tabR + slot * cte;
+            J.trf = T.trfR + slot * ctr;
         }
-    };
-    if (E.lg) {
+    }
+    {
         TimedLaunch tl(c, QPC_K_FACTOR, c->fstream);
-        for (int op : {EP_X1, EP_Y1}) sym_tables(op, c->fxL, c->restart_l);
-    } else {
-        TimedLaunch tl(c, QPC_K_FACTOR, c->fstream);
-        for (int op = 0; op < 4; ++op) {
-            const double* eig = E.eig + op * ML + E.p0;
-            const int64_t slot = ep_slot(op, 0);
-            if (ep_is_d(op))
-                qpc::launch_factor_asy(c->fstream, c->fxD, eig, sc + ep_sc(op, 0), 2, (int)np, c->geo,
-                                       T.tabD + slot * np * te, 0, c->restart_d);
-            else
-                sym_tables(op, c->fxR, 0);
-        }
-        qpc::launch_transfer_r(c->fstream, T.tabD, T.trfD, (int)(4 * np), c->geo);
+        qpc::launch_factor_jobs(c->fstream, jobs, n, 2, c->geo);
     }
     TRY(launch_check(c, "ep factor"));
     QPC_HIP_CHECK(c, hipEventRecord(T.ready, c->fstream));
@@ -950,16 +939,17 @@ int ep_run(qpc_ctx* c, bool lg, const double* atx, const double* aty, int64_t nt
 int ep_step(qpc_ctx* c, bool lg, double ax_i, double ax_f, double ay_i, double ay_f) {
     if (!c) return QPC_E_ARG;
     TRY(ep_ready(c, false, lg));
-    QPC_HIP_CHECK(c, hipStreamSynchronize(c->stream));
-    QPC_HIP_CHECK(c, hipStreamSynchronize(c->fstream));
+    auto& E = c->ep;
     const double ax[2] = {ax_i, ax_f}, ay[2] = {ay_i, ay_f};
     TRY(ep_set_scalars(c, ax, ay, 1));
-    TRY(ep_factor(c, 0, 0));
-    QPC_HIP_CHECK(c, hipStreamWaitEvent(c->stream, c->ep.set[0].ready, 0));
-    TRY(lg ? lg_do_step(c, 0, 0, false, false) : ep_do_step(c, 0, 0, false, false));
-    QPC_HIP_CHECK(c, hipEventRecord(c->ep.set[0].freed, c->stream));
-    c->ep.set[0].pending = true;
-    QPC_HIP_CHECK(c, hipStreamSynchronize(c->stream));
+    // the two table sets in turn: a call's tables are factorised beside the previous call's sweeps
+    const int set = E.step_set;
+    E.step_set = 1 - set;
+    TRY(ep_factor(c, set, 0));
+    QPC_HIP_CHECK(c, hipStreamWaitEvent(c->stream, E.set[set].ready, 0));
+    TRY(lg ? lg_do_step(c, set, 0, false, false) : ep_do_step(c, set, 0, false, false));
+    QPC_HIP_CHECK(c, hipEventRecord(E.set[set].freed, c->stream));
+    E.set[set].pending = true;
     return QPC_OK;
 }
 

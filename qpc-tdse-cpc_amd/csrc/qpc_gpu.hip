@@ -260,21 +260,14 @@ int set_run_scalars(qpc_ctx* c, const double* a, int64_t n, int64_t stride = 0) 
 // factorisations of the coupling sweeps for run time points [t0, t0+n) into
 // table set ts from position pos on, on fstream once the steps that read the
 // set before are done
-int factor_batch(qpc_ctx* c, int ts, int64_t t0, int64_t n, int64_t pos = 0, bool wait_set = true,
-                 bool split = false) {
-    if (pos + n > c->tb_cap) {
+int factor_batch(qpc_ctx* c, int ts, int64_t t0, int64_t n) {
+    if (n > c->tb_cap) {
         c->set_error("factor batch larger than its capacity");
         return QPC_E_ARG;
     }
-    const qpc_ctx::TableSet& S = c->ts[ts];
-    qpc_ctx::TableSet T = S;  // the set's tables from position pos on
-    T.tabD = S.tabD + pos * tabsz_r(c);
-    T.trfD = S.trfD + pos * trfsz_r(c);
-    T.tabR = S.tabR + pos * tabsz_c(c);
-    T.trfR = S.trfR + pos * trfsz_c(c);
-    if (wait_set && T.pending) QPC_HIP_CHECK(c, hipStreamWaitEvent(c->fstream, T.freed, 0));
-    // the R-part tables and transfer sets first (ready_r), then the D-part's
-    // (ready): a step reads the R part of its t_f tables before the D part
+    const qpc_ctx::TableSet& T = c->ts[ts];
+    if (T.pending) QPC_HIP_CHECK(c, hipStreamWaitEvent(c->fstream, T.freed, 0));
+    // the R-part tables and transfer sets first, then the D-part's
     {
         TimedLaunch tl(c, QPC_K_FACTOR, c->fstream);
         const int64_t ML = c->ML;
@@ -304,28 +297,39 @@ int factor_batch(qpc_ctx* c, int ts, int64_t t0, int64_t n, int64_t pos = 0, boo
             qpc::launch_transfer_c(c->fstream, T.tabR, T.trfR, (int)(n * ML), c->geo);
     }
     TRY(launch_check(c, "factor_batch"));
-    QPC_HIP_CHECK(c, hipEventRecord(S.ready_r, c->fstream));
-    // split (a per-step call's one time point): the D part on its own stream,
-    // after everything queued on fstream before this call's R part
-    hipStream_t ds = split && c->gauge != 1 ? c->dstream : c->fstream;
-    if (ds != c->fstream) QPC_HIP_CHECK(c, hipStreamWaitEvent(ds, c->put_done, 0));
     if (c->gauge != 1) {
-        TimedLaunch tl(c, QPC_K_FACTOR, ds);
+        TimedLaunch tl(c, QPC_K_FACTOR, c->fstream);
         const int64_t ML = c->ML;
         if (c->batch)
-            qpc::launch_factor_asy(ds, c->fxD, c->d_e + t0 * ML, c->d_ones, (int)n, (int)ML, c->geo, T.tabD,
+            qpc::launch_factor_asy(c->fstream, c->fxD, c->d_e + t0 * ML, c->d_ones, (int)n, (int)ML, c->geo, T.tabD,
                                    ML, c->restart_d);
         else
-            qpc::launch_factor_asy(ds, c->fxD, c->yeig, c->d_ifdt + t0, (int)n, (int)ML, c->geo, T.tabD, 0,
+            qpc::launch_factor_asy(c->fstream, c->fxD, c->yeig, c->d_ifdt + t0, (int)n, (int)ML, c->geo, T.tabD, 0,
                                    c->restart_d);
-        qpc::launch_transfer_r(ds, T.tabD, T.trfD, (int)(n * ML), c->geo);
+        qpc::launch_transfer_r(c->fstream, T.tabD, T.trfD, (int)(n * ML), c->geo);
         TRY(launch_check(c, "factor_batch"));
     }
-    QPC_HIP_CHECK(c, hipEventRecord(S.ready, ds));
-    if (ds != c->fstream) {
-        // later work on fstream (the next call's tables) comes after this D part
-        QPC_HIP_CHECK(c, hipStreamWaitEvent(c->fstream, S.ready, 0));
+    QPC_HIP_CHECK(c, hipEventRecord(T.ready, c->fstream));
+    return QPC_OK;
+}
+
+// tables of a per-step call's time point (scalars dD, dR) at position pos of
+// table set 0, on fstream
+int factor_step(qpc_ctx* c, int pos, double dD, double dR) {
+    const qpc_ctx::TableSet& T = c->ts[0];
+    const bool lg = c->gauge == 1, shared = !lg && c->n_rprim > 0;
+    const int ML = (int)c->ML;
+    const qpc::FactorJob jobs[2] = {
+        {0, shared ? (int)c->n_rprim : ML, lg ? c->restart_l : 0, lg ? c->fxL : c->fxR,
+         lg ? c->yeig : shared ? c->qeig_prim : c->qeig, {dR, 0.0}, T.tabR + pos * tabsz_c(c), T.trfR + pos * trfsz_c(c),
+         ML},
+        {1, ML, c->restart_d, c->fxD, c->yeig, {dD, 0.0}, T.tabD + pos * tabsz_r(c), T.trfD + pos * trfsz_r(c), ML}};
+    {
+        TimedLaunch tl(c, QPC_K_FACTOR, c->fstream);
+        qpc::launch_factor_jobs(c->fstream, jobs, lg ? 1 : 2, 1, c->geo);
     }
+    TRY(launch_check(c, "factor_step"));
+    QPC_HIP_CHECK(c, hipEventRecord(T.ready, c->fstream));
     return QPC_OK;
 }
 
@@ -338,15 +342,6 @@ int release_set(qpc_ctx* c, int ts) {
     QPC_HIP_CHECK(c, hipEventRecord(c->ts[ts].freed, c->stream));
     c->ts[ts].pending = true;
     return QPC_OK;
-}
-
-// two scalars written by the device (queued with the values, so the host
-// can go on at once)
-__global__ void k_put2(double* p, double v, double* q, double w) {
-    if (threadIdx.x == 0) {
-        *p = v;
-        *q = w;
-    }
 }
 
 // one with-field step (propagator_cn_hc_vgwz::propagate, cn_1e.hpp:682-709)
@@ -363,7 +358,7 @@ __global__ void k_put2(double* p, double v, double* q, double w) {
 // rotations per step drop out; the result differs from the sequence with
 // both rotations by rounding only.
 int do_step(qpc_ctx* c, int ts, int64_t t0, int64_t ti, int64_t tf, bool in_y = false, bool out_y = false,
-            bool mask_in_y = false, hipEvent_t wait_r = nullptr, hipEvent_t wait_d = nullptr) {
+            bool mask_in_y = false, hipEvent_t wait_f = nullptr) {
     cplx* X = c->coef;
     cplx* Y = c->tmpc;
     cplx* Z = c->spare;
@@ -379,10 +374,9 @@ int do_step(qpc_ctx* c, int ts, int64_t t0, int64_t ti, int64_t tf, bool in_y = 
     TRY(solve_free(c, Y, Z));                // prop_hc.propagate0
     TRY(rot_cplx(c, c->rtQ, Z, Y));      // tran_z1.construct
     // (a per-step call: the t_f tables are factorised while the first half runs)
-    if (wait_r) QPC_HIP_CHECK(c, hipStreamWaitEvent(c->stream, wait_r, 0));
+    if (wait_f) QPC_HIP_CHECK(c, hipStreamWaitEvent(c->stream, wait_f, 0));
     TRY(solve_R(c, ts, t0, tf, Y, Z));               // prop_z1.propagate1(A_f)
     TRY(rot_cplx(c, c->rtMh, Z, Y));    // z2_2_z1.eliminate
-    if (wait_d) QPC_HIP_CHECK(c, hipStreamWaitEvent(c->stream, wait_d, 0));
     TRY(solve_D(c, ts, t0, tf, Y, Z));               // prop_z2.propagate2(A_f)
     if (out_y) {
         // stay in P_Y's basis for the next step, with the absorber applied there
@@ -400,7 +394,7 @@ int do_step(qpc_ctx* c, int ts, int64_t t0, int64_t ti, int64_t tf, bool in_y = 
 
 // one length-gauge step (propagator_cn_hc_lgwz::propagate, cn_1e.hpp:598-613)
 // with run time points ti (E(t_i)) and tf (E(t_f)); coef ends in c->coef
-int do_step_lg(qpc_ctx* c, int ts, int64_t t0, int64_t ti, int64_t tf, hipEvent_t wait_r = nullptr) {
+int do_step_lg(qpc_ctx* c, int ts, int64_t t0, int64_t ti, int64_t tf, hipEvent_t wait_f = nullptr) {
     cplx* X = c->coef;
     cplx* Y = c->tmpc;
     cplx* Z = c->spare;
@@ -409,7 +403,7 @@ int do_step_lg(qpc_ctx* c, int ts, int64_t t0, int64_t ti, int64_t tf, hipEvent_
     TRY(rot_real(c, c->rtYt, Z, X));           // tran_z1.eliminate
     TRY(solve_free(c, X, Y));                  // prop_hc.propagate0
     TRY(rot_real(c, c->rtY, Y, Z));            // tran_z1.construct
-    if (wait_r) QPC_HIP_CHECK(c, hipStreamWaitEvent(c->stream, wait_r, 0));
+    if (wait_f) QPC_HIP_CHECK(c, hipStreamWaitEvent(c->stream, wait_f, 0));
     TRY(solve_L(c, ts, t0, tf, Z, Y));         // prop_z1.propagate1(ez_tf)
     TRY(rot_real(c, c->rtYt, Y, X));           // tran_z1.eliminate
     return QPC_OK;
@@ -631,11 +625,8 @@ static int create_impl(const qpc_dims* d, int64_t n_shots, int64_t tb_cap, qpc_c
     if ((rc = qpc_host::resolve_scratch(c))) return fail(rc);
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) return fail(QPC_E_HIP);
     if (hipStreamCreateWithFlags(&c->fstream, hipStreamNonBlocking) != hipSuccess) return fail(QPC_E_HIP);
-    if (hipStreamCreateWithFlags(&c->dstream, hipStreamNonBlocking) != hipSuccess) return fail(QPC_E_HIP);
-    if (hipEventCreateWithFlags(&c->put_done, hipEventDisableTiming) != hipSuccess) return fail(QPC_E_HIP);
     for (auto& T : c->ts)
         if (hipEventCreateWithFlags(&T.ready, hipEventDisableTiming) != hipSuccess ||
-            hipEventCreateWithFlags(&T.ready_r, hipEventDisableTiming) != hipSuccess ||
             hipEventCreateWithFlags(&T.freed, hipEventDisableTiming) != hipSuccess)
             return fail(QPC_E_HIP);
     const size_t band = (size_t)c->N * c->ne;
@@ -681,7 +672,7 @@ int qpc_destroy(qpc_ctx* c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->fstream) (void)hipStreamSynchronize(c->fstream);
     for (hipEvent_t e : c->ev) (void)hipEventDestroy(e);
-    for (hipEvent_t e : c->slot_read)
+    for (hipEvent_t e : c->step_done)
         if (e) (void)hipEventDestroy(e);
     if (c->rmap) (void)hipFree(c->rmap);
     if (c->rorder) (void)hipFree(c->rorder);
@@ -691,7 +682,6 @@ int qpc_destroy(qpc_ctx* c) {
     if (c->d_eprim) (void)hipFree(c->d_eprim);
     for (auto& T : c->ts) {
         if (T.ready) (void)hipEventDestroy(T.ready);
-        if (T.ready_r) (void)hipEventDestroy(T.ready_r);
         if (T.freed) (void)hipEventDestroy(T.freed);
         void* tp[] = {T.tabD, T.trfD, T.tabR, T.trfR};
         for (void* p : tp)
@@ -718,7 +708,7 @@ int qpc_destroy(qpc_ctx* c) {
             for (void* p : tp)
                 if (p) (void)hipFree(p);
         }
-        void* ep_ptrs[] = {E.eig,  E.tx1,  E.ty2,     E.x1x2,     E.x2y1,     E.y1y2,     E.ty1,      E.d_sc,
+        void* ep_ptrs[] = {E.eig,  E.tx1,  E.ty2,     E.x1x2,     E.x2y1,     E.y1y2,     E.ty1,
                            E.perm, E.lmap, E.ty2p,    E.ty1p,     E.rmap[0],  E.rmap[1],  E.rmap[2],  E.rmap[3],
                            E.eprim[0], E.eprim[1], E.eprim[2], E.eprim[3], E.ord[0], E.ord[1], E.ord[2],
                            E.ord[3]};
@@ -727,8 +717,6 @@ int qpc_destroy(qpc_ctx* c) {
     }
     if (c->stream) (void)hipStreamDestroy(c->stream);
     if (c->fstream) (void)hipStreamDestroy(c->fstream);
-    if (c->dstream) (void)hipStreamDestroy(c->dstream);
-    if (c->put_done) (void)hipEventDestroy(c->put_done);
     delete c;
     return QPC_OK;
 }
@@ -1318,13 +1306,16 @@ int run_impl(qpc_ctx* c, const double* atab, int64_t stride, int64_t nt_field, i
 // tables of that time point are kept and a call factorises A(t_f) alone,
 // into the one of three positions of table set 0 that the previous step did
 // not read: that factorisation waits only for the step before the previous
-// one (event slot_read) and so runs beside the previous step.  Nothing
-// waits on the host: the new scalars are written and the tables factorised
-// on the second stream, the step waits for them with an event.
+// one (step_done) and so runs beside the previous step.  Nothing waits on the
+// host.  A call of a small grid is bound by the host's queueing: the scalars
+// go by value, both operators' tables are one launch and their transfer sets
+// another, and a call records and waits for two events each.
+// (16 steps and absorber calls at N = 1000, L = 31: 3.09 -> 2.80 ms; 4 at
+// N = 240, L = 6: 0.79 -> 0.65 ms.)
 int step_impl(qpc_ctx* c, int gauge, double a_i, double a_f) {
     TRY(ready(c, false));
     TRY(alloc_zsets(c));
-    for (auto& e : c->slot_read)
+    for (auto& e : c->step_done)
         if (!e) QPC_HIP_CHECK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
     const bool reuse = c->step_slot >= 0 && c->step_gauge == gauge && c->gauge == gauge && a_i == c->step_a &&
                        c->run_cap >= 3 && c->h_dD.size() >= 3;
@@ -1354,12 +1345,9 @@ int step_impl(qpc_ctx* c, int gauge, double a_i, double a_f) {
         }
         c->h_dD[tf] = dD;
         c->h_dR[tf] = dR;
-        if (c->slot_rec[tf]) QPC_HIP_CHECK(c, hipStreamWaitEvent(c->fstream, c->slot_read[tf], 0));
-        hipLaunchKernelGGL(k_put2, dim3(1), dim3(64), 0, c->fstream, c->d_ifdt + tf, dD, c->d_ifdt + c->run_cap + tf,
-                           dR);
-        TRY(launch_check(c, "step scalars"));
-        QPC_HIP_CHECK(c, hipEventRecord(c->put_done, c->fstream));
-        TRY(factor_batch(c, 0, tf, 1, tf, false, true));
+        if (c->slot_read[tf] >= 0)
+            QPC_HIP_CHECK(c, hipStreamWaitEvent(c->fstream, c->step_done[c->slot_read[tf]], 0));
+        TRY(factor_step(c, tf, dD, dR));
     } else {
         // a fresh pair: scalars of both time points (and room for a third;
         // the streams are idle after set_run_scalars), tables at positions 0
@@ -1371,20 +1359,14 @@ int step_impl(qpc_ctx* c, int gauge, double a_i, double a_f) {
     // a fresh pair waits for both time points' tables; with the t_i tables
     // kept from the previous call (already waited for), the step waits for
     // the t_f tables only where it first reads them
-    hipEvent_t wr = nullptr, wd = nullptr;
-    if (reuse) {
-        wr = c->ts[0].ready_r;
-        wd = c->ts[0].ready;
-    } else {
-        TRY(use_set(c, 0));
-    }
-    if (gauge == 1) TRY(do_step_lg(c, 0, 0, ti, tf, wr));
-    else TRY(do_step(c, 0, 0, ti, tf, false, false, false, wr, wd));
-    for (int k : {ti, tf}) {
-        QPC_HIP_CHECK(c, hipEventRecord(c->slot_read[k], c->stream));
-        c->slot_rec[k] = true;
-    }
-    TRY(release_set(c, 0));
+    hipEvent_t wf = nullptr;
+    if (reuse) wf = c->ts[0].ready;
+    else TRY(use_set(c, 0));
+    if (gauge == 1) TRY(do_step_lg(c, 0, 0, ti, tf, wf));
+    else TRY(do_step(c, 0, 0, ti, tf, false, false, false, wf));
+    QPC_HIP_CHECK(c, hipEventRecord(c->step_done[c->step_next], c->stream));
+    c->slot_read[ti] = c->slot_read[tf] = c->step_next;
+    c->step_next = (c->step_next + 1) % 3;
     c->step_slot = tf;
     c->step_a = a_f;
     c->step_gauge = gauge;

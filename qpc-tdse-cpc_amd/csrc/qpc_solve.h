@@ -213,6 +213,22 @@ void launch_factor_sym(hipStream_t s, const cplx* fx, const double* eig, const d
 void launch_factor_asy(hipStream_t s, const cplx* fx, const double* eig, const double* ifdt, int nt, int nch, Geom geo,
                        double* tab, int64_t eig_tstride = 0, int restart = 0);
 
+// Tables and transfer sets of at most kFactorJobs operators for nt <= 2 time
+// points whose scalars are given by value: table (t, ch) of a job at
+// t * tstride + ch, e = eig[ch] * ifdt[t].  Few tables are one launch for the
+// factors and one for the transfer sets, whatever the number of operators.
+constexpr int kFactorJobs = 4;
+struct FactorJob {
+    int real;  // 1: S + e X (real LU rows), 0: S + i e X (complex symmetric)
+    int nch, restart;
+    const cplx* fx;
+    const double* eig;
+    double ifdt[2];
+    void *tab, *trf;
+    int64_t tstride;
+};
+void launch_factor_jobs(hipStream_t s, const FactorJob* jobs, int n, int nt, Geom geo);
+
 // ---- host ------------------------------------------------------------------
 // Reach of the recurrences of A = S + e X (row-major bands N*(p+1)): asym 0,
 // A = S + i e X with X symmetric; asym 1, A = S + e X with X antisymmetric

@@ -839,13 +839,11 @@ __device__ inline double tsub(double a, double t, double x) { return fma(-t, x, 
 __device__ inline cplx tsub(cplx a, cplx t, cplx x) { return tmsub(a, t, x); }
 
 template <class TF, int P>
-__global__ __launch_bounds__(kLane) void k_transfer(const cplx* __restrict__ tab, TF* __restrict__ trf, Geom geo,
-                                                    int64_t stride) {
+__device__ inline void transfer_cols(const cplx* __restrict__ tab, TF* __restrict__ trf, Geom geo, int64_t t) {
     using F = TabFmt<TF, P>;
     constexpr int NC = trf_cols<TF, P>(), RB = 4;
     const int grp = blockIdx.y % trf_groups<TF, P>();
     const int g = blockIdx.y / trf_groups<TF, P>() * kLane + threadIdx.x;
-    const int64_t t = (int64_t)blockIdx.z * stride + blockIdx.x;  // table index
     if (g >= geo.P) return;
     const int dir = F::SYM ? 0 : grp, c0 = F::SYM ? grp * NC : 0;
     const cplx* T0 = tab + t * F::units(geo) + (dir ? F::boff * kLane : 0);
@@ -891,6 +889,11 @@ __global__ __launch_bounds__(kLane) void k_transfer(const cplx* __restrict__ tab
 #pragma unroll
         for (int c = 0; c < NC; ++c)
             if (c0 + c < P) out[(int64_t)(q * P + c0 + c) * kLane] = H[q][c];
+}
+template <class TF, int P>
+__global__ __launch_bounds__(kLane) void k_transfer(const cplx* __restrict__ tab, TF* __restrict__ trf, Geom geo,
+                                                    int64_t stride) {
+    transfer_cols<TF, P>(tab, trf, geo, (int64_t)blockIdx.z * stride + blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -1011,9 +1014,19 @@ __device__ inline double fmulx(double a, double b) { return a * b; }
 __device__ inline cplx fsubx(cplx a, cplx t, cplx x) { return tmsub(a, t, x); }
 __device__ inline double fsubx(double a, double t, double x) { return fma(-t, x, a); }
 
+// a table's scalar e: its eigenvalue times its time point's ifdt, from the
+// device or (ifdt null, at most two time points) by value
+struct FactorScal {
+    const double *eig, *ifdt;
+    int64_t eig_tstride;
+    double v[2];
+    __device__ double at(int t, int ch) const {
+        return eig[(int64_t)t * eig_tstride + ch] * (ifdt ? ifdt[t] : t ? v[1] : v[0]);
+    }
+};
+
 template <int SYM, int P>
-__global__ __launch_bounds__(kLane, P == 7 ? 2 : 1) void k_factor(const cplx* __restrict__ fx, const double* __restrict__ eig,
-                                                  int64_t eig_tstride, const double* __restrict__ ifdt, Geom geo,
+__global__ __launch_bounds__(kLane, P == 7 ? 2 : 1) void k_factor(const cplx* __restrict__ fx, FactorScal sc0, Geom geo,
                                                   int restart, cplx* __restrict__ tab, int64_t tstride) {
     using T = typename FactorTypes<SYM>::T;
     constexpr int NE = P + 1;
@@ -1024,7 +1037,7 @@ __global__ __launch_bounds__(kLane, P == 7 ? 2 : 1) void k_factor(const cplx* __
     const int ch = blockIdx.y, t = blockIdx.z;
     if (g >= geo.P) return;
     const int FP = factor_cols(geo);
-    const double e = eig[(int64_t)t * eig_tstride + ch] * ifdt[t];
+    const double e = sc0.at(t, ch);
     // SYM 0 writes complex symmetric rows [E_1..E_P, 1/pivot] (for a symmetric
     // matrix the unit upper factor's rows are the columns of L in A = L D L^T);
     // SYM 1 writes real LU rows (forward: the multipliers of the rows below, backward: u)
@@ -1163,18 +1176,15 @@ template <int P>
 constexpr int factor_pe() { return P == 7 ? 8 : 10; }
 inline __host__ __device__ int factor_row_blocks(int above) { return (above + kPM - 1) / kPM + kFactorQ + 1; }
 
+// rows of partitions [g0, g0 + kFactorQ) of one table
 template <int SYM, int P>
-__global__ __launch_bounds__(kLane) void k_factor_row(const cplx* __restrict__ fx, const double* __restrict__ eig,
-                                                      int64_t eig_tstride, const double* __restrict__ ifdt, Geom geo,
-                                                      int above, cplx* __restrict__ tab, int64_t tstride) {
+__device__ inline void factor_row(const cplx* __restrict__ fx, double e, Geom geo, int g0, int above,
+                                  cplx* __restrict__ tab) {
     using T = typename FactorTypes<SYM>::T;
     constexpr int NE = P + 1, PE = factor_pe<P>();
     constexpr int ROW = TabFmt<T, P>::row;
     extern __shared__ __align__(16) double sh[];  // [2][columns][PE]: re, im or upper, lower
-    const int g0 = blockIdx.x * kFactorQ;
-    const int ch = blockIdx.y, t = blockIdx.z;
     const int FP = factor_cols(geo);
-    const double e = eig[(int64_t)t * eig_tstride + ch] * ifdt[t];
     const int ln = threadIdx.x, cl = ln & 7, hf = (ln >> 3) & 1;
     // stage whole blocks of kPM columns from block b0 on, a lane per (block, entry)
     const int nb = factor_row_blocks(above), b0 = g0 - (nb - kFactorQ - 1), half = nb * kPM * PE;
@@ -1205,7 +1215,7 @@ __global__ __launch_bounds__(kLane) void k_factor_row(const cplx* __restrict__ f
     const int first = (g - b0) * kPM - above;  // first row of the restarted elimination
     const double* up = sh + first * PE + (SYM == 0 ? hf * half : 0);
     const double* lo = sh + first * PE + half;
-    char* Tg = (char*)(tab + ((int64_t)t * tstride + ch) * TabFmt<T, P>::units(geo) + part_col<T, P>(g));
+    char* Tg = (char*)(tab + part_col<T, P>(g));
     double w[8];
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
@@ -1281,6 +1291,44 @@ __global__ __launch_bounds__(kLane) void k_factor_row(const cplx* __restrict__ f
     for (; i < above; i += 8) round(i, std::false_type{});
 #pragma unroll 1
     for (; i < above + kPM; i += 8) round(i, std::true_type{});
+}
+
+template <int SYM, int P>
+__global__ __launch_bounds__(kLane) void k_factor_row(const cplx* __restrict__ fx, FactorScal sc, Geom geo, int above,
+                                                      cplx* __restrict__ tab, int64_t tstride) {
+    using T = typename FactorTypes<SYM>::T;
+    const int ch = blockIdx.y, t = blockIdx.z;
+    factor_row<SYM, P>(fx, sc.at(t, ch), geo, blockIdx.x * kFactorQ, above,
+                       tab + ((int64_t)t * tstride + ch) * TabFmt<T, P>::units(geo));
+}
+// The tables, and their transfer sets, of several operators in one launch each:
+// a step called by itself waits for all of them (four operators of N = 361,
+// M = 9, L = 9 in turn: 115 us of its 515).
+struct FactorJobs {
+    FactorJob j[kFactorJobs];
+    int n;
+};
+template <int P>
+__global__ __launch_bounds__(kLane) void k_factor_jobs(FactorJobs a, Geom geo) {
+    int ch = blockIdx.y, k = 0;
+    while (k + 1 < a.n && ch >= a.j[k].nch) ch -= a.j[k++].nch;
+    const FactorJob& J = a.j[k];
+    const int t = blockIdx.z, g0 = blockIdx.x * kFactorQ;
+    const double e = J.eig[ch] * (t ? J.ifdt[1] : J.ifdt[0]);
+    const int64_t q = (int64_t)t * J.tstride + ch;
+    const int above = (J.restart + 7) / 8 * 8;
+    if (J.real) factor_row<1, P>(J.fx, e, geo, g0, above, (cplx*)J.tab + q * TabFmt<double, P>::units(geo));
+    else factor_row<0, P>(J.fx, e, geo, g0, above, (cplx*)J.tab + q * TabFmt<cplx, P>::units(geo));
+}
+template <int P>
+__global__ __launch_bounds__(kLane) void k_transfer_jobs(FactorJobs a, Geom geo) {
+    static_assert(trf_groups<cplx, P>() == trf_groups<double, P>(), "one grid");
+    int ch = blockIdx.x, k = 0;
+    while (k + 1 < a.n && ch >= a.j[k].nch) ch -= a.j[k++].nch;
+    const FactorJob& J = a.j[k];
+    const int64_t q = (int64_t)blockIdx.z * J.tstride + ch;
+    if (J.real) transfer_cols<double, P>((const cplx*)J.tab, (double*)J.trf, geo, q);
+    else transfer_cols<cplx, P>((const cplx*)J.tab, (cplx*)J.trf, geo, q);
 }
 
 // fx[(s * (p+1) + j) * FP + g] = {S, X}(c-j, c) of column c = 24 g + s, zero
@@ -1487,33 +1535,82 @@ void launch_factor_bands(hipStream_t s, const double* S, const double* X, cplx* 
     hipLaunchKernelGGL(k_factor_bands, dim3((total + 255) / 256), dim3(256), 0, s, S, X, fx, geo.N, geo.hw + 1,
                        factor_cols(geo));
 }
+// restart rows and waves within k_factor_row's range
+static int row_above(int restart) { return ((restart > 0 ? restart : kRestart) + 7) / 8 * 8; }
+static int row_groups(const Geom& geo) { return (geo.P + kFactorQ - 1) / kFactorQ; }
+static bool row_fits(const Geom& geo, int64_t tables, int above) {
+    return row_groups(geo) * tables <= kFactorRowWaves && above <= kFactorRowAbove;
+}
+template <int P>
+static size_t row_lds(int above) { return sizeof(double) * 2 * factor_row_blocks(above) * kPM * factor_pe<P>(); }
+
 template <int SYM, int P>
-static void factor_launch_p(hipStream_t s, const cplx* fx, const double* eig, const double* ifdt, int nt, int nch,
-                            Geom geo, cplx* tab, int64_t eig_tstride, int rs, int64_t ts) {
-    const int above = (rs + 7) / 8 * 8;
-    const int64_t groups = (geo.P + kFactorQ - 1) / kFactorQ;
-    if (groups * nch * nt <= kFactorRowWaves && above <= kFactorRowAbove)
-        hipLaunchKernelGGL((k_factor_row<SYM, P>), dim3((unsigned)groups, nch, nt), dim3(kLane),
-                           sizeof(double) * 2 * factor_row_blocks(above) * kPM * factor_pe<P>(), s, fx, eig, eig_tstride, ifdt,
-                           geo, above, tab, ts);
+static void factor_launch_p(hipStream_t s, const cplx* fx, const FactorScal& sc, int nt, int nch, Geom geo, cplx* tab,
+                            int restart, int64_t ts) {
+    const int above = row_above(restart);
+    if (row_fits(geo, (int64_t)nch * nt, above))
+        hipLaunchKernelGGL((k_factor_row<SYM, P>), dim3(row_groups(geo), nch, nt), dim3(kLane), row_lds<P>(above), s, fx,
+                           sc, geo, above, tab, ts);
     else
-        hipLaunchKernelGGL((k_factor<SYM, P>), dim3(geo.NG, nch, nt), dim3(kLane), 0, s, fx, eig, eig_tstride, ifdt,
-                           geo, rs, tab, ts);
+        hipLaunchKernelGGL((k_factor<SYM, P>), dim3(geo.NG, nch, nt), dim3(kLane), 0, s, fx, sc, geo,
+                           restart > 0 ? restart : kRestart, tab, ts);
 }
 template <int SYM>
-static void factor_launch(hipStream_t s, const cplx* fx, const double* eig, const double* ifdt, int nt, int nch, Geom geo,
-                          cplx* tab, int64_t eig_tstride, int restart, int64_t ts) {
-    const int rs = restart > 0 ? restart : kRestart;
-    if (geo.hw == 8) factor_launch_p<SYM, 8>(s, fx, eig, ifdt, nt, nch, geo, tab, eig_tstride, rs, ts);
-    else factor_launch_p<SYM, 7>(s, fx, eig, ifdt, nt, nch, geo, tab, eig_tstride, rs, ts);
+static void factor_launch(hipStream_t s, const cplx* fx, const FactorScal& sc, int nt, int nch, Geom geo, cplx* tab,
+                          int restart, int64_t ts) {
+    if (geo.hw == 8) factor_launch_p<SYM, 8>(s, fx, sc, nt, nch, geo, tab, restart, ts);
+    else factor_launch_p<SYM, 7>(s, fx, sc, nt, nch, geo, tab, restart, ts);
 }
 void launch_factor_sym(hipStream_t s, const cplx* fx, const double* eig, const double* ifdt, int nt, int nch, Geom geo,
                        cplx* tab, int64_t eig_tstride, int restart, int64_t tab_tstride) {
-    factor_launch<0>(s, fx, eig, ifdt, nt, nch, geo, tab, eig_tstride, restart, tab_tstride > 0 ? tab_tstride : nch);
+    factor_launch<0>(s, fx, FactorScal{eig, ifdt, eig_tstride, {}}, nt, nch, geo, tab, restart,
+                     tab_tstride > 0 ? tab_tstride : nch);
 }
 void launch_factor_asy(hipStream_t s, const cplx* fx, const double* eig, const double* ifdt, int nt, int nch, Geom geo,
                        double* tab, int64_t eig_tstride, int restart) {
-    factor_launch<1>(s, fx, eig, ifdt, nt, nch, geo, (cplx*)tab, eig_tstride, restart, nch);
+    factor_launch<1>(s, fx, FactorScal{eig, ifdt, eig_tstride, {}}, nt, nch, geo, (cplx*)tab, restart, nch);
+}
+
+template <int P>
+static void factor_jobs(hipStream_t s, const FactorJobs& a, int nt, const Geom& geo) {
+    int rows = 0, above = 0;
+    bool fit = true;  // each by itself: together they take no longer than one after the other
+    for (int k = 0; k < a.n; ++k) {
+        rows += a.j[k].nch;
+        above = std::max(above, row_above(a.j[k].restart));
+        fit = fit && row_fits(geo, (int64_t)a.j[k].nch * nt, row_above(a.j[k].restart));
+    }
+    if (fit) {
+        hipLaunchKernelGGL(k_factor_jobs<P>, dim3(row_groups(geo), rows, nt), dim3(kLane), row_lds<P>(above), s, a, geo);
+        hipLaunchKernelGGL(k_transfer_jobs<P>, dim3(rows, geo.NG * trf_groups<cplx, P>(), nt), dim3(kLane), 0, s, a, geo);
+        return;
+    }
+    for (int k = 0; k < a.n; ++k) {
+        const FactorJob& J = a.j[k];
+        const FactorScal sc{J.eig, nullptr, 0, {J.ifdt[0], J.ifdt[1]}};
+        const dim3 tg(J.nch, geo.NG * trf_groups<cplx, P>(), nt);
+        if (J.real) {
+            factor_launch_p<1, P>(s, J.fx, sc, nt, J.nch, geo, (cplx*)J.tab, J.restart, J.tstride);
+            hipLaunchKernelGGL((k_transfer<double, P>), tg, dim3(kLane), 0, s, (const cplx*)J.tab, (double*)J.trf, geo,
+                               J.tstride);
+        } else {
+            factor_launch_p<0, P>(s, J.fx, sc, nt, J.nch, geo, (cplx*)J.tab, J.restart, J.tstride);
+            hipLaunchKernelGGL((k_transfer<cplx, P>), tg, dim3(kLane), 0, s, (const cplx*)J.tab, (cplx*)J.trf, geo,
+                               J.tstride);
+        }
+    }
+}
+void launch_factor_jobs(hipStream_t s, const FactorJob* jobs, int n, int nt, Geom geo) {
+    FactorJobs a{};
+    for (int k = 0; k < n && a.n < kFactorJobs; ++k)
+        if (jobs[k].nch > 0) {
+            a.j[a.n] = jobs[k];
+            if (a.j[a.n].restart <= 0) a.j[a.n].restart = kRestart;
+            ++a.n;
+        }
+    if (a.n == 0) return;
+    if (geo.hw == 8) factor_jobs<8>(s, a, nt, geo);
+    else factor_jobs<7>(s, a, nt, geo);
 }
 
 // ---------------------------------------------------------------------------

@@ -101,3 +101,33 @@ def test_batched_and_single_time_points_agree(p):
     print(f"  rel L2 {err:.2e}", flush=True)
     assert err <= 1e-12
     prop.close()
+
+
+@pytest.mark.parametrize("gauge", ["vgwr", "lgwr"])
+def test_queued_elliptical_steps_match_the_run(gauge):
+    """Elliptical steps called one by one return when queued, each call's
+    tables in the other of two sets: seven steps in a row against the run's."""
+    import pyoracle as po
+    M, L, N, n = 5, 6, 150, 7
+    print(f"case: queued elliptical steps {gauge}", flush=True)
+    o, prop = _pair(N, 7, L, M, -2)
+    f = 0.6 if gauge == "vgwr" else 0.05
+    ax, ay = (f * np.cos(0.4 * np.arange(n + 1) + ph) for ph in (0.0, 1.1))
+    if gauge == "vgwr":
+        prop.upload_angular_ep(po.ep_angular(M, L, -2))
+        step, run = prop.propagate_ep, prop.run_ep
+    else:
+        prop.upload_angular_lgwr(po.lgwr_angular(M, L, -2))
+        step, run = prop.propagate_lgwr, prop.run_lgwr
+    c = mixed_state(o, seed=3, amp=0.3)
+    prop.set_state(c)
+    run(ax, ay, n, 0, n, use_mask=True)
+    ref = prop.get_state().copy()
+    prop.set_state(c)
+    for k in range(n):
+        step(ax[k], ax[k + 1], ay[k], ay[k + 1])
+        prop.mask()
+    err = rel_l2(prop.get_state(), ref)
+    print(f"  rel L2 {err:.2e}", flush=True)
+    assert err <= 1e-12
+    prop.close()
