@@ -674,6 +674,8 @@ int qpc_destroy(qpc_ctx* c) {
     for (hipEvent_t e : c->ev) (void)hipEventDestroy(e);
     for (hipEvent_t e : c->step_done)
         if (e) (void)hipEventDestroy(e);
+    if (c->kev) (void)hipEventDestroy(c->kev);
+    if (c->kab) (void)hipHostFree(c->kab);
     if (c->rmap) (void)hipFree(c->rmap);
     if (c->rorder) (void)hipFree(c->rorder);
     if (c->dorder.d) (void)hipFree(c->dorder.d);
@@ -694,7 +696,7 @@ int qpc_destroy(qpc_ctx* c) {
                     c->rpow1d, c->sxR, c->sxD, c->sxL, c->fxR, c->fxD, c->fxL, c->tsf_ib, c->tsf_b0, c->tsf_br, c->tsf_kr, c->tsf_ckt,
                     c->tsf_j0, c->tsf_jr, c->tsf_pm, c->tsf_Y, c->tsf_tmp, c->tsf_work, c->tsf_stx, c->tsf_sty,
                     c->tsf_pm1, c->tsf_pm2, c->rtY, c->rtYt, c->rtM, c->rtMh, c->rtQ, c->rtQh,
-                    c->Wp, c->ppart, c->pchan, c->pcnt, c->pout, c->Hd, c->q10, c->kU, c->kpart, c->kcoef,
+                    c->Wp, c->ppart, c->pchan, c->pcnt, c->pout, c->Hd, c->q10, c->kU, c->kpart, c->kcoef, c->knorm,
                     c->souter, c->accel, c->hist, c->red4, c->obs_tmp, c->pcs_Wp, c->pcs_part, c->pcs_chan,
                     c->pcs_cnt, c->pcs_cps, c->pcs_out, c->pcs_lmd};
     for (void* p : ptrs)
@@ -1635,19 +1637,6 @@ int qpc_upload_krylov(qpc_ctx* c, const double* H, const double* y10, const doub
 }
 
 namespace {
-// sum_ml <v|S|v> with the per-channel partials of k_norm, summed in order
-int snorm(qpc_ctx* c, const cplx* v, double* out) {
-    qpc::launch_norm(c->stream, c->S, v, c->red, c->ML, c->N, c->p);
-    TRY(launch_check(c, "snorm"));
-    std::vector<double> h(c->ML);
-    QPC_HIP_CHECK(c, hipMemcpyAsync(h.data(), c->red, sizeof(double) * c->ML, hipMemcpyDeviceToHost, c->stream));
-    QPC_HIP_CHECK(c, hipStreamSynchronize(c->stream));
-    double s = 0.0;
-    for (int64_t i = 0; i < c->ML; ++i) s += h[i];
-    *out = s;
-    return QPC_OK;
-}
-
 // propagate_sub (la_1e.hpp:157-182) for the leading m x m block of the
 // Lanczos tridiagonal (a, b): xs = b0 Z e^{-i dt Lambda} Z^T e0
 int lanczos_coefs(int64_t m, const std::vector<double>& a, const std::vector<double>& b, double dt,
@@ -1688,79 +1677,73 @@ int krylov_core(qpc_ctx* c, double az, double dt, int64_t kstart, int64_t kmax, 
     QPC_HIP_CHECK(c, hipStreamSynchronize(c->fstream));
     if (kmax + 2 > c->kry_cap) {
         QPC_HIP_CHECK(c, hipStreamSynchronize(c->stream));
-        void* old[] = {c->kU, c->kpart, c->kcoef};
+        void* old[] = {c->kU, c->kpart, c->kcoef, c->knorm};
         for (void* p : old)
             if (p) QPC_HIP_CHECK(c, hipFree(p));
+        if (c->kab) QPC_HIP_CHECK(c, hipHostFree(c->kab));
         c->kU = c->kpart = c->kcoef = nullptr;
+        c->knorm = c->kab = nullptr;
         c->kry_cap = 0;
         int rc = QPC_OK;
         if ((rc = dev_alloc(c, &c->kU, (size_t)(kmax + 2) * n)) ||
             (rc = dev_alloc(c, &c->kpart, (size_t)(kmax + 2) * qpc::kDotBlocks)) ||
-            (rc = dev_alloc(c, &c->kcoef, (size_t)(kmax + 2))))
+            (rc = dev_alloc(c, &c->kcoef, (size_t)(kmax + 2))) || (rc = dev_alloc(c, &c->knorm, qpc::kNormBlocks)))
             return rc;
+        QPC_HIP_CHECK(c, hipHostMalloc((void**)&c->kab, sizeof(double) * 2 * (kmax + 2)));
+        if (!c->kev) QPC_HIP_CHECK(c, hipEventCreateWithFlags(&c->kev, hipEventDisableTiming));
         c->kry_cap = kmax + 2;
     }
     TimedLaunch tl(c, QPC_K_KRYLOV);
     auto U = [&](int64_t i) { return c->kU + i * n; };
-    cplx* T = c->vbuf;  // H u_{k-1}
+    cplx* T = c->vbuf;   // H u_{k-1}
+    cplx* W = c->tmpc;   // S^-1 T
+    cplx* V = c->spare;  // the next vector before its normalisation
     std::vector<double> a(kmax + 2, 0.0), b(kmax + 2, 0.0);
-    std::vector<cplx> x(kmax + 2), part((size_t)(kmax + 2) * qpc::kDotBlocks), xs;
+    std::vector<cplx> xs;
     const qpc::TabMap tm{1, (int)c->L, (int)c->m0};
-    // construct_sub (la_1e.hpp:134-154)
-    QPC_HIP_CHECK(c, hipMemcpyAsync(U(0), c->coef, sizeof(cplx) * n, hipMemcpyDeviceToDevice, c->stream));
-    double nrm = 0.0;
-    TRY(snorm(c, U(0), &nrm));
-    if (!(nrm > 0.0)) {
-        c->set_error("zero state");
-        return QPC_E_NUMERIC;
-    }
-    nrm = std::sqrt(nrm);
-    qpc::launch_scale(c->stream, U(0), 1.0 / nrm, n);
-    b[0] = nrm;
-    // Lanczos loop (la_1e.hpp:318-328), orthogonalize_ip (:195-240)
-    bool more = true;
+    const int N = (int)c->N, ML = (int)c->ML, p = (int)c->p;
+    // construct_sub (la_1e.hpp:134-154): the norm of the state
+    qpc::launch_axpy_norm(c->stream, nullptr, 0, 0, nullptr, nullptr, c->Sd, c->coef, nullptr, N, ML, p, c->knorm);
+    // Lanczos loop (la_1e.hpp:318-328), orthogonalize_ip (:195-240).  Vector k
+    // is queued whole; then the host waits for its norm b[k] (there after the
+    // first of its kernels) and judges the k vectors before it while the rest
+    // of its kernels run: those are wasted once, when the subspace ends.
     int64_t m = 0;
-    while (more && m < kmax) {
-        qpc::launch_hmul(c->stream, c->Hd, c->rinvd, c->rdifd, c->y10, c->q10, az, (int)c->M, (int)c->L, (int)c->m0,
-                         (int)c->N, (int)c->p, U(m), T);
-        const int64_t k = ++m;
-        qpc::launch_dots(c->stream, c->kU, n, (int)k, T, n, c->kpart);
-        TRY(launch_check(c, "krylov dots"));
-        QPC_HIP_CHECK(c, hipMemcpyAsync(part.data(), c->kpart, sizeof(cplx) * k * qpc::kDotBlocks,
-                                        hipMemcpyDeviceToHost, c->stream));
-        // S \ (H u_{k-1}) into u_k, channel by channel (chol(S) tables)
-        qpc::launch_bsolve_r(c->stream, qpc::RHS_RBAND, c->tab_mask, c->trf_mask, tm, T, U(k), (int)c->ML, c->geo);
-        QPC_HIP_CHECK(c, hipStreamSynchronize(c->stream));
-        std::vector<cplx> cf(k);
-        for (int64_t i = 0; i < k; ++i) {
-            cplx s = {0.0, 0.0};
-            for (int q = 0; q < qpc::kDotBlocks; ++q) s += part[(size_t)i * qpc::kDotBlocks + q];
-            x[i] = s;
-            const bool use = i == k - 1 || (s.re * s.re + s.im * s.im) > 4e-27;
-            cf[i] = use ? s : cplx{0.0, 0.0};
-        }
-        QPC_HIP_CHECK(c, hipMemcpyAsync(c->kcoef, cf.data(), sizeof(cplx) * k, hipMemcpyHostToDevice, c->stream));
-        qpc::launch_axpy_multi(c->stream, c->kU, n, (int)k, c->kcoef, U(k), n);
-        double nk = 0.0;
-        TRY(snorm(c, U(k), &nk));  // synchronises: cf may be released after
-        bool stop = false;
-        if (nk < 1e-13) {
-            nk = 0.0;
-            stop = true;
+    for (int64_t k = 0;; ++k) {
+        if (k < kmax) {
+            qpc::launch_hmul(c->stream, c->Hd, c->rinvd, c->rdifd, c->y10, c->q10, az, (int)c->M, (int)c->L, (int)c->m0,
+                             N, p, k ? V : c->coef, c->knorm, k == 0, c->kab + 2 * k + 1, U(k), T);
+            QPC_HIP_CHECK(c, hipEventRecord(c->kev, c->stream));
+            qpc::launch_dots(c->stream, c->kU, n, (int)k + 1, T, n, c->kpart);
+            // S \ (H u_k), channel by channel (chol(S) tables)
+            qpc::launch_bsolve_r(c->stream, qpc::RHS_RBAND, c->tab_mask, c->trf_mask, tm, T, W, ML, c->geo);
+            qpc::launch_axpy_norm(c->stream, c->kU, n, (int)k + 1, c->kpart, c->kab + 2 * k, c->Sd, W, V, N, ML, p,
+                                  c->knorm);
         } else {
-            nk = std::sqrt(nk);
-            qpc::launch_scale(c->stream, U(k), 1.0 / nk, n);
+            qpc::launch_norm_final(c->stream, N, ML, c->knorm, c->kab + 2 * k + 1);
+            QPC_HIP_CHECK(c, hipEventRecord(c->kev, c->stream));
         }
-        a[k - 1] = x[k - 1].re;
-        b[k] = nk;
-        more = !stop;
+        TRY(launch_check(c, "krylov vector"));
+        QPC_HIP_CHECK(c, hipEventSynchronize(c->kev));
+        const volatile double* ab_h = c->kab;
+        b[k] = ab_h[2 * k + 1];
+        if (k == 0) {
+            if (!(b[0] > 0.0)) {
+                c->set_error("zero state");
+                return QPC_E_NUMERIC;
+            }
+            continue;
+        }
+        m = k;
+        a[k - 1] = ab_h[2 * k - 2];
+        if (b[k] == 0.0 || k == kmax) break;
         // subspace extension judged by the a-posteriori estimate
-        if (more && tol >= 0.0 && k >= kstart) {
+        if (tol >= 0.0 && k >= kstart) {
             if (lanczos_coefs(k, a, b, dt, xs)) {
                 c->set_error("tridiagonal eigen-solve failed");
                 return QPC_E_NUMERIC;
             }
-            if (estimate(k, xs) <= tol) more = false;
+            if (estimate(k, xs) <= tol) break;
         }
     }
     if (lanczos_coefs(m, a, b, dt, xs)) {

@@ -131,3 +131,26 @@ def test_queued_elliptical_steps_match_the_run(gauge):
     print(f"  rel L2 {err:.2e}", flush=True)
     assert err <= 1e-12
     prop.close()
+
+
+@pytest.mark.parametrize("p", [7, 8])
+@pytest.mark.parametrize("N,L,kmax", [(18, 1, 1), (33, 2, 3), (127, 3, 8), (128, 3, 9), (129, 2, 8), (255, 1, 8),
+                                      (256, 3, 2), (257, 3, 8), (700, 2, 12)])
+def test_krylov_step_at_tile_edges(N, L, kmax, p):
+    """The Lanczos vector's kernels around their tiles of 128 and 256 rows
+    (with p rows on either side), one channel and several, subspaces from one
+    vector on.  Bar: 1e-10, as the other sizes' in test_gpu_parity."""
+    import pyoracle as po
+    print(f"case: krylov edges N={N} L={L} p={p} kmax={kmax}", flush=True)
+    o, prop = _pair(N, p, L)
+    prop.upload_krylov(o.get(po.QOR_H), o.get(po.QOR_Y10), o.get(po.QOR_Q10))
+    c = mixed_state(o, seed=N + p, amp=0.3)
+    ref = c.copy()
+    _, m_o, eps_o, ab_o = o.krylov_step(ref, 0.7, 0.002, kmax=kmax)
+    prop.set_state(c)
+    _, m, eps = prop.krylov_step(0.7, 0.002, kmax=kmax)
+    err = rel_l2(prop.get_state(), ref)
+    print(f"  m={m}/{m_o} eps={eps:.2e}/{eps_o:.2e} rel L2 {err:.2e}", flush=True)
+    assert m == m_o
+    assert err <= 1e-10
+    prop.close()
