@@ -266,8 +266,6 @@ __device__ inline double sinexp(int which, int m, int l) {
     if (which == 3) return -sqrt(q((double)(l + m) * (l + m - 1), (double)(2 * l + 1) * (2 * l - 1)));
     return +sqrt(q((double)(l - m + 2) * (l - m + 1), (double)(2 * l + 1) * (2 * l + 3)));
 }
-__device__ inline cplx cmulc(cplx a, cplx b) { return mulc(a, b); }  // a * conj(b)
-
 // the observables of launch_observe for one channel per block: partial q of
 // channel iml at red[q * ML + iml].  observable_r (observable/1e.hpp:76-126):
 // channel (m, l) couples to (m+1, l+-1) in observe_rm (sinexp1 outer,
@@ -275,90 +273,174 @@ __device__ inline cplx cmulc(cplx a, cplx b) { return mulc(a, b); }  // a * conj
 // for l-1), the partner channel existing when in_check finds it in the grid
 // (dimension/1e.hpp:97-100); the channel's share of <x> is Re(rm + rp)/2 and
 // of <y> Im(rp - rm)/2.
-__global__ __launch_bounds__(kRedThreads) void k_observe(ObsBands b, int flags, const cplx* __restrict__ coef,
+//
+// A recorded run waits for this kernel before every step, and a channel's rows
+// are few: what bounds it is the latency of its loads.  One thread takes a row
+// (1024 at a time) with the stored upper half of the symmetric bands, a row of
+// contiguous entries requested at once: sum_i conj(x_i) (B y)_i is the sum
+// over the pairs (i, i + j).  The partners of a coupling are added up first,
+// so that each band is applied to one vector, from LDS; bands of one coupling
+// share the pairs' products.  N = 1000, L = 31, four observables: 10.9 us, the
+// sum over the channels 4.4 us (15 entries per row and vector, gathered with a
+// stride of a row: 54 and 7.6 us).
+constexpr int kObsThreads = 1024;
+struct ObsCouple {
+    const cplx* p[2];  // partners (null: none) and their coefficients
+    double c[2];
+    __device__ cplx at(int r) const {
+        cplx t = {0.0, 0.0};
+        if (p[0]) t += p[0][r] * c[0];
+        if (p[1]) t += p[1][r] * c[1];
+        return t;
+    }
+};
+// row i of a band: the diagonal and the entries to its right
+template <int NE>
+__device__ inline void obs_band(double (&b)[NE], const double* __restrict__ B, int i) {
+    if constexpr (NE % 2 == 0) {  // (a row's address is a multiple of 16 bytes)
+        const double2* q = (const double2*)(B + (int64_t)i * NE);
+#pragma unroll
+        for (int k = 0; k < NE / 2; ++k) {
+            const double2 v = q[k];
+            b[2 * k] = v.x;
+            b[2 * k + 1] = v.y;
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < NE; ++k) b[k] = B[(int64_t)i * NE + k];
+    }
+}
+// sums of K values over the waves of the block; thread q < K returns value q
+template <int K>
+__device__ inline double obs_sums(double (&v)[K], double (*sw)[kObsThreads / 64]) {
+#pragma unroll
+    for (int st = 32; st > 0; st >>= 1)
+#pragma unroll
+        for (int q = 0; q < K; ++q) v[q] += __shfl_xor(v[q], st);
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int q = 0; q < K; ++q) sw[q][threadIdx.x >> 6] = v[q];
+    __syncthreads();
+    double a = 0.0;
+    if ((int)threadIdx.x < K)
+        for (int w = 0; w < kObsThreads / 64; ++w) a += sw[threadIdx.x][w];
+    return a;
+}
+
+// XY: observable_r (flags 16, 32), else the z observables (flags 1, 2, 4, 8)
+template <int NE, bool XY>
+__global__ __launch_bounds__(kObsThreads) void k_observe(ObsBands b, int flags, const cplx* __restrict__ coef,
                                                          double* __restrict__ red, int M, int L, int m0, int N,
-                                                         int ne, int ML) {
-    const int iml = blockIdx.x;
+                                                         int ML) {
+    constexpr int NY = XY ? 2 : 1, K = XY ? 8 : 4;
+    __shared__ cplx sx[kObsThreads + NE], sy[NY][kObsThreads + NE];
+    __shared__ double sw[K][kObsThreads / 64];
+    const int iml = blockIdx.x, tid = threadIdx.x;
     const int im = iml / L, il = iml % L;
     const int m = im + m0, l = il + (m < 0 ? -m : m);
     const cplx* x = coef + (int64_t)iml * N;
-    const cplx* base = coef + (int64_t)im * L * N;
-    const cplx* lo = il > 0 ? base + (int64_t)(il - 1) * N : nullptr;
-    const cplx* hi = il + 1 < L ? base + (int64_t)(il + 1) * N : nullptr;
-    const double ylo = il > 0 ? b.y10[im * L + il - 1] : 0.0, yhi = il + 1 < L ? b.y10[im * L + il] : 0.0;
-    // observable_r partners: k = 0, 1 (rm: m+1, l+1 / l-1), k = 2, 3 (rp: m-1, l+1 / l-1)
-    const cplx* nb[4] = {nullptr, nullptr, nullptr, nullptr};
-    double nc[4] = {0.0, 0.0, 0.0, 0.0};
-    if (flags & 48) {
-        const int dm[4] = {+1, +1, -1, -1}, dl[4] = {+1, -1, +1, -1}, fw[4] = {1, 2, 4, 3};
-        for (int k = 0; k < 4; ++k) {
-            const int im2 = im + dm[k];
-            if (im2 < 0 || im2 >= M) continue;
-            const int m2 = im2 + m0;
-            const int il2 = l + dl[k] - (m2 < 0 ? -m2 : m2);
-            if (il2 < 0 || il2 >= L) continue;
-            nb[k] = coef + ((int64_t)im2 * L + il2) * N;
-            nc[k] = sinexp(fw[k], m, l);
-        }
+    ObsCouple cp[NY];  // z: l -+ 1; XY: rm (m+1) and rp (m-1), l+1 and l-1 each
+    if constexpr (!XY) {
+        cp[0].p[0] = il > 0 ? x - N : nullptr;
+        cp[0].p[1] = il + 1 < L ? x + N : nullptr;
+        cp[0].c[0] = il > 0 && (flags & 6) ? b.y10[iml - 1] : 0.0;
+        cp[0].c[1] = il + 1 < L && (flags & 6) ? b.y10[iml] : 0.0;
+    } else {
+        const int fw[2][2] = {{1, 2}, {4, 3}};
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const int im2 = im + (f ? -1 : 1), m2 = im2 + m0;
+                const int il2 = l + (k ? -1 : 1) - (m2 < 0 ? -m2 : m2);
+                const bool in = im2 >= 0 && im2 < M && il2 >= 0 && il2 < L;
+                cp[f].p[k] = in ? coef + ((int64_t)im2 * L + il2) * N : nullptr;
+                cp[f].c[k] = in ? sinexp(fw[f][k], m, l) : 0.0;
+            }
     }
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    cplx rr[2][2] = {{{0.0, 0.0}, {0.0, 0.0}}, {{0.0, 0.0}, {0.0, 0.0}}};  // [R or A][rm or rp]
-    for (int i = threadIdx.x; i < N; i += blockDim.x) {
-        const cplx xi = x[i];
-        if (flags & 1) acc[0] += mulc(band_row(b.S, x, i, N, ne), xi).re;
-        if (flags & 2) {
-            if (lo) acc[1] += mulc(band_row(b.R, lo, i, N, ne), xi).re * ylo;
-            if (hi) acc[1] += mulc(band_row(b.R, hi, i, N, ne), xi).re * yhi;
+    const bool own = !XY && (flags & 9), cross = XY || (flags & 6);
+    double acc[K] = {};
+    for (int r0 = 0; r0 < N; r0 += kObsThreads) {
+        const int i = r0 + tid, ic = min(i, N - 1);
+        // bands of the two kinds: {S, W} with x itself, {R, A} with the partners
+        double bs[NE], bw[NE], br[NE], ba[NE];
+        if (!XY && (flags & 1)) obs_band<NE>(bs, b.S, ic);
+        if (!XY && (flags & 8)) obs_band<NE>(bw, b.W, ic);
+        if (flags & (XY ? 16 : 2)) obs_band<NE>(br, b.R, ic);
+        if (flags & (XY ? 32 : 4)) obs_band<NE>(ba, b.A, ic);
+        for (int e = tid; e < kObsThreads + NE; e += kObsThreads) {
+            const int r = r0 + e;
+            sx[e] = r < N ? x[r] : cplx{0.0, 0.0};
+            if (cross)
+#pragma unroll
+                for (int f = 0; f < NY; ++f) sy[f][e] = r < N ? cp[f].at(r) : cplx{0.0, 0.0};
         }
-        if (flags & 4) {
-            if (lo) acc[2] += mulc(band_row(b.A, lo, i, N, ne), xi).re * ylo;
-            if (hi) acc[2] += mulc(band_row(b.A, hi, i, N, ne), xi).re * yhi;
-        }
-        if (flags & 8) acc[3] += mulc(band_row(b.W, x, i, N, ne), xi).re;
-        for (int f = 0; f < 2; ++f) {
-            if (!(flags & (16 << f))) continue;
-            const double* band = f ? b.A : b.R;
-            for (int k = 0; k < 4; ++k)
-                if (nb[k]) rr[f][k / 2] += cmulc(band_row(band, nb[k], i, N, ne), xi) * nc[k];
-        }
-    }
-    for (int q = 0; q < 4; ++q)
-        if (flags & (1 << q)) {
-            const double s = block_sum(acc[q]);
-            if (threadIdx.x == 0) red[(int64_t)q * ML + iml] = s;
-            __syncthreads();  // block_sum's buffer is reused by the next sum
-        }
-    for (int f = 0; f < 2; ++f)
-        if (flags & (16 << f)) {
-            double v[4];
-            v[0] = block_sum(rr[f][0].re);
-            __syncthreads();
-            v[1] = block_sum(rr[f][0].im);
-            __syncthreads();
-            v[2] = block_sum(rr[f][1].re);
-            __syncthreads();
-            v[3] = block_sum(rr[f][1].im);
-            __syncthreads();
-            if (threadIdx.x == 0) {
-                red[(int64_t)(4 + 2 * f) * ML + iml] = 0.5 * (v[0] + v[2]);  // Re(rm + rp) / 2
-                red[(int64_t)(5 + 2 * f) * ML + iml] = 0.5 * (v[3] - v[1]);  // Im(rp - rm) / 2
+        __syncthreads();
+        if (i < N) {
+            const cplx xi = sx[tid];
+#pragma unroll
+            for (int j = 0; j < NE; ++j) {
+                const cplx xj = sx[tid + j];
+                if (own) {
+                    const double d = (j ? 2.0 : 1.0) * (xi.re * xj.re + xi.im * xj.im);
+                    if (flags & 1) acc[0] += bs[j] * d;
+                    if (flags & 8) acc[3] += bw[j] * d;
+                }
+                if (cross)
+#pragma unroll
+                    for (int f = 0; f < NY; ++f) {
+                        // y_{i+j} conj(x_i), and for j > 0 y_i conj(x_{i+j})
+                        const cplx yj = sy[f][tid + j], yi = sy[f][tid];
+                        double re = yj.re * xi.re + yj.im * xi.im, im = yj.im * xi.re - yj.re * xi.im;
+                        if (j) {
+                            re += yi.re * xj.re + yi.im * xj.im;
+                            im += yi.im * xj.re - yi.re * xj.im;
+                        }
+                        if constexpr (!XY) {
+                            if (flags & 2) acc[1] += br[j] * re;
+                            if (flags & 4) acc[2] += ba[j] * re;
+                        } else {
+                            // Re(rm + rp) / 2 and Im(rp - rm) / 2
+                            if (flags & 16) {
+                                acc[2 * f] += br[j] * re;
+                                acc[2 * f + 1] += br[j] * im;
+                            }
+                            if (flags & 32) {
+                                acc[4 + 2 * f] += ba[j] * re;
+                                acc[5 + 2 * f] += ba[j] * im;
+                            }
+                        }
+                    }
             }
         }
-}
-
-// out[q] = sum over channels of red[q * ML + ch] (strided partials, then a
-// fixed tree); 0 where the observable is not requested
-__device__ inline bool obs_slot_on(int flags, int q) { return q < 4 ? (flags >> q) & 1 : (flags >> (4 + (q - 4) / 2)) & 1; }
-__global__ __launch_bounds__(kRedThreads) void k_observe_sum(const double* __restrict__ red, int flags, int ML,
-                                                             double* __restrict__ out) {
-    for (int q = 0; q < kObs; ++q) {
-        double a = 0.0;
-        if (obs_slot_on(flags, q))
-            for (int i = threadIdx.x; i < ML; i += blockDim.x) a += red[(int64_t)q * ML + i];
-        const double s = block_sum(a);
-        if (threadIdx.x == 0) out[q] = s;
         __syncthreads();
     }
+    const double s = obs_sums<K>(acc, sw);
+    if constexpr (!XY) {
+        if (tid < 4 && (flags & (1 << tid))) red[(int64_t)tid * ML + iml] = s;
+    } else if (tid < 64) {
+        // thread 4 f + {0, 1, 2, 3}: Re rm, Im rm, Re rp, Im rp of observable f
+        const double o = __shfl(s, (int)threadIdx.x + 2);
+        const int f = tid / 4, k = tid % 4;
+        if (tid < 8 && k < 2 && (flags & (16 << f)))
+            red[(int64_t)(4 + 2 * f + k) * ML + iml] = k ? 0.5 * (o - s) : 0.5 * (s + o);
+    }
+}
+
+// out[q] = sum over channels of red[q * ML + ch], a wave per observable
+// (strided partials, then a fixed tree); 0 where the observable is not requested
+__device__ inline bool obs_slot_on(int flags, int q) { return q < 4 ? (flags >> q) & 1 : (flags >> (4 + (q - 4) / 2)) & 1; }
+__global__ __launch_bounds__(64 * kObs) void k_observe_sum(const double* __restrict__ red, int flags, int ML,
+                                                           double* __restrict__ out) {
+    const int q = threadIdx.x >> 6, l = threadIdx.x & 63;
+    double a = 0.0;
+    if (obs_slot_on(flags, q)) {
+#pragma unroll 8
+        for (int i = l; i < ML; i += 64) a += red[(int64_t)q * ML + i];
+    }
+#pragma unroll
+    for (int st = 32; st > 0; st >>= 1) a += __shfl_xor(a, st);
+    if (l == 0) out[q] = a;
 }
 
 }  // namespace
@@ -443,12 +525,20 @@ void launch_dipole_z(hipStream_t s, const double* rband, const double* y10, cons
                        (int)N, (int)(p + 1));
 }
 
+template <int NE>
+static void observe_launch(hipStream_t s, const ObsBands& b, int flags, const cplx* coef, double* red, double* out,
+                           int M, int L, int m0, int N) {
+    const int ML = M * L;
+    if (flags & 15)
+        hipLaunchKernelGGL((k_observe<NE, false>), dim3(ML), dim3(kObsThreads), 0, s, b, flags, coef, red, M, L, m0, N, ML);
+    if (flags & 48)
+        hipLaunchKernelGGL((k_observe<NE, true>), dim3(ML), dim3(kObsThreads), 0, s, b, flags, coef, red, M, L, m0, N, ML);
+    hipLaunchKernelGGL(k_observe_sum, dim3(1), dim3(64 * kObs), 0, s, red, flags, ML, out);
+}
 void launch_observe(hipStream_t s, const ObsBands& b, int flags, const cplx* coef, double* red, double* out,
                     int64_t M, int64_t L, int64_t m0, int64_t N, int64_t p) {
-    const int ML = (int)(M * L);
-    hipLaunchKernelGGL(k_observe, dim3((unsigned)ML), dim3(kRedThreads), 0, s, b, flags, coef, red, (int)M, (int)L,
-                       (int)m0, (int)N, (int)(p + 1), ML);
-    hipLaunchKernelGGL(k_observe_sum, dim3(1), dim3(kRedThreads), 0, s, red, flags, ML, out);
+    if (p == 8) observe_launch<9>(s, b, flags, coef, red, out, (int)M, (int)L, (int)m0, (int)N);
+    else observe_launch<8>(s, b, flags, coef, red, out, (int)M, (int)L, (int)m0, (int)N);
 }
 
 

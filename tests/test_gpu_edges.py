@@ -154,3 +154,31 @@ def test_krylov_step_at_tile_edges(N, L, kmax, p):
     assert m == m_o
     assert err <= 1e-10
     prop.close()
+
+
+@pytest.mark.parametrize("p", [7, 8])
+@pytest.mark.parametrize("N", [18, 40, 1023, 1024, 1025, 1031, 2049])
+def test_recorded_observables_at_block_edges(N, p):
+    """All eight recorded observables of a state around the 1024 rows that a
+    block takes at a time (with p rows after them), three m blocks.  Bars as
+    the single observables' in test_gpu_observe."""
+    import pyoracle as po
+    import qpc_gpu
+    print(f"case: observables edges N={N} p={p}", flush=True)
+    L, M, m0 = 3, 3, -1
+    cfg = shape(N, L, 0.2 * N, M=M, m0=m0, p=p)
+    o, prop = _pair(N, p, L, M, m0)
+    st = qpc_gpu.Setup(N, p, L, M, m0, cfg["dt"], 0.0, cfg["rmax"], 1.0, 1.0, cfg["mask_rmin"], cfg["mask_rmax"],
+                       cfg["mask_fact"])
+    prop.upload_outer(st.get(qpc_gpu.SETUP_SOUTER))
+    prop.upload_accel(o.get(po.QOR_DVDR))
+    c = mixed_state(o, seed=N + p, amp=0.5)
+    prop.set_state(c)
+    prop.record(qpc_gpu.REC_ALL, 1)
+    prop.run(np.zeros(2), 0, 0, 1, use_mask=False)
+    h = prop.record_read()[0]
+    ref = [o.norm(c), o.dipole_z(c, 0), o.dipole_z(c, 1), o.outer_norm(c, cfg["mask_rmin"]), *o.dipole_xy(c, 0),
+           *o.dipole_xy(c, 1)]
+    for g, r in zip(h, ref):
+        assert abs(g - r) <= 1e-12 * max(1.0, abs(r))
+    prop.close()
