@@ -108,29 +108,36 @@ __device__ inline cplx cj_if(bool c, cplx v) { return c ? cplx{v.re, -v.im} : v;
 // under a branch compiles to a load-and-wait pair.  The sums keep their
 // order; the extra terms add exact zeros.
 
+// entry i of diagonal j: a uniform address per diagonal and one offset
+template <class T>
+__device__ inline T diag_at(const T* D, int j, int N, int i) {
+    return *(const T*)((const char*)(D + (int64_t)j * N) + (unsigned)i * (unsigned)sizeof(T));
+}
+
 // Row i < N of a per-table complex band (diagonal-major, B(i, i+k) =
 // U[k*N + i], zero where i + k >= N): its entries, then (B z)_i from
-// zl[j-1] = z_{i-j} (j = 1..P) and zu[k] = z_{i+k} (k = 0..P)
+// z(d) = z_{i+d}, |d| <= P
 template <int P>
 struct CBandRow {
     cplx ul[P], uu[P + 1];
     __device__ inline void load(const cplx* __restrict__ U, int i, int N) {
 #pragma unroll
-        for (int j = 1; j <= P; ++j) ul[j - 1] = U[(int64_t)j * N + max(i - j, 0)];
+        for (int j = 1; j <= P; ++j) ul[j - 1] = diag_at(U, j, N, max(i - j, 0));
 #pragma unroll
-        for (int k = 0; k <= P; ++k) uu[k] = U[(int64_t)k * N + i];
+        for (int k = 0; k <= P; ++k) uu[k] = diag_at(U, k, N, i);
     }
     // explicit fused multiply-adds, so that every kernel forming the row
     // rounds it alike (a complex product leaves the contraction open)
-    __device__ inline cplx apply(const cplx (&zl)[P], const cplx (&zu)[P + 1], int i) const {
+    template <class Z>
+    __device__ inline cplx apply(Z z, int i) const {
         cplx v = {0.0, 0.0};
 #pragma unroll
         for (int j = 1; j <= P; ++j) {
             const cplx u = i - j >= 0 ? ul[j - 1] : cplx{0.0, 0.0};
-            v = tmac(v, u, zl[j - 1]);
+            v = tmac(v, u, z(-j));
         }
 #pragma unroll
-        for (int k = 0; k <= P; ++k) v = tmac(v, uu[k], zu[k]);
+        for (int k = 0; k <= P; ++k) v = tmac(v, uu[k], z(k));
         return v;
     }
 };
@@ -146,24 +153,23 @@ struct SBandRow {
     __device__ inline void load(const RhsArgs& ra, int i, int N) {
 #pragma unroll
         for (int j = 1; j <= P; ++j) {
-            const int64_t k = (int64_t)j * N + max(i - j, 0);
             if constexpr (SX) {
-                const cplx q = ra.sx[k];
+                const cplx q = diag_at(ra.sx, j, N, max(i - j, 0));
                 sl[j - 1] = q.re;
                 xl[j - 1] = q.im;
             } else {
-                sl[j - 1] = ra.rband[k];
+                sl[j - 1] = diag_at(ra.rband, j, N, max(i - j, 0));
                 xl[j - 1] = 0.0;
             }
         }
 #pragma unroll
         for (int k = 0; k <= P; ++k) {
             if constexpr (SX) {
-                const cplx q = ra.sx[(int64_t)k * N + i];
+                const cplx q = diag_at(ra.sx, k, N, i);
                 su[k] = q.re;
                 xu[k] = q.im;
             } else {
-                su[k] = ra.rband[(int64_t)k * N + i];
+                su[k] = diag_at(ra.rband, k, N, i);
                 xu[k] = 0.0;
             }
         }
@@ -171,18 +177,21 @@ struct SBandRow {
         for (int j = 1; j <= P; ++j)
             if (i - j < 0) sl[j - 1] = xl[j - 1] = 0.0;
     }
-    // (B z)_i from zlo[j-1] = z_{i-j}, zup[k] = z_{i+k}; e = eig * ifdt of the channel
-    __device__ inline cplx apply(const cplx (&zlo)[P], const cplx (&zup)[P + 1], double e) const {
+    // (B z)_i from z(d) = z_{i+d}, |d| <= P; e = eig * ifdt of the channel
+    template <class Z>
+    __device__ inline cplx apply(Z z, double e) const {
         cplx sz = {0.0, 0.0}, zl = {0.0, 0.0}, zu = {0.0, 0.0};
 #pragma unroll
         for (int j = 1; j <= P; ++j) {
-            sz += sl[j - 1] * zlo[j - 1];
-            if (SX) zl += xl[j - 1] * zlo[j - 1];
+            const cplx v = z(-j);
+            sz += sl[j - 1] * v;
+            if (SX) zl += xl[j - 1] * v;
         }
 #pragma unroll
         for (int k = 0; k <= P; ++k) {
-            sz += su[k] * zup[k];
-            if (SX) zu += xu[k] * zup[k];
+            const cplx v = z(k);
+            sz += su[k] * v;
+            if (SX) zu += xu[k] * v;
         }
         if (RHS == RHS_SX_SYM) {
             // a = S - ifet X with ifet = i*e:  v = Sz - i e (Xz)
@@ -470,6 +479,11 @@ __device__ inline const lcplx* carried(const lcplx* sE, const lcplx* sS, int PK)
     return PK > 1 ? sS + ((PK - 1) & 1) * P * kSt : sE;
 }
 
+template <int... I, class F>
+__device__ inline void each(std::integer_sequence<int, I...>, F f) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+
 // v = B z for per-table bands (RHS_CBAND), one lane per (row, channel)
 template <int P>
 __global__ __launch_bounds__(256) void k_rhs(RhsArgs ra, TabMap tm, const cplx* __restrict__ zin,
@@ -480,12 +494,7 @@ __global__ __launch_bounds__(256) void k_rhs(RhsArgs ra, TabMap tm, const cplx* 
     CBandRow<P> b;
     b.load(ra.cband + (int64_t)table_of(tm, ch) * (P + 1) * N, i, N);
     const cplx* z = zin + (int64_t)ch * N;
-    cplx zl[P], zu[P + 1];
-#pragma unroll
-    for (int j = 1; j <= P; ++j) zl[j - 1] = z[max(i - j, 0)];
-#pragma unroll
-    for (int k = 0; k <= P; ++k) zu[k] = z[min(i + k, N - 1)];
-    vout[(int64_t)ch * N + i] = b.apply(zl, zu, i);
+    vout[(int64_t)ch * N + i] = b.apply([&](int d) { return z[min(max(i + d, 0), N - 1)]; }, i);
 }
 
 // v = B z for bands shared by every channel (RHS_RBAND, RHS_SX_*): a lane
@@ -504,13 +513,8 @@ __global__ __launch_bounds__(256) void k_rhs_shared(RhsArgs ra, const cplx* __re
         const int ch = blockIdx.y * kRhsCG + c;
         if (ch < nch) {
             const cplx* z = zin + (int64_t)ch * N;
-            cplx zlo[P], zup[P + 1];
-#pragma unroll
-            for (int j = 1; j <= P; ++j) zlo[j - 1] = z[max(i - j, 0)];
-#pragma unroll
-            for (int k = 0; k <= P; ++k) zup[k] = z[min(i + k, N - 1)];
             const double e = SBandRow<RHS, P>::SX ? ra.eig[ch] * ra.ifdt : 0.0;
-            vout[(int64_t)ch * N + i] = b.apply(zlo, zup, e);
+            vout[(int64_t)ch * N + i] = b.apply([&](int d) { return z[min(max(i + d, 0), N - 1)]; }, e);
         }
     }
 }
@@ -718,13 +722,10 @@ __global__ __launch_bounds__(kLane * (STAGED ? kWavesStaged : 1)) void k_bsolve(
             const double e = cj ? -e0 : e0;
             auto form = [&](const Row& b, int k) {
                 const int i = min(ht + k * HT, NR - 1);  // (a row past the last repeats the last)
-                cplx zl[P], zu[P + 1], v;
-#pragma unroll
-                for (int j = 1; j <= P; ++j) zl[j - 1] = sz[i + P - j];
-#pragma unroll
-                for (int q = 0; q <= P; ++q) zu[q] = sz[i + P + q];
-                if constexpr (ROLE == RHS_CBAND) v = b.apply(zl, zu, row_at(k));
-                else v = b.apply(zl, zu, e);
+                cplx v;
+                auto zat = [&](int d) -> cplx { return sz[i + P + d]; };
+                if constexpr (ROLE == RHS_CBAND) v = b.apply(zat, row_at(k));
+                else v = b.apply(zat, e);
                 // rows from N on are padding: v = 0
                 if (i < nrow) sv[row_slot(i % kPM, i / kPM)] = lc(i < nv ? v : cplx{0.0, 0.0});
             };
@@ -773,6 +774,324 @@ __global__ __launch_bounds__(kLane * (STAGED ? kWavesStaged : 1)) void k_bsolve(
     cplx* xo = zout + (int64_t)ch * N + r0;
 #pragma unroll 6
     for (int i = i0 + tid; i < i1; i += NTH) xo[i] = cj_if(cj, sv[row_slot(i % kPM, i / kPM)]);
+}
+
+// The same solve with eight lanes per partition, for channels of at most
+// kSplitParts partitions, whose lanes k_bsolve's wave would leave idle.  Lane l
+// owns rows l, l + 8 and l + 16 of its partition.  Going down, the row's value
+// is broadcast to the eight (two DPP moves per double) and each lane subtracts
+// its multiple from the row it gathers next: P products per row in one
+// instruction each, and the chain of a row is a broadcast and two FMAs.  The
+// lane that owned the row starts its next one from zero: its coefficient is 1
+// (P = 8: row s itself reaches row s + 8, so the lane's sum is set to zero).
+// Going up is the same from the last row, with the rows' own coefficients.
+// The state a partition hands down is what the eight lanes have gathered for
+// the first rows of the next one.  A lane's 24 coefficients per direction stay
+// in registers for both passes, its rows too: LDS holds the rows of z for the
+// right-hand side, P rows on either side, and the states of the carries, which
+// each lane runs for its own entry (row l of the transfer matrix).
+//
+// Forward rows of a real table are scaled by the target row's 1/u as they are
+// loaded (y_i = r_i v_i - sum (r_i F) y); the rows beyond the partition are not,
+// their state is.
+//
+// A pass takes 1.4 k cycles (k_bsolve: 6.5 k), so what bounds it is the loads:
+// every table entry twice, the band entries of three rows per lane.  Longer
+// channels would wait for them as long (N = 1500: no gain) and, with one
+// work-group per compute unit, on grids of many channels longer.  R, D, free
+// and mask solves of 6 channels of N = 240: 12.2 / 11.1 / 12.1 / 9.4 us (k_bsolve
+// 21.6 / 18.0 / 21.4 / 17.0); whole passes at 32 partitions: 31 channels step by
+// step 5.3 -> 4.3 ms, 2400 batched ones 36.0 -> 31.1; at 42 (N = 1000) 651
+// channels are 15 % slower, hence the line.
+//
+// FUSE: as k_bsolve's; with one segment src and zout may be the same.
+constexpr int kSplit = 8;                     // lanes per partition
+constexpr int kSplitParts = 32;               // partitions up to which they are used
+constexpr int kOwn = kPM / kSplit;            // rows per lane
+constexpr int kSt8 = kSplit + 1;              // a state's entries in LDS, odd for the banks
+static_assert(kPM % kSplit == 0 && kSplit == 8, "lane layout");
+
+template <int L>
+__device__ inline double bcast8(double v) {  // lane L of each eight
+    const long long b = __double_as_longlong(v);
+    const long long a = __builtin_amdgcn_mov_dpp(b, 0x150 + L, 0xf, 0xf, true);
+    return __longlong_as_double(__builtin_amdgcn_update_dpp(a, b, 0x158 + L, 0xf, 0xc, false));
+}
+template <int L>
+__device__ inline cplx bcast8(cplx v) { return {bcast8<L>(v.re), bcast8<L>(v.im)}; }
+__device__ inline cplx pick(bool c, cplx a, cplx b) { return {c ? a.re : b.re, c ? a.im : b.im}; }
+__device__ inline double pick(bool c, double a, double b) { return c ? a : b; }
+// keeps a value where it is computed: put off to its use, it would keep its
+// operands alive until then
+__device__ inline void keep(cplx& v) { asm volatile("" : "+v"(v.re), "+v"(v.im)); }
+
+// A lane's coefficients.  ld: byte offset of coefficient k = 1..P of row `row`
+// (relative to the table's partition column), element P the diagonal
+template <class TF, int P>
+struct LaneTab {
+    using F = TabFmt<TF, P>;
+    static constexpr unsigned kUnit = kLane * 16u, kRow = F::row * kUnit;
+    __device__ static unsigned elem(int e) {  // element e = 0..P of a row
+        if constexpr (F::SYM) return (unsigned)e * kUnit;
+        else return (unsigned)(e >> 1) * kUnit + (unsigned)(e & 1) * 8u;
+    }
+    __device__ static TF at(const char* base, unsigned off) { return *(const TF*)(base + off); }
+};
+
+// rows down through the partition: z the own rows' right-hand sides, acc what
+// the partition above contributes (in) and what this one does to the next
+// (out), y the own rows
+template <class TF, int P>
+__device__ inline void rows_down(const TF (&C)[kPM], const cplx (&z)[kOwn], cplx (&y)[kOwn], cplx& acc, int l) {
+    each(std::make_integer_sequence<int, kPM>{}, [&](auto sc) {
+        constexpr int s = decltype(sc)::value, t = s / kSplit, r = s % kSplit;
+        if constexpr (r == 0) acc = {acc.re + z[t].re, acc.im + z[t].im};
+        const cplx x = bcast8<r>(acc);
+        y[t] = pick(l == r, acc, y[t]);
+        keep(y[t]);
+        if constexpr (P == 8) acc = pick(l == r, cplx{0.0, 0.0}, acc);
+        acc = tmsub(acc, C[s], x);
+    });
+}
+// rows up; acc: what the partition below contributes to the last eight
+template <class TF, int P>
+__device__ inline void rows_up(const TF (&C)[kPM], const cplx (&y)[kOwn], cplx (&x)[kOwn], cplx acc, int l) {
+    each(std::make_integer_sequence<int, kPM>{}, [&](auto sc) {
+        constexpr int s = kPM - 1 - decltype(sc)::value, t = s / kSplit, r = s % kSplit;
+        if constexpr (r == kSplit - 1) acc = {acc.re + y[t].re, acc.im + y[t].im};
+        const cplx v = bcast8<r>(acc);
+        x[t] = pick(l == r, acc, x[t]);
+        keep(x[t]);
+        if constexpr (P == 8) acc = pick(l == r, cplx{0.0, 0.0}, acc);
+        acc = tmsub(acc, C[s], v);
+    });
+}
+
+// The incoming states from the pass-A end states e: s_g <- e_g + T_g s_{g-1}
+// (g+1 backward), PK - 1 times from s = e, so that s_{g-1} holds the PK
+// partitions before g, the same sums as Horner's rule over them.  Entry l of
+// slot q at q * kSt8 + l; slot nb is the neighbour's, or the zero slot.  Returns
+// the neighbour's incoming state.
+// (par: which buffer comes first, so that a direction's first is not the
+// other's last, which lanes may still be reading)
+template <class TF, int P>
+__device__ inline const lcplx* carry(lcplx (*sS)[(kSplitParts + 1) * kSt8], const TF (&t)[P], cplx e, int own, int nb, int PK,
+                                     int par) {
+    cplx a = e;
+#pragma unroll 1
+    for (int k = 1;; ++k) {
+        lcplx* buf = sS[(k + par) & 1];
+        buf[own] = lc(a);
+        __syncthreads();
+        if (k == PK) return buf + nb * kSt8;
+        cplx in[P];
+#pragma unroll
+        for (int c = 0; c < P; ++c) in[c] = buf[nb * kSt8 + c];
+        a = e;
+#pragma unroll
+        for (int c = 0; c < P; ++c) a = tmac(a, t[c], in[c]);
+    }
+}
+
+// row r of the direction's matrix
+template <class TF, int P>
+__device__ inline void trf_row(TF (&t)[P], const TF* T, unsigned off, int dir, int r) {
+    constexpr bool SYM = TabFmt<TF, P>::SYM;
+    const bool tr = SYM && dir;
+    const unsigned o = off + (unsigned)((SYM ? 0 : dir * P * P) + (tr ? r : r * P)) * kLane * (unsigned)sizeof(TF);
+#pragma unroll
+    for (int c = 0; c < P; ++c) t[c] = *(const TF*)((const char*)(T + (tr ? c * P : c) * kLane) + o);
+}
+
+template <class TF, int ROLE, bool FUSE, int P>
+__global__ __launch_bounds__(kSplitParts * kSplit) void k_bsolve8(const cplx* __restrict__ tab, const TF* __restrict__ trf,
+                                                           TabMap tm, const cplx* __restrict__ src,
+                                                           cplx* __restrict__ zout, Geom geo, int SN, int PK,
+                                                           RhsArgs ra) {
+    using F = TabFmt<TF, P>;
+    using LT = LaneTab<TF, P>;
+    constexpr bool SYM = F::SYM;
+    constexpr int KZ = 4;  // staged rows per thread: 24 per eight threads, and 2 P
+    __shared__ lcplx sz[FUSE ? kPM * kSplitParts + 2 * P : 1];  // z rows [r0 - P, r0 + nrow + P), zero outside [0, N)
+    __shared__ lcplx sS[2][(kSplitParts + 1) * kSt8];            // states
+
+    int ch = blockIdx.y, seg = blockIdx.x;
+    if (tm.order) {
+        const int o = tm.order[blockIdx.y * gridDim.x + blockIdx.x];
+        ch = o >> 8;
+        seg = o & 255;
+    }
+    const int N = geo.N, NP = geo.P;
+    const int k0 = seg * SN, k1 = min(NP, k0 + SN);         // owned partitions [k0, k1)
+    const int ga = max(0, k0 - PK), gb = min(NP, k1 + PK);  // staged partitions [ga, gb)
+    const int n = gb - ga;
+    const int tid = threadIdx.x, q = tid / kSplit, l = tid % kSplit;
+    // this lane's partition; slots past the staged ones repeat the last (their
+    // rows and states are not used)
+    const int g = min(ga + q, gb - 1);
+    const int tabid = table_of(tm, ch);
+    const bool cj = conj_of(tm, ch);
+    const int r0 = ga * kPM;  // first staged row
+    const int i0 = g * kPM + l;
+    const char* T = (const char*)(tab + (int64_t)tabid * F::units(geo));
+    const unsigned off = part_off<TF, P>(g);
+    const TF* TR = trf + (int64_t)tabid * F::trf_elems(geo);
+    const unsigned toff = trf_off<TF, P>(g);
+    const int own = q * kSt8 + l, lp = min(l, P - 1);
+
+    if (tid < 2 * kSt8) sS[tid / kSt8][kSplitParts * kSt8 + tid % kSt8] = lcplx{0.0, 0.0};
+    // requests: z, the first band row, the forward coefficients
+    using Row = std::conditional_t<ROLE == RHS_CBAND, CBandRow<P>, SBandRow<ROLE, P>>;
+    Row band;
+    auto load_band = [&](int t) {
+        const int i = min(i0 + kSplit * t, N - 1);
+        if constexpr (ROLE == RHS_CBAND) band.load(ra.cband + (int64_t)tabid * (P + 1) * N, i, N);
+        else band.load(ra, i, N);
+    };
+    cplx z[kOwn], zr[FUSE ? KZ : 1];
+    if constexpr (FUSE) {
+        const cplx* zc = src + (int64_t)ch * N;
+#pragma unroll
+        for (int k = 0; k < KZ; ++k) zr[k] = zc[min(max(r0 - P + tid + k * (int)blockDim.x, 0), N - 1)];
+        load_band(0);
+    } else {
+#pragma unroll
+        for (int t = 0; t < kOwn; ++t) z[t] = src[(int64_t)ch * N + min(i0 + kSplit * t, N - 1)];
+    }
+    TF C[kPM], dg[kOwn], tr[P];
+    auto load_down = [&](int t) {
+#pragma unroll
+        for (int r = 0; r < kSplit; ++r)
+            C[t * kSplit + r] = LT::at(T + t * kSplit * LT::kRow, off + r * LT::kRow + LT::elem((l - r - 1) & 7));
+        dg[t] = LT::at(T + t * kSplit * LT::kRow, off + l * LT::kRow + LT::elem(P));
+    };
+    // (the right-hand side's operands leave room for two thirds of them)
+    constexpr int T0 = FUSE ? 2 : kOwn;
+#pragma unroll
+    for (int t = 0; t < T0; ++t) load_down(t);
+    if constexpr (FUSE) {
+        const int nz = n * kPM + 2 * P, zlo = r0 - P;
+#pragma unroll
+        for (int k = 0; k < KZ; ++k) {
+            const int j = tid + k * blockDim.x, row = zlo + j;
+            if (j < nz) sz[j] = lc(row >= 0 && row < N ? cj_if(cj, zr[k]) : cplx{0.0, 0.0});
+        }
+        __syncthreads();
+        // staged row i is channel row r0 + i, its z_{r0+i+d} sits at sz[i + P +
+        // d]; a conjugate channel forms its table's right-hand side (scalar -e)
+        const double e0 = ROLE == RHS_SX_SYM || ROLE == RHS_SX_ASY ? ra.eig[ch] * ra.ifdt : 0.0;
+        const double e = cj ? -e0 : e0;
+#pragma unroll 1
+        for (int t = 0; t < kOwn; ++t) {
+            const int i = i0 + kSplit * t;
+            const lcplx* zs = sz + (i - r0 + P);
+            cplx v;
+            // four rows of z at a time: all fifteen would leave too few registers for the coefficients
+            auto zat = [&](int d) -> cplx {
+                if (d % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+                return zs[d];
+            };
+            if constexpr (ROLE == RHS_CBAND) v = band.apply(zat, min(i, N - 1));
+            else v = band.apply(zat, e);
+            if (i >= N) v = cplx{0.0, 0.0};  // padding
+#pragma unroll
+            for (int k = 0; k + 1 < kOwn; ++k) z[k] = z[k + 1];
+            z[kOwn - 1] = v;
+            keep(v);  // (before the next row's entries are requested)
+            __builtin_amdgcn_sched_barrier(0);
+            if (t + 1 < kOwn) load_band(t + 1);
+        }
+    } else {
+#pragma unroll
+        for (int t = 0; t < kOwn; ++t) z[t] = i0 + kSplit * t < N ? cj_if(cj, z[t]) : cplx{0.0, 0.0};
+    }
+#pragma unroll
+    for (int t = T0; t < kOwn; ++t) load_down(t);
+    trf_row<TF, P>(tr, TR, toff, 0, lp);
+
+    // Coefficients of the way up: row 8 t + r reaches lane l's row of its eight
+    // or of the eight above (the first rows' wrap around: the partition's last
+    // eight, which the partition below reaches).  The last rows' are requested
+    // here (a real table's all), the others once the way down has left room.
+    TF D[kPM];
+    auto load_up = [&](int t) {
+#pragma unroll
+        for (int r = kSplit - 1; r >= 0; --r) {
+            const bool same = P == 7 ? l <= r : l < r;
+            const unsigned o = off + (unsigned)F::boff * LT::kUnit + LT::elem((r - l - 1) & 7);
+            const int row = t ? (same ? l + kSplit : l) : (same ? l : kPM - kSplit + l);
+            D[t * kSplit + r] = LT::at(T + (t ? t - 1 : 0) * kSplit * LT::kRow, o + (unsigned)row * LT::kRow);
+        }
+    };
+    constexpr int T1 = SYM ? (P == 7 ? 2 : kOwn) : 0;
+#pragma unroll
+    for (int t = kOwn - 1; t >= T1; --t) load_up(t);
+    // down: pass A from the zero state, carry, pass B
+    if constexpr (!SYM) {
+#pragma unroll
+        for (int t = 0; t < kOwn; ++t) {
+            z[t] = {dg[t] * z[t].re, dg[t] * z[t].im};
+#pragma unroll
+            for (int r = 0; r < kSplit; ++r) {
+                // the row that lane l gathers after row 8 t + r: its own of this eight, or of the next
+                const double up = t + 1 < kOwn ? dg[t + 1 < kOwn ? t + 1 : t] : 1.0;
+                C[t * kSplit + r] *= l > r ? dg[t] : up;
+            }
+        }
+    }
+    if constexpr (P == 7) {
+#pragma unroll
+        for (int s = 0; s < kPM; ++s) C[s] = pick(l == s % kSplit, tone(TF{}), C[s]);
+    }
+    cplx y[kOwn], acc = {0.0, 0.0};
+#pragma unroll
+    for (int t = 0; t < kOwn; ++t) y[t] = acc;
+#pragma unroll 1
+    for (int pass = 0;; ++pass) {
+        rows_down<TF, P>(C, z, y, acc, l);
+        if (pass) break;
+        const lcplx* in = carry<TF, P>(sS, tr, acc, own, q > 0 && q < n ? q - 1 : kSplitParts, PK, 0);
+        acc = l < P ? (cplx)in[l] : cplx{0.0, 0.0};
+        if constexpr (!SYM) acc = {dg[0] * acc.re, dg[0] * acc.im};
+    }
+    // up
+#pragma unroll
+    for (int t = T1 - 1; t >= 0; --t) load_up(t);
+    trf_row<TF, P>(tr, TR, toff, 1, lp);
+#pragma unroll
+    for (int t = 0; t < kOwn; ++t) {
+        if constexpr (SYM) {
+            y[t] = tmulf(dg[t], y[t]);
+        } else {
+            const TF d = LT::at(T + t * kSplit * LT::kRow, off + (unsigned)F::boff * LT::kUnit + l * LT::kRow + LT::elem(P));
+            y[t] = {d * y[t].re, d * y[t].im};
+        }
+    }
+    cplx x[kOwn];
+    if constexpr (P == 7) {
+#pragma unroll
+        for (int s = kPM - 1; s >= 0; --s) D[s] = pick(l == s % kSplit, tone(TF{}), D[s]);
+    }
+#pragma unroll
+    for (int t = 0; t < kOwn; ++t) x[t] = {0.0, 0.0};
+    acc = {0.0, 0.0};
+#pragma unroll 1
+    for (int pass = 0;; ++pass) {
+        rows_up<TF, P>(D, y, x, acc, l);
+        if (pass) break;
+        const lcplx* in = carry<TF, P>(sS, tr, x[0], own, q + 1 < n ? q + 1 : kSplitParts, PK, PK);
+        // the first P rows of the partition below, seen from this one's last eight
+#pragma unroll
+        for (int i = P - 1; i >= 0; --i) {
+            const bool on = P == 7 ? l > i : l >= i;
+            acc = tmsub(acc, pick(on, D[i], tzero(TF{})), (cplx)in[i]);
+        }
+    }
+    cplx* xo = zout + (int64_t)ch * N;
+    if (q >= k0 - ga && q < k1 - ga)
+#pragma unroll
+        for (int t = 0; t < kOwn; ++t)
+            if (i0 + kSplit * t < N) xo[i0 + kSplit * t] = cj_if(cj, x[t]);
 }
 
 // Sequential solve x = U^-1 L^-1 v over all N rows, one lane per channel:
@@ -1161,10 +1480,6 @@ __device__ inline double swap8(double v) {  // lane l ^ 8 in the banks of four l
     const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(h, h, 0x128, 0xf, BANKS, false);
     return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
 }
-template <int... I, class F>
-__device__ inline void each(std::integer_sequence<int, I...>, F f) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
 constexpr int kFactorQ = 4;  // partitions per wave
 // Used up to this many waves (six per compute unit, the most its LDS holds:
 // 650 waves take 18 us, 3200 78 us and 5600 118 us where k_factor takes 35 to
@@ -1438,6 +1753,25 @@ static void bsolve(hipStream_t s, const TF* tab, const TF* trf, TabMap tm, const
     const int sn = seg_parts(geo, PK);
     const int nseg = (geo.P + sn - 1) / sn;
     if (tm.order && nseg != tm.order_nseg) tm.order = nullptr;  // built for another launch shape
+    if (geo.P <= kSplitParts) {
+        // eight lanes per partition; the right-hand side in the launch unless another work-group may still read
+        // rows of z that one writes
+        const dim3 grid8(nseg, nch), block((std::min(geo.P, nseg > 1 ? sn + 2 * PK : sn) + 7) / 8 * kLane);
+        if (ra) {
+            const uintptr_t a0 = (uintptr_t)zin, b0 = (uintptr_t)zout;
+            const uintptr_t len = sizeof(cplx) * (uintptr_t)nch * geo.N;
+            if (a0 + len <= b0 || b0 + len <= a0 || (nseg == 1 && a0 == b0)) {
+                hipLaunchKernelGGL((k_bsolve8<TF, ROLE, true, P>), grid8, block, 0, s, (const cplx*)tab, trf, tm, zin,
+                                   zout, geo, sn, PK, *ra);
+                return;
+            }
+            rhs_launch<P>(s, ROLE, *ra, tm, zin, vbuf, nch, geo);
+            zin = vbuf;
+        }
+        hipLaunchKernelGGL((k_bsolve8<TF, ROLE, false, P>), grid8, block, 0, s, (const cplx*)tab, trf, tm, zin, zout, geo,
+                           sn, PK, RhsArgs{});
+        return;
+    }
     // staged grids form the right-hand side in the launch when z and x do not overlap
     const bool staged = (int64_t)nseg * nch <= geo.stage_grid;
     const dim3 grid(nseg, nch);

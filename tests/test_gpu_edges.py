@@ -182,3 +182,33 @@ def test_recorded_observables_at_block_edges(N, p):
     for g, r in zip(h, ref):
         assert abs(g - r) <= 1e-12 * max(1.0, abs(r))
     prop.close()
+
+
+@pytest.mark.parametrize("p", [7, 8])
+@pytest.mark.parametrize("N", [192, 745, 767, 768, 769, 793])
+def test_steps_where_the_solve_changes_kernel(N, p):
+    """Channels of up to 32 partitions (768 rows) have eight lanes per
+    partition in the solves, longer ones one: steps on either side of the line
+    against the oracle, and the same bits however the channel is segmented."""
+    print(f"case: solve kernels N={N} p={p}", flush=True)
+    o, prop = _pair(N, p, 3, M=3, m0=-1)
+    c = mixed_state(o, seed=N + p, amp=0.3)
+    ref = c.copy()
+    out = []
+    for seg in (0, 1, 3):
+        prop.set_tune(seg_add=seg)
+        prop.set_state(c)
+        for a in ((0.7, 0.9), (0.9, -0.4)):
+            prop.propagate(*a)
+        prop.propagate()
+        prop.mask()
+        out.append(prop.get_state().copy())
+    for a in ((0.7, 0.9), (0.9, -0.4)):
+        o.step(ref, *a)
+    o.step_free(ref)
+    o.mask(ref)
+    err = rel_l2(out[0], ref)
+    print(f"  rel L2 {err:.2e}", flush=True)
+    assert err <= 1e-12
+    assert all(np.array_equal(x, out[0]) for x in out[1:])
+    prop.close()
