@@ -415,8 +415,9 @@ int  qpc_run_lgwr(qpc_ctx* ctx, const double* extab, const double* eytab, int64_
  * segments, one work-group each; seg_add adds segments beyond the fewest
  * that hold them (more work-groups, each with the carry's halo partitions
  * again), and grids of at most stage_grid work-groups stage table rows in
- * LDS, with eight waves per work-group.  Neither changes the result (the
- * segments are exact, the two paths share their arithmetic).
+ * LDS, with eight waves per work-group, or give each partition eight lanes
+ * (channels of up to 32 partitions have them on every grid).  Neither changes
+ * the result (the segments are exact, the paths share their arithmetic).
  * qpc_autotune runs the with-field steps [it0, it0+nsteps) of the field
  * table (as qpc_run, or qpc_run_batch with its stride for a batch context;
  * stride is ignored otherwise) once per candidate, seg_add 0..3 x stage_grid
@@ -443,9 +444,9 @@ int  qpc_autotune(qpc_ctx* ctx, const double* atab, int64_t stride, int64_t nt_f
  * `which` (QPC_K_*) queued afterwards, up to max_launches; qpc_timing_end
  * waits and returns the number of timed launches and their mean duration in
  * ms.  The solve classes time the right-hand side B z and the partitioned
- * triangular solve of one CN factor: one launch (k_bsolve forming B z while
- * it stages) on grids of at most 512 work-groups with distinct input and
- * output, else the banded product (k_rhs*) followed by the solve. */
+ * triangular solve of one CN factor: one launch (k_bsolve or k_bsolve8 forming
+ * B z) on grids of at most 512 work-groups, and for channels of up to 32
+ * partitions on every grid, with distinct input and output, else the banded product (k_rhs*) followed by the solve. */
 #define QPC_K_CN_D     0   /* CN factor of a coupling step, D-part (prop_z2) */
 #define QPC_K_CN_R     1   /* CN factor of a coupling step, R-part (prop_z1) */
 #define QPC_K_FREE     2   /* field-free CN factor (prop_hc)         */

@@ -22,7 +22,8 @@
 //
 // Rows are cut into partitions of kPM rows (the last one padded with identity
 // rows: F = G = E = 0, rdf = rdb = rD = 1, v = 0, which leaves rows < N
-// exact).  One lane owns one partition.  Pass A runs each partition from a
+// exact).  One lane owns a partition, or eight (the same arithmetic; short
+// channels and small grids).  Pass A runs each partition from a
 // zero state; the true incoming state is recovered from the pass-A end
 // states of the PK preceding partitions through the partitions' p x p
 // transfer matrices (state independent, built with the tables); pass B
@@ -72,7 +73,9 @@ constexpr int kRestart = 64;
 inline bool width_supported(int p) { return p == 7 || p == 8; }
 
 // grids of at most this many solve work-groups stage table rows in LDS
-// (eight waves per work-group, the right-hand side formed in the launch)
+// (eight waves per work-group, the right-hand side formed in the launch), or
+// run with eight lanes per partition where that leaves one work-group to a
+// compute unit (kSplitGrid)
 constexpr int64_t kStageGrid = 512;
 
 // units (two doubles) per direction of a real LU row: p coefficients and a diagonal
@@ -145,7 +148,7 @@ struct TabMap {
 constexpr int kMapConj = 1 << 30, kMapIdx = kMapConj - 1;
 constexpr int kXcds = 8;
 // segments per channel of the partitioned solve for this launch shape and
-// carry depth (bsolve's choice; 0 when the carry is too deep for it and the
+// carry depth (bsolve's choice with one lane per partition; 0 when the carry is too deep for it and the
 // solve runs sequentially), and the XCD-grouping order of its
 // work-groups for channels whose tables are tab[ch] (nch channels)
 int solve_segments(const Geom& geo, int pk);
@@ -165,7 +168,7 @@ void launch_bsolve_r(hipStream_t s, int role, const double* tab, const double* t
                      cplx* zout, int nch, Geom geo, int pk = 0);
 
 // v = B z (the RhsKind role with the bands of ra) and x = A^-1 v in one call.
-// On grids that stage table rows in LDS, and when zin and zout do not
+// On small grids (kStageGrid) and for short channels, when zin and zout do not
 // overlap, the solve forms v itself; otherwise launch_rhs writes v into vbuf
 // (nch * N) and the solve reads it.
 void launch_rsolve_c(hipStream_t s, int role, const RhsArgs& ra, const cplx* tab, const cplx* trf, TabMap tm,

@@ -207,20 +207,21 @@ struct SBandRow {
 
 // ---------------------------------------------------------------------------
 // One table row of one partition and direction in registers (UF units).
-// Forward (state acc[k]: what the rows above contribute to row s + k, to be
-// added to its right-hand side): the row's value leaves the window and its
-// multiples go to the P rows below.  The state a partition hands on is what
-// its rows contribute to the first P rows of the next.
+// Forward (acc[k]: the right-hand side of row s + k less what the rows above
+// contribute): the row's value leaves the window, its multiples go to the P
+// rows below, and row s + P enters with its right-hand side vn.  The state a
+// partition hands on is what its rows contribute to the first P rows of the
+// next, whose own right-hand sides enter as zero.
 template <class TF, int P>
-__device__ inline cplx fwd_row(const cplx (&c)[TabFmt<TF, P>::UF], cplx v, cplx (&acc)[P]) {
+__device__ inline cplx fwd_row(const cplx (&c)[TabFmt<TF, P>::UF], cplx vn, cplx (&acc)[P]) {
     using F = TabFmt<TF, P>;
-    const cplx z = {v.re + acc[0].re, v.im + acc[0].im};
+    const cplx z = acc[0];
     cplx y;  // what the lower rows' updates take, and the stored row
     if constexpr (F::SYM) y = z;
     else y = {F::diag(c) * z.re, F::diag(c) * z.im};
 #pragma unroll
     for (int k = 1; k < P; ++k) acc[k - 1] = tmsub(acc[k], F::coef(c, k), y);
-    acc[P - 1] = tmsub(cplx{0.0, 0.0}, F::coef(c, P), y);
+    acc[P - 1] = tmsub(vn, F::coef(c, P), y);
     if constexpr (F::SYM) return tmulf(F::diag(c), z);
     else return y;
 }
@@ -284,16 +285,21 @@ constexpr int kRowStride = kPM + 1, kRowPad = 4;
 constexpr int kRowSlots = kLane * kRowStride + 2 * kRowPad;
 __device__ inline int row_slot(int s, int ln) { return kRowPad + ln * kRowStride + s; }
 
-// the rows of one block: v[r] the row's value, written to wb[r]; the block's
-// registers are refilled from LDS (l: this lane's units) or the table (p)
+// the rows of one block, written to wb[r]; the block's registers are refilled
+// from LDS (l: this lane's units) or the table (p).  Forward, row r of the
+// block takes in the right-hand side v[r] of the row P below; nv: the four rows
+// from 12 below the block's first (with P = 7 one row of them waits in v[RB]).
 template <class TF, int P, bool L>
-__device__ inline void fwd_block(BlockRegs<TF, P>& c, cplx (&v)[Blocks<TF, P>::RB], const lcplx* rb, lcplx* wb,
+__device__ inline void fwd_block(BlockRegs<TF, P>& c, cplx (&v)[Blocks<TF, P>::RB + 1], const lcplx* nv, lcplx* wb,
                                  const lcplx* l, const cplx* p, unsigned off, cplx (&acc)[P]) {
     using B = Blocks<TF, P>;
+    static_assert(P == B::RB + 3 || P == B::RB + 4, "the rows that nv holds");
 #pragma unroll
     for (int r = 0; r < B::RB; ++r) {
         const cplx y = fwd_row<TF, P>(c[r], v[r], acc);
-        v[r] = rb[B::RB + r];
+        if constexpr (P == 8) v[r] = nv[r];
+        else v[r] = r ? (cplx)nv[r > 0 ? r - 1 : 0] : v[B::RB];
+        if (P == 7 && r == B::RB - 1) v[B::RB] = nv[B::RB - 1];
         wb[r] = lc(y);
 #pragma unroll
         for (int u = 0; u < B::UF; ++u)
@@ -321,18 +327,24 @@ __device__ inline void bwd_block(BlockRegs<TF, P>& c, cplx (&v)[Blocks<TF, P>::R
 // One pass over the rows of slot ln (rows: its first row; T: the direction's
 // units of the table, uniform).  c holds the first block at entry and the
 // block at `after` at the end.  Rows are written to `out` (their own place, or
-// a scrap block of RB rows when ostep is 0).
+// a scrap block of RB rows when ostep is 0).  zeros: RB zero rows, for those
+// past the partition.
 template <class TF, int P, bool STAGED>
 __device__ inline void fwd_pass(BlockRegs<TF, P>& c, const cplx* T, unsigned off, const lcplx* sL,
-                                const lcplx* rows, lcplx* out, int ostep, cplx (&acc)[P], const cplx* after) {
+                                const lcplx* rows, lcplx* out, int ostep, cplx (&acc)[P], const cplx* after,
+                                const lcplx* zeros) {
     using B = Blocks<TF, P>;
-    cplx v[B::RB];
+    cplx v[B::RB + 1];
 #pragma unroll
-    for (int r = 0; r < B::RB; ++r) v[r] = rows[r];
+    for (int r = 0; r < P; ++r) acc[r] += (cplx)rows[r];
+#pragma unroll
+    for (int r = 0; r < B::RB + (P == 7); ++r) v[r] = rows[P + r];
+    constexpr int AHEAD = 3;  // blocks from the one in hand to the rows read while it runs
+    int left = B::NB - AHEAD;
     if constexpr (STAGED) {
 #pragma unroll 1
         for (int i = 0; i < B::LB1 - B::LB0; ++i) {
-            fwd_block<TF, P, true>(c, v, rows, out, sL, nullptr, 0, acc);
+            fwd_block<TF, P, true>(c, v, left-- > 0 ? rows + AHEAD * B::RB : zeros, out, sL, nullptr, 0, acc);
             rows += B::RB;
             out += ostep;
             sL += B::RB * B::UF * kLane;
@@ -342,7 +354,8 @@ __device__ inline void fwd_pass(BlockRegs<TF, P>& c, const cplx* T, unsigned off
     T += (int64_t)G0 * B::RB * B::UT * kLane;
 #pragma unroll 1
     for (int i = 0; i < GN; ++i) {
-        fwd_block<TF, P, false>(c, v, rows, out, nullptr, i == GN - 1 ? after : T, off, acc);
+        fwd_block<TF, P, false>(c, v, left-- > 0 ? rows + AHEAD * B::RB : zeros, out, nullptr, i == GN - 1 ? after : T,
+                                off, acc);
         rows += B::RB;
         out += ostep;
         T += B::RB * B::UT * kLane;
@@ -542,10 +555,10 @@ __global__ __launch_bounds__(256) void k_rhs_shared(RhsArgs ra, const cplx* __re
 // wave per work-group, several per compute unit, which hide each other's
 // loads.
 // Measured per launch, R, D, free and mask solves (with, in
-// brackets, four waves that shared the passes' loads through LDS): 21.6 / 18.0 / 21.4 / 17.0 us at N = 240
-// (29.6 / 22.2 / 30 / 20.7), 26.9 / 25.0 / 28.7 / 19.2 us at N = 3000 with 81
-// channels (32.2 / 27.6 / 33.8 / 22.8).  Of the 55 k cycles of a symmetric solve the
-// passes take 27 k (two thirds of it the issue of their own arithmetic), the
+// brackets, four waves that shared the passes' loads through LDS): 26.9 / 25.0 /
+// 28.7 / 19.2 us at N = 3000 with 81 channels (32.2 / 27.6 / 33.8 / 22.8).  Of the
+// 55 k cycles of a symmetric solve the passes take 27 k (two thirds of it the
+// issue of their own arithmetic), the
 // carries 7 k and the loads with the right-hand side 20 k.
 //
 // FUSE (STAGED): src is the state z and the work-group forms v = B z itself
@@ -560,7 +573,8 @@ struct StageLds {
     static constexpr int NZ = kPM * kLane + 2 * P;
     static constexpr int scrap = 2 * P * kSt;
     static constexpr int sz = NZ > scrap + kLane * Blocks<TF, P>::RB ? NZ : scrap + kLane * Blocks<TF, P>::RB;
-    static constexpr int bytes = 16 * (sz + kRowSlots + P * kSt + Blocks<TF, P>::LR * Blocks<TF, P>::UT * kLane);
+    static constexpr int bytes =
+        16 * (sz + kRowSlots + P * kSt + Blocks<TF, P>::LR * Blocks<TF, P>::UT * kLane + Blocks<TF, P>::RB);
     static_assert(bytes <= 160 * 1024, "LDS budget");
 };
 
@@ -578,6 +592,7 @@ __global__ __launch_bounds__(kLane * (STAGED ? kWavesStaged : 1)) void k_bsolve(
     // z rows [r0 - P, r0 + NZ - P) (FUSE; zero outside [0, N)); then carry states and scrap rows
     __shared__ lcplx sz[STAGED ? S::sz : kLane * B::RB];
     __shared__ lcplx sT[STAGED ? B::LR * B::UT * kLane : 1];    // staged table rows
+    __shared__ lcplx s0[B::RB];                                 // zero rows
 
     int ch = blockIdx.y, seg = blockIdx.x;
     if (tm.order) {
@@ -610,6 +625,7 @@ __global__ __launch_bounds__(kLane * (STAGED ? kWavesStaged : 1)) void k_bsolve(
     if (w == 0) {
         BlockRegs<TF, P> c;
         cplx h[P];
+        if (ln < B::RB) s0[ln] = lcplx{0.0, 0.0};
         const lcplx* sL = sT + ln;
         lcplx* scrap = sz + (STAGED ? S::scrap : 0) + ln * B::RB;
         if constexpr (STAGED) {
@@ -652,7 +668,7 @@ __global__ __launch_bounds__(kLane * (STAGED ? kWavesStaged : 1)) void k_bsolve(
         // forward: pass A from the zero state, carry, pass B
 #pragma unroll 1
         for (int pass = 0;; ++pass) {
-            fwd_pass<TF, P, STAGED>(c, T, off, sL, rows, pass ? rows : scrap, pass ? B::RB : 0, h, pass ? Tb0 : T);
+            fwd_pass<TF, P, STAGED>(c, T, off, sL, rows, pass ? rows : scrap, pass ? B::RB : 0, h, pass ? Tb0 : T, s0);
             if (pass) break;
             if constexpr (STAGED) {
 #pragma unroll
@@ -776,37 +792,35 @@ __global__ __launch_bounds__(kLane * (STAGED ? kWavesStaged : 1)) void k_bsolve(
     for (int i = i0 + tid; i < i1; i += NTH) xo[i] = cj_if(cj, sv[row_slot(i % kPM, i / kPM)]);
 }
 
-// The same solve with eight lanes per partition, for channels of at most
-// kSplitParts partitions, whose lanes k_bsolve's wave would leave idle.  Lane l
-// owns rows l, l + 8 and l + 16 of its partition.  Going down, the row's value
-// is broadcast to the eight (two DPP moves per double) and each lane subtracts
-// its multiple from the row it gathers next: P products per row in one
-// instruction each, and the chain of a row is a broadcast and two FMAs.  The
-// lane that owned the row starts its next one from zero: its coefficient is 1
-// (P = 8: row s itself reaches row s + 8, so the lane's sum is set to zero).
-// Going up is the same from the last row, with the rows' own coefficients.
-// The state a partition hands down is what the eight lanes have gathered for
-// the first rows of the next one.  A lane's 24 coefficients per direction stay
-// in registers for both passes, its rows too: LDS holds the rows of z for the
-// right-hand side, P rows on either side, and the states of the carries, which
-// each lane runs for its own entry (row l of the transfer matrix).
+// The same solve, bit for bit, with eight lanes per partition, for channels of
+// at most kSplitParts partitions and for longer ones on small grids, where
+// k_bsolve's waves would leave lanes or compute units idle.  Lane l owns rows l,
+// l + 8 and l + 16 of its partition.  Going down, the row's value is broadcast
+// to the eight (two DPP moves per double) and each lane subtracts its multiple
+// from the row it gathers next, which it began with the row's right-hand side:
+// P products per row in one instruction each, and the chain of a row is a
+// broadcast and two FMAs.  Going up is the same from the last row, with the
+// rows' own coefficients.  The state a partition hands down is what the eight
+// lanes have gathered for the first rows of the next one.  A lane's 24
+// coefficients per direction stay in registers for both passes, its rows too:
+// LDS holds the rows of z for the right-hand side, P rows on either side, and
+// the states of the carries, which each lane runs for its own entry (row l of
+// the transfer matrix).
 //
-// Forward rows of a real table are scaled by the target row's 1/u as they are
-// loaded (y_i = r_i v_i - sum (r_i F) y); the rows beyond the partition are not,
-// their state is.
-//
-// A pass takes 1.4 k cycles (k_bsolve: 6.5 k), so what bounds it is the loads:
-// every table entry twice, the band entries of three rows per lane.  Longer
-// channels would wait for them as long (N = 1500: no gain) and, with one
-// work-group per compute unit, on grids of many channels longer.  R, D, free
-// and mask solves of 6 channels of N = 240: 12.2 / 11.1 / 12.1 / 9.4 us (k_bsolve
-// 21.6 / 18.0 / 21.4 / 17.0); whole passes at 32 partitions: 31 channels step by
-// step 5.3 -> 4.3 ms, 2400 batched ones 36.0 -> 31.1; at 42 (N = 1000) 651
-// channels are 15 % slower, hence the line.
+// A pass takes 1.6 k cycles (k_bsolve: 6.5 k), so what bounds it is the loads:
+// every table entry twice, the band entries of three rows per lane.  More
+// partitions to a work-group would wait for them as long as k_bsolve does (64 at
+// N = 1500: no gain), and so would two work-groups to a compute unit.  R, D, free
+// and mask solves of 6 channels of N = 240: 12.3 / 11.2 / 12.2 / 9.5 us (k_bsolve
+// 21.6 / 18.0 / 21.4 / 17.0).  At 32 partitions 31 channels step by step 5.3 ->
+// 4.3 ms, 2400 batched ones 36.0 -> 31.1.  Longer channels, a step of one
+// segment or more each, k_bsolve before: 31 channels of N = 1000 155 -> 118 us,
+// 41 of N = 1500 167 -> 127, 51 of N = 2000 175 -> 143, 30 of N = 3000 170 -> 134.
 //
 // FUSE: as k_bsolve's; with one segment src and zout may be the same.
 constexpr int kSplit = 8;                     // lanes per partition
 constexpr int kSplitParts = 32;               // partitions up to which they are used
+constexpr int64_t kSplitGrid = 256;           // work-groups of longer channels, one per compute unit
 constexpr int kOwn = kPM / kSplit;            // rows per lane
 constexpr int kSt8 = kSplit + 1;              // a state's entries in LDS, odd for the banks
 static_assert(kPM % kSplit == 0 && kSplit == 8, "lane layout");
@@ -820,7 +834,6 @@ __device__ inline double bcast8(double v) {  // lane L of each eight
 template <int L>
 __device__ inline cplx bcast8(cplx v) { return {bcast8<L>(v.re), bcast8<L>(v.im)}; }
 __device__ inline cplx pick(bool c, cplx a, cplx b) { return {c ? a.re : b.re, c ? a.im : b.im}; }
-__device__ inline double pick(bool c, double a, double b) { return c ? a : b; }
 // keeps a value where it is computed: put off to its use, it would keep its
 // operands alive until then
 __device__ inline void keep(cplx& v) { asm volatile("" : "+v"(v.re), "+v"(v.im)); }
@@ -841,29 +854,67 @@ struct LaneTab {
 // rows down through the partition: z the own rows' right-hand sides, acc what
 // the partition above contributes (in) and what this one does to the next
 // (out), y the own rows
-template <class TF, int P>
-__device__ inline void rows_down(const TF (&C)[kPM], const cplx (&z)[kOwn], cplx (&y)[kOwn], cplx& acc, int l) {
+template <int P>
+__device__ inline void rows_down(const cplx (&C)[kPM], const cplx (&z)[kOwn], cplx (&y)[kOwn], cplx& acc, int l) {
+    acc = {acc.re + z[0].re, acc.im + z[0].im};
     each(std::make_integer_sequence<int, kPM>{}, [&](auto sc) {
         constexpr int s = decltype(sc)::value, t = s / kSplit, r = s % kSplit;
-        if constexpr (r == 0) acc = {acc.re + z[t].re, acc.im + z[t].im};
         const cplx x = bcast8<r>(acc);
         y[t] = pick(l == r, acc, y[t]);
         keep(y[t]);
-        if constexpr (P == 8) acc = pick(l == r, cplx{0.0, 0.0}, acc);
-        acc = tmsub(acc, C[s], x);
+        cplx next = {0.0, 0.0};
+        if constexpr (t + 1 < kOwn) next = z[t + 1];
+        acc = tmsub(pick(l == r, next, acc), C[s], x);
     });
 }
-// rows up; acc: what the partition below contributes to the last eight
-template <class TF, int P>
-__device__ inline void rows_up(const TF (&C)[kPM], const cplx (&y)[kOwn], cplx (&x)[kOwn], cplx acc, int l) {
+// rows up; acc: the last eight's y less what the partition below contributes
+template <int P>
+__device__ inline void rows_up(const cplx (&C)[kPM], const cplx (&y)[kOwn], cplx (&x)[kOwn], cplx acc, int l) {
     each(std::make_integer_sequence<int, kPM>{}, [&](auto sc) {
         constexpr int s = kPM - 1 - decltype(sc)::value, t = s / kSplit, r = s % kSplit;
-        if constexpr (r == kSplit - 1) acc = {acc.re + y[t].re, acc.im + y[t].im};
         const cplx v = bcast8<r>(acc);
         x[t] = pick(l == r, acc, x[t]);
         keep(x[t]);
-        if constexpr (P == 8) acc = pick(l == r, cplx{0.0, 0.0}, acc);
-        acc = tmsub(acc, C[s], v);
+        if constexpr (s > 0) {
+            if constexpr (t > 0) acc = pick(l == r, y[t - 1], acc);
+            acc = tmsub(acc, C[s], v);
+        }
+    });
+}
+
+// The same for real tables, whose coefficients leave room for two of each:
+// C[s] where lane l still gathers its row of this eight (l past row s), B[s]
+// where it gathers the next eight's, zero elsewhere.  Then no value is picked:
+// two products for eight moves (a step of 6 channels of N = 240 83 -> 80 us).
+template <int P>
+__device__ inline void rows_down_r(const double (&C)[kPM], const double (&B)[kPM], const double (&dg)[kOwn],
+                                   const cplx (&z)[kOwn], cplx (&y)[kOwn], cplx& acc) {
+    cplx a[kOwn + 1];
+    a[0] = {acc.re + z[0].re, acc.im + z[0].im};
+#pragma unroll
+    for (int t = 1; t < kOwn; ++t) a[t] = z[t];
+    a[kOwn] = {0.0, 0.0};
+    each(std::make_integer_sequence<int, kPM>{}, [&](auto sc) {
+        constexpr int s = decltype(sc)::value, t = s / kSplit, r = s % kSplit;
+        const cplx x = bcast8<r>(cplx{dg[t] * a[t].re, dg[t] * a[t].im});
+        if constexpr (r < kSplit - 1) a[t] = tmsub(a[t], C[s], x);
+        if constexpr (r > 0 || P == 8) a[t + 1] = tmsub(a[t + 1], B[s], x);
+    });
+#pragma unroll
+    for (int t = 0; t < kOwn; ++t) y[t] = {dg[t] * a[t].re, dg[t] * a[t].im};
+    acc = a[kOwn];
+}
+template <int P>
+__device__ inline void rows_up_r(const double (&C)[kPM], const double (&B)[kPM], const cplx (&y)[kOwn],
+                                 cplx (&x)[kOwn], cplx acc) {
+    x[kOwn - 1] = acc;
+#pragma unroll
+    for (int t = 0; t + 1 < kOwn; ++t) x[t] = y[t];
+    each(std::make_integer_sequence<int, kPM>{}, [&](auto sc) {
+        constexpr int s = kPM - 1 - decltype(sc)::value, t = s / kSplit, r = s % kSplit;
+        const cplx v = bcast8<r>(x[t]);
+        if constexpr (r > 0) x[t] = tmsub(x[t], C[s], v);
+        if constexpr (t > 0 && (r < kSplit - 1 || P == 8)) x[t > 0 ? t - 1 : 0] = tmsub(x[t > 0 ? t - 1 : 0], B[s], v);
     });
 }
 
@@ -906,8 +957,8 @@ __device__ inline void trf_row(TF (&t)[P], const TF* T, unsigned off, int dir, i
 template <class TF, int ROLE, bool FUSE, int P>
 __global__ __launch_bounds__(kSplitParts * kSplit) void k_bsolve8(const cplx* __restrict__ tab, const TF* __restrict__ trf,
                                                            TabMap tm, const cplx* __restrict__ src,
-                                                           cplx* __restrict__ zout, Geom geo, int SN, int PK,
-                                                           RhsArgs ra) {
+                                                           cplx* __restrict__ zout, Geom geo, int SN, int SX,
+                                                           int PK, RhsArgs ra) {
     using F = TabFmt<TF, P>;
     using LT = LaneTab<TF, P>;
     constexpr bool SYM = F::SYM;
@@ -922,7 +973,8 @@ __global__ __launch_bounds__(kSplitParts * kSplit) void k_bsolve8(const cplx* __
         seg = o & 255;
     }
     const int N = geo.N, NP = geo.P;
-    const int k0 = seg * SN, k1 = min(NP, k0 + SN);         // owned partitions [k0, k1)
+    // owned partitions [k0, k1): SN, the first segment's SX more, the last one's what is left
+    const int k0 = seg ? SX + seg * SN : 0, k1 = seg == (int)gridDim.x - 1 ? NP : SX + (seg + 1) * SN;
     const int ga = max(0, k0 - PK), gb = min(NP, k1 + PK);  // staged partitions [ga, gb)
     const int n = gb - ga;
     const int tid = threadIdx.x, q = tid / kSplit, l = tid % kSplit;
@@ -1027,32 +1079,27 @@ __global__ __launch_bounds__(kSplitParts * kSplit) void k_bsolve8(const cplx* __
 #pragma unroll
     for (int t = kOwn - 1; t >= T1; --t) load_up(t);
     // down: pass A from the zero state, carry, pass B
+    TF B[SYM ? 1 : kPM];
     if constexpr (!SYM) {
 #pragma unroll
-        for (int t = 0; t < kOwn; ++t) {
-            z[t] = {dg[t] * z[t].re, dg[t] * z[t].im};
-#pragma unroll
-            for (int r = 0; r < kSplit; ++r) {
-                // the row that lane l gathers after row 8 t + r: its own of this eight, or of the next
-                const double up = t + 1 < kOwn ? dg[t + 1 < kOwn ? t + 1 : t] : 1.0;
-                C[t * kSplit + r] *= l > r ? dg[t] : up;
-            }
+        for (int s = 0; s < kPM; ++s) {
+            B[s] = (P == 8 ? l <= s % kSplit : l < s % kSplit) ? C[s] : 0.0;
+            C[s] = l > s % kSplit ? C[s] : 0.0;
         }
-    }
-    if constexpr (P == 7) {
+    } else if constexpr (P == 7) {
 #pragma unroll
-        for (int s = 0; s < kPM; ++s) C[s] = pick(l == s % kSplit, tone(TF{}), C[s]);
+        for (int s = 0; s < kPM; ++s) C[s] = pick(l == s % kSplit, tzero(TF{}), C[s]);
     }
     cplx y[kOwn], acc = {0.0, 0.0};
 #pragma unroll
     for (int t = 0; t < kOwn; ++t) y[t] = acc;
 #pragma unroll 1
     for (int pass = 0;; ++pass) {
-        rows_down<TF, P>(C, z, y, acc, l);
+        if constexpr (SYM) rows_down<P>(C, z, y, acc, l);
+        else rows_down_r<P>(C, B, dg, z, y, acc);
         if (pass) break;
         const lcplx* in = carry<TF, P>(sS, tr, acc, own, q > 0 && q < n ? q - 1 : kSplitParts, PK, 0);
         acc = l < P ? (cplx)in[l] : cplx{0.0, 0.0};
-        if constexpr (!SYM) acc = {dg[0] * acc.re, dg[0] * acc.im};
     }
     // up
 #pragma unroll
@@ -1068,23 +1115,31 @@ __global__ __launch_bounds__(kSplitParts * kSplit) void k_bsolve8(const cplx* __
         }
     }
     cplx x[kOwn];
-    if constexpr (P == 7) {
+    if constexpr (!SYM) {
 #pragma unroll
-        for (int s = kPM - 1; s >= 0; --s) D[s] = pick(l == s % kSplit, tone(TF{}), D[s]);
+        for (int s = kPM - 1; s >= 0; --s) {
+            B[s] = (P == 8 ? l >= s % kSplit : l > s % kSplit) ? D[s] : 0.0;
+            D[s] = l < s % kSplit ? D[s] : 0.0;
+        }
+    } else if constexpr (P == 7) {
+#pragma unroll
+        for (int s = kPM - 1; s >= 0; --s) D[s] = pick(l == s % kSplit, tzero(TF{}), D[s]);
     }
 #pragma unroll
     for (int t = 0; t < kOwn; ++t) x[t] = {0.0, 0.0};
-    acc = {0.0, 0.0};
+    acc = y[kOwn - 1];
 #pragma unroll 1
     for (int pass = 0;; ++pass) {
-        rows_up<TF, P>(D, y, x, acc, l);
+        if constexpr (SYM) rows_up<P>(D, y, x, acc, l);
+        else rows_up_r<P>(D, B, y, x, acc);
         if (pass) break;
         const lcplx* in = carry<TF, P>(sS, tr, x[0], own, q + 1 < n ? q + 1 : kSplitParts, PK, PK);
         // the first P rows of the partition below, seen from this one's last eight
 #pragma unroll
         for (int i = P - 1; i >= 0; --i) {
             const bool on = P == 7 ? l > i : l >= i;
-            acc = tmsub(acc, pick(on, D[i], tzero(TF{})), (cplx)in[i]);
+            if constexpr (SYM) acc = tmsub(acc, pick(on, D[i], tzero(TF{})), (cplx)in[i]);
+            else acc = tmsub(acc, B[i], (cplx)in[i]);
         }
     }
     cplx* xo = zout + (int64_t)ch * N;
@@ -1112,15 +1167,16 @@ __global__ __launch_bounds__(64) void k_seqsolve(const cplx* __restrict__ tab, T
     const cplx* v = vin + (int64_t)ch * N;
     cplx* x = zout + (int64_t)ch * N;
     cplx h[P];
+    auto vat = [&](int i) { return i < N ? cj_if(cj, v[min(i, N - 1)]) : cplx{0.0, 0.0}; };
 #pragma unroll
-    for (int j = 0; j < P; ++j) h[j] = {0.0, 0.0};
+    for (int j = 0; j < P; ++j) h[j] = vat(j);
     for (int i0 = 0; i0 < N; i0 += RB) {
         cplx c[RB][F::UF], vr[RB];
 #pragma unroll
         for (int b = 0; b < RB; ++b) {
             const int i = min(i0 + b, N - 1);
             row_g<TF, P, F::UF>(c[b], T0, part_off<TF, P>(i / kPM), i % kPM);
-            vr[b] = cj_if(cj, v[i]);
+            vr[b] = vat(i0 + b + P);
         }
 #pragma unroll
         for (int b = 0; b < RB; ++b)
@@ -1736,6 +1792,34 @@ void solve_order(const int* tab, int nch, int nseg, int* order) {
     }
 }
 
+// The launch of the solve with eight lanes per partition.  Channels of at most
+// kSplitParts partitions always run it; longer ones are cut into the fewest
+// work-groups of that many partitions, halos included (the outer segments have
+// a halo on one side only and own that many more), evened out, if no more than
+// kSplitGrid work-groups result.  One step, N = 1000, k_bsolve against eight
+// lanes: 100 channels (200 work-groups) 184 / 152 us, 128 (256) 194 / 166, 140
+// (280) 200 / 214; N = 1500: 80 channels (240) 183 / 149, 86 (258) 186 / 195.
+struct SplitGrid {
+    int nseg = 0, sn = 0, sx = 0, parts = 0;  // nseg 0: not this launch; parts: the most of a work-group
+};
+static SplitGrid split_grid(const Geom& geo, int nch, int pk) {
+    SplitGrid g;
+    if (geo.P <= kSplitParts) {
+        g.sn = seg_parts(geo, pk);
+        g.nseg = (geo.P + g.sn - 1) / g.sn;
+        g.parts = std::min(geo.P, g.nseg > 1 ? g.sn + 2 * pk : g.sn);
+        return g;
+    }
+    const int own = kSplitParts - 2 * pk;  // of an inner segment
+    if (own < 1) return g;
+    const int n = (geo.P - 2 * pk + own - 1) / own + std::max(0, geo.seg_add);
+    const int64_t grid = (int64_t)n * nch;
+    if (grid > kSplitGrid || grid > geo.stage_grid) return g;
+    const int w = (geo.P + 2 * pk * (n - 1) + n - 1) / n, sn = w - 2 * pk;
+    if (sn < 1 || pk + (n - 1) * sn >= geo.P) return g;  // (more segments than they can share)
+    return {n, sn, pk, w};
+}
+
 template <class TF, int ROLE, int P>
 static void bsolve(hipStream_t s, const TF* tab, const TF* trf, TabMap tm, const cplx* zin, cplx* vbuf,
                    cplx* zout, int nch, Geom geo, const RhsArgs* ra, int pk) {
@@ -1750,26 +1834,27 @@ static void bsolve(hipStream_t s, const TF* tab, const TF* trf, TabMap tm, const
                            geo, nch);
         return;
     }
-    const int sn = seg_parts(geo, PK);
-    const int nseg = (geo.P + sn - 1) / sn;
+    const SplitGrid g8 = split_grid(geo, nch, PK);
+    const int sn = g8.nseg ? g8.sn : seg_parts(geo, PK);
+    const int nseg = g8.nseg ? g8.nseg : (geo.P + sn - 1) / sn;
     if (tm.order && nseg != tm.order_nseg) tm.order = nullptr;  // built for another launch shape
-    if (geo.P <= kSplitParts) {
-        // eight lanes per partition; the right-hand side in the launch unless another work-group may still read
+    if (g8.nseg) {
+        // the right-hand side in the launch unless another work-group may still read
         // rows of z that one writes
-        const dim3 grid8(nseg, nch), block((std::min(geo.P, nseg > 1 ? sn + 2 * PK : sn) + 7) / 8 * kLane);
+        const dim3 grid8(nseg, nch), block((g8.parts + 7) / 8 * kLane);
         if (ra) {
             const uintptr_t a0 = (uintptr_t)zin, b0 = (uintptr_t)zout;
             const uintptr_t len = sizeof(cplx) * (uintptr_t)nch * geo.N;
             if (a0 + len <= b0 || b0 + len <= a0 || (nseg == 1 && a0 == b0)) {
                 hipLaunchKernelGGL((k_bsolve8<TF, ROLE, true, P>), grid8, block, 0, s, (const cplx*)tab, trf, tm, zin,
-                                   zout, geo, sn, PK, *ra);
+                                   zout, geo, sn, g8.sx, PK, *ra);
                 return;
             }
             rhs_launch<P>(s, ROLE, *ra, tm, zin, vbuf, nch, geo);
             zin = vbuf;
         }
         hipLaunchKernelGGL((k_bsolve8<TF, ROLE, false, P>), grid8, block, 0, s, (const cplx*)tab, trf, tm, zin, zout, geo,
-                           sn, PK, RhsArgs{});
+                           sn, g8.sx, PK, RhsArgs{});
         return;
     }
     // staged grids form the right-hand side in the launch when z and x do not overlap

@@ -212,3 +212,32 @@ def test_steps_where_the_solve_changes_kernel(N, p):
     assert err <= 1e-12
     assert all(np.array_equal(x, out[0]) for x in out[1:])
     prop.close()
+
+
+@pytest.mark.parametrize("N,p", [(769, 7), (1000, 8), (1537, 7), (1801, 8), (2305, 7)])
+def test_steps_whichever_solve_kernel_runs(N, p):
+    """Long channels on small grids are cut into segments with eight lanes per
+    partition, on large ones run with one: the same bits either way, and the
+    oracle's steps."""
+    print(f"case: solve kernels on long channels N={N} p={p}", flush=True)
+    o, prop = _pair(N, p, 3, M=3, m0=-1)
+    c = mixed_state(o, seed=N + p, amp=0.3)
+    ref = c.copy()
+    out = []
+    for seg, grid in ((0, 512), (3, 512), (0, 0), (1, 0)):
+        prop.set_tune(seg_add=seg, stage_grid=grid)
+        prop.set_state(c)
+        for a in ((0.7, 0.9), (0.9, -0.4)):
+            prop.propagate(*a)
+        prop.propagate()
+        prop.mask()
+        out.append(prop.get_state().copy())
+    for a in ((0.7, 0.9), (0.9, -0.4)):
+        o.step(ref, *a)
+    o.step_free(ref)
+    o.mask(ref)
+    err = rel_l2(out[0], ref)
+    print(f"  rel L2 {err:.2e}", flush=True)
+    assert err <= 1e-12
+    assert all(np.array_equal(x, out[0]) for x in out[1:])
+    prop.close()
