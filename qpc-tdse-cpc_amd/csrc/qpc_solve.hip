@@ -810,17 +810,17 @@ __global__ __launch_bounds__(kLane * (STAGED ? kWavesStaged : 1)) void k_bsolve(
 // A pass takes 1.6 k cycles (k_bsolve: 6.5 k), so what bounds it is the loads:
 // every table entry twice, the band entries of three rows per lane.  More
 // partitions to a work-group would wait for them as long as k_bsolve does (64 at
-// N = 1500: no gain), and so would two work-groups to a compute unit.  R, D, free
-// and mask solves of 6 channels of N = 240: 12.3 / 11.2 / 12.2 / 9.5 us (k_bsolve
-// 21.6 / 18.0 / 21.4 / 17.0).  At 32 partitions 31 channels step by step 5.3 ->
-// 4.3 ms, 2400 batched ones 36.0 -> 31.1.  Longer channels, a step of one
-// segment or more each, k_bsolve before: 31 channels of N = 1000 155 -> 118 us,
-// 41 of N = 1500 167 -> 127, 51 of N = 2000 175 -> 143, 30 of N = 3000 170 -> 134.
+// N = 1500: no gain), and so would two work-groups to a compute unit; fewer wait
+// less (split_grid).  R, D, free and mask solves of 6 channels of N = 240: 12.3 /
+// 11.2 / 12.2 / 9.5 us (k_bsolve 21.6 / 18.0 / 21.4 / 17.0).  At 32 partitions,
+// uncut, 31 channels step by step 5.3 -> 4.3 ms, 2400 batched ones 36.0 -> 31.1.
+// A step of longer channels, k_bsolve before: 31 of N = 1000 155 -> 102 us, 41 of
+// N = 1500 167 -> 118, 51 of N = 2000 175 -> 140, 30 of N = 3000 170 -> 132.
 //
 // FUSE: as k_bsolve's; with one segment src and zout may be the same.
 constexpr int kSplit = 8;                     // lanes per partition
 constexpr int kSplitParts = 32;               // partitions up to which they are used
-constexpr int64_t kSplitGrid = 256;           // work-groups of longer channels, one per compute unit
+constexpr int64_t kSplitGrid = 256;           // work-groups of a cut grid, one per compute unit
 constexpr int kOwn = kPM / kSplit;            // rows per lane
 constexpr int kSt8 = kSplit + 1;              // a state's entries in LDS, odd for the banks
 static_assert(kPM % kSplit == 0 && kSplit == 8, "lane layout");
@@ -1792,32 +1792,53 @@ void solve_order(const int* tab, int nch, int nseg, int* order) {
     }
 }
 
-// The launch of the solve with eight lanes per partition.  Channels of at most
-// kSplitParts partitions always run it; longer ones are cut into the fewest
-// work-groups of that many partitions, halos included (the outer segments have
-// a halo on one side only and own that many more), evened out, if no more than
-// kSplitGrid work-groups result.  One step, N = 1000, k_bsolve against eight
-// lanes: 100 channels (200 work-groups) 184 / 152 us, 128 (256) 194 / 166, 140
-// (280) 200 / 214; N = 1500: 80 channels (240) 183 / 149, 86 (258) 186 / 195.
+// The launch of the solve with eight lanes per partition: channels of at most
+// kSplitParts partitions always run it, longer ones if they can be cut into
+// work-groups of that many partitions, halos included, of which no more than
+// kSplitGrid result (the outer segments have a halo on one side only and own
+// that many more partitions).  One step, N = 1000, k_bsolve against eight lanes:
+// 100 channels (200 work-groups) 184 / 152 us, 128 (256) 194 / 166, 140 (280)
+// 200 / 214; N = 1500: 80 channels (240) 183 / 149, 86 (258) 186 / 195.
+//
+// Within these work-groups, the fewest segments that leave each the fewest
+// waves (short channels too, unless the solve is in place, where one segment
+// keeps the right-hand side in the launch): a step of 8 channels of N = 1000
+// takes 105 us with four waves each, 99 / 94 / 87 as the operators' solves come
+// down to three and two, and does not change in between.
 struct SplitGrid {
     int nseg = 0, sn = 0, sx = 0, parts = 0;  // nseg 0: not this launch; parts: the most of a work-group
+    int waves() const { return (parts + 7) / 8; }
 };
-static SplitGrid split_grid(const Geom& geo, int nch, int pk) {
-    SplitGrid g;
-    if (geo.P <= kSplitParts) {
-        g.sn = seg_parts(geo, pk);
-        g.nseg = (geo.P + g.sn - 1) / g.sn;
-        g.parts = std::min(geo.P, g.nseg > 1 ? g.sn + 2 * pk : g.sn);
+static SplitGrid split_grid(const Geom& geo, int nch, int pk, bool in_place) {
+    const bool whole = geo.P <= kSplitParts;
+    auto cut = [&](int n) {
+        SplitGrid g;
+        const int w = (geo.P + 2 * pk * (n - 1) + n - 1) / n, sn = w - 2 * pk;
+        if (w <= kSplitParts && sn >= 1 && pk + (n - 1) * sn < geo.P) g = {n, sn, pk, w};
         return g;
+    };
+    SplitGrid best;
+    if (!whole || !in_place) {
+        const int most = (int)std::min<int64_t>(geo.P, std::min(kSplitGrid, geo.stage_grid) / std::max(1, nch));
+        int waves = whole ? (geo.P + 7) / 8 : kSplitParts / 8 + 1;
+        for (int n = 2; n <= most; ++n) {
+            const SplitGrid g = cut(n);
+            if (g.nseg && g.waves() < waves) {
+                best = g;
+                waves = g.waves();
+            }
+        }
+        if (best.nseg && geo.seg_add > 0 && best.nseg + geo.seg_add <= most) {
+            const SplitGrid g = cut(best.nseg + geo.seg_add);
+            if (g.nseg) best = g;
+        }
     }
-    const int own = kSplitParts - 2 * pk;  // of an inner segment
-    if (own < 1) return g;
-    const int n = (geo.P - 2 * pk + own - 1) / own + std::max(0, geo.seg_add);
-    const int64_t grid = (int64_t)n * nch;
-    if (grid > kSplitGrid || grid > geo.stage_grid) return g;
-    const int w = (geo.P + 2 * pk * (n - 1) + n - 1) / n, sn = w - 2 * pk;
-    if (sn < 1 || pk + (n - 1) * sn >= geo.P) return g;  // (more segments than they can share)
-    return {n, sn, pk, w};
+    if (whole && !best.nseg) {
+        best.sn = seg_parts(geo, pk);
+        best.nseg = (geo.P + best.sn - 1) / best.sn;
+        best.parts = std::min(geo.P, best.nseg > 1 ? best.sn + 2 * pk : best.sn);
+    }
+    return best;
 }
 
 template <class TF, int ROLE, int P>
@@ -1834,7 +1855,7 @@ static void bsolve(hipStream_t s, const TF* tab, const TF* trf, TabMap tm, const
                            geo, nch);
         return;
     }
-    const SplitGrid g8 = split_grid(geo, nch, PK);
+    const SplitGrid g8 = split_grid(geo, nch, PK, ra && zin == zout);
     const int sn = g8.nseg ? g8.sn : seg_parts(geo, PK);
     const int nseg = g8.nseg ? g8.nseg : (geo.P + sn - 1) / sn;
     if (tm.order && nseg != tm.order_nseg) tm.order = nullptr;  // built for another launch shape
