@@ -7,9 +7,9 @@
 // uses them, the norm it leaves in partial sums is finished by the next
 // vector's k_hmul, which also normalises the vector, and the tridiagonal goes
 // to host memory that the device writes.
-// A vector now takes 40 us, 30 of them in its four kernels: k_hmul 4.9 us (was
-// 11.3), k_dots 4, the solve 14.4, k_axpy_norm 6.4 (6.2 with 8.6 for the norm
-// and 2.2 for the scaling).
+// A vector now takes 37 us, 25 of them in its four kernels: k_hmul 4.9 us (was
+// 11.3), k_dots 4.2, the solve 8.6 (21), k_axpy_norm 6.8 (6.2 with 8.6 for the
+// norm and 2.2 for the scaling).
 #include "qpc_krylov.h"
 
 #include <algorithm>
