@@ -161,7 +161,7 @@ struct qpc_ctx {
     std::vector<double> h_e;             // host copy of d_e
     bool have_outer = false;
     cplx *kU = nullptr, *kpart = nullptr, *kcoef = nullptr;
-    double* knorm = nullptr;       // partial sums of a squared norm
+    double *ktab = nullptr, *ktrf = nullptr;  // chol(S) tables of the Lanczos vectors' solves
     double* kab = nullptr;         // tridiagonal a_i at 2 i, b_i at 2 i + 1 (host memory, written by the device)
     hipEvent_t kev = nullptr;      // a vector's b is there
     int64_t kry_cap = 0;

@@ -696,7 +696,7 @@ int qpc_destroy(qpc_ctx* c) {
                     c->rpow1d, c->sxR, c->sxD, c->sxL, c->fxR, c->fxD, c->fxL, c->tsf_ib, c->tsf_b0, c->tsf_br, c->tsf_kr, c->tsf_ckt,
                     c->tsf_j0, c->tsf_jr, c->tsf_pm, c->tsf_Y, c->tsf_tmp, c->tsf_work, c->tsf_stx, c->tsf_sty,
                     c->tsf_pm1, c->tsf_pm2, c->rtY, c->rtYt, c->rtM, c->rtMh, c->rtQ, c->rtQh,
-                    c->Wp, c->ppart, c->pchan, c->pcnt, c->pout, c->Hd, c->q10, c->kU, c->kpart, c->kcoef, c->knorm,
+                    c->Wp, c->ppart, c->pchan, c->pcnt, c->pout, c->Hd, c->q10, c->kU, c->kpart, c->kcoef, c->ktab, c->ktrf,
                     c->souter, c->accel, c->hist, c->red4, c->obs_tmp, c->pcs_Wp, c->pcs_part, c->pcs_chan,
                     c->pcs_cnt, c->pcs_cps, c->pcs_out, c->pcs_lmd};
     for (void* p : ptrs)
@@ -763,6 +763,7 @@ int qpc_upload_radial(qpc_ctx* c, const double* S, const double* chol, const dou
     // absorber solve tables from chol(S) and their partition transfers
     qpc::launch_tab_chol(c->stream, c->chol, c->tab_mask, c->geo);
     qpc::launch_transfer_r(c->stream, c->tab_mask, c->trf_mask, 1, c->geo);
+    if (c->ktrf) qpc::launch_ssolve_tables(c->stream, c->chol, c->ktab, c->ktrf, c->geo);
     TRY(launch_check(c, "mask tables"));
     QPC_HIP_CHECK(c, hipStreamSynchronize(c->stream));
     c->have_radial = true;
@@ -1623,6 +1624,12 @@ int qpc_upload_krylov(qpc_ctx* c, const double* H, const double* y10, const doub
     const size_t nl = (size_t)c->lmax + 1, band = (size_t)c->N * c->ne, ml = (size_t)c->ML;
     int rc = QPC_OK;
     if (!c->Hd && ((rc = dev_alloc(c, &c->Hd, nl * band)) || (rc = dev_alloc(c, &c->q10, ml)))) return rc;
+    if (!c->ktrf) {
+        // (upload_radial renews them from then on)
+        if (!c->ktab && (rc = dev_alloc(c, &c->ktab, (size_t)qpc::ssolve_tab_elems(c->geo)))) return rc;
+        if ((rc = dev_alloc(c, &c->ktrf, (size_t)qpc::ssolve_trf_elems(c->geo)))) return rc;
+        if (c->have_radial) qpc::launch_ssolve_tables(c->stream, c->chol, c->ktab, c->ktrf, c->geo);
+    }
     double* tmp = nullptr;
     if ((rc = dev_alloc(c, &tmp, nl * band))) return rc;
     DevTemp guard{tmp};
@@ -1677,17 +1684,17 @@ int krylov_core(qpc_ctx* c, double az, double dt, int64_t kstart, int64_t kmax, 
     QPC_HIP_CHECK(c, hipStreamSynchronize(c->fstream));
     if (kmax + 2 > c->kry_cap) {
         QPC_HIP_CHECK(c, hipStreamSynchronize(c->stream));
-        void* old[] = {c->kU, c->kpart, c->kcoef, c->knorm};
+        void* old[] = {c->kU, c->kpart, c->kcoef};
         for (void* p : old)
             if (p) QPC_HIP_CHECK(c, hipFree(p));
         if (c->kab) QPC_HIP_CHECK(c, hipHostFree(c->kab));
         c->kU = c->kpart = c->kcoef = nullptr;
-        c->knorm = c->kab = nullptr;
+        c->kab = nullptr;
         c->kry_cap = 0;
         int rc = QPC_OK;
         if ((rc = dev_alloc(c, &c->kU, (size_t)(kmax + 2) * n)) ||
             (rc = dev_alloc(c, &c->kpart, (size_t)(kmax + 2) * qpc::kDotBlocks)) ||
-            (rc = dev_alloc(c, &c->kcoef, (size_t)(kmax + 2))) || (rc = dev_alloc(c, &c->knorm, qpc::kNormBlocks)))
+            (rc = dev_alloc(c, &c->kcoef, (size_t)(kmax + 2))))
             return rc;
         QPC_HIP_CHECK(c, hipHostMalloc((void**)&c->kab, sizeof(double) * 2 * (kmax + 2)));
         if (!c->kev) QPC_HIP_CHECK(c, hipEventCreateWithFlags(&c->kev, hipEventDisableTiming));
@@ -1696,14 +1703,12 @@ int krylov_core(qpc_ctx* c, double az, double dt, int64_t kstart, int64_t kmax, 
     TimedLaunch tl(c, QPC_K_KRYLOV);
     auto U = [&](int64_t i) { return c->kU + i * n; };
     cplx* T = c->vbuf;   // H u_{k-1}
-    cplx* W = c->tmpc;   // S^-1 T
-    cplx* V = c->spare;  // the next vector before its normalisation
+    cplx* V = c->spare;  // S^-1 T, then the next vector before its normalisation
     std::vector<double> a(kmax + 2, 0.0), b(kmax + 2, 0.0);
     std::vector<cplx> xs;
-    const qpc::TabMap tm{1, (int)c->L, (int)c->m0};
     const int N = (int)c->N, ML = (int)c->ML, p = (int)c->p;
     // construct_sub (la_1e.hpp:134-154): the norm of the state
-    qpc::launch_axpy_norm(c->stream, nullptr, 0, 0, nullptr, nullptr, c->Sd, c->coef, nullptr, N, ML, p, c->knorm);
+    qpc::launch_axpy_norm(c->stream, nullptr, 0, 0, nullptr, nullptr, c->Sd, c->coef, N, ML, p, c->red);
     // Lanczos loop (la_1e.hpp:318-328), orthogonalize_ip (:195-240).  Vector k
     // is queued whole; then the host waits for its norm b[k] (there after the
     // first of its kernels) and judges the k vectors before it while the rest
@@ -1712,15 +1717,14 @@ int krylov_core(qpc_ctx* c, double az, double dt, int64_t kstart, int64_t kmax, 
     for (int64_t k = 0;; ++k) {
         if (k < kmax) {
             qpc::launch_hmul(c->stream, c->Hd, c->rinvd, c->rdifd, c->y10, c->q10, az, (int)c->M, (int)c->L, (int)c->m0,
-                             N, p, k ? V : c->coef, c->knorm, k == 0, c->kab + 2 * k + 1, U(k), T);
+                             N, p, k ? V : c->coef, c->red, k == 0, c->kab + 2 * k + 1, U(k), T);
             QPC_HIP_CHECK(c, hipEventRecord(c->kev, c->stream));
             qpc::launch_dots(c->stream, c->kU, n, (int)k + 1, T, n, c->kpart);
-            // S \ (H u_k), channel by channel (chol(S) tables)
-            qpc::launch_bsolve_r(c->stream, qpc::RHS_RBAND, c->tab_mask, c->trf_mask, tm, T, W, ML, c->geo);
-            qpc::launch_axpy_norm(c->stream, c->kU, n, (int)k + 1, c->kpart, c->kab + 2 * k, c->Sd, W, V, N, ML, p,
-                                  c->knorm);
+            // S \ (H u_k), channel by channel
+            qpc::launch_ssolve(c->stream, c->ktab, c->ktrf, T, V, ML, c->geo);
+            qpc::launch_axpy_norm(c->stream, c->kU, n, (int)k + 1, c->kpart, c->kab + 2 * k, c->Sd, V, N, ML, p, c->red);
         } else {
-            qpc::launch_norm_final(c->stream, N, ML, c->knorm, c->kab + 2 * k + 1);
+            qpc::launch_norm_final(c->stream, ML, c->red, c->kab + 2 * k + 1);
             QPC_HIP_CHECK(c, hipEventRecord(c->kev, c->stream));
         }
         TRY(launch_check(c, "krylov vector"));

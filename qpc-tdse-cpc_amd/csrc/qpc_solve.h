@@ -156,18 +156,11 @@ void solve_order(const int* tab, int nch, int nseg, int* order);
 
 // v = B z for nch channels (vout: nch * N)
 void launch_rhs(hipStream_t s, int rhs, const RhsArgs& ra, TabMap tm, const cplx* zin, cplx* vout, int nch, Geom geo);
-// x = A^-1 v for nch channels; tab/trf hold the tables and transfer sets of
-// every table id, strides geo.ctab_elems (complex symmetric) or
-// geo.tab_elems (real LU) and geo.ctrf_elems or geo.trf_elems; role is the RhsKind of the
-// operator (kernel name only).  vin and zout may not alias.  pk is the carry
-// depth in partitions (0: the operator's default, kPKS or kPKD; > kPKMax:
-// the sequential solve).
-void launch_bsolve_c(hipStream_t s, int role, const cplx* tab, const cplx* trf, TabMap tm, const cplx* vin,
-                     cplx* zout, int nch, Geom geo, int pk = 0);
-void launch_bsolve_r(hipStream_t s, int role, const double* tab, const double* trf, TabMap tm, const cplx* vin,
-                     cplx* zout, int nch, Geom geo, int pk = 0);
-
-// v = B z (the RhsKind role with the bands of ra) and x = A^-1 v in one call.
+// v = B z (the RhsKind role with the bands of ra) and x = A^-1 v for nch
+// channels; tab/trf hold the tables and transfer sets of every table id,
+// strides geo.ctab_elems (complex symmetric) or geo.tab_elems (real LU) and
+// geo.ctrf_elems or geo.trf_elems.  pk is the carry depth in partitions (0: the
+// operator's default, kPKS or kPKD; > kPKMax: the sequential solve).
 // On small grids (kStageGrid) and for short channels, when zin and zout do not
 // overlap, the solve forms v itself; otherwise launch_rhs writes v into vbuf
 // (nch * N) and the solve reads it.

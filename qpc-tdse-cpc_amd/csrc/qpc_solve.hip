@@ -1843,90 +1843,66 @@ static SplitGrid split_grid(const Geom& geo, int nch, int pk, bool in_place) {
 
 template <class TF, int ROLE, int P>
 static void bsolve(hipStream_t s, const TF* tab, const TF* trf, TabMap tm, const cplx* zin, cplx* vbuf,
-                   cplx* zout, int nch, Geom geo, const RhsArgs* ra, int pk) {
+                   cplx* zout, int nch, Geom geo, const RhsArgs& ra, int pk) {
     const int PK = pk > 0 ? pk : (ROLE == RHS_SX_ASY ? kPKD : kPKS);
     if (PK > kPKMax) {
         // the carry would reach further than a work-group holds: sequential solve
-        if (ra) {
-            rhs_launch<P>(s, ROLE, *ra, tm, zin, vbuf, nch, geo);
-            zin = vbuf;
-        }
-        hipLaunchKernelGGL((k_seqsolve<TF, P>), dim3((nch + 63) / 64), dim3(64), 0, s, (const cplx*)tab, tm, zin, zout,
+        rhs_launch<P>(s, ROLE, ra, tm, zin, vbuf, nch, geo);
+        hipLaunchKernelGGL((k_seqsolve<TF, P>), dim3((nch + 63) / 64), dim3(64), 0, s, (const cplx*)tab, tm, vbuf, zout,
                            geo, nch);
         return;
     }
-    const SplitGrid g8 = split_grid(geo, nch, PK, ra && zin == zout);
+    const SplitGrid g8 = split_grid(geo, nch, PK, zin == zout);
     const int sn = g8.nseg ? g8.sn : seg_parts(geo, PK);
     const int nseg = g8.nseg ? g8.nseg : (geo.P + sn - 1) / sn;
     if (tm.order && nseg != tm.order_nseg) tm.order = nullptr;  // built for another launch shape
-    if (g8.nseg) {
-        // the right-hand side in the launch unless another work-group may still read
-        // rows of z that one writes
-        const dim3 grid8(nseg, nch), block((g8.parts + 7) / 8 * kLane);
-        if (ra) {
-            const uintptr_t a0 = (uintptr_t)zin, b0 = (uintptr_t)zout;
-            const uintptr_t len = sizeof(cplx) * (uintptr_t)nch * geo.N;
-            if (a0 + len <= b0 || b0 + len <= a0 || (nseg == 1 && a0 == b0)) {
-                hipLaunchKernelGGL((k_bsolve8<TF, ROLE, true, P>), grid8, block, 0, s, (const cplx*)tab, trf, tm, zin,
-                                   zout, geo, sn, g8.sx, PK, *ra);
-                return;
-            }
-            rhs_launch<P>(s, ROLE, *ra, tm, zin, vbuf, nch, geo);
-            zin = vbuf;
-        }
-        hipLaunchKernelGGL((k_bsolve8<TF, ROLE, false, P>), grid8, block, 0, s, (const cplx*)tab, trf, tm, zin, zout, geo,
-                           sn, g8.sx, PK, RhsArgs{});
-        return;
-    }
-    // staged grids form the right-hand side in the launch when z and x do not overlap
-    const bool staged = (int64_t)nseg * nch <= geo.stage_grid;
+    // z and x apart: another work-group never reads rows of z that one writes
+    const uintptr_t a0 = (uintptr_t)zin, b0 = (uintptr_t)zout, len = sizeof(cplx) * (uintptr_t)nch * geo.N;
+    const bool apart = a0 + len <= b0 || b0 + len <= a0;
     const dim3 grid(nseg, nch);
-    if (ra) {
-        // right-hand side formed in the solve (staged grids, disjoint z and x)
-        const uintptr_t a0 = (uintptr_t)zin, b0 = (uintptr_t)zout;
-        const uintptr_t len = sizeof(cplx) * (uintptr_t)nch * geo.N;
-        if (staged && (a0 + len <= b0 || b0 + len <= a0)) {
-            hipLaunchKernelGGL((k_bsolve<TF, ROLE, true, true, P>), grid, dim3(kLane * kWavesStaged), 0, s,
-                               (const cplx*)tab, trf, tm, zin, zout, geo, sn, PK, *ra);
+    if (g8.nseg) {
+        const dim3 block((g8.parts + 7) / 8 * kLane);
+        if (apart || (nseg == 1 && a0 == b0)) {
+            hipLaunchKernelGGL((k_bsolve8<TF, ROLE, true, P>), grid, block, 0, s, (const cplx*)tab, trf, tm, zin, zout,
+                               geo, sn, g8.sx, PK, ra);
             return;
         }
-        rhs_launch<P>(s, ROLE, *ra, tm, zin, vbuf, nch, geo);
-        zin = vbuf;
+        rhs_launch<P>(s, ROLE, ra, tm, zin, vbuf, nch, geo);
+        hipLaunchKernelGGL((k_bsolve8<TF, ROLE, false, P>), grid, block, 0, s, (const cplx*)tab, trf, tm, vbuf, zout,
+                           geo, sn, g8.sx, PK, RhsArgs{});
+        return;
     }
+    const bool staged = (int64_t)nseg * nch <= geo.stage_grid;
+    if (staged && apart) {
+        hipLaunchKernelGGL((k_bsolve<TF, ROLE, true, true, P>), grid, dim3(kLane * kWavesStaged), 0, s,
+                           (const cplx*)tab, trf, tm, zin, zout, geo, sn, PK, ra);
+        return;
+    }
+    rhs_launch<P>(s, ROLE, ra, tm, zin, vbuf, nch, geo);
     if (staged)
         hipLaunchKernelGGL((k_bsolve<TF, ROLE, true, false, P>), grid, dim3(kLane * kWavesStaged), 0, s,
-                           (const cplx*)tab, trf, tm, zin, zout, geo, sn, PK, RhsArgs{});
+                           (const cplx*)tab, trf, tm, vbuf, zout, geo, sn, PK, RhsArgs{});
     else
         hipLaunchKernelGGL((k_bsolve<TF, ROLE, false, false, P>), grid, dim3(kLane), 0, s, (const cplx*)tab, trf, tm,
-                           zin, zout, geo, sn, PK, RhsArgs{});
+                           vbuf, zout, geo, sn, PK, RhsArgs{});
 }
 
 template <class TF, int ROLE>
 static void bsolve_w(hipStream_t s, const TF* tab, const TF* trf, TabMap tm, const cplx* zin, cplx* vbuf, cplx* zout,
-                     int nch, Geom geo, const RhsArgs* ra, int pk) {
+                     int nch, Geom geo, const RhsArgs& ra, int pk) {
     if (geo.hw == 8) bsolve<TF, ROLE, 8>(s, tab, trf, tm, zin, vbuf, zout, nch, geo, ra, pk);
     else bsolve<TF, ROLE, 7>(s, tab, trf, tm, zin, vbuf, zout, nch, geo, ra, pk);
 }
 
-void launch_bsolve_c(hipStream_t s, int role, const cplx* tab, const cplx* trf, TabMap tm, const cplx* vin,
-                     cplx* zout, int nch, Geom geo, int pk) {
-    if (role == RHS_CBAND) bsolve_w<cplx, RHS_CBAND>(s, tab, trf, tm, vin, nullptr, zout, nch, geo, nullptr, pk);
-    else bsolve_w<cplx, RHS_SX_SYM>(s, tab, trf, tm, vin, nullptr, zout, nch, geo, nullptr, pk);
-}
-void launch_bsolve_r(hipStream_t s, int role, const double* tab, const double* trf, TabMap tm, const cplx* vin,
-                     cplx* zout, int nch, Geom geo, int pk) {
-    if (role == RHS_RBAND) bsolve_w<double, RHS_RBAND>(s, tab, trf, tm, vin, nullptr, zout, nch, geo, nullptr, pk);
-    else bsolve_w<double, RHS_SX_ASY>(s, tab, trf, tm, vin, nullptr, zout, nch, geo, nullptr, pk);
-}
 void launch_rsolve_c(hipStream_t s, int role, const RhsArgs& ra, const cplx* tab, const cplx* trf, TabMap tm,
                      const cplx* zin, cplx* vbuf, cplx* zout, int nch, Geom geo, int pk) {
-    if (role == RHS_CBAND) bsolve_w<cplx, RHS_CBAND>(s, tab, trf, tm, zin, vbuf, zout, nch, geo, &ra, pk);
-    else bsolve_w<cplx, RHS_SX_SYM>(s, tab, trf, tm, zin, vbuf, zout, nch, geo, &ra, pk);
+    if (role == RHS_CBAND) bsolve_w<cplx, RHS_CBAND>(s, tab, trf, tm, zin, vbuf, zout, nch, geo, ra, pk);
+    else bsolve_w<cplx, RHS_SX_SYM>(s, tab, trf, tm, zin, vbuf, zout, nch, geo, ra, pk);
 }
 void launch_rsolve_r(hipStream_t s, int role, const RhsArgs& ra, const double* tab, const double* trf, TabMap tm,
                      const cplx* zin, cplx* vbuf, cplx* zout, int nch, Geom geo, int pk) {
-    if (role == RHS_RBAND) bsolve_w<double, RHS_RBAND>(s, tab, trf, tm, zin, vbuf, zout, nch, geo, &ra, pk);
-    else bsolve_w<double, RHS_SX_ASY>(s, tab, trf, tm, zin, vbuf, zout, nch, geo, &ra, pk);
+    if (role == RHS_RBAND) bsolve_w<double, RHS_RBAND>(s, tab, trf, tm, zin, vbuf, zout, nch, geo, ra, pk);
+    else bsolve_w<double, RHS_SX_ASY>(s, tab, trf, tm, zin, vbuf, zout, nch, geo, ra, pk);
 }
 
 void launch_transfer_c(hipStream_t s, const cplx* tab, cplx* trf, int ntab, Geom geo) {
