@@ -160,6 +160,7 @@ struct qpc_ctx {
     double *d_e = nullptr, *d_ones = nullptr;
     std::vector<double> h_e;             // host copy of d_e
     bool have_outer = false;
+    // kU: kmax + 2 vectors, the Lanczos vectors and behind them the next one before its normalisation
     cplx *kU = nullptr, *kpart = nullptr, *kcoef = nullptr;
     double *ktab = nullptr, *ktrf = nullptr;  // chol(S) tables of the Lanczos vectors' solves
     double* kab = nullptr;         // tridiagonal a_i at 2 i, b_i at 2 i + 1 (host memory, written by the device)

@@ -1702,8 +1702,10 @@ int krylov_core(qpc_ctx* c, double az, double dt, int64_t kstart, int64_t kmax, 
     }
     TimedLaunch tl(c, QPC_K_KRYLOV);
     auto U = [&](int64_t i) { return c->kU + i * n; };
+    // scratch is vbuf and kU alone: the callers keep a state in spare
+    // (qpc_krylov_propagate's before the step)
     cplx* T = c->vbuf;   // H u_{k-1}
-    cplx* V = c->spare;  // S^-1 T, then the next vector before its normalisation
+    cplx* V = U(kmax);   // S^-1 T, then the next vector before its normalisation
     std::vector<double> a(kmax + 2, 0.0), b(kmax + 2, 0.0);
     std::vector<cplx> xs;
     const int N = (int)c->N, ML = (int)c->ML, p = (int)c->p;

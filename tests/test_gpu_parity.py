@@ -411,3 +411,47 @@ def test_step_by_step_loop_matches_oracle_run(gauge):
     err = rel_l2(prop.get_state(), c)
     print(f"  {gauge}: rel L2 = {err:.3e}", flush=True)
     assert err <= 1e-12
+
+
+@pytest.mark.parametrize("controlled", [False, True])
+def test_rejected_krylov_steps_start_again_from_the_state_before(controlled):
+    """kmax too small for dt_base: qpc_krylov_propagate rejects steps, restores
+    the state before each and halves them.  The accepted steps, recorded, are
+    replayed as CF4 Magnus steps of converged oracle exponentials.  Bar: 1e-10,
+    as without rejections (an accepted exponential leaves out at most 1e-12 of
+    the state, and there are a few tens)."""
+    import os
+    import qpc_gpu
+    import pyoracle as po
+    cfg = shape(400, 8, 80.0)
+    print(f"case: rejected Krylov steps N=400 L=8, controlled {controlled}", flush=True)
+    o = make_oracle(cfg)
+    prop = _gpu_prop(o, cfg)
+    prop.upload_krylov(o.get(po.QOR_H), o.get(po.QOR_Y10), o.get(po.QOR_Q10))
+    net = None
+    if controlled:
+        st = qpc_gpu.Setup(400, 7, 8, 1, 0, 0.05, 0.0, 80.0, 1.0, 1.0, 60.0, 80.0, 0.125)
+        prop.upload_outer(st.get(qpc_gpu.SETUP_SOUTER))
+        net = qpc_gpu.Mlp(seed=1)
+        net.params = np.load(os.path.join(os.path.dirname(qpc_gpu.__file__), "krylov_controller_params.npy"))
+    pulse = (cfg["e0"], cfg["w0"], cfg["nc"], 0.0, 0.0)
+    c = mixed_state(o, seed=47, amp=0.1)
+    prop.set_state(c)
+    t0, T = 150.0, 0.2
+    stats, rec = prop.krylov_propagate(pulse, t0, t0 + T, 0.04, 1e-24, kmin=8, kmax=30, net=net, record=256,
+                                       record_ab=False)
+    hs = rec["h"]
+    print(f"  stats {stats}; h in [{hs.min():.4g}, {hs.max():.4g}]", flush=True)
+    assert stats["rejected"] > 0 and len(hs) == stats["steps"] and abs(hs.sum() - T) < 1e-12
+    r3 = np.sqrt(3.0)
+    a1, a2 = (3 - 2 * r3) / 12, (3 + 2 * r3) / 12
+    A = lambda t: po.sinen2(*pulse, t)
+    t = t0
+    for h in hs:
+        A1, A2 = A(t + (0.5 - r3 / 6) * h), A(t + (0.5 + r3 / 6) * h)
+        for a in (2 * (a2 * A1 + a1 * A2), 2 * (a1 * A1 + a2 * A2)):
+            o.krylov_step(c, a, h / 2, kmax=64)
+        t += h
+    err = rel_l2(prop.get_state(), c)
+    print(f"  rel L2 = {err:.3e}", flush=True)
+    assert err <= 1e-10
