@@ -1348,7 +1348,7 @@ __global__ __launch_bounds__(256) void k_band_diag(const T* __restrict__ src, T*
 // ---------------------------------------------------------------------------
 // LU of A = S + ifet X in the reference's elimination order
 // (propagate.hpp:33-86), one lane per (time point, channel, partition).  A
-// lane restarts the elimination `restart` rows above its partition (as if the
+// lane restarts the elimination `above` rows above its partition (as if the
 // matrix began there) and writes the table rows of its own partition.
 //
 // The elimination is right-looking: the lane keeps the window of the Schur
@@ -1365,6 +1365,16 @@ __global__ __launch_bounds__(256) void k_band_diag(const T* __restrict__ src, T*
 // k_factor_row.  A batch is bound by the products and the table
 // writes: 32 time points of N = 3000, 41 tables of S + i e X 167 us (was
 // 434), 81 of S + e X 307 us (was 596).
+//
+// Both kernels start the same number of rows above a partition, whole rounds of
+// either (8 rows; 12 and 8 for p = 8), so that a table's bits do not depend on
+// how many are built together.
+constexpr int restart_round(int p) { return p == 7 ? 8 : 24; }
+static int restart_rows(int p, int restart) {
+    const int r = restart_round(p);
+    return ((restart > 0 ? restart : kRestart) + r - 1) / r * r;
+}
+
 template <int SYM>
 struct FactorTypes;
 template <>
@@ -1402,12 +1412,12 @@ struct FactorScal {
 
 template <int SYM, int P>
 __global__ __launch_bounds__(kLane, P == 7 ? 2 : 1) void k_factor(const cplx* __restrict__ fx, FactorScal sc0, Geom geo,
-                                                  int restart, cplx* __restrict__ tab, int64_t tstride) {
+                                                  int above, cplx* __restrict__ tab, int64_t tstride) {
     using T = typename FactorTypes<SYM>::T;
     constexpr int NE = P + 1;
     // slots: a divisor of kPM, so that the rounds of rows end with the partition
     constexpr int RS = P == 7 ? 8 : 12;
-    static_assert(RS > P && kPM % RS == 0, "slot count");
+    static_assert(RS > P && kPM % RS == 0 && restart_round(P) % RS == 0, "slot count");
     const int g = blockIdx.x * kLane + threadIdx.x;
     const int ch = blockIdx.y, t = blockIdx.z;
     if (g >= geo.P) return;
@@ -1419,8 +1429,7 @@ __global__ __launch_bounds__(kLane, P == 7 ? 2 : 1) void k_factor(const cplx* __
     constexpr int ROW = TabFmt<T, P>::row;
     cplx* Tg = tab + ((int64_t)t * tstride + ch) * TabFmt<T, P>::units(geo) + part_col<T, P>(g);
     const int r0 = g * kPM;
-    // whole rounds of RS rows above the partition (r0 is a multiple of RS too)
-    const int above = (restart + RS - 1) / RS * RS;
+    // (whole rounds of RS rows; r0 is a multiple of RS too)
     const int start = r0 > above ? r0 - above : 0;
     // column entries of the band from column `start` on
     int sc = start % kPM, gc = start / kPM;
@@ -1687,9 +1696,8 @@ __global__ __launch_bounds__(kLane) void k_factor_jobs(FactorJobs a, Geom geo) {
     const int t = blockIdx.z, g0 = blockIdx.x * kFactorQ;
     const double e = J.eig[ch] * (t ? J.ifdt[1] : J.ifdt[0]);
     const int64_t q = (int64_t)t * J.tstride + ch;
-    const int above = (J.restart + 7) / 8 * 8;
-    if (J.real) factor_row<1, P>(J.fx, e, geo, g0, above, (cplx*)J.tab + q * TabFmt<double, P>::units(geo));
-    else factor_row<0, P>(J.fx, e, geo, g0, above, (cplx*)J.tab + q * TabFmt<cplx, P>::units(geo));
+    if (J.real) factor_row<1, P>(J.fx, e, geo, g0, J.restart, (cplx*)J.tab + q * TabFmt<double, P>::units(geo));
+    else factor_row<0, P>(J.fx, e, geo, g0, J.restart, (cplx*)J.tab + q * TabFmt<cplx, P>::units(geo));
 }
 template <int P>
 __global__ __launch_bounds__(kLane) void k_transfer_jobs(FactorJobs a, Geom geo) {
@@ -1951,8 +1959,7 @@ void launch_factor_bands(hipStream_t s, const double* S, const double* X, cplx* 
     hipLaunchKernelGGL(k_factor_bands, dim3((total + 255) / 256), dim3(256), 0, s, S, X, fx, geo.N, geo.hw + 1,
                        factor_cols(geo));
 }
-// restart rows and waves within k_factor_row's range
-static int row_above(int restart) { return ((restart > 0 ? restart : kRestart) + 7) / 8 * 8; }
+// waves and restart rows within k_factor_row's range
 static int row_groups(const Geom& geo) { return (geo.P + kFactorQ - 1) / kFactorQ; }
 static bool row_fits(const Geom& geo, int64_t tables, int above) {
     return row_groups(geo) * tables <= kFactorRowWaves && above <= kFactorRowAbove;
@@ -1963,13 +1970,13 @@ static size_t row_lds(int above) { return sizeof(double) * 2 * factor_row_blocks
 template <int SYM, int P>
 static void factor_launch_p(hipStream_t s, const cplx* fx, const FactorScal& sc, int nt, int nch, Geom geo, cplx* tab,
                             int restart, int64_t ts) {
-    const int above = row_above(restart);
+    const int above = restart_rows(P, restart);
     if (row_fits(geo, (int64_t)nch * nt, above))
         hipLaunchKernelGGL((k_factor_row<SYM, P>), dim3(row_groups(geo), nch, nt), dim3(kLane), row_lds<P>(above), s, fx,
                            sc, geo, above, tab, ts);
     else
-        hipLaunchKernelGGL((k_factor<SYM, P>), dim3(geo.NG, nch, nt), dim3(kLane), 0, s, fx, sc, geo,
-                           restart > 0 ? restart : kRestart, tab, ts);
+        hipLaunchKernelGGL((k_factor<SYM, P>), dim3(geo.NG, nch, nt), dim3(kLane), 0, s, fx, sc, geo, above,
+                           tab, ts);
 }
 template <int SYM>
 static void factor_launch(hipStream_t s, const cplx* fx, const FactorScal& sc, int nt, int nch, Geom geo, cplx* tab,
@@ -1993,8 +2000,8 @@ static void factor_jobs(hipStream_t s, const FactorJobs& a, int nt, const Geom& 
     bool fit = true;  // each by itself: together they take no longer than one after the other
     for (int k = 0; k < a.n; ++k) {
         rows += a.j[k].nch;
-        above = std::max(above, row_above(a.j[k].restart));
-        fit = fit && row_fits(geo, (int64_t)a.j[k].nch * nt, row_above(a.j[k].restart));
+        above = std::max(above, a.j[k].restart);
+        fit = fit && row_fits(geo, (int64_t)a.j[k].nch * nt, a.j[k].restart);
     }
     if (fit) {
         hipLaunchKernelGGL(k_factor_jobs<P>, dim3(row_groups(geo), rows, nt), dim3(kLane), row_lds<P>(above), s, a, geo);
@@ -2021,7 +2028,7 @@ void launch_factor_jobs(hipStream_t s, const FactorJob* jobs, int n, int nt, Geo
     for (int k = 0; k < n && a.n < kFactorJobs; ++k)
         if (jobs[k].nch > 0) {
             a.j[a.n] = jobs[k];
-            if (a.j[a.n].restart <= 0) a.j[a.n].restart = kRestart;
+            a.j[a.n].restart = restart_rows(geo.hw, jobs[k].restart);
             ++a.n;
         }
     if (a.n == 0) return;

@@ -241,3 +241,28 @@ def test_steps_whichever_solve_kernel_runs(N, p):
     assert err <= 1e-12
     assert all(np.array_equal(x, out[0]) for x in out[1:])
     prop.close()
+
+
+@pytest.mark.parametrize("p", [7, 8])
+def test_tables_have_the_same_bits_however_many_are_factorised(p):
+    """A run factorises its time points' tables together (17 time points of 20
+    and 40 tables), a step one time point's, by different kernels.  With a
+    recorded observable the run hands the whole state over between steps as the
+    single calls do, so that equal tables give equal states in every bit."""
+    import qpc_gpu
+    N, L, nt = 600, 40, 16
+    print(f"case: bits of batched and single tables N={N} L={L} p={p}", flush=True)
+    o, prop = _pair(N, p, L)
+    a = 0.8 * np.sin(0.3 * np.arange(nt + 1)) + 0.1
+    c = mixed_state(o, seed=p, amp=0.3)
+    prop.set_state(c)
+    prop.record(qpc_gpu.REC_NORM, nt)
+    prop.run(a, nt, 0, nt, use_mask=False)
+    ref = prop.get_state().copy()
+    prop.set_state(c)
+    for k in range(nt):
+        prop.propagate(a[k], a[k + 1])
+    got = prop.get_state()
+    print(f"  rel L2 {rel_l2(got, ref):.2e}", flush=True)
+    assert np.array_equal(got, ref)
+    prop.close()
