@@ -1357,6 +1357,7 @@ int step_impl(qpc_ctx* c, int gauge, double a_i, double a_f) {
         // and 1 once every step that read the set is done
         const double a[3] = {a_i, a_f, a_f};
         TRY(set_run_scalars(c, a, 3));
+        for (int& e : c->slot_read) e = -1;  // nothing reads a position any more
         TRY(factor_batch(c, 0, 0, 2));
     }
     // a fresh pair waits for both time points' tables; with the t_i tables
