@@ -1356,6 +1356,7 @@ int step_impl(qpc_ctx* c, int gauge, double a_i, double a_f) {
         // the streams are idle after set_run_scalars), tables at positions 0
         // and 1 once every step that read the set is done
         const double a[3] = {a_i, a_f, a_f};
+        c->step_slot = -1;  // (the scalars are overwritten even where the values are refused)
         TRY(set_run_scalars(c, a, 3));
         for (int& e : c->slot_read) e = -1;  // nothing reads a position any more
         TRY(factor_batch(c, 0, 0, 2));

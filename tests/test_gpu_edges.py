@@ -266,3 +266,28 @@ def test_tables_have_the_same_bits_however_many_are_factorised(p):
     print(f"  rel L2 {rel_l2(got, ref):.2e}", flush=True)
     assert np.array_equal(got, ref)
     prop.close()
+
+
+@pytest.mark.parametrize("gauge", ["vg", "lg"])
+def test_refused_step_leaves_the_next_one_right(gauge):
+    """A step with a non-finite field value is refused; the loop goes on from
+    the step before it, whose last time point's tables and scalars are kept."""
+    import qpc_gpu
+    N, L = 240, 4
+    print(f"case: refused step {gauge}", flush=True)
+    o, prop = _pair(N, 7, L)
+    step, ref_step = (prop.propagate, o.step) if gauge == "vg" else (prop.propagate_lg, o.step_lg)
+    f = 0.9 if gauge == "vg" else 0.05
+    c = mixed_state(o, seed=5, amp=0.3)
+    prop.set_state(c)
+    step(f, 0.8 * f)
+    for bad in ((0.5 * f, np.nan), (np.inf, 0.5 * f), (0.8 * f, np.nan)):
+        with pytest.raises(qpc_gpu.QpcError):
+            step(*bad)
+    step(0.8 * f, 0.6 * f)
+    for a in ((f, 0.8 * f), (0.8 * f, 0.6 * f)):
+        ref_step(c, *a)
+    err = rel_l2(prop.get_state(), c)
+    print(f"  rel L2 {err:.2e}", flush=True)
+    assert err <= 1e-12
+    prop.close()
