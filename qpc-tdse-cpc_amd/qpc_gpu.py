@@ -868,7 +868,7 @@ class ShotBuckets:
         for p, g, Lb in zip(self.props, self.groups, self.Lb):
             blk = p.get_state()
             for q, k in enumerate(g):
-                out[k] = blk[q * Lb * self.N:q * Lb * self.N + self.ldim[k] * self.N]  # (blk is nobody else's)
+                out[k] = blk[q * Lb * self.N:q * Lb * self.N + self.ldim[k] * self.N].copy()
         return out
 
     def run_batch(self, atab, nt_field, it0, it1, use_mask=True, sync=True):
