@@ -470,7 +470,7 @@ int ep_sweep(qpc_ctx* c, int set, int64_t k, int op, int tf, cplx* buf) {
                                 : qpc::TabMap{0, (int)c->L, (int)c->m0};
     // the work-groups of a row's segments and of a shared table's rows on one XCD
     const int pk = E.lg ? c->pk_l : ep_is_d(op) ? c->pk_d : qpc::kPKS;
-    const int nseg = qpc::solve_segments(c->geo, pk);
+    const int nseg = qpc::solve_segments(c->geo, (int)np, pk, true);
     if (nseg > 0 && nseg != E.ord_nseg[op] && (int64_t)E.rtab_h[op].size() == np) {
         E.ord_h[op].assign((size_t)np * nseg, 0);
         qpc::solve_order(E.rtab_h[op].data(), (int)np, nseg, E.ord_h[op].data());

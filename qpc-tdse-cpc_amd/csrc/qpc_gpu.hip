@@ -36,7 +36,7 @@ inline int64_t trfsz_c(const qpc_ctx* c) { return c->ML * c->geo.ctrf_elems; }
 // tab(ch) (qpc::solve_order), rebuilt when the segments per channel change
 template <class TabOf>
 int wg_order(qpc_ctx* c, qpc_ctx::WgOrder& o, int pk, TabOf tab_of, qpc::TabMap& tm) {
-    const int nseg = qpc::solve_segments(c->geo, pk);
+    const int nseg = qpc::solve_segments(c->geo, (int)c->ML, pk, false);
     if (nseg == 0) return QPC_OK;  // sequential solve
     if (nseg != o.nseg) {
         std::vector<int> tab((size_t)c->ML);
@@ -78,7 +78,7 @@ int solve_R(qpc_ctx* c, int ts, int64_t t0, int64_t t, const cplx* in, cplx* out
                                     : qpc::TabMap{0, (int)c->L, (int)c->m0};
     if (c->n_rprim > 0) {
         // the channels of a shared table on one XCD, so that its rows are read once per L2
-        const int nseg = qpc::solve_segments(c->geo, qpc::kPKS);
+        const int nseg = qpc::solve_segments(c->geo, (int)c->ML, qpc::kPKS, false);
         if (nseg != c->rorder_nseg) {
             const size_t n = (size_t)c->ML * nseg;
             c->rorder_h.assign(n, 0);

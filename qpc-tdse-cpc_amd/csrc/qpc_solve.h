@@ -147,11 +147,11 @@ struct TabMap {
 };
 constexpr int kMapConj = 1 << 30, kMapIdx = kMapConj - 1;
 constexpr int kXcds = 8;
-// segments per channel of the partitioned solve for this launch shape and
-// carry depth (bsolve's choice with one lane per partition; 0 when the carry is too deep for it and the
-// solve runs sequentially), and the XCD-grouping order of its
+// segments per channel of the partitioned solve of nch channels at this carry
+// depth (0 when the carry is too deep for it and the solve runs sequentially),
+// with z and x the same (in_place) or apart, and the XCD-grouping order of its
 // work-groups for channels whose tables are tab[ch] (nch channels)
-int solve_segments(const Geom& geo, int pk);
+int solve_segments(const Geom& geo, int nch, int pk, bool in_place);
 void solve_order(const int* tab, int nch, int nseg, int* order);
 
 // v = B z for nch channels (vout: nch * N)

@@ -1772,12 +1772,6 @@ static int seg_parts(const Geom& geo, int pk) {
     return (geo.P + nseg - 1) / nseg;
 }
 
-int solve_segments(const Geom& geo, int pk) {
-    if (pk > kPKMax) return 0;  // the sequential solve: no segments
-    const int sn = seg_parts(geo, pk);
-    return (geo.P + sn - 1) / sn;
-}
-
 void solve_order(const int* tab, int nch, int nseg, int* order) {
     // (table, segment, channel) ascending, dealt to the XCDs in contiguous
     // chunks; XCD x's k-th work-group has linear id x + kXcds k
@@ -1847,6 +1841,14 @@ static SplitGrid split_grid(const Geom& geo, int nch, int pk, bool in_place) {
         best.parts = std::min(geo.P, best.nseg > 1 ? best.sn + 2 * pk : best.sn);
     }
     return best;
+}
+
+int solve_segments(const Geom& geo, int nch, int pk, bool in_place) {
+    if (pk > kPKMax) return 0;  // the sequential solve: no segments
+    const SplitGrid g8 = split_grid(geo, nch, pk, in_place);
+    if (g8.nseg) return g8.nseg;
+    const int sn = seg_parts(geo, pk);
+    return (geo.P + sn - 1) / sn;
 }
 
 template <class TF, int ROLE, int P>
