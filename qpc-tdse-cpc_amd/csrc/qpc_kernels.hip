@@ -294,9 +294,10 @@ struct ObsCouple {
         return t;
     }
 };
-// row i of a band: the diagonal and the entries to its right
+// row i of a band: the diagonal and the entries to its right, zero past the
+// matrix whatever the array holds there
 template <int NE>
-__device__ inline void obs_band(double (&b)[NE], const double* __restrict__ B, int i) {
+__device__ inline void obs_band(double (&b)[NE], const double* __restrict__ B, int i, int N) {
     if constexpr (NE % 2 == 0) {  // (a row's address is a multiple of 16 bytes)
         const double2* q = (const double2*)(B + (int64_t)i * NE);
 #pragma unroll
@@ -309,6 +310,9 @@ __device__ inline void obs_band(double (&b)[NE], const double* __restrict__ B, i
 #pragma unroll
         for (int k = 0; k < NE; ++k) b[k] = B[(int64_t)i * NE + k];
     }
+#pragma unroll
+    for (int k = 1; k < NE; ++k)
+        if (i + k >= N) b[k] = 0.0;
 }
 // sums of K values over the waves of the block; thread q < K returns value q
 template <int K>
@@ -364,10 +368,10 @@ __global__ __launch_bounds__(kObsThreads) void k_observe(ObsBands b, int flags, 
         const int i = r0 + tid, ic = min(i, N - 1);
         // bands of the two kinds: {S, W} with x itself, {R, A} with the partners
         double bs[NE], bw[NE], br[NE], ba[NE];
-        if (!XY && (flags & 1)) obs_band<NE>(bs, b.S, ic);
-        if (!XY && (flags & 8)) obs_band<NE>(bw, b.W, ic);
-        if (flags & (XY ? 16 : 2)) obs_band<NE>(br, b.R, ic);
-        if (flags & (XY ? 32 : 4)) obs_band<NE>(ba, b.A, ic);
+        if (!XY && (flags & 1)) obs_band<NE>(bs, b.S, ic, N);
+        if (!XY && (flags & 8)) obs_band<NE>(bw, b.W, ic, N);
+        if (flags & (XY ? 16 : 2)) obs_band<NE>(br, b.R, ic, N);
+        if (flags & (XY ? 32 : 4)) obs_band<NE>(ba, b.A, ic, N);
         for (int e = tid; e < kObsThreads + NE; e += kObsThreads) {
             const int r = r0 + e;
             sx[e] = r < N ? x[r] : cplx{0.0, 0.0};
