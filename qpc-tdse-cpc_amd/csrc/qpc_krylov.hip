@@ -57,6 +57,7 @@ __global__ __launch_bounds__(kTile) void k_hmul(const double* __restrict__ Hd, c
         hu[k] = H[(int64_t)k * N + ic];
         fu[k] = Fd[(int64_t)k * N + ic];
         gu[k] = Gd[(int64_t)k * N + ic];
+        if (ic + k >= N) hu[k] = fu[k] = gu[k] = 0.0;  // past the matrix, whatever the caller's arrays hold there
     }
 #pragma unroll
     for (int j = 1; j <= P; ++j) {

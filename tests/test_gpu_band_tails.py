@@ -1,6 +1,6 @@
 """The last rows of a band array have entries past the matrix (row i, diagonal
-j with i + j >= N).  Whatever a caller's arrays hold there, the observables are
-those of the matrix: the same bits as with zeros."""
+j with i + j >= N).  Whatever a caller's arrays hold there, the observables and
+the Lanczos vectors are those of the matrix: the same bits as with zeros."""
 import numpy as np
 import pytest
 
@@ -40,4 +40,24 @@ def test_observables_do_not_see_entries_past_the_matrix(N, p):
         out.append(prop.record_read()[0].copy())
         prop.close()
     print(f"  {out[0]}\n  {out[1]}", flush=True)
+    assert np.all(np.isfinite(out[0])) and np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("c", [dict(N=250, p=7, L=5, M=1, m0=0, kmax=64), dict(N=400, p=8, L=3, M=3, m0=-1, kmax=64)],
+                         ids=lambda c: "N{N}_p{p}".format(**c))
+def test_lanczos_vectors_do_not_see_entries_past_the_matrix(c):
+    import qpc_gpu
+    from test_gpu_krylov_order import operators
+    N, p = c["N"], c["p"]
+    print(f"case: band tails, Krylov N={N} p={p}", flush=True)
+    S, ch, F, G, H, y10, q10, z = operators(c)
+    out = []
+    for value in (0.0, np.nan):
+        prop = qpc_gpu.Propagator(N, p, c["L"], c["M"], c["m0"], 0.05)
+        prop.upload_radial(*[with_tail(b, N, p, value) for b in (S, ch, F, G, F, S)])
+        prop.upload_krylov(with_tail(H, N, p, value), y10, q10)
+        prop.set_state(z)
+        m, _, ab = prop.krylov_step_adaptive(0.75, 0.03125, c["kmax"], c["kmax"], 0.0)
+        out.append(np.concatenate([ab.ravel(), prop.get_state().view(np.float64).ravel()]))
+        prop.close()
     assert np.all(np.isfinite(out[0])) and np.array_equal(out[0], out[1])
