@@ -1800,7 +1800,8 @@ void solve_order(const int* tab, int nch, int nseg, int* order) {
 // kSplitGrid result (the outer segments have a halo on one side only and own
 // that many more partitions).  One step, N = 1000, k_bsolve against eight lanes:
 // 100 channels (200 work-groups) 184 / 152 us, 128 (256) 194 / 166, 140 (280)
-// 200 / 214; N = 1500: 80 channels (240) 183 / 149, 86 (258) 186 / 195.
+// 200 / 214; N = 1500: 80 channels (240) 183 / 149, 86 (258) 186 / 195 (with the
+// work-groups of one table on one XCD the cut ones take 150, 160 and 146).
 //
 // Within these work-groups, the fewest segments that leave each the fewest
 // waves (short channels too, unless the solve is in place, where one segment
@@ -1843,6 +1844,11 @@ static SplitGrid split_grid(const Geom& geo, int nch, int pk, bool in_place) {
     return best;
 }
 
+// (The count is the launch's own, cut or not, so that an order built for it is
+// used: a cut launch is bound by its loads, and without the order the channels
+// of one table lie on different XCDs.  31 channels of N = 1000, HBM reads per R /
+// D / free launch 6.1 / 6.5 / 17.3 -> 2.6 / 3.7 / 5.5 MB, a step of a run 106.8 ->
+// 105.1 us; 41 of N = 1500 120.5 -> 117.4, 128 of N = 1000 165.7 -> 160.5.)
 int solve_segments(const Geom& geo, int nch, int pk, bool in_place) {
     if (pk > kPKMax) return 0;  // the sequential solve: no segments
     const SplitGrid g8 = split_grid(geo, nch, pk, in_place);
