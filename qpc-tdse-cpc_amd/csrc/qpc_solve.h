@@ -11,7 +11,7 @@
 //   forward   y_i = rdf_i * (v_i - sum_{j=1..p} F_j(i-j) y_{i-j})
 //   backward  x_i = rdb_i * y_i   - sum_{k=1..p} G_k(i) x_{i+k}
 // F_k(i) is the entry of column i of L in row i + k: a row done, its multiples
-// go to the p rows below.
+// go to the p rows below, which gather them and add v_i last (for its rounding).
 //
 // Complex symmetric tables (R-part sweeps S + i e X with X symmetric, and the
 // field-free S + i dt/2 H_l), A = L D L^T with L unit lower, p+1 coefficients

@@ -207,21 +207,28 @@ struct SBandRow {
 
 // ---------------------------------------------------------------------------
 // One table row of one partition and direction in registers (UF units).
-// Forward (acc[k]: the right-hand side of row s + k less what the rows above
-// contribute): the row's value leaves the window, its multiples go to the P
-// rows below, and row s + P enters with its right-hand side vn.  The state a
-// partition hands on is what its rows contribute to the first P rows of the
-// next, whose own right-hand sides enter as zero.
+// Forward (acc[k]: what the rows above contribute to row s + k): the row's value
+// is its right-hand side v with what it has gathered, its multiples go to the P
+// rows below, and row s + P enters with nothing.  The state a partition hands on
+// is what its rows contribute to the first P rows of the next.
+//
+// The right-hand side comes last for the sake of its rounding: the farthest
+// rows' products are the first to be added, and a sum that began with v would
+// round each of them at v's size.  Errors of a free / mask solve of N = 240 (p =
+// 7) against 80-bit arithmetic: 1.24e-14 / 2.52e-14; with v first 1.42e-14 /
+// 3.32e-14; with v first and the nearest row's product next 1.23e-14 / 2.49e-14,
+// but then every product waits for the row above.  Launches take the same time
+// to 0.5%.
 template <class TF, int P>
-__device__ inline cplx fwd_row(const cplx (&c)[TabFmt<TF, P>::UF], cplx vn, cplx (&acc)[P]) {
+__device__ inline cplx fwd_row(const cplx (&c)[TabFmt<TF, P>::UF], cplx v, cplx (&acc)[P]) {
     using F = TabFmt<TF, P>;
-    const cplx z = acc[0];
+    const cplx z = {v.re + acc[0].re, v.im + acc[0].im};
     cplx y;  // what the lower rows' updates take, and the stored row
     if constexpr (F::SYM) y = z;
     else y = {F::diag(c) * z.re, F::diag(c) * z.im};
 #pragma unroll
     for (int k = 1; k < P; ++k) acc[k - 1] = tmsub(acc[k], F::coef(c, k), y);
-    acc[P - 1] = tmsub(vn, F::coef(c, P), y);
+    acc[P - 1] = tmsub(cplx{0.0, 0.0}, F::coef(c, P), y);
     if constexpr (F::SYM) return tmulf(F::diag(c), z);
     else return y;
 }
@@ -286,20 +293,16 @@ constexpr int kRowSlots = kLane * kRowStride + 2 * kRowPad;
 __device__ inline int row_slot(int s, int ln) { return kRowPad + ln * kRowStride + s; }
 
 // the rows of one block, written to wb[r]; the block's registers are refilled
-// from LDS (l: this lane's units) or the table (p).  Forward, row r of the
-// block takes in the right-hand side v[r] of the row P below; nv: the four rows
-// from 12 below the block's first (with P = 7 one row of them waits in v[RB]).
+// from LDS (l: this lane's units) or the table (p), v[r] from the next block's
+// rows at nv
 template <class TF, int P, bool L>
-__device__ inline void fwd_block(BlockRegs<TF, P>& c, cplx (&v)[Blocks<TF, P>::RB + 1], const lcplx* nv, lcplx* wb,
+__device__ inline void fwd_block(BlockRegs<TF, P>& c, cplx (&v)[Blocks<TF, P>::RB], const lcplx* nv, lcplx* wb,
                                  const lcplx* l, const cplx* p, unsigned off, cplx (&acc)[P]) {
     using B = Blocks<TF, P>;
-    static_assert(P == B::RB + 3 || P == B::RB + 4, "the rows that nv holds");
 #pragma unroll
     for (int r = 0; r < B::RB; ++r) {
         const cplx y = fwd_row<TF, P>(c[r], v[r], acc);
-        if constexpr (P == 8) v[r] = nv[r];
-        else v[r] = r ? (cplx)nv[r > 0 ? r - 1 : 0] : v[B::RB];
-        if (P == 7 && r == B::RB - 1) v[B::RB] = nv[B::RB - 1];
+        v[r] = nv[r];
         wb[r] = lc(y);
 #pragma unroll
         for (int u = 0; u < B::UF; ++u)
@@ -327,25 +330,19 @@ __device__ inline void bwd_block(BlockRegs<TF, P>& c, cplx (&v)[Blocks<TF, P>::R
 // One pass over the rows of slot ln (rows: its first row; T: the direction's
 // units of the table, uniform).  c holds the first block at entry and the
 // block at `after` at the end.  Rows are written to `out` (their own place, or
-// a scrap block of RB rows when ostep is 0).  zeros: RB zero rows, for those
-// past the partition.
+// a scrap block of RB rows when ostep is 0).
 template <class TF, int P, bool STAGED>
 __device__ inline void fwd_pass(BlockRegs<TF, P>& c, const cplx* T, unsigned off, const lcplx* sL,
-                                const lcplx* rows, lcplx* out, int ostep, cplx (&acc)[P], const cplx* after,
-                                const lcplx* zeros) {
+                                const lcplx* rows, lcplx* out, int ostep, cplx (&acc)[P], const cplx* after) {
     using B = Blocks<TF, P>;
-    cplx v[B::RB + 1];
+    cplx v[B::RB];
 #pragma unroll
-    for (int r = 0; r < P; ++r) acc[r] += (cplx)rows[r];
-#pragma unroll
-    for (int r = 0; r < B::RB + (P == 7); ++r) v[r] = rows[P + r];
-    constexpr int AHEAD = 3;  // blocks from the one in hand to the rows read while it runs
-    int left = B::NB - AHEAD;
+    for (int r = 0; r < B::RB; ++r) v[r] = rows[r];
     if constexpr (STAGED) {
 #pragma unroll 1
         for (int i = 0; i < B::LB1 - B::LB0; ++i) {
-            fwd_block<TF, P, true>(c, v, left-- > 0 ? rows + AHEAD * B::RB : zeros, out, sL, nullptr, 0, acc);
             rows += B::RB;
+            fwd_block<TF, P, true>(c, v, rows, out, sL, nullptr, 0, acc);
             out += ostep;
             sL += B::RB * B::UF * kLane;
         }
@@ -354,9 +351,8 @@ __device__ inline void fwd_pass(BlockRegs<TF, P>& c, const cplx* T, unsigned off
     T += (int64_t)G0 * B::RB * B::UT * kLane;
 #pragma unroll 1
     for (int i = 0; i < GN; ++i) {
-        fwd_block<TF, P, false>(c, v, left-- > 0 ? rows + AHEAD * B::RB : zeros, out, nullptr, i == GN - 1 ? after : T,
-                                off, acc);
         rows += B::RB;
+        fwd_block<TF, P, false>(c, v, rows, out, nullptr, i == GN - 1 ? after : T, off, acc);
         out += ostep;
         T += B::RB * B::UT * kLane;
     }
@@ -574,7 +570,7 @@ struct StageLds {
     static constexpr int scrap = 2 * P * kSt;
     static constexpr int sz = NZ > scrap + kLane * Blocks<TF, P>::RB ? NZ : scrap + kLane * Blocks<TF, P>::RB;
     static constexpr int bytes =
-        16 * (sz + kRowSlots + P * kSt + Blocks<TF, P>::LR * Blocks<TF, P>::UT * kLane + Blocks<TF, P>::RB);
+        16 * (sz + kRowSlots + P * kSt + Blocks<TF, P>::LR * Blocks<TF, P>::UT * kLane);
     static_assert(bytes <= 160 * 1024, "LDS budget");
 };
 
@@ -592,7 +588,6 @@ __global__ __launch_bounds__(kLane * (STAGED ? kWavesStaged : 1)) void k_bsolve(
     // z rows [r0 - P, r0 + NZ - P) (FUSE; zero outside [0, N)); then carry states and scrap rows
     __shared__ lcplx sz[STAGED ? S::sz : kLane * B::RB];
     __shared__ lcplx sT[STAGED ? B::LR * B::UT * kLane : 1];    // staged table rows
-    __shared__ lcplx s0[B::RB];                                 // zero rows
 
     int ch = blockIdx.y, seg = blockIdx.x;
     if (tm.order) {
@@ -625,7 +620,6 @@ __global__ __launch_bounds__(kLane * (STAGED ? kWavesStaged : 1)) void k_bsolve(
     if (w == 0) {
         BlockRegs<TF, P> c;
         cplx h[P];
-        if (ln < B::RB) s0[ln] = lcplx{0.0, 0.0};
         const lcplx* sL = sT + ln;
         lcplx* scrap = sz + (STAGED ? S::scrap : 0) + ln * B::RB;
         if constexpr (STAGED) {
@@ -668,7 +662,7 @@ __global__ __launch_bounds__(kLane * (STAGED ? kWavesStaged : 1)) void k_bsolve(
         // forward: pass A from the zero state, carry, pass B
 #pragma unroll 1
         for (int pass = 0;; ++pass) {
-            fwd_pass<TF, P, STAGED>(c, T, off, sL, rows, pass ? rows : scrap, pass ? B::RB : 0, h, pass ? Tb0 : T, s0);
+            fwd_pass<TF, P, STAGED>(c, T, off, sL, rows, pass ? rows : scrap, pass ? B::RB : 0, h, pass ? Tb0 : T);
             if (pass) break;
             if constexpr (STAGED) {
 #pragma unroll
@@ -797,10 +791,10 @@ __global__ __launch_bounds__(kLane * (STAGED ? kWavesStaged : 1)) void k_bsolve(
 // k_bsolve's waves would leave lanes or compute units idle.  Lane l owns rows l,
 // l + 8 and l + 16 of its partition.  Going down, the row's value is broadcast
 // to the eight (two DPP moves per double) and each lane subtracts its multiple
-// from the row it gathers next, which it began with the row's right-hand side:
-// P products per row in one instruction each, and the chain of a row is a
-// broadcast and two FMAs.  Going up is the same from the last row, with the
-// rows' own coefficients.  The state a partition hands down is what the eight
+// from the row it gathers next: P products per row in one instruction each, and
+// the chain of a row is the sum with its right-hand side, a broadcast and two
+// FMAs.  Going up is the same from the last row, which begin with their values,
+// with the rows' own coefficients.  The state a partition hands down is what the eight
 // lanes have gathered for the first rows of the next one.  A lane's 24
 // coefficients per direction stay in registers for both passes, its rows too:
 // LDS holds the rows of z for the right-hand side, P rows on either side, and
@@ -851,20 +845,18 @@ struct LaneTab {
     __device__ static TF at(const char* base, unsigned off) { return *(const TF*)(base + off); }
 };
 
-// rows down through the partition: z the own rows' right-hand sides, acc what
-// the partition above contributes (in) and what this one does to the next
-// (out), y the own rows
+// rows down through the partition: z the own rows' right-hand sides, each added
+// when its row is done (fwd_row), acc what the partition above contributes (in)
+// and what this one does to the next (out), y the own rows
 template <int P>
 __device__ inline void rows_down(const cplx (&C)[kPM], const cplx (&z)[kOwn], cplx (&y)[kOwn], cplx& acc, int l) {
-    acc = {acc.re + z[0].re, acc.im + z[0].im};
     each(std::make_integer_sequence<int, kPM>{}, [&](auto sc) {
         constexpr int s = decltype(sc)::value, t = s / kSplit, r = s % kSplit;
-        const cplx x = bcast8<r>(acc);
-        y[t] = pick(l == r, acc, y[t]);
+        const cplx w = {z[t].re + acc.re, z[t].im + acc.im};
+        const cplx x = bcast8<r>(w);
+        y[t] = pick(l == r, w, y[t]);
         keep(y[t]);
-        cplx next = {0.0, 0.0};
-        if constexpr (t + 1 < kOwn) next = z[t + 1];
-        acc = tmsub(pick(l == r, next, acc), C[s], x);
+        acc = tmsub(pick(l == r, cplx{0.0, 0.0}, acc), C[s], x);
     });
 }
 // rows up; acc: the last eight's y less what the partition below contributes
@@ -890,18 +882,17 @@ template <int P>
 __device__ inline void rows_down_r(const double (&C)[kPM], const double (&B)[kPM], const double (&dg)[kOwn],
                                    const cplx (&z)[kOwn], cplx (&y)[kOwn], cplx& acc) {
     cplx a[kOwn + 1];
-    a[0] = {acc.re + z[0].re, acc.im + z[0].im};
+    a[0] = acc;
 #pragma unroll
-    for (int t = 1; t < kOwn; ++t) a[t] = z[t];
-    a[kOwn] = {0.0, 0.0};
+    for (int t = 1; t <= kOwn; ++t) a[t] = {0.0, 0.0};
     each(std::make_integer_sequence<int, kPM>{}, [&](auto sc) {
         constexpr int s = decltype(sc)::value, t = s / kSplit, r = s % kSplit;
-        const cplx x = bcast8<r>(cplx{dg[t] * a[t].re, dg[t] * a[t].im});
+        const cplx x = bcast8<r>(cplx{dg[t] * (z[t].re + a[t].re), dg[t] * (z[t].im + a[t].im)});
         if constexpr (r < kSplit - 1) a[t] = tmsub(a[t], C[s], x);
         if constexpr (r > 0 || P == 8) a[t + 1] = tmsub(a[t + 1], B[s], x);
     });
 #pragma unroll
-    for (int t = 0; t < kOwn; ++t) y[t] = {dg[t] * a[t].re, dg[t] * a[t].im};
+    for (int t = 0; t < kOwn; ++t) y[t] = {dg[t] * (z[t].re + a[t].re), dg[t] * (z[t].im + a[t].im)};
     acc = a[kOwn];
 }
 template <int P>
@@ -1169,14 +1160,14 @@ __global__ __launch_bounds__(64) void k_seqsolve(const cplx* __restrict__ tab, T
     cplx h[P];
     auto vat = [&](int i) { return i < N ? cj_if(cj, v[min(i, N - 1)]) : cplx{0.0, 0.0}; };
 #pragma unroll
-    for (int j = 0; j < P; ++j) h[j] = vat(j);
+    for (int j = 0; j < P; ++j) h[j] = {0.0, 0.0};
     for (int i0 = 0; i0 < N; i0 += RB) {
         cplx c[RB][F::UF], vr[RB];
 #pragma unroll
         for (int b = 0; b < RB; ++b) {
             const int i = min(i0 + b, N - 1);
             row_g<TF, P, F::UF>(c[b], T0, part_off<TF, P>(i / kPM), i % kPM);
-            vr[b] = vat(i0 + b + P);
+            vr[b] = vat(i0 + b);
         }
 #pragma unroll
         for (int b = 0; b < RB; ++b)
