@@ -551,8 +551,8 @@ __global__ __launch_bounds__(256) void k_rhs_shared(RhsArgs ra, const cplx* __re
 // wave per work-group, several per compute unit, which hide each other's
 // loads.
 // Measured per launch, R, D, free and mask solves (with, in
-// brackets, four waves that shared the passes' loads through LDS): 26.9 / 25.0 /
-// 28.7 / 19.2 us at N = 3000 with 81 channels (32.2 / 27.6 / 33.8 / 22.8).  Of the
+// brackets, four waves that shared the passes' loads through LDS): 27.0 / 25.2 /
+// 28.9 / 19.3 us at N = 3000 with 81 channels (32.2 / 27.6 / 33.8 / 22.8).  Of the
 // 55 k cycles of a symmetric solve the passes take 27 k (two thirds of it the
 // issue of their own arithmetic), the
 // carries 7 k and the loads with the right-hand side 20 k.
@@ -810,8 +810,8 @@ __global__ __launch_bounds__(kLane * (STAGED ? kWavesStaged : 1)) void k_bsolve(
 // every table entry twice, the band entries of three rows per lane.  More
 // partitions to a work-group would wait for them as long as k_bsolve does (64 at
 // N = 1500: no gain), and so would two work-groups to a compute unit; fewer wait
-// less (split_grid).  R, D, free and mask solves of 6 channels of N = 240: 13.1 /
-// 10.6 / 12.2 / 9.7 us (k_bsolve 21.6 / 18.0 / 21.4 / 17.0).  At 32 partitions,
+// less (split_grid).  R, D, free and mask solves of 6 channels of N = 240: 13.2 /
+// 11.4 / 12.7 / 9.7 us (k_bsolve 21.6 / 18.0 / 21.4 / 17.0).  At 32 partitions,
 // uncut, 31 channels step by step 5.3 -> 4.3 ms, 2400 batched ones 36.0 -> 31.1.
 // A step of longer channels, k_bsolve before: 31 of N = 1000 155 -> 102 us, 41 of
 // N = 1500 167 -> 118, 51 of N = 2000 175 -> 140, 30 of N = 3000 170 -> 132.
