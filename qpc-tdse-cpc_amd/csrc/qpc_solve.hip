@@ -1148,7 +1148,8 @@ __global__ __launch_bounds__(kSplitParts * kSplit) void k_bsolve8(const cplx* __
 // Sequential solve x = U^-1 L^-1 v over all N rows, one lane per channel:
 // the fallback for carries deeper than kPKMax partitions (exact for any
 // operator the tables hold).  Table rows are fetched in blocks of RB rows,
-// every load of a block issued before its first use; zout holds y between
+// every load of a block issued before its first use and none under a branch
+// (rows from N on repeat the last and are left out); zout holds y between
 // the two passes.
 template <class TF, int P>
 __global__ __launch_bounds__(64) void k_seqsolve(const cplx* __restrict__ tab, TabMap tm, const cplx* __restrict__ vin,
@@ -1163,7 +1164,6 @@ __global__ __launch_bounds__(64) void k_seqsolve(const cplx* __restrict__ tab, T
     const cplx* v = vin + (int64_t)ch * N;
     cplx* x = zout + (int64_t)ch * N;
     cplx h[P];
-    auto vat = [&](int i) { return i < N ? cj_if(cj, v[min(i, N - 1)]) : cplx{0.0, 0.0}; };
 #pragma unroll
     for (int j = 0; j < P; ++j) h[j] = {0.0, 0.0};
     for (int i0 = 0; i0 < N; i0 += RB) {
@@ -1172,7 +1172,7 @@ __global__ __launch_bounds__(64) void k_seqsolve(const cplx* __restrict__ tab, T
         for (int b = 0; b < RB; ++b) {
             const int i = min(i0 + b, N - 1);
             row_g<TF, P, F::UF>(c[b], T0, part_off<TF, P>(i / kPM), i % kPM);
-            vr[b] = vat(i0 + b);
+            vr[b] = cj_if(cj, v[i]);
         }
 #pragma unroll
         for (int b = 0; b < RB; ++b)
